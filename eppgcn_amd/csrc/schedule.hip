@@ -24,15 +24,28 @@
 //     wtail[w]   index of the partial sum for what wave w still holds at its last slot, or -1
 //     touched    one bit per vertex: the row has at least one slot
 //     frow/fptr  rows that have partial sums and the range of each; the partial sums are numbered row by row,
-//                in stream order inside a row, so that summing a range in order gives the same bits every run
+//                inside a row those of its piece ends, then those of the waves' tails, each in the caller's group order
+//                (the stream's too when the columns of a row ascend), so that summing a range in order gives the
+//                same bits every run
 // and a header with the counts.  A plan with empty groups gets no stream form (header.valid = 0).
 //
 // The re-ordering changes no result, only which groups run together.  It depends on the graph
 // and the groups alone: a caller builds it once and passes it to every aggregation call.
 //
-// Everything is written here: the keys, a stable least-significant-digit radix sort of the
-// (key, group index) pairs (8 bits per pass: tile histograms, one look-back scan, stable scatter with
-// ballot-based ranks), the look-back scan of the group sizes, the flags and the column copy.
+// How a plan is built (launch_build_plan), all on the device and without a host read-back:
+//   plan_init      clears the scan states, the two row bitmaps and the header
+//   plan_keys      per group, in the caller's order: row, adjacency, sort key, the digit counts of the first radix pass
+//   radix passes   stable least-significant-digit sort of (key, group index); none for a plan in one block
+//   plan_order     per plan entry: one look-back scan over (slots, piece ends) gives the slot offsets and the piece
+//                  numbers together; writes ptr / row / flags and the extent of every piece
+//   plan_fill      per 2048 slots: the column copy with the piece-end flags, cev, wtail preset
+//   plan_partials  per group, in the caller's order again: which pieces leave partial sums, numbered by two
+//                  look-back scans side by side.  A row's groups are neighbours in this order, so the numbers come out
+//                  row by row without sorting the pieces by row (a three-pass sort of 8 M candidates before)
+//   plan_targets   writes erow / wtail from those numbers and completes the header
+// Every kernel streams its arrays once; what used to be 46 launches, four of them radix passes over 8 M keys, is 9.  R-MAT
+// scale 22, both paths and the forward groups of a two-layer run (7.8 + 5.9 + 1.7 M groups, 132 + 126 + 13 M slots):
+// 6.0 -> 2.2 ms for the three plans; scale 20 (8.8 + 7.3 + 0.9 M slots): 1.3 -> 0.35 ms.
 #include <atomic>
 #include <cstring>
 
@@ -42,61 +55,7 @@ namespace eppgcn {
 
 static size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
-// ---------------------------------------------------------------- kernels
-// Sort key of group p: the column block of its first slot, except that all groups of a short row
-// (at most `keep_slots` slots in at most kMaxRowWalk groups) share the key of the row's first group:
-// such a row stays together in the plan, is summed in registers and written once with plain stores,
-// instead of leaving one partial sum per column block to be combined with atomics (measured at group
-// size 31: the atomics of rows with 2..16 groups cost more than the L2 hits of their later groups
-// save; the bound is in slots because a row's gathers, not its groups, are what a block can speed up:
-// with groups of 4-8 slots a bound in groups spread rows of 40 slots and lost up to 2x at 256 columns).
-constexpr int kMaxRowWalk = 64;
-__global__ __launch_bounds__(256) void plan_keys_kernel(const int* __restrict__ part_ptr, const int* __restrict__ col,
-                                                       const int* __restrict__ part2node, const int* __restrict__ ids,
-                                                       int num_parts, int shift, int keep_slots, int classes,
-                                                       unsigned* __restrict__ keys)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= num_parts) return;
-    const int beg = part_ptr[p];
-    const int end = part_ptr[p + 1];
-    if (end <= beg) { keys[p] = 0u; return; }
-    const int row = part2node ? part2node[p] : ids[beg];
-    auto same_row = [&](int j) {
-        const int b = part_ptr[j];
-        if (part_ptr[j + 1] <= b) return false;
-        return (part2node ? part2node[j] : ids[b]) == row;
-    };
-    int start = p;
-    for (int k = 0; k < kMaxRowWalk && start > 0 && same_row(start - 1); ++k) --start;
-    const bool start_found = !(start > 0 && same_row(start - 1));
-    int last = p;
-    while (last + 1 < num_parts && last + 1 - start < kMaxRowWalk && same_row(last + 1)) ++last;
-    const bool end_found = !(last + 1 < num_parts && same_row(last + 1));
-    const bool short_row = keep_slots > 0 && start_found && end_found && last - start + 1 <= kMaxRowWalk &&
-                           part_ptr[last + 1] - part_ptr[start] <= keep_slots;
-    const int key_col = short_row ? col[part_ptr[start]] : col[beg];
-    unsigned key = static_cast<unsigned>(key_col) >> shift;
-    if (classes) {
-        // second key: length class of a row that is a single group (a class = one gather step of 8
-        // slots), so that the groups a wave works on in one round take the same number of steps;
-        // rows of several groups consist of full groups but for the last one: class 3
-        const int len = end - beg;
-        const int cls = (short_row && start == last) ? min(3, (len - 1) >> 3) : 3;
-        key = (key << 2) | static_cast<unsigned>(cls);
-    }
-    keys[p] = key;
-}
-
-__global__ __launch_bounds__(256) void plan_sizes_kernel(const int* __restrict__ part_ptr, const int* __restrict__ order,
-                                                        int num_parts, int* __restrict__ sizes)
-{
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= num_parts) return;
-    const int p = order[q];
-    sizes[q] = part_ptr[p + 1] - part_ptr[p];
-}
-
+// ---------------------------------------------------------------- look-back scan (radix offsets)
 // Exclusive prefix sum of `in[0..n)` into `out[0..n]` (out[n] = total): single pass, decoupled
 // look-back over tiles of 2048.
 constexpr int kScanBlock = 256;
@@ -145,13 +104,13 @@ __global__ __launch_bounds__(kScanBlock) void exclusive_scan_kernel(const int* _
 }
 
 // ---------------------------------------------------------------- stable radix sort of (key, index) pairs
-// One pass sorts by the 8-bit digit (key >> shift) & 255 and keeps the order of equal digits, so
-// passes from the least significant digit upwards sort by the whole key, equal keys staying in index
-// order.  A tile is kSortTile consecutive elements, element (round r, thread t) of tile T being
-// T * kSortTile + r * 256 + t, so that (round, wave, lane) order is index order.
-//   radix_hist_kernel     hist[d * tiles + T] = elements of tile T with digit d
+// One pass sorts by the digit (key >> shift) & (digits - 1), digits = 2^bits <= 256, and keeps the order of equal
+// digits, so passes from the least significant digit upwards sort by the whole key, equal keys staying in index order.
+// A tile is kSortTile consecutive elements, element (round r, thread t) of tile T being T * kSortTile + r * 256 + t, so
+// that (round, wave, lane) order is index order.
+//   plan_keys_kernel / radix_hist_kernel   hist[d * tiles + T] = elements of tile T with digit d
 //   exclusive_scan_kernel over hist (digit-major): where (digit d, tile T) starts in the output
-//   radix_scatter_kernel  rank of an element among the equal digits of its wave from eight ballots,
+//   radix_scatter_kernel  rank of an element among the equal digits of its wave from one ballot per digit bit,
 //                         counts per (round, wave, digit) in LDS, prefix over (round, wave) per digit
 constexpr int kSortBlock = 256;
 constexpr int kSortRounds = 8;
@@ -159,7 +118,7 @@ constexpr int kSortTile = kSortBlock * kSortRounds;
 constexpr int kDigits = 256;
 
 __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const unsigned* __restrict__ keys, int n, int shift,
-                                                                int num_tiles, int* __restrict__ hist)
+                                                                int digits, int num_tiles, int* __restrict__ hist)
 {
     __shared__ int s_hist[kDigits];
     s_hist[threadIdx.x] = 0;
@@ -168,24 +127,27 @@ __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const unsigned* 
 #pragma unroll
     for (int r = 0; r < kSortRounds; ++r) {
         const long long i = base + r * kSortBlock + threadIdx.x;
-        if (i < n) atomicAdd(&s_hist[(keys[i] >> shift) & (kDigits - 1)], 1);
+        if (i < n) atomicAdd(&s_hist[(keys[i] >> shift) & (digits - 1)], 1);
     }
     __syncthreads();
-    hist[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x] = s_hist[threadIdx.x];
+    if (static_cast<int>(threadIdx.x) < digits)
+        hist[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x] = s_hist[threadIdx.x];
 }
 
-// vals_in == nullptr: the value of element i is i (first pass)
+// vals_in == nullptr: the value of element i is i (first pass); keys_out == nullptr: the last pass, whose keys nobody reads
 __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigned* __restrict__ keys_in,
                                                                    const int* __restrict__ vals_in,
                                                                    unsigned* __restrict__ keys_out,
-                                                                   int* __restrict__ vals_out, int n, int shift,
+                                                                   int* __restrict__ vals_out, int n, int shift, int bits,
                                                                    int num_tiles, const int* __restrict__ offsets)
 {
     constexpr int kWaves = kSortBlock / kWave;
     __shared__ int s_count[kSortRounds * kWaves][kDigits];      // per (round, wave): elements of each digit
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < kSortRounds * kWaves * kDigits; i += kSortBlock) (&s_count[0][0])[i] = 0;
+    const int digits = 1 << bits;
+    for (int i = threadIdx.x; i < kSortRounds * kWaves * digits; i += kSortBlock)
+        s_count[i >> bits][i & (digits - 1)] = 0;
     __syncthreads();
     const long long base = static_cast<long long>(blockIdx.x) * kSortTile;
     unsigned key[kSortRounds];
@@ -193,13 +155,15 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigne
 #pragma unroll
     for (int r = 0; r < kSortRounds; ++r) {
         const long long i = base + r * kSortBlock + threadIdx.x;
-        const bool valid = i < n;
-        key[r] = valid ? keys_in[i] : 0u;
-        const unsigned d = (key[r] >> shift) & (kDigits - 1);
-        // lanes of the wave holding the same digit: intersect the ballots of the eight digit bits
-        uint64_t peers = __ballot(valid);
+        key[r] = i < n ? keys_in[i] : 0u;
+    }
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+    for (int r = 0; r < kSortRounds; ++r) {
+        const bool valid = base + r * kSortBlock + threadIdx.x < n;
+        const unsigned d = (key[r] >> shift) & (digits - 1);
+        // lanes of the wave holding the same digit: intersect the ballots of the digit's bits
+        uint64_t peers = __ballot(valid);
+        for (int b = 0; b < bits; ++b) {
             const uint64_t set = __ballot(((d >> b) & 1u) != 0);
             peers &= ((d >> b) & 1u) ? set : ~set;
         }
@@ -207,7 +171,8 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigne
         if (valid && rank[r] == 0) s_count[r * kWaves + wave][d] = __popcll(peers);
     }
     __syncthreads();
-    {   // thread d: exclusive prefix of digit d over the (round, wave) pairs, on top of the tile's global offset
+    if (static_cast<int>(threadIdx.x) < digits) {
+        // thread d: exclusive prefix of digit d over the (round, wave) pairs, on top of the tile's global offset
         int run = offsets[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x];
 #pragma unroll
         for (int q = 0; q < kSortRounds * kWaves; ++q) {
@@ -221,55 +186,43 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigne
     for (int r = 0; r < kSortRounds; ++r) {
         const long long i = base + r * kSortBlock + threadIdx.x;
         if (i < n) {
-            const unsigned d = (key[r] >> shift) & (kDigits - 1);
+            const unsigned d = (key[r] >> shift) & (digits - 1);
             const int dst = s_count[r * kWaves + wave][d] + rank[r];
-            keys_out[dst] = key[r];
-            vals_out[dst] = vals_in ? vals_in[i] : static_cast<int>(i);
-        }
-    }
-}
-
-// row, flags and the column copy of every plan entry; a team of 8 lanes per group.
-__global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ part_ptr, const int* __restrict__ col,
-                                                       const int* __restrict__ part2node, const int* __restrict__ ids,
-                                                       const int* __restrict__ order, int num_parts, PlanView plan)
-{
-    constexpr int kTeam = 8;
-    const long long t = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const long long q = t / kTeam;
-    const int tl = static_cast<int>(t % kTeam);
-    if (q >= num_parts) return;
-    const int p = order[q];
-    const int beg = part_ptr[p];
-    const int end = part_ptr[p + 1];
-    const int dst = plan.ptr[q];
-    for (int i = tl; i < end - beg; i += kTeam) plan.col[dst + i] = col[beg + i];
-    if (tl == 0) {
-        int row = 0;
-        bool prev = false, next = false;
-        if (end > beg) {
-            if (part2node) {
-                row = part2node[p];
-                prev = p > 0 && part2node[p - 1] == row;
-                next = p + 1 < num_parts && part2node[p + 1] == row;
-            } else {
-                row = ids[beg];
-                prev = beg > 0 && ids[beg - 1] == row;
-                next = p + 1 < num_parts && ids[end] == row;
+            if (dst >= 0 && dst < n) {                          // false only after a stalled scan
+                if (keys_out) keys_out[dst] = key[r];
+                vals_out[dst] = vals_in ? vals_in[i] : static_cast<int>(i);
             }
         }
-        const bool joins_left = prev && q > 0 && order[q - 1] == p - 1;
-        const bool joins_right = next && q + 1 < num_parts && order[q + 1] == p + 1;
-        if (end > beg && !prev && !next) atomicOr(plan.single + (row >> 5), 1u << (row & 31));
-        plan.row[q] = row;
-        plan.flags[q] = static_cast<uint8_t>((prev ? 1 : 0) | (next ? 2 : 0) | (joins_left ? 4 : 0) | (joins_right ? 8 : 0));
     }
 }
 
-// ---------------------------------------------------------------- stream form
-__global__ void stream_init_kernel(StreamHeader* h, int num_parts, int num_slots, int num_nodes, int generation)
+// ---------------------------------------------------------------- plan kernels
+struct PlanScans {            // states of the look-back scans of one build, inside the workspace
+    ScanState* sort;          // radix offsets
+    ScanState* order;         // plan_order
+    ScanState* partials;      // plan_partials (two descriptor arrays: ends and tails, rows)
+    uint64_t *sort_desc, *order_desc, *ends_desc, *rows_desc;
+    int sort_tiles, order_tiles;
+};
+
+// one launch clears everything a build counts on being clear
+__global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanScans sc, uint32_t* __restrict__ single,
+                                                        uint32_t* __restrict__ touched, int words, int num_parts,
+                                                        int num_slots, int num_nodes, int generation)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+    const int stride = gridDim.x * blockDim.x;
+    const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int i = i0; i < words; i += stride) { single[i] = 0u; touched[i] = 0u; }
+    for (int i = i0; i < sc.sort_tiles; i += stride) sc.sort_desc[i] = kTileEmpty;
+    for (int i = i0; i < sc.order_tiles; i += stride) {
+        sc.order_desc[i] = kTileEmpty;
+        sc.ends_desc[i] = kTileEmpty;
+        sc.rows_desc[i] = kTileEmpty;
+    }
+    if (i0 == 0) {
+        *sc.sort = ScanState{};
+        *sc.order = ScanState{};
+        *sc.partials = ScanState{};
         StreamHeader z = {};
         z.empty_rows = num_nodes;
         z.magic = kPlanMagic;
@@ -281,199 +234,509 @@ __global__ void stream_init_kernel(StreamHeader* h, int num_parts, int num_slots
     }
 }
 
-// is_end[q]: plan entry q is the last of its piece
-__global__ __launch_bounds__(256) void stream_ends_kernel(PlanView plan, int num_parts, int* __restrict__ is_end,
-                                                         StreamHeader* h)
+// Sets bit (row & 31) of map[row >> 5] for the lanes with `set`: the lanes of a wave whose rows share a word (rows ascend
+// along the groups, so they are neighbours) combine their bits first, one atomic per run.  One atomic per group, as before,
+// was most of the old classification kernel (0.7 ms per run at R-MAT scale 22).
+__device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ map, int row, bool set)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= num_parts) return;
-    const bool nonempty = plan.ptr[q + 1] > plan.ptr[q];
-    is_end[q] = nonempty && (plan.flags[q] & 8) == 0;
-    if (!nonempty) h->empty_groups = 1;
-}
-
-// ends_before[q] = pieces that end before entry q (exclusive scan of is_end; [P] = number of pieces).  Piece e:
-// first[e] = its first slot | bit 31 when the row has groups before it, last[e] = its last slot,
-// erow[e] = its row | bit 31 when the row has groups after it; the last slot is flagged in col.
-__global__ __launch_bounds__(256) void stream_pieces_kernel(PlanView plan, int num_parts,
-                                                           const int* __restrict__ ends_before, int* __restrict__ first,
-                                                           int* __restrict__ last, int* __restrict__ erow, StreamHeader* h)
-{
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q == 0) h->num_events = ends_before[num_parts];
-    if (q >= num_parts) return;
-    const int beg = plan.ptr[q], end = plan.ptr[q + 1];
-    if (end <= beg) return;
-    const int f = plan.flags[q];
-    const int e = ends_before[q];
-    if (e < 0 || e >= num_parts) return;          // only after a stalled scan (the plan is then refused)
-    if ((f & 4) == 0) first[e] = beg | ((f & 1) ? static_cast<int>(kStreamFlag) : 0);
-    if ((f & 8) == 0) {
-        last[e] = end - 1;
-        erow[e] = plan.row[q] | ((f & 2) ? static_cast<int>(kStreamFlag) : 0);
-        plan.col[end - 1] |= static_cast<int>(kStreamFlag);
-    }
-}
-
-// number of pieces whose last slot lies before `slot`
-__device__ __forceinline__ int pieces_before(const int* __restrict__ last, int num_events, int slot)
-{
-    int lo = 0, hi = num_events;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (last[mid] < slot) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-}
-
-// Candidates for a partial sum: piece e at index e, the tail of wave w at index P + w.  key = the row for a real
-// candidate, num_nodes otherwise (sorts behind every row).  Also: plain pieces get their row in erow, every piece
-// marks its row as touched, wtail is preset to -1, the padding of col is written.
-__global__ __launch_bounds__(256) void stream_classify_kernel(PlanView plan, StreamView sv, int num_parts, int num_slots,
-                                                             int padded_slots, int num_nodes,
-                                                             const int* __restrict__ first, const int* __restrict__ last,
-                                                             unsigned* __restrict__ keys)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int num_waves = padded_slots / kStreamWave;
-    // "gathers nothing": an id whose row lies behind every table, in swizzled row order too
-    if (i < padded_slots - num_slots) plan.col[num_slots + i] = static_cast<int>(swizzle_padded_rows(num_nodes));
-    if (i >= num_parts + num_waves) return;
-    if (sv.header->empty_groups) { keys[i] = static_cast<unsigned>(num_nodes); if (i >= num_parts) sv.wtail[i - num_parts] = -1; return; }
-    const int num_events = sv.header->num_events;
-    unsigned key = static_cast<unsigned>(num_nodes);
-    if (i < num_parts) {
-        if (i < num_events) {
-            const int a = first[i], b = last[i], r = sv.erow[i];
-            const int row = r & kStreamIdMask;
-            const bool whole = a >= 0 && r >= 0;
-            const bool partial = !whole || (a & kStreamIdMask) < b / kStreamWave * kStreamWave;
-            if (row < num_nodes) atomicOr(sv.touched + (row >> 5), 1u << (row & 31));
-            if (partial) key = static_cast<unsigned>(row);
-            else sv.erow[i] = row;
-        }
-    } else {
-        const int w = i - num_parts;
-        sv.wtail[w] = -1;
-        const long long at = static_cast<long long>(w + 1) * kStreamWave - 1;
-        if (at < num_slots && plan.col[at] >= 0) {
-            const int e = pieces_before(last, num_events, static_cast<int>(at));
-            if (e < num_events) key = static_cast<unsigned>(sv.erow[e] & kStreamIdMask);
-        }
-    }
-    keys[i] = key;
-}
-
-__global__ __launch_bounds__(256) void stream_cev_kernel(StreamView sv, int num_slots, int padded_slots,
-                                                        const int* __restrict__ last)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c > padded_slots / kStreamChunk) return;
-    if (sv.header->empty_groups) { sv.cev[c] = 0; return; }
-    const int num_events = sv.header->num_events;
-    const long long pos = static_cast<long long>(c) * kStreamChunk;
-    const int e = pos >= num_slots ? num_events : pieces_before(last, num_events, static_cast<int>(pos));
-    const bool inside = pos > 0 && pos < num_slots && !(e > 0 && last[e - 1] == pos - 1);
-    sv.cev[c] = e | (inside ? static_cast<int>(kStreamFlag) : 0);
-}
-
-// sorted candidates: position k of a real one is the index of its partial sum
-__global__ __launch_bounds__(256) void stream_assign_kernel(StreamView sv, int num_parts, int total, int num_nodes,
-                                                           const unsigned* __restrict__ sorted_keys,
-                                                           const int* __restrict__ order, int* __restrict__ is_head)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= total) return;
-    const unsigned key = sorted_keys[k];
-    int head = 0;
-    if (key < static_cast<unsigned>(num_nodes) && !sv.header->empty_groups) {
-        const int src = order[k];
-        if (src >= 0 && src < num_parts) sv.erow[src] = static_cast<int>(kStreamFlag) | k;
-        else if (src >= num_parts && src < total) sv.wtail[src - num_parts] = k;
-        head = k == 0 || sorted_keys[k - 1] != key;
-        if (k + 1 == total || sorted_keys[k + 1] >= static_cast<unsigned>(num_nodes)) sv.header->num_partials = k + 1;
-    }
-    is_head[k] = head;
-}
-
-__global__ __launch_bounds__(256) void stream_fix_rows_kernel(StreamView sv, int total, int num_nodes,
-                                                             const unsigned* __restrict__ sorted_keys,
-                                                             const int* __restrict__ is_head, const int* __restrict__ heads_before)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= total || !is_head[k]) return;
-    const int j = heads_before[k];
-    if (j < 0 || j >= num_nodes) return;          // only after a stalled scan
-    sv.frow[j] = static_cast<int>(sorted_keys[k]);
-    sv.fptr[j] = k;
-}
-
-__global__ __launch_bounds__(256) void stream_count_rows_kernel(StreamView sv, int words)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    int c = i < words ? __popc(sv.touched[i]) : 0;
+    const int lane = lane_id();
+    const int word = set ? row >> 5 : -1;
+    uint32_t bits = set ? 1u << (row & 31) : 0u;
+    const int prev = __shfl_up(word, 1, kWave);
+    const uint64_t heads = __ballot(lane == 0 || prev != word);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, kWave);
-    if ((threadIdx.x & (kWave - 1)) == 0 && c) atomicSub(&sv.header->empty_rows, c);
+    for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t other = static_cast<uint32_t>(__shfl_down(static_cast<int>(bits), off, kWave));
+        const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);      // run heads in lanes lane+1 .. lane+off
+        if (lane + off < kWave && between == 0) bits |= other;
+    }
+    if (((heads >> lane) & 1ull) && bits) atomicOr(map + word, bits);
 }
 
-__global__ void stream_finish_kernel(StreamView sv, const int* __restrict__ heads_before, int total, int num_nodes,
-                                     const ScanState* a, const ScanState* b)
+// Per group p: rowp[p] (0 for an empty group), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the
+// group has slots; the row bitmaps; the sort key and the digit counts of the first radix pass (keys == nullptr: the plan
+// keeps the caller's order).
+// Sort key of group p: the column block of its first slot, except that all groups of a short row
+// (at most `keep_slots` slots in at most kMaxRowWalk groups) share the key of the row's first group:
+// such a row stays together in the plan, is summed in registers and written once with plain stores,
+// instead of leaving one partial sum per column block (measured at group size 31: the partial sums of rows with 2..16
+// groups cost more than the L2 hits of their later groups save; the bound is in slots because a row's gathers, not its
+// groups, are what a block can speed up: with groups of 4-8 slots a bound in groups spread rows of 40 slots and lost up
+// to 2x at 256 columns).
+// The walk to the ends of a row stops as soon as the row cannot be short any more: with the usual group sizes that is
+// after two or three groups, where a hub's groups walked 64 neighbours each way before (0.55 -> 0.28 ms for the 7.8 M
+// forward groups of R-MAT scale 22).  What is left is one 64-byte sector of `col` (and of `ids`) per group.
+constexpr int kMaxRowWalk = 64;
+__global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
+    const int* __restrict__ part_ptr, const int* __restrict__ col, const int* __restrict__ part2node,
+    const int* __restrict__ ids, int num_parts, int num_nodes, int shift, int keep_slots, int classes, int digits,
+    int num_tiles, unsigned* __restrict__ keys, int* __restrict__ hist, int* __restrict__ rowp, uint8_t* __restrict__ info,
+    uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    StreamHeader* h = sv.header;
-    const int num_fix = h->empty_groups ? 0 : min(max(heads_before[total], 0), num_nodes);
-    h->num_fix = num_fix;
-    sv.fptr[num_fix] = h->num_partials;
-    h->error = (a->error || b->error) ? 1 : 0;
-    h->valid = (!h->empty_groups && !h->error) ? 1 : 0;
+    __shared__ int s_hist[kDigits];
+    s_hist[threadIdx.x] = 0;
+    __syncthreads();
+    const long long base = static_cast<long long>(blockIdx.x) * kSortTile;
+    int beg[kSortRounds], end[kSortRounds], row[kSortRounds], before[kSortRounds], after[kSortRounds];
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        const long long p = base + r * kSortBlock + threadIdx.x;
+        beg[r] = p < num_parts ? part_ptr[p] : 0;
+        end[r] = p < num_parts ? part_ptr[p + 1] : 0;
+    }
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        const int p = static_cast<int>(base) + r * kSortBlock + static_cast<int>(threadIdx.x);
+        const bool some = end[r] > beg[r];
+        row[r] = 0;
+        before[r] = after[r] = -1;
+        if (some) {
+            if (part2node) {
+                row[r] = part2node[p];
+                if (p > 0) before[r] = part2node[p - 1];
+                if (p + 1 < num_parts) after[r] = part2node[p + 1];
+            } else {
+                row[r] = ids[beg[r]];
+                if (beg[r] > 0) before[r] = ids[beg[r] - 1];
+                if (p + 1 < num_parts) after[r] = ids[end[r]];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kSortRounds; ++r) {
+        const long long pl = base + r * kSortBlock + threadIdx.x;
+        const int p = static_cast<int>(pl);
+        const bool have = pl < num_parts;
+        const bool some = end[r] > beg[r];
+        const bool prev = some && before[r] == row[r], next = some && after[r] == row[r];
+        if (have) {
+            rowp[p] = row[r];
+            info[p] = static_cast<uint8_t>((prev ? 1 : 0) | (next ? 2 : 0) | (some ? 4 : 0));
+            if (!some) h->empty_groups = 1;
+        }
+        const bool in_range = some && row[r] >= 0 && row[r] < num_nodes;
+        or_row_bits(touched, row[r], in_range);
+        or_row_bits(single, row[r], in_range && !prev && !next);
+        if (!keys || !have) continue;
+        unsigned key = 0u;
+        if (some) {
+            auto same_row = [&](int j) {
+                const int b = part_ptr[j];
+                if (part_ptr[j + 1] <= b) return false;
+                return (part2node ? part2node[j] : ids[b]) == row[r];
+            };
+            int start = p, last = p;
+            bool short_row = keep_slots > 0 && end[r] - beg[r] <= keep_slots;
+            int first_slot = beg[r], past = end[r];
+            while (short_row && start > 0 && same_row(start - 1)) {
+                first_slot = part_ptr[--start];
+                short_row = past - first_slot <= keep_slots && p - start < kMaxRowWalk;
+            }
+            while (short_row && last + 1 < num_parts && same_row(last + 1)) {
+                past = part_ptr[++last + 1];
+                short_row = past - first_slot <= keep_slots && last - start < kMaxRowWalk;
+            }
+            key = static_cast<unsigned>(col[short_row ? first_slot : beg[r]]) >> shift;
+            if (classes) {
+                // second key: length class of a row that is a single group (a class = one gather step of 8
+                // slots), so that the groups a wave works on in one round take the same number of steps;
+                // rows of several groups consist of full groups but for the last one: class 3
+                const int cls = (short_row && start == last) ? min(3, (end[r] - beg[r] - 1) >> 3) : 3;
+                key = (key << 2) | static_cast<unsigned>(cls);
+            }
+        }
+        keys[p] = key;
+        atomicAdd(&s_hist[key & (digits - 1)], 1);
+    }
+    if (!keys) return;
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < digits)
+        hist[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x] = s_hist[threadIdx.x];
+}
+
+// Tiles of the two scans over the groups: entry (round r, thread t) of tile T is T * kPlanTile + r * 512 + t, so that every
+// array is read and written with full-width accesses and (round, wave, lane) order is entry order; the 64 (round, wave)
+// sums of a tile are scanned by one wave.  8 consecutive entries per thread instead: 0.63
+// and 0.26 ms for the two kernels over 15.4 M groups, against 0.45 and 0.22.  (The tile ids of a look-back
+// scan come from one device counter at 12 ns each: tiles of 4096 keep that below 25 us for 8 M groups.)
+constexpr int kPlanBlock = 512;
+constexpr int kPlanItems = 8;
+constexpr int kPlanTile = kPlanBlock * kPlanItems;
+constexpr int kPlanWaves = kPlanBlock / kWave;
+static_assert(kPlanItems * kPlanWaves == kWave, "one wave scans the (round, wave) sums of a tile");
+constexpr int kFillTile = 2048;            // slots a workgroup of plan_fill_kernel writes
+static_assert(kFillTile % kStreamWave == 0 && kFillTile % kStreamChunk == 0, "cev and wtail entries belong to one fill tile");
+
+// Plan entry q holds group order[q] (order == nullptr: group q).  One scan carries (slots, piece ends) packed as
+// ends * 2^31 + slots.  Piece e: first[e] = its first slot | bit 31 when the row has groups before it, last[e] = its last
+// slot, erow[e] = its row, event_of[p] = e for the group p that ends it and -1 for every other group.
+// tile_q[t] = the plan entry that holds slot t * kFillTile.
+__global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
+    const int* __restrict__ part_ptr, const int* __restrict__ order, const int* __restrict__ rowp,
+    const uint8_t* __restrict__ info, int num_parts, int num_slots, int num_tiles, PlanView plan, StreamView sv,
+    int* __restrict__ src, int* __restrict__ ends_before, int* __restrict__ first, int* __restrict__ last,
+    int* __restrict__ event_of, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode)
+{
+    __shared__ int s_tile;
+    __shared__ uint64_t s_sum[kPlanItems * kPlanWaves];
+    const int tile = acquire_tile(st, &s_tile);
+    if (tile >= num_tiles) return;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x >> 6;
+    const long long q0 = static_cast<long long>(tile) * kPlanTile + threadIdx.x;
+    int p[kPlanItems], left[kPlanItems], right[kPlanItems];      // group of the entry and of its neighbours (-1: none)
+    auto group_at = [&](long long q) {
+        if (q < 0 || q >= num_parts) return -1;
+        const int g = order ? order[q] : static_cast<int>(q);
+        return g >= 0 && g < num_parts ? g : 0;                   // out of range only after a stalled scan of the sort
+    };
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        const long long q = q0 + r * kPlanBlock;
+        p[r] = group_at(q);
+        left[r] = group_at(q - 1);
+        right[r] = group_at(q + 1);
+    }
+    int beg[kPlanItems], size[kPlanItems], row[kPlanItems];
+    unsigned f[kPlanItems];
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        const int g = p[r];
+        beg[r] = g >= 0 ? part_ptr[g] : 0;
+        size[r] = g >= 0 ? part_ptr[g + 1] : 0;
+        row[r] = g >= 0 ? rowp[g] : 0;
+        f[r] = g >= 0 ? info[g] : 0u;
+    }
+    int at[kPlanItems], eb[kPlanItems];
+    unsigned is_end = 0u;
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        size[r] = max(size[r] - beg[r], 0);
+        const bool joins_left = (f[r] & 1u) && left[r] >= 0 && left[r] == p[r] - 1;
+        const bool joins_right = (f[r] & 2u) && right[r] >= 0 && right[r] == p[r] + 1;
+        const bool ends = (f[r] & 4u) && !joins_right;
+        f[r] = (f[r] & 3u) | (joins_left ? 4u : 0u) | (joins_right ? 8u : 0u);
+        is_end |= ends ? 1u << r : 0u;
+        const uint64_t ballot = __ballot(ends);
+        const int incl = wave_inclusive_scan(size[r]);
+        at[r] = incl - size[r];
+        eb[r] = ballot_rank(ballot);
+        if (lane == kWave - 1) s_sum[r * kPlanWaves + wave] = (static_cast<uint64_t>(__popcll(ballot)) << 31) + static_cast<uint64_t>(incl);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const uint64_t mine = s_sum[lane];
+        const uint64_t incl = wave_inclusive_scan_u64(mine);
+        const uint64_t total = static_cast<uint64_t>(__shfl(static_cast<long long>(incl), kWave - 1, kWave));
+        const uint64_t excl = tile_lookback(desc, st, tile, total, mode);
+        s_sum[lane] = excl + incl - mine;
+        if (tile == num_tiles - 1 && lane == 0) {
+            const uint64_t all = excl + total;
+            plan.ptr[num_parts] = static_cast<int>(all & 0x7fffffffull);
+            sv.header->num_events = min(static_cast<int>(all >> 31), num_parts);
+            const int fill_tiles = (num_slots + kFillTile - 1) / kFillTile;
+            for (int t = static_cast<int>(((all & 0x7fffffffull) + kFillTile - 1) / kFillTile); t < fill_tiles; ++t)
+                tile_q[t] = num_parts - 1;              // slots the caller counted and no group covers
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        if (p[r] < 0) continue;
+        const int q = static_cast<int>(q0) + r * kPlanBlock;
+        const uint64_t before = s_sum[r * kPlanWaves + wave];
+        const int slot = at[r] + static_cast<int>(before & 0x7fffffffull);
+        const int e = eb[r] + static_cast<int>(before >> 31);
+        const bool ends = (is_end >> r) & 1u;
+        plan.ptr[q] = slot;
+        plan.row[q] = row[r];
+        plan.flags[q] = static_cast<uint8_t>(f[r]);
+        src[q] = beg[r];
+        ends_before[q] = e;
+        event_of[p[r]] = ends ? e : -1;
+        if (size[r] == 0) continue;
+        if ((f[r] & 4u) == 0 && e < num_parts) first[e] = slot | ((f[r] & 1u) ? static_cast<int>(kStreamFlag) : 0);
+        if (ends && e < num_parts) {
+            last[e] = slot + size[r] - 1;
+            sv.erow[e] = row[r];
+        }
+        for (long long t = (static_cast<long long>(slot) + kFillTile - 1) / kFillTile;
+             t * kFillTile < min(static_cast<long long>(slot) + size[r], static_cast<long long>(num_slots)); ++t)
+            tile_q[t] = q;
+    }
+}
+
+// A workgroup writes kFillTile consecutive slots of plan.col: the plan entry (and so the source) of a slot is a prefix
+// population count over a bit map of the entries' starts in LDS, loads and stores are coalesced whatever the group
+// lengths are (a team of 8 lanes per group before: 0.52 -> 0.34 ms for 132 M slots, 1.06 GB read and written).
+__global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ col, PlanView plan, StreamView sv,
+                                                       const int* __restrict__ src, const int* __restrict__ ends_before,
+                                                       const int* __restrict__ tile_q, int num_parts, int num_slots,
+                                                       int padded_slots, int num_nodes, int num_fill_tiles, PlanScans sc)
+{
+    constexpr int kItems = kFillTile / 256;
+    constexpr int kWords = kFillTile / 64;
+    __shared__ unsigned long long s_start[kWords];      // bit i: an entry starts at slot base + i (i > 0)
+    __shared__ unsigned long long s_last[kWords];       // bit i: slot base + i is the last of a piece
+    __shared__ int s_before[kWords];                    // entry starts before each word
+    __shared__ int s_delta[kFillTile + 1];              // source slot - plan slot of every entry of the tile
+    if (sc.sort->error || sc.order->error) return;      // the offsets are not to be trusted; the plan is refused
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x >> 6;
+    const int base = blockIdx.x * kFillTile;
+    const int covered = min(plan.ptr[num_parts], num_slots);      // slots behind the groups' own gather nothing, as the padding
+    const int q_lo = tile_q[blockIdx.x];
+    const int q_hi = static_cast<int>(blockIdx.x) + 1 < num_fill_tiles ? tile_q[blockIdx.x + 1] : num_parts - 1;
+    const int count = q_hi - q_lo + 1;
+    const bool by_bits = sv.header->empty_groups == 0 && count <= kFillTile + 1;
+    if (threadIdx.x < kWords) { s_start[threadIdx.x] = 0ull; s_last[threadIdx.x] = 0ull; }
+    __syncthreads();
+    for (int i = threadIdx.x; i < count; i += 256) {
+        const int q = q_lo + i;
+        const int a = plan.ptr[q], b = plan.ptr[q + 1];
+        if (by_bits) s_delta[i] = src[q] - a;
+        const int s = a - base, l = b - 1 - base;
+        if (i > 0 && s > 0 && s < kFillTile) atomicOr(&s_start[s >> 6], 1ull << (s & 63));
+        if (b > a && (plan.flags[q] & 8) == 0 && l >= 0 && l < kFillTile) atomicOr(&s_last[l >> 6], 1ull << (l & 63));
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int pc = lane < kWords ? __popcll(s_start[lane]) : 0;
+        const int incl = wave_inclusive_scan(pc);
+        if (lane < kWords) s_before[lane] = incl - pc;
+    }
+    __syncthreads();
+    // plan entry of slot base + i, relative to q_lo
+    auto owner = [&](int i) -> int {
+        if (by_bits) {
+            const unsigned long long upto = (i & 63) == 63 ? ~0ull : (2ull << (i & 63)) - 1ull;
+            return s_before[i >> 6] + __popcll(s_start[i >> 6] & upto);
+        }
+        int a = 0, b = count;                           // empty groups: the last entry that starts at or before the slot
+        while (b - a > 1) {
+            const int mid = (a + b) >> 1;
+            if (plan.ptr[q_lo + mid] <= base + i) a = mid; else b = mid;
+        }
+        return a;
+    };
+    int v[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int i = k * 256 + static_cast<int>(threadIdx.x);
+        // "gathers nothing": an id whose row lies behind every table, in swizzled row order too
+        v[k] = static_cast<int>(swizzle_padded_rows(num_nodes));
+        if (base + i < covered) {
+            const int o = owner(i);
+            const int delta = by_bits ? s_delta[o] : src[q_lo + o] - plan.ptr[q_lo + o];
+            v[k] = __builtin_nontemporal_load(col + base + i + delta);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int i = k * 256 + static_cast<int>(threadIdx.x);
+        const bool flagged = (s_last[i >> 6] >> (i & 63)) & 1ull;
+        if (base + i < padded_slots) plan.col[base + i] = v[k] | (flagged ? static_cast<int>(kStreamFlag) : 0);
+    }
+    if (threadIdx.x < kFillTile / kStreamWave) {
+        const int w = base / kStreamWave + threadIdx.x;
+        if (w < padded_slots / kStreamWave) sv.wtail[w] = -1;
+    }
+    const bool closing = static_cast<int>(blockIdx.x) + 1 == num_fill_tiles;       // writes the entry behind the last slot too
+    if (threadIdx.x <= kFillTile / kStreamChunk) {
+        const int i = static_cast<int>(threadIdx.x) * kStreamChunk;
+        const int pos = base + i;
+        const bool mine = i < kFillTile ? pos < padded_slots || (closing && pos == padded_slots) : closing && pos == padded_slots;
+        if (mine) {
+            int e = sv.header->num_events;
+            bool inside = false;
+            if (pos < covered) {
+                const int q = q_lo + owner(i);
+                e = ends_before[q];
+                inside = pos > 0 && (plan.ptr[q] < pos || (plan.flags[q] & 4) != 0);
+            }
+            sv.cev[pos / kStreamChunk] = e | (inside ? static_cast<int>(kStreamFlag) : 0);
+        }
+    }
+}
+
+// Which pieces leave partial sums, and how many: a piece that is not all of its row, or that crosses from one wave's
+// slots into the next, leaves one at its end, and one more per wave boundary it crosses (what that wave still holds at
+// its last slot).  Group p (in the caller's order) speaks for the piece it ends.  Two scans run side by side, wave 0's
+// over (tails, ends) packed as tails * 2^31 + ends, wave 1's over (rows with slots, rows with partial sums).
+// The partial sums of row j of the fix list are numbered ends first, then tails: its range starts at ends + tails before
+// its first group.  fix_of[p] = j or -1; ends_at / tails_at[p] the counts before p; ends0 / tails0[j] those before row j.
+__global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
+    const int* __restrict__ rowp, const uint8_t* __restrict__ info, const int* __restrict__ event_of,
+    const int* __restrict__ first, const int* __restrict__ last, int num_parts, int num_nodes, int num_tiles,
+    StreamView sv, int* __restrict__ fix_of, int* __restrict__ ends_at, int* __restrict__ tails_at,
+    int* __restrict__ ends0, int* __restrict__ tails0, int* __restrict__ ends_total, PlanScans sc, unsigned mode)
+{
+    __shared__ int s_tile;
+    __shared__ uint64_t s_sum[2][kPlanItems * kPlanWaves];
+    if (sc.sort->error || sc.order->error || sv.header->empty_groups) return;      // no stream form
+    const int tile = acquire_tile(sc.partials, &s_tile);
+    if (tile >= num_tiles) return;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x >> 6;
+    const long long p0 = static_cast<long long>(tile) * kPlanTile + threadIdx.x;
+    int e[kPlanItems], a[kPlanItems], b[kPlanItems], tails[kPlanItems], tails_before[kPlanItems];
+    bool more[kPlanItems];                              // the row has groups after this one
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        const long long p = p0 + r * kPlanBlock;
+        e[r] = p < num_parts ? event_of[p] : -1;
+        more[r] = p < num_parts && (info[p] & 2u) != 0;
+    }
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        a[r] = e[r] >= 0 ? first[e[r]] : -1;
+        b[r] = e[r] >= 0 ? last[e[r]] : 0;
+    }
+    unsigned partial = 0u, head = 0u;
+    int ends_before[kPlanItems], rows_before[kPlanItems];
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        const bool begins = a[r] >= 0;                  // the row's first piece
+        tails[r] = e[r] >= 0 ? b[r] / kStreamWave - (a[r] & kStreamIdMask) / kStreamWave : 0;
+        const bool part = e[r] >= 0 && (!begins || more[r] || tails[r] > 0);
+        partial |= part ? 1u << r : 0u;
+        head |= part && begins ? 1u << r : 0u;
+        const uint64_t parts = __ballot(part), heads = __ballot(part && begins), rows = __ballot(begins);
+        ends_before[r] = ballot_rank(parts);
+        rows_before[r] = ballot_rank(heads);
+        int incl = 0;
+        if (__any(tails[r] > 0)) incl = wave_inclusive_scan(tails[r]);       // few waves see a piece that crosses
+        tails_before[r] = incl - tails[r];
+        if (lane == kWave - 1) {
+            s_sum[0][r * kPlanWaves + wave] = (static_cast<uint64_t>(incl) << 31) + static_cast<uint64_t>(__popcll(parts));
+            s_sum[1][r * kPlanWaves + wave] = (static_cast<uint64_t>(__popcll(rows)) << 31) + static_cast<uint64_t>(__popcll(heads));
+        }
+    }
+    __syncthreads();
+    if (wave < 2) {
+        const uint64_t mine = s_sum[wave][lane];
+        const uint64_t incl = wave_inclusive_scan_u64(mine);
+        const uint64_t total = static_cast<uint64_t>(__shfl(static_cast<long long>(incl), kWave - 1, kWave));
+        const uint64_t excl = tile_lookback(wave == 0 ? sc.ends_desc : sc.rows_desc, sc.partials, tile, total, mode);
+        s_sum[wave][lane] = excl + incl - mine;
+        if (tile == num_tiles - 1 && lane == 0) {
+            const uint64_t all = excl + total;
+            const int low = static_cast<int>(all & 0x7fffffffull), high = static_cast<int>(all >> 31);
+            if (wave == 0) {
+                sv.header->num_partials = low + high;
+                *ends_total = low;
+            } else {
+                sv.header->num_fix = min(low, min(num_nodes, num_parts));
+                sv.header->empty_rows = num_nodes - high;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPlanItems; ++r) {
+        const long long p = p0 + r * kPlanBlock;
+        if (p >= num_parts) continue;
+        const bool part = (partial >> r) & 1u, begins = (head >> r) & 1u;
+        int j = -1;
+        if (part) {
+            const uint64_t x = s_sum[0][r * kPlanWaves + wave], y = s_sum[1][r * kPlanWaves + wave];
+            const int ea = ends_before[r] + static_cast<int>(x & 0x7fffffffull);
+            const int ta = tails_before[r] + static_cast<int>(x >> 31);
+            j = rows_before[r] + static_cast<int>(y & 0x7fffffffull) - (begins ? 0 : 1);
+            if (begins && j < num_nodes && j < num_parts) {
+                sv.frow[j] = rowp[p];
+                sv.fptr[j] = ea + ta;
+                ends0[j] = ea;
+                tails0[j] = ta;
+            }
+            ends_at[p] = ea;
+            tails_at[p] = ta;
+        }
+        fix_of[p] = j;
+    }
+}
+
+// The number of every partial sum into erow (a piece's end) and wtail (a wave's tail); the header is completed.
+__global__ __launch_bounds__(256) void plan_targets_kernel(StreamView sv, const int* __restrict__ event_of,
+                                                          const int* __restrict__ first, const int* __restrict__ last,
+                                                          const int* __restrict__ fix_of, const int* __restrict__ ends_at,
+                                                          const int* __restrict__ tails_at, const int* __restrict__ ends0,
+                                                          const int* __restrict__ tails0, const int* __restrict__ ends_total,
+                                                          int num_parts, int num_waves, PlanScans sc)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool error = sc.sort->error || sc.order->error || sc.partials->error;
+    const bool usable = !error && sv.header->empty_groups == 0;
+    if (p == 0) {
+        sv.header->error = error ? 1 : 0;
+        sv.header->valid = usable ? 1 : 0;
+        if (usable) sv.fptr[sv.header->num_fix] = sv.header->num_partials;
+    }
+    if (!usable || p >= num_parts) return;
+    const int j = fix_of[p];
+    if (j < 0) return;
+    const int e = event_of[p];
+    sv.erow[e] = static_cast<int>(kStreamFlag) | (ends_at[p] + tails0[j]);
+    const int w0 = (first[e] & kStreamIdMask) / kStreamWave, tails = last[e] / kStreamWave - w0;
+    if (tails > 0) {
+        const int at = (j + 1 < sv.header->num_fix ? ends0[j + 1] : *ends_total) + tails_at[p];
+        for (int k = 0; k < tails && w0 + k < num_waves; ++k) sv.wtail[w0 + k] = at + k;
+    }
 }
 
 // ---------------------------------------------------------------- host
-static size_t scan_state_bytes(long long n)
+static size_t scan_state_bytes(long long n, int tile)
 {
-    const long long tiles = (n + kScanTile - 1) / kScanTile;
+    const long long tiles = (n + tile - 1) / tile;
     return align256(sizeof(ScanState) + sizeof(uint64_t) * static_cast<size_t>(tiles > 0 ? tiles : 1));
 }
 
-static long long sort_tiles(long long n) { return (n + kSortTile - 1) / kSortTile; }
-// histogram | its exclusive scan (one more entry) | state of that scan
-static size_t sort_temp_bytes(long long n)
+static long long tiles_of(long long n, int tile) { return (n + tile - 1) / tile; }
+
+// Workspace of a build: ten arrays of num_parts + 1 ints (some used twice, the later use in brackets), the adjacency
+// bytes, the fill tiles' first entries, the radix histogram and its offsets, the scan states.
+struct PlanTemp {
+    int *keys_a, *keys_b, *order_a, *order_b, *rowp, *src, *ends_before, *first, *last, *event_of;
+    int *fix_of, *ends_at, *tails_at, *ends0, *tails0;      // = keys_a, keys_b, the spare order array, src, ends_before
+    uint8_t* info;
+    int *tile_q, *hist, *offsets, *ends_total;
+    PlanScans scans;
+    size_t bytes;
+};
+static PlanTemp plan_temp(char* base, long long num_parts, long long num_slots)
 {
-    const long long entries = sort_tiles(n) * kDigits;
-    return 2 * align256(sizeof(int) * static_cast<size_t>(entries + 1)) + scan_state_bytes(entries);
+    PlanTemp t;
+    size_t at = 0;
+    auto take = [&](size_t bytes) { char* p = base + at; at += align256(bytes); return p; };
+    const size_t slab = sizeof(int) * (static_cast<size_t>(num_parts) + 1);
+    int** arrays[] = {&t.keys_a, &t.keys_b, &t.order_a, &t.order_b, &t.rowp, &t.src, &t.ends_before, &t.first, &t.last, &t.event_of};
+    for (int** a : arrays) *a = reinterpret_cast<int*>(take(slab));
+    t.info = reinterpret_cast<uint8_t*>(take(static_cast<size_t>(num_parts)));
+    t.tile_q = reinterpret_cast<int*>(take(sizeof(int) * static_cast<size_t>(tiles_of(stream_padded_slots(num_slots), kFillTile) + 1)));
+    const long long entries = tiles_of(num_parts, kSortTile) * kDigits;
+    t.hist = reinterpret_cast<int*>(take(sizeof(int) * static_cast<size_t>(entries + 1)));
+    t.offsets = reinterpret_cast<int*>(take(sizeof(int) * static_cast<size_t>(entries + 1)));
+    auto state = [&](ScanState** st, uint64_t** desc, long long n, int tile) {
+        char* p = take(scan_state_bytes(n, tile));
+        *st = reinterpret_cast<ScanState*>(p);
+        *desc = reinterpret_cast<uint64_t*>(p + sizeof(ScanState));
+    };
+    state(&t.scans.sort, &t.scans.sort_desc, entries, kScanTile);
+    state(&t.scans.order, &t.scans.order_desc, num_parts, kPlanTile);
+    state(&t.scans.partials, &t.scans.ends_desc, num_parts, kPlanTile);
+    t.scans.rows_desc = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * static_cast<size_t>(tiles_of(num_parts, kPlanTile))));
+    t.ends_total = reinterpret_cast<int*>(take(sizeof(int)));
+    t.scans.order_tiles = static_cast<int>(tiles_of(num_parts, kPlanTile));
+    t.scans.sort_tiles = 0;
+    t.fix_of = t.keys_a; t.ends_at = t.keys_b; t.tails_at = nullptr; t.ends0 = t.src; t.tails0 = t.ends_before;
+    t.bytes = at;
+    return t;
 }
 
-// The stream form sorts one candidate per plan entry and per wave of the stream kernel.
-static long long plan_sort_capacity(long long num_parts, long long num_slots)
-{
-    return (num_parts > 0 ? num_parts : 0) + stream_padded_slots(num_slots) / kStreamWave;
-}
-
-// workspace layout: six arrays of plan_sort_capacity + 1 ints (keys, sorted keys, two index arrays, sizes, one
-// more for the stream form) | scan state | sort temporaries
-constexpr int kPlanSlabs = 6;
 size_t plan_workspace_bytes(long long num_parts, long long num_slots)
 {
     if (num_parts <= 0) return 256;
-    const long long cap = plan_sort_capacity(num_parts, num_slots);
-    return kPlanSlabs * align256(sizeof(int) * (static_cast<size_t>(cap) + 1)) + scan_state_bytes(cap + 1) +
-           sort_temp_bytes(cap) + 256;
-}
-
-// where launch_build_plan keeps the state of its look-back scans inside the workspace
-static size_t plan_scan_state_offset(long long num_parts, long long num_slots)
-{
-    return kPlanSlabs * align256(sizeof(int) * (static_cast<size_t>(plan_sort_capacity(num_parts, num_slots)) + 1));
-}
-
-// ... and the state of the scans inside its radix sorts (one state for all passes; the stall flag survives them)
-static size_t plan_sort_state_offset(long long num_parts, long long num_slots)
-{
-    const long long cap = plan_sort_capacity(num_parts, num_slots);
-    const long long entries = sort_tiles(cap) * kDigits;
-    return plan_scan_state_offset(num_parts, num_slots) + scan_state_bytes(cap + 1) +
-           2 * align256(sizeof(int) * static_cast<size_t>(entries + 1));
+    return plan_temp(nullptr, num_parts, num_slots).bytes;
 }
 
 int workspace_pitch(int dim);   // aggregate.hip
@@ -516,118 +779,12 @@ int schedule_shift(int dim)
     return shift;
 }
 
-// keep_error: a later scan over the same state must not wipe the stall flag of an earlier one
-__global__ void plan_scan_init_kernel(ScanState* st, uint64_t* desc, int num_tiles, bool keep_error)
+// a later scan over the same state must not wipe the stall flag of an earlier one
+__global__ void plan_scan_init_kernel(ScanState* st, uint64_t* desc, int num_tiles)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < num_tiles) desc[i] = kTileEmpty;
-    if (i == 0) {
-        st->counter = 0;
-        if (!keep_error) st->error = 0;
-        st->counts[0] = st->counts[1] = 0;
-        st->overflow = 0;
-    }
-}
-
-// out[0..n] = exclusive prefix sums of in[0..n) (out[n] = total), with the scan state at `state`
-static int launch_exclusive_scan(const int* in, int* out, long long n, void* state, hipStream_t stream,
-                                 bool keep_error = false)
-{
-    ScanState* st = static_cast<ScanState*>(state);
-    uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
-    const int tiles = static_cast<int>((n + kScanTile - 1) / kScanTile);
-    hipLaunchKernelGGL(plan_scan_init_kernel, dim3((tiles + 255) / 256), dim3(256), 0, stream, st, desc, tiles, keep_error);
-    EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(exclusive_scan_kernel, dim3(tiles), dim3(kScanBlock), 0, stream, in, out, static_cast<int>(n),
-                       tiles, st, desc, scan_mode());
-    EPPGCN_HIP(hipGetLastError());
-    return kOk;
-}
-
-// Sorts the pairs (keys[i], i) by the low `bits` bits of the key, stably; the sorted indices end up in
-// `order`.  keys_a is overwritten; keys_b, vals_tmp and temp are scratch.
-static int stable_sort_by_key(unsigned* keys_a, unsigned* keys_b, int* vals_tmp, int* order, int n, int bits, void* temp,
-                              void* state, hipStream_t stream, unsigned** sorted_keys = nullptr, bool keep_error = false)
-{
-    const int tiles = static_cast<int>(sort_tiles(n));
-    const long long entries = static_cast<long long>(tiles) * kDigits;
-    char* t = static_cast<char*>(temp);
-    int* hist = reinterpret_cast<int*>(t);
-    int* offsets = reinterpret_cast<int*>(t + align256(sizeof(int) * static_cast<size_t>(entries + 1)));
-    const int passes = bits <= 8 ? 1 : (bits + 7) / 8;
-    // the last pass must write `order`: with an even number of passes the first one writes the temporary
-    unsigned* kin = keys_a;
-    unsigned* kout = keys_b;
-    const int* vin = nullptr;
-    for (int pass = 0; pass < passes; ++pass) {
-        int* vout = ((passes - pass) % 2 == 1) ? order : vals_tmp;
-        const int shift = pass * 8;
-        hipLaunchKernelGGL(radix_hist_kernel, dim3(tiles), dim3(kSortBlock), 0, stream, kin, n, shift, tiles, hist);
-        EPPGCN_HIP(hipGetLastError());
-        if (int rc = launch_exclusive_scan(hist, offsets, entries, state, stream, keep_error || pass > 0)) return rc;
-        hipLaunchKernelGGL(radix_scatter_kernel, dim3(tiles), dim3(kSortBlock), 0, stream, kin, vin, kout, vout, n, shift,
-                           tiles, offsets);
-        EPPGCN_HIP(hipGetLastError());
-        unsigned* tk = kin; kin = kout; kout = tk;
-        vin = vout;
-    }
-    if (sorted_keys) *sorted_keys = kin;
-    return kOk;
-}
-
-static int launch_build_stream(PlanView v, StreamView sv, int num_parts, long long num_slots, int num_nodes, char* base,
-                               size_t slab, ScanState* st, ScanState* sort_st, void* temp, int generation,
-                               hipStream_t stream)
-{
-    const int padded = static_cast<int>(stream_padded_slots(num_slots));
-    const int num_waves = padded / kStreamWave;
-    const int total = num_parts + num_waves;
-    int* is_end = reinterpret_cast<int*>(base);                       // later: scratch of the sort
-    int* ends_before = reinterpret_cast<int*>(base + slab);           // later: second key array of the sort
-    int* first = reinterpret_cast<int*>(base + 2 * slab);             // later: is_head
-    int* last = reinterpret_cast<int*>(base + 3 * slab);              // later: heads_before
-    unsigned* keys = reinterpret_cast<unsigned*>(base + 4 * slab);
-    int* order = reinterpret_cast<int*>(base + 5 * slab);
-    const auto blocks = [](long long n) { return dim3(static_cast<unsigned>((n + 255) / 256 > 0 ? (n + 255) / 256 : 1)); };
-    hipLaunchKernelGGL(stream_init_kernel, dim3(1), dim3(64), 0, stream, sv.header, num_parts,
-                       static_cast<int>(num_slots), num_nodes, generation);
-    EPPGCN_HIP(hipGetLastError());
-    if (int rc = launch_zero_words(sv.touched, plan_single_words(num_nodes), stream)) return rc;
-    hipLaunchKernelGGL(stream_ends_kernel, blocks(num_parts), dim3(256), 0, stream, v, num_parts, is_end, sv.header);
-    EPPGCN_HIP(hipGetLastError());
-    if (int rc = launch_exclusive_scan(is_end, ends_before, num_parts, st, stream, true)) return rc;
-    hipLaunchKernelGGL(stream_pieces_kernel, blocks(num_parts), dim3(256), 0, stream, v, num_parts, ends_before, first, last,
-                       sv.erow, sv.header);
-    EPPGCN_HIP(hipGetLastError());
-    const long long classify_threads = total > padded - num_slots ? total : padded - num_slots;
-    hipLaunchKernelGGL(stream_classify_kernel, blocks(classify_threads), dim3(256), 0, stream, v, sv, num_parts,
-                       static_cast<int>(num_slots), padded, num_nodes, first, last, keys);
-    EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(stream_cev_kernel, blocks(padded / kStreamChunk + 1), dim3(256), 0, stream, sv,
-                       static_cast<int>(num_slots), padded, last);
-    EPPGCN_HIP(hipGetLastError());
-    int bits = 1;
-    while (bits < 31 && (1ll << bits) <= num_nodes) ++bits;           // the key num_nodes needs a digit too
-    unsigned* sorted_keys = nullptr;
-    if (int rc = stable_sort_by_key(keys, reinterpret_cast<unsigned*>(ends_before), is_end, order, total, bits, temp, sort_st,
-                                    stream, &sorted_keys, true))
-        return rc;
-    int* is_head = first;
-    int* heads_before = last;
-    hipLaunchKernelGGL(stream_assign_kernel, blocks(total), dim3(256), 0, stream, sv, num_parts, total, num_nodes, sorted_keys,
-                       order, is_head);
-    EPPGCN_HIP(hipGetLastError());
-    if (int rc = launch_exclusive_scan(is_head, heads_before, total, st, stream, true)) return rc;
-    hipLaunchKernelGGL(stream_fix_rows_kernel, blocks(total), dim3(256), 0, stream, sv, total, num_nodes, sorted_keys,
-                       is_head, heads_before);
-    EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(stream_count_rows_kernel, blocks(static_cast<long long>(plan_single_words(num_nodes))), dim3(256), 0,
-                       stream, sv, static_cast<int>(plan_single_words(num_nodes)));
-    EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(stream_finish_kernel, dim3(1), dim3(64), 0, stream, sv, heads_before, total, num_nodes, st,
-                       sort_st);
-    EPPGCN_HIP(hipGetLastError());
-    return kOk;
+    if (i == 0) st->counter = 0;
 }
 
 // Every build gets a number of its own (> 0): it is written into the plan's header and remembered by the host with the
@@ -653,44 +810,85 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
         set_error("build_plan: plan buffer smaller than eppgcn_plan_bytes(num_parts, num_slots, num_nodes)");
         return kErrInvalidArgument;
     }
-    if (num_slots >= (1ll << 31) - kStreamWave) {
+    if (num_slots >= (1ll << 31) - kFillTile) {
         set_error("build_plan: slot count beyond 32-bit offsets");
         return kErrInvalidArgument;
     }
-    const long long cap = plan_sort_capacity(num_parts, num_slots);
-    const size_t slab = align256(sizeof(int) * (static_cast<size_t>(cap) + 1));
-    char* base = static_cast<char*>(workspace);
-    unsigned* keys_in = reinterpret_cast<unsigned*>(base);
-    unsigned* keys_out = reinterpret_cast<unsigned*>(base + slab);
-    int* order_tmp = reinterpret_cast<int*>(base + 2 * slab);
-    int* order = reinterpret_cast<int*>(base + 3 * slab);
-    int* sizes = reinterpret_cast<int*>(base + 4 * slab);
-    ScanState* st = reinterpret_cast<ScanState*>(base + plan_scan_state_offset(num_parts, num_slots));
-    void* temp = base + kPlanSlabs * slab + scan_state_bytes(cap + 1);
-    ScanState* sort_st = reinterpret_cast<ScanState*>(base + plan_sort_state_offset(num_parts, num_slots));
-    int bits = 1;
-    while (bits < 30 && (static_cast<long long>(num_nodes) >> shift) >= (1ll << bits)) ++bits;
-    if (length_classes) bits += 2;
     if (plan_workspace_bytes(num_parts, num_slots) > workspace_bytes) {
         set_error("build_plan: workspace smaller than eppgcn_plan_workspace_bytes(num_parts, num_slots)");
         return kErrInvalidArgument;
     }
-    const unsigned blocks = static_cast<unsigned>((num_parts + 255) / 256);
-    hipLaunchKernelGGL(plan_keys_kernel, dim3(blocks), dim3(256), 0, stream, part_ptr, col, part2node, ids, num_parts,
-                       shift, keep_rows * 32, length_classes, keys_in);
+    PlanTemp t = plan_temp(static_cast<char*>(workspace), num_parts, num_slots);
+    const PlanView v = plan_view(plan, num_parts, num_nodes);
+    const StreamView sv = stream_view(plan, num_parts, num_slots, num_nodes);
+    const int slots = static_cast<int>(num_slots), padded = static_cast<int>(stream_padded_slots(num_slots));
+    const int words = static_cast<int>(plan_single_words(num_nodes));
+
+    // significant key bits; a plan in one block without length classes keeps the caller's order and needs no sort
+    int bits = 0;
+    while (bits < 30 && (static_cast<long long>(num_nodes > 0 ? num_nodes - 1 : 0) >> shift) >= (1ll << bits)) ++bits;
+    if (length_classes) bits += 2;
+    const int passes = (bits + 7) / 8;
+    const int sort_tiles = static_cast<int>(tiles_of(num_parts, kSortTile));
+    auto pass_bits = [&](int pass) { return bits - 8 * pass < 8 ? bits - 8 * pass : 8; };
+    t.scans.sort_tiles = passes ? static_cast<int>(tiles_of(static_cast<long long>(sort_tiles) << pass_bits(0), kScanTile)) : 0;
+
+    int init_blocks = (words + 255) / 256;
+    if (init_blocks > 512) init_blocks = 512;
+    if (init_blocks < 8) init_blocks = 8;
+    hipLaunchKernelGGL(plan_init_kernel, dim3(init_blocks), dim3(256), 0, stream, sv.header, t.scans, v.single, sv.touched, words,
+                       num_parts, slots, num_nodes, next_plan_generation());
     EPPGCN_HIP(hipGetLastError());
-    if (int rc = stable_sort_by_key(keys_in, keys_out, order_tmp, order, num_parts, bits, temp, sort_st, stream)) return rc;
-    hipLaunchKernelGGL(plan_sizes_kernel, dim3(blocks), dim3(256), 0, stream, part_ptr, order, num_parts, sizes);
+    unsigned* keys_in = reinterpret_cast<unsigned*>(t.keys_a);
+    unsigned* keys_out = reinterpret_cast<unsigned*>(t.keys_b);
+    hipLaunchKernelGGL(plan_keys_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, part_ptr, col, part2node, ids,
+                       num_parts, num_nodes, shift > 31 ? 31 : shift, keep_rows * 32, length_classes,
+                       passes ? 1 << pass_bits(0) : 1, sort_tiles, passes ? keys_in : nullptr, t.hist, t.rowp, t.info, v.single,
+                       sv.touched, sv.header);
     EPPGCN_HIP(hipGetLastError());
-    PlanView v = plan_view(plan, num_parts, num_nodes);
-    if (int rc = launch_zero_words(v.single, plan_single_words(num_nodes), stream)) return rc;
-    if (int rc = launch_exclusive_scan(sizes, v.ptr, num_parts, st, stream)) return rc;
-    const long long threads = static_cast<long long>(num_parts) * 8;
-    hipLaunchKernelGGL(plan_fill_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
-                       part_ptr, col, part2node, ids, order, num_parts, v);
+    int* order = nullptr;
+    int* spare = t.order_b;
+    for (int pass = 0; pass < passes; ++pass) {
+        const int nb = pass_bits(pass), digits = 1 << nb;
+        const long long entries = static_cast<long long>(sort_tiles) * digits;
+        const int scan_tiles = static_cast<int>(tiles_of(entries, kScanTile));
+        if (pass > 0) {
+            hipLaunchKernelGGL(plan_scan_init_kernel, dim3((scan_tiles + 255) / 256), dim3(256), 0, stream, t.scans.sort,
+                               t.scans.sort_desc, scan_tiles);
+            hipLaunchKernelGGL(radix_hist_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, keys_in, num_parts, 8 * pass,
+                               digits, sort_tiles, t.hist);
+            EPPGCN_HIP(hipGetLastError());
+        }
+        hipLaunchKernelGGL(exclusive_scan_kernel, dim3(scan_tiles), dim3(kScanBlock), 0, stream, t.hist, t.offsets,
+                           static_cast<int>(entries), scan_tiles, t.scans.sort, t.scans.sort_desc, scan_mode());
+        EPPGCN_HIP(hipGetLastError());
+        int* out = order == t.order_a ? t.order_b : t.order_a;
+        hipLaunchKernelGGL(radix_scatter_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, keys_in, order,
+                           pass + 1 < passes ? keys_out : nullptr, out, num_parts, 8 * pass, nb, sort_tiles, t.offsets);
+        EPPGCN_HIP(hipGetLastError());
+        unsigned* k = keys_in; keys_in = keys_out; keys_out = k;
+        order = out;
+        spare = out == t.order_a ? t.order_b : t.order_a;
+    }
+    t.tails_at = spare;
+    hipLaunchKernelGGL(plan_order_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, part_ptr, order, t.rowp, t.info,
+                       num_parts, slots, t.scans.order_tiles, v, sv, t.src, t.ends_before, t.first, t.last, t.event_of,
+                       t.tile_q, t.scans.order, t.scans.order_desc, scan_mode());
     EPPGCN_HIP(hipGetLastError());
-    return launch_build_stream(v, stream_view(plan, num_parts, num_slots, num_nodes), num_parts, num_slots, num_nodes, base,
-                               slab, st, sort_st, temp, next_plan_generation(), stream);
+    if (padded > 0) {
+        const int fill_tiles = static_cast<int>(tiles_of(padded, kFillTile));
+        hipLaunchKernelGGL(plan_fill_kernel, dim3(fill_tiles), dim3(256), 0, stream, col, v, sv, t.src, t.ends_before, t.tile_q,
+                           num_parts, slots, padded, num_nodes, fill_tiles, t.scans);
+        EPPGCN_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(plan_partials_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, t.rowp, t.info, t.event_of,
+                       t.first, t.last, num_parts, num_nodes, t.scans.order_tiles, sv, t.fix_of, t.ends_at, t.tails_at,
+                       t.ends0, t.tails0, t.ends_total, t.scans, scan_mode());
+    EPPGCN_HIP(hipGetLastError());
+    hipLaunchKernelGGL(plan_targets_kernel, dim3((num_parts + 255) / 256), dim3(256), 0, stream, sv, t.event_of, t.first, t.last,
+                       t.fix_of, t.ends_at, t.tails_at, t.ends0, t.tails0, t.ends_total, num_parts, padded / kStreamWave, t.scans);
+    EPPGCN_HIP(hipGetLastError());
+    return kOk;
 }
 
 // ---------------------------------------------------------------- what the host knows about built plans

@@ -1,0 +1,73 @@
+"""GPU tests of the plan builder where its tiles end: group counts around the tiles of its two scans, slot counts around
+a fill tile and a wave, groups longer than a fill tile, empty rows between them, one block and several.  The stream arrays
+are held, entry by entry, against the plain construction of tests/test_gpu_stream.py."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import c_oracle as co
+from tests.test_gpu_stream import check_stream_form, dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def api():
+    from eppgcn_amd import capi
+    capi.load()
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    return capi
+
+
+def csr_of(degrees, seed):
+    """CSR with these row lengths, columns ascending inside a row (repeats allowed)."""
+    degrees = np.asarray(degrees, np.int64)
+    indptr = np.concatenate([[0], np.cumsum(degrees)]).astype(np.int32)
+    n = degrees.size
+    col = np.random.default_rng(seed).integers(0, n, int(indptr[-1]))
+    rows = np.repeat(np.arange(n), degrees)
+    col = col[np.lexsort((col, rows))].astype(np.int32)
+    return indptr, col
+
+
+def degrees_of(kind):
+    rng = np.random.default_rng(17)
+    if kind.startswith("ones"):                      # one group per row: exactly that many groups and slots
+        return np.ones(int(kind[4:]), np.int64)
+    if kind == "long":                               # groups and pieces longer than fill tiles and waves
+        return np.array([5000, 0, 0, 1, 2047, 2049, 512, 511, 513, 0, 1, 4096], np.int64)
+    if kind == "mixed":                              # several tiles of groups, empty rows, rows of one to many groups
+        d = rng.integers(0, 40, 12000)
+        d[rng.random(12000) < 0.3] = 0
+        d[[7, 4000, 11999]] = [9000, 3000, 1500]
+        return d
+    raise ValueError(kind)
+
+
+@pytest.mark.parametrize("kind,ps", [("ones1", 1), ("ones511", 3), ("ones512", 3), ("ones2047", 3), ("ones2048", 1),
+                                     ("ones2049", 8), ("ones4095", 2), ("ones4096", 2), ("ones4097", 2), ("ones8193", 1),
+                                     ("long", 4), ("long", 6000), ("mixed", 1), ("mixed", 7), ("mixed", 32)])
+@pytest.mark.parametrize("shift", [0, 5, 31])
+def test_stream_form_at_tile_edges(api, kind, ps, shift):
+    indptr, col = csr_of(degrees_of(kind), 3)
+    n = indptr.size - 1
+    pp, p2n = co.build_part(ps, indptr)
+    plan = api.build_plan(dev(pp), dev(col), p2n.size, col.size, n, 16, part2node=dev(p2n), block_shift=shift)
+    check_stream_form(api, plan, n)
+
+
+def test_slots_no_group_covers_gather_nothing(api):
+    """A column array longer than what the groups cover: the slots behind the last group are padding."""
+    indptr, col = csr_of(degrees_of("mixed"), 5)
+    n = indptr.size - 1
+    pp, p2n = co.build_part(16, indptr)
+    longer = np.concatenate([col, np.zeros(3000, np.int32)])
+    plan = api.build_plan(dev(pp), dev(longer), p2n.size, longer.size, n, 16, part2node=dev(p2n))
+    got = plan.stream_view()["col"].cpu().numpy()
+    assert np.all(got[col.size:] == (n + 4095) // 4096 * 4096)
+    rng = np.random.default_rng(1)
+    x = rng.integers(-4, 5, (n, 16)).astype(np.float32)
+    ones = np.ones(n, np.float32)
+    out = api.spmm_forward(dev(x), dev(longer), dev(ones), dev(pp), dev(p2n), part_size=16, plan=plan)
+    assert api.last_call_used_stream()
+    assert np.array_equal(out.cpu().numpy(), co.spmm_f64(x, indptr, col, ones).astype(np.float32))
