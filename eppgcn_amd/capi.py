@@ -31,6 +31,7 @@ EXPORTS = [
     "eppgcn_plan_workspace_floats", "eppgcn_set_stream_mode", "eppgcn_last_call_used_stream",
     "eppgcn_update_forward_table", "eppgcn_feature_workspace_row", "eppgcn_plan_release", "eppgcn_aggregation_status",
     "eppgcn_ours_backward_rows", "eppgcn_update_backward_rows",
+    "eppgcn_mark_gathered_rows_scratch", "eppgcn_mark_gathered_rows_scratch_bytes",
 ]
 
 ABI_VERSION = 16      # what eppgcn_abi_version() of a matching library returns
@@ -72,6 +73,10 @@ def load():
     lib.eppgcn_ours_backward.argtypes = [p, p, p, p, p, p, i, i, i, i, i, i, i, p, sz, p, p, p]
     lib.eppgcn_mark_gathered_rows.argtypes = [p, i64, i, p, p, C.POINTER(i64), p]
     lib.eppgcn_mark_gathered_rows.restype = i
+    lib.eppgcn_mark_gathered_rows_scratch.argtypes = [p, i64, i, p, p, C.POINTER(i64), p, sz, p]
+    lib.eppgcn_mark_gathered_rows_scratch.restype = i
+    lib.eppgcn_mark_gathered_rows_scratch_bytes.argtypes = [i64]
+    lib.eppgcn_mark_gathered_rows_scratch_bytes.restype = sz
     lib.eppgcn_mask_forward.argtypes = [p, p, p, p, p, p, p, i, i64, i, i, i, p]
     lib.eppgcn_compact_workspace_bytes.argtypes = [i64]
     lib.eppgcn_compact_workspace_bytes.restype = sz
@@ -523,8 +528,10 @@ def mark_gathered_rows(edge_list, valid_len: int, num_nodes: int):
         raise EppgcnError("edge_list is shorter than valid_len")
     bitmap = torch.empty((int(num_nodes) + 31) // 32 + 1, dtype=torch.int32, device=edge_list.device)
     count = C.c_int64(0)
-    _check(lib.eppgcn_mark_gathered_rows(_ptr(edge_list), int(valid_len), int(num_nodes), _ptr(bitmap),
-                                         _ptr(bitmap[-1:]), C.byref(count), _stream()))
+    nbytes = lib.eppgcn_mark_gathered_rows_scratch_bytes(int(num_nodes))
+    scratch = _workspace(nbytes, edge_list.device)
+    _check(lib.eppgcn_mark_gathered_rows_scratch(_ptr(edge_list), int(valid_len), int(num_nodes), _ptr(bitmap),
+                                                 _ptr(bitmap[-1:]), C.byref(count), _ptr(scratch), nbytes, _stream()))
     return bitmap[:-1], int(count.value)
 
 

@@ -54,7 +54,8 @@ int launch_mark_compact(const int*, const int*, const int*, const uint8_t*, uint
 int launch_split(bool, const int*, int, int, int*, int*, long long, bool, void*, hipStream_t);
 int launch_count_nonzero(const int*, long long, int*, hipStream_t);
 int launch_ginfo_hist(const int*, long long, int*, hipStream_t);
-int launch_mark_listed_rows(const int*, long long, long long, uint32_t*, int*, hipStream_t);
+size_t mark_listed_rows_scratch_bytes(long long);
+int launch_mark_listed_rows(const int*, long long, long long, uint32_t*, int*, uint8_t*, hipStream_t);
 // ---- errors
 static thread_local std::string g_last_error;
 void set_error(const std::string& msg) { g_last_error = msg; }
@@ -325,14 +326,15 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers, 
     return kOk;
 }
 
-int eppgcn_mark_gathered_rows(const int32_t* edge_list, int64_t valid_len, int num_nodes, uint32_t* bitmap,
-                              int32_t* d_count, int64_t* h_count, void* stream)
+static int mark_gathered_call(const int32_t* edge_list, int64_t valid_len, int num_nodes, uint32_t* bitmap,
+                              int32_t* d_count, int64_t* h_count, void* scratch, void* stream)
 {
     EPPGCN_REQUIRE(valid_len >= 0 && valid_len < (1ll << 31) && num_nodes >= 0, "lengths must be non-negative int32");
     EPPGCN_REQUIRE(d_count && (num_nodes == 0 || bitmap) && (valid_len == 0 || edge_list), "null pointer");
     EPPGCN_REQUIRE(aligned(bitmap, 4) && aligned(d_count, 4), "bitmap and counter must be 4-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (int rc = launch_mark_listed_rows(edge_list, valid_len, num_nodes, bitmap, d_count, s)) return rc;
+    if (int rc = launch_mark_listed_rows(edge_list, valid_len, num_nodes, bitmap, d_count, static_cast<uint8_t*>(scratch), s))
+        return rc;
     if (h_count) {
         int v = 0;
         EPPGCN_HIP(hipMemcpyAsync(&v, d_count, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -340,6 +342,25 @@ int eppgcn_mark_gathered_rows(const int32_t* edge_list, int64_t valid_len, int n
         *h_count = v;
     }
     return kOk;
+}
+
+int eppgcn_mark_gathered_rows(const int32_t* edge_list, int64_t valid_len, int num_nodes, uint32_t* bitmap,
+                              int32_t* d_count, int64_t* h_count, void* stream)
+{
+    return mark_gathered_call(edge_list, valid_len, num_nodes, bitmap, d_count, h_count, nullptr, stream);
+}
+
+size_t eppgcn_mark_gathered_rows_scratch_bytes(int64_t num_nodes)
+{
+    return num_nodes <= 0 ? 0 : mark_listed_rows_scratch_bytes(num_nodes);
+}
+
+int eppgcn_mark_gathered_rows_scratch(const int32_t* edge_list, int64_t valid_len, int num_nodes, uint32_t* bitmap,
+                                      int32_t* d_count, int64_t* h_count, void* scratch, size_t scratch_bytes, void* stream)
+{
+    EPPGCN_REQUIRE(num_nodes <= 0 || (scratch && aligned(scratch, 16)), "scratch must be 16-byte aligned");
+    EPPGCN_REQUIRE(num_nodes <= 0 || scratch_bytes >= mark_listed_rows_scratch_bytes(num_nodes), "scratch too small");
+    return mark_gathered_call(edge_list, valid_len, num_nodes, bitmap, d_count, h_count, scratch, stream);
 }
 
 int eppgcn_count_nonzero(const int32_t* node_deg, int64_t length, int32_t* d_count, int64_t* h_count, void* stream)

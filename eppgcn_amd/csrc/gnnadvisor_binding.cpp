@@ -202,9 +202,12 @@ const PathChoice& path_choice(const Tensor& part_pointer, const Tensor& edge_lis
                  g_plan_policy > 0 || 2 * valid_len >= edge_list.numel(), part_pointer, edge_list, Tensor()};
     auto bitmap = torch::empty({(static_cast<int64_t>(num_nodes) + 31) / 32 + 1}, edge_list.options());
     int64_t distinct = 0;
-    check(eppgcn_mark_gathered_rows(i32(edge_list), valid_len, num_nodes,
-                                    reinterpret_cast<uint32_t*>(bitmap.data_ptr<int32_t>()),
-                                    bitmap.data_ptr<int32_t>() + bitmap.numel() - 1, &distinct, stream_of(edge_list)),
+    const size_t scratch_bytes = eppgcn_mark_gathered_rows_scratch_bytes(num_nodes);
+    auto scratch = workspace(scratch_bytes, edge_list);
+    check(eppgcn_mark_gathered_rows_scratch(i32(edge_list), valid_len, num_nodes,
+                                            reinterpret_cast<uint32_t*>(bitmap.data_ptr<int32_t>()),
+                                            bitmap.data_ptr<int32_t>() + bitmap.numel() - 1, &distinct, scratch.data_ptr(),
+                                            scratch_bytes, stream_of(edge_list)),
           "mark_gathered_rows");
     if (2 * distinct < num_nodes) c.gathered = bitmap;
     g_path_choices.push_front(std::move(c));
