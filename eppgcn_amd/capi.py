@@ -24,7 +24,8 @@ EXPORTS = [
     "eppgcn_clear_time", "eppgcn_get_time_ms", "eppgcn_set_team_size", "eppgcn_set_rounds", "eppgcn_set_plan_shift", "eppgcn_set_plan_keep_rows",
     "eppgcn_feature_workspace_pitch", "eppgcn_update_forward", "eppgcn_update_backward_input",
     "eppgcn_update_workspace_bytes", "eppgcn_update_backward_weight", "eppgcn_update_supported", "eppgcn_update_backward",
-    "eppgcn_mark_compact_workspace_bytes", "eppgcn_mark_compact", "eppgcn_set_plan_length_classes",
+    "eppgcn_mark_compact_workspace_bytes", "eppgcn_mark_compact", "eppgcn_mark_path_workspace_bytes", "eppgcn_mark_path",
+    "eppgcn_set_plan_length_classes",
     "eppgcn_mark_gathered_rows", "eppgcn_set_wide_index", "eppgcn_wave64_back_part_size",
     "eppgcn_compact_back_edge_static", "eppgcn_compact_back_edge_static_max_length",
     "eppgcn_auto_back_part_size", "eppgcn_scan_status", "eppgcn_plan_status", "eppgcn_set_scan_test_mode",
@@ -133,6 +134,10 @@ def load():
     lib.eppgcn_mark_compact_workspace_bytes.restype = sz
     lib.eppgcn_mark_compact.argtypes = [p, p, p, p, p, p, p, p, i, i64, i, p, sz, p, C.POINTER(i64), p]
     lib.eppgcn_mark_compact.restype = i
+    lib.eppgcn_mark_path_workspace_bytes.argtypes = [i64, i64]
+    lib.eppgcn_mark_path_workspace_bytes.restype = sz
+    lib.eppgcn_mark_path.argtypes = [p, p, p, p, p, p, p, p, p, i, i64, i, i, p, sz, C.POINTER(i64), p]
+    lib.eppgcn_mark_path.restype = i
     lib.eppgcn_feature_workspace_pitch.argtypes = [i]
     lib.eppgcn_feature_workspace_pitch.restype = i
     lib.eppgcn_update_supported.argtypes = [i, i]
@@ -660,6 +665,33 @@ def mark_compact(part2node, part_ptr, column_index, src_mask, ngh_mask, node_deg
                                    _ptr(node_degs), _ptr(out_id), _ptr(out_edge), part2node.numel(), length,
                                    int(bool(is_last_layer)), _ptr(ws), nbytes, None, C.byref(v), _stream()))
     return out_id, out_edge, int(v.value)
+
+
+def mark_path(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool):
+    """``mark_compact`` with what ``count_nonzero`` and ``mark_gathered_rows`` say about the path ->
+    (id int32[E], edge_list int32[E], valid_len, valid_nodes, gathered rows bitmap int32[(N+31)//32], gathered rows)."""
+    lib = load()
+    _dev(part2node, torch.int32, "part2node"); _dev(part_ptr, torch.int32, "part_ptr")
+    _dev(column_index, torch.int32, "column_index"); _dev(node_degs, torch.int32, "node_degs")
+    src = _mask_bytes(src_mask, "src_mask")
+    ngh = _mask_bytes(ngh_mask, "ngh_mask")
+    n, length, dev = node_degs.numel(), column_index.numel(), column_index.device
+    if n > 0 and (src is None or src.numel() < n):
+        raise EppgcnError("src_mask must have one entry per vertex")
+    if not is_last_layer and n > 0 and (ngh is None or ngh.numel() < n):
+        raise EppgcnError("ngh_mask must have one entry per vertex")
+    if part_ptr.numel() < part2node.numel() + 1:
+        raise EppgcnError("part_ptr needs num_parts + 1 entries")
+    out_id = torch.empty(length, dtype=torch.int32, device=dev)
+    out_edge = torch.empty(length, dtype=torch.int32, device=dev)
+    bitmap = torch.empty((n + 31) // 32, dtype=torch.int32, device=dev)
+    nbytes = lib.eppgcn_mark_path_workspace_bytes(length, n)
+    ws = _workspace(nbytes, dev)
+    counts = (C.c_int64 * 3)()
+    _check(lib.eppgcn_mark_path(_ptr(part2node), _ptr(part_ptr), _ptr(column_index), _ptr(src), _ptr(ngh), _ptr(node_degs),
+                                _ptr(out_id), _ptr(out_edge), _ptr(bitmap), part2node.numel(), length, n,
+                                int(bool(is_last_layer)), _ptr(ws), nbytes, counts, _stream()))
+    return out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
 
 
 def count_nonzero(node_deg) -> int:

@@ -49,6 +49,10 @@ int launch_compact_mask_static(const int*, int*, const int*, int*, long long, vo
 int static_compact_workspace(void**);
 int read_aggregation_status(hipStream_t);
 size_t mark_compact_workspace_bytes(long long);
+size_t mark_path_workspace_bytes(long long, long long);
+uint8_t* mark_path_scratch(void*, long long, long long);
+int launch_mark_path(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, uint32_t*, int,
+                     long long, int, int, void*, hipStream_t);
 int launch_mark_compact(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, int, long long,
                         int, void*, hipStream_t);
 int launch_split(bool, const int*, int, int, int*, int*, long long, bool, void*, hipStream_t);
@@ -322,6 +326,59 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers, 
         ScanState host;
         if (int rc = read_state(workspace, s, &host)) return rc;
         *h_valid_len = host.counts[0];
+    }
+    return kOk;
+}
+
+size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes)
+{
+    return mark_path_workspace_bytes(num_edges < 0 ? 0 : num_edges, num_nodes < 0 ? 0 : num_nodes);
+}
+
+int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                     const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
+                     uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, void* workspace,
+                     size_t workspace_bytes, int64_t* counts, void* stream)
+{
+    EPPGCN_REQUIRE(num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
+                   "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
+    EPPGCN_REQUIRE(counts, "null pointer");
+    EPPGCN_REQUIRE(workspace && aligned(workspace, 16), "workspace must be 16-byte aligned");
+    EPPGCN_REQUIRE(workspace_bytes >= mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
+    EPPGCN_REQUIRE(num_edges == 0 || (out_id && out_edge), "null output pointer");
+    EPPGCN_REQUIRE(num_nodes == 0 || gathered_rows, "null output pointer");
+    EPPGCN_REQUIRE(num_parts == 0 || (part2node && part_pointers && column_index && src_mask && node_degs), "null pointer");
+    EPPGCN_REQUIRE(is_last || num_parts == 0 || ngh_mask, "ngh_mask is required unless this is the last layer");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    counts[0] = counts[1] = counts[2] = 0;
+    if (num_parts == 0 || num_edges == 0 || num_nodes == 0) {
+        if (num_nodes > 0)
+            if (int rc = launch_zero_words(gathered_rows, (static_cast<size_t>(num_nodes) + 31) / 32, s)) return rc;
+        if (num_edges > 0) {
+            if (int rc = launch_zero_words(out_id, static_cast<size_t>(num_edges), s)) return rc;
+            if (int rc = launch_zero_words(out_edge, static_cast<size_t>(num_edges), s)) return rc;
+        }
+        EPPGCN_HIP(hipStreamSynchronize(s));
+        return kOk;
+    }
+    {
+        KernelTimer timer(s, &g_mask_ms);
+        if (int rc = launch_mark_path(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+                                      gathered_rows, num_parts, num_edges, num_nodes, is_last ? 1 : 0, workspace, s))
+            return rc;
+    }
+    ScanState host;
+    if (int rc = read_state(workspace, s, &host)) return rc;
+    counts[0] = host.counts[0];
+    counts[1] = host.pad[2];
+    counts[2] = host.pad[0];
+    if (host.pad[1]) {          // a marked vertex without a kept self-loop: the gathered rows have to be looked for
+        ScanState* st = static_cast<ScanState*>(workspace);
+        if (int rc = launch_mark_listed_rows(out_edge, counts[0], num_nodes, gathered_rows, &st->pad[0],
+                                             mark_path_scratch(workspace, num_edges, num_nodes), s))
+            return rc;
+        if (int rc = read_state(workspace, s, &host)) return rc;
+        counts[2] = host.pad[0];
     }
     return kOk;
 }

@@ -52,6 +52,43 @@ void set_scan_test_mode(unsigned spin_limit, int mute_first_tile)
     g_scan_mode.store((spin_limit & 0x7fffffffu) | (mute_first_tile ? 0x80000000u : 0u));
 }
 
+// ================================================================ shared pieces
+// Counts end in one atomic per workgroup.  Device-scope atomics on one address serialise at about 12 ns
+// each: with one per wave, a million vertices took 50 us of which 45 were the 4096 additions (now 5).
+__device__ __forceinline__ void add_block_count(int local, int* __restrict__ d_count)
+{
+    __shared__ int s_part[4];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
+    if ((threadIdx.x & (kWave - 1)) == 0) s_part[threadIdx.x / kWave] = local;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int sum = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+        if (sum) atomicAdd(d_count, sum);
+    }
+}
+
+// bit j of the result: byte j of x is not zero
+__device__ __forceinline__ unsigned nonzero_bytes(unsigned x)
+{
+    const unsigned top = (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u;
+    return ((top >> 7) * 0x01020408u) >> 24 & 0xfu;
+}
+
+// Zeros from word `from` to word `end` by threads i0 < stride: 16-byte stores between the aligned ends.
+__device__ __forceinline__ void zero_from(int* __restrict__ p, long long from, long long end, long long i0, long long stride)
+{
+    typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+    if (from >= end) return;
+    const long long head = min(end - from, static_cast<long long>((16 - reinterpret_cast<uintptr_t>(p + from) % 16) % 16 / 4));
+    const long long vecs = (end - from - head) / 4;
+    uintx4* v = reinterpret_cast<uintx4*>(p + from + head);
+    for (long long i = i0; i < vecs; i += stride) __builtin_nontemporal_store(uintx4{0u, 0u, 0u, 0u}, v + i);
+    const long long tail = from + head + 4 * vecs;
+    if (i0 < head) p[from + i0] = 0;
+    if (i0 < end - tail) p[tail + i0] = 0;
+}
+
 // ================================================================ path marking
 // A wave owns 64 consecutive forward groups (one per lane) and walks the contiguous slot range
 // they cover 64 slots at a time, so that the column ids are read and the edge marks written
@@ -208,26 +245,42 @@ __global__ __launch_bounds__(kCompactBlock) void compact_mask_kernel(
     }
 }
 
-// ================================================================ fused marking + compaction
-// One pass over the slots does what mask_forward_kernel followed by compact_mask_kernel do, without
-// the E-entry edge mask between them: a tile of 4096 consecutive slots finds the group (hence the
-// row) of every slot from a bit map of the group starts inside the tile (prefix population count;
-// tile_groups_kernel finds each tile's first group beforehand), decides keep = src_mask[col],
-// marks the neighbour masks, counts kept slots per row from wave ballots (one atomic per run of
-// equal rows in a wave), and compacts (row, col) of the kept slots with the same ballot ranks and
-// look-back prefix as compact_mask_kernel.
-
-// first[t] = last group starting at or before slot t * kCompactTile; first[num_tiles] = last group
-__global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_parts, int num_tiles,
-                                   int* __restrict__ first)
+// ================================================================ marking + compaction in one pass
+// One pass over the slots does what mask_forward_kernel followed by compact_mask_kernel do, without the E-entry edge
+// mask between them.  A tile is kMarkBlock * kItems consecutive slots; slot k * kMarkBlock + t of the tile belongs to
+// thread t, so word k * (waves) + wave of every 64-slot bit map is one ballot and words are in slot order.
+//   - the column ids of a thread's slots are loaded first (kItems loads in flight), then their mask entries;
+//   - the row of a slot comes from a bit map of the group starts inside the tile (prefix population count; the tile's
+//     first group was found by mark_tiles_kernel) and the rows of the tile's groups, staged in LDS;
+//   - kept slots per group are differences of the prefix counts of the kept bit map, added over the groups of a row in a
+//     wave, one atomic per (wave, row): a hub of 600 thousand slots costs 40 tiles a few atomics each, where one per 64
+//     slots queued ten thousand on one address;
+//   - (row, col) of the kept slots go out at look-back prefix + word prefix + ballot rank.
+// What bounds it: the random reads of the source mask, one cache line per slot that misses the vector cache.  kBits: the
+// mask is read as a bit map (packed once per call), which lets eight times as many vertices share a line.
+// Tile ids come from one device counter at 12 ns each: 16384 slots per tile keep that below 0.1 ms for 132 M slots;
+// inputs of a few million slots take tiles of 4096 so that every CU has work.
+constexpr int kMarkBlock = 512;
+constexpr int kMarkWaves = kMarkBlock / kWave;
+constexpr int kMarkItemsLarge = 32, kMarkItemsSmall = 8;
+constexpr int kMarkStagedRows = 4096;     // groups of a tile whose rows are staged (more: read where they are needed)
+static_assert(kMarkBlock * kMarkItemsSmall >= kCompactTile, "the workspace is sized for tiles of kCompactTile slots");
+constexpr long long kMarkLargeLength = 4ll << 20;
+__host__ __device__ constexpr int mark_tile_slots(long long length)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    return kMarkBlock * (length >= kMarkLargeLength ? kMarkItemsLarge : kMarkItemsSmall);
+}
+
+// first[t] = last group starting at or before slot t * tile_slots; first[num_tiles] = last group
+__device__ __forceinline__ void find_tile_groups(const int* __restrict__ part_ptr, int num_parts, int num_tiles,
+                                                 int tile_slots, int* __restrict__ first, int t)
+{
     if (t > num_tiles) return;
     if (t == num_tiles) {
         first[t] = num_parts - 1;
         return;
     }
-    const long long slot = static_cast<long long>(t) * kCompactTile;
+    const long long slot = static_cast<long long>(t) * tile_slots;
     int a = 0, b = num_parts;                 // part_ptr[a] <= slot is assumed for a = 0
     while (b - a > 1) {
         const int mid = a + (b - a) / 2;
@@ -236,119 +289,156 @@ __global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_par
     first[t] = a;
 }
 
-__global__ __launch_bounds__(kCompactBlock) void mark_compact_kernel(
-    const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
-    const uint8_t* __restrict__ src_mask, uint8_t* __restrict__ ngh_mask, int* __restrict__ node_degs,
-    int* __restrict__ out_id, int* __restrict__ out_edge, int num_parts, int length, int num_tiles, int is_last,
-    const int* __restrict__ tile_first, ScanState* st, uint64_t* desc, unsigned mode)
+__global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_parts, int num_tiles, int tile_slots,
+                                   int* __restrict__ first)
 {
+    find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+template <int kItems, bool kBits>
+__global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
+    const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
+    const uint8_t* __restrict__ src_bytes, const uint32_t* __restrict__ src_bits, uint8_t* __restrict__ ngh_mask,
+    int* __restrict__ node_degs, int* __restrict__ out_id, int* __restrict__ out_edge, uint8_t* __restrict__ self_kept,
+    int num_parts, int length, int num_tiles, int is_last, const int* __restrict__ tile_first, ScanState* st,
+    uint64_t* desc, unsigned mode)
+{
+    constexpr int kTile = kMarkBlock * kItems;
+    constexpr int kWords = kTile / 64;
+    constexpr int kPerLane = (kWords + kWave - 1) / kWave;     // words a lane of the scanning wave adds up
+    constexpr int kChunk = kItems < 16 ? kItems : 16;
+    static_assert(kWords % kWave == 0, "the words of a tile are divided evenly over one wave");
     __shared__ int s_tile;
-    __shared__ int s_count[kWave];
     __shared__ int s_prefix;
-    __shared__ unsigned long long s_bits[kCompactTile / 64];   // bit p: a group starts at slot base + p
-    __shared__ int s_word_prefix[kCompactTile / 64];     // group starts before each 64-slot word
     __shared__ int s_starts_in_tile;
-    if (threadIdx.x < kCompactTile / 64) s_bits[threadIdx.x] = 0ull;
+    __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
+    __shared__ unsigned long long s_kept[kWords];      // bit p: slot base + p is kept
+    __shared__ int s_starts_before[kWords];            // group starts before each word
+    __shared__ int s_kept_before[kWords + 1];          // kept slots before each word; [kWords] = all of the tile
+    __shared__ unsigned s_row[kMarkStagedRows];        // rows of the tile's groups; bit 31: the row is in the source mask
+    for (int i = threadIdx.x; i < kWords; i += kMarkBlock) s_starts[i] = 0ull;
     if (threadIdx.x == 0) s_starts_in_tile = 0;
-    const int tile = acquire_tile(st, &s_tile);          // contains the barrier that publishes the zeros
+    const int tile = acquire_tile(st, &s_tile);        // contains the barrier that publishes the zeros
     if (tile >= num_tiles) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
-    const long long base = static_cast<long long>(tile) * kCompactTile;
-    const int g_lo = tile_first[tile];
-    const int g_cnt = tile_first[tile + 1] - g_lo + 1;
+    const long long base = static_cast<long long>(tile) * kTile;
+    auto in_src = [&](int v) {
+        if constexpr (kBits) return ((src_bits[static_cast<unsigned>(v) >> 5] >> (v & 31)) & 1u) != 0u;
+        else return src_bytes[v] != 0;
+    };
+
     // slots outside [part_ptr[0], part_ptr[num_parts]) belong to no group and are never kept
     const int owned_lo = part_ptr[0];
-    const int owned_hi = part_ptr[num_parts];
-    // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
-    // When no two groups start at the same slot (no empty groups, as build_part guarantees) that
-    // number is a prefix population count over a 4096-bit map of group starts; otherwise every
-    // slot does a binary search over the group starts in global memory.
+    const int owned_hi = min(part_ptr[num_parts], length);
+    int c[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const long long idx = base + k * kMarkBlock + threadIdx.x;
+        c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
+    }
+    const int g_lo = tile_first[tile];
+    const int g_cnt = tile_first[tile + 1] - g_lo + 1;
+    const bool staged = g_cnt <= kMarkStagedRows;
+    const int before = part_ptr[g_lo] < base ? 1 : 0;    // g_lo itself starts before the tile
     {
         int mine = 0;
-        for (int i = threadIdx.x; i < g_cnt; i += kCompactBlock) {
-            const long long p = part_ptr[g_lo + i] - base;
-            if (p >= 0 && p < kCompactTile) {
-                atomicOr(&s_bits[p >> 6], 1ull << (p & 63));
+        for (int i = threadIdx.x; i < g_cnt; i += kMarkBlock) {
+            const int start = part_ptr[g_lo + i];
+            const int row = part2node[g_lo + i];
+            const long long p = start - base;
+            if (p >= 0 && p < kTile) {
+                atomicOr(&s_starts[p >> 6], 1ull << (p & 63));
                 ++mine;
             }
+            const bool marked = !is_last && in_src(row);
+            if (staged) s_row[i] = static_cast<unsigned>(row) | (marked ? 0x80000000u : 0u);
+            if (marked && part_ptr[g_lo + i + 1] > start) ngh_mask[row] = 1;
         }
         if (mine) atomicAdd(&s_starts_in_tile, mine);
     }
     __syncthreads();
+    // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
+    // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
+    // population count over the map of group starts; otherwise every slot does a binary search over the group starts.
     if (wave == 0) {
-        const int pc = __popcll(s_bits[lane]);
-        const int incl = wave_inclusive_scan(pc);
-        s_word_prefix[lane] = incl - pc;
+        int n[kPerLane], sum = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) {
+            n[j] = __popcll(s_starts[lane * kPerLane + j]);
+            sum += n[j];
+        }
+        const int incl = wave_inclusive_scan(sum);
+        int run = incl - sum;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) {
+            s_starts_before[lane * kPerLane + j] = run;
+            run += n[j];
+        }
         if (lane == kWave - 1 && incl != s_starts_in_tile) s_starts_in_tile = -1;   // duplicate starts
     }
     __syncthreads();
     const bool by_bits = s_starts_in_tile >= 0;
-    const int before = part_ptr[g_lo] < base ? 1 : 0;    // g_lo itself starts before the tile
-
-    // phases with all loads of one kind issued together: a ballot inside the item loop would make
-    // every item wait for its own gather (16 dependent memory round trips per tile)
-    int v[kCompactItems], c[kCompactItems], rows[kCompactItems];
-    bool ok[kCompactItems], keep[kCompactItems], row_src[kCompactItems];
-#pragma unroll
-    for (int k = 0; k < kCompactItems; ++k) {
-        const long long idx = base + k * kCompactBlock + threadIdx.x;
-        ok[k] = idx < length && idx >= owned_lo && idx < owned_hi;
-        c[k] = ok[k] ? col[idx] : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kCompactItems; ++k) {
-        rows[k] = -1;
-        if (ok[k]) {
-            const int e = static_cast<int>(base + k * kCompactBlock + threadIdx.x);
-            int a = 0, b = g_cnt;
-            if (by_bits) {
-                const int p = k * kCompactBlock + threadIdx.x;
-                const unsigned long long upto = (p & 63) == 63 ? ~0ull : (2ull << (p & 63)) - 1ull;
-                a = before + s_word_prefix[p >> 6] + __popcll(s_bits[p >> 6] & upto) - 1;
-            } else {
-                while (b - a > 1) {
-                    const int mid = (a + b) >> 1;
-                    if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
-                }
+    auto row_of = [&](int k) {                            // row of this thread's slot k; bit 31 as in s_row
+        int a = 0;
+        if (by_bits) {
+            const int word = k * kMarkWaves + wave;
+            const unsigned long long upto = lane == 63 ? ~0ull : (2ull << lane) - 1ull;
+            a = before + s_starts_before[word] + __popcll(s_starts[word] & upto) - 1;
+        } else {
+            const int e = static_cast<int>(base + k * kMarkBlock + threadIdx.x);
+            int b = g_cnt;
+            while (b - a > 1) {
+                const int mid = (a + b) >> 1;
+                if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
             }
-            rows[k] = part2node[g_lo + a];
         }
-    }
+        if (staged) return s_row[a];
+        const int row = part2node[g_lo + a];
+        return static_cast<unsigned>(row) | (!is_last && in_src(row) ? 0x80000000u : 0u);
+    };
+
 #pragma unroll
-    for (int k = 0; k < kCompactItems; ++k) {
-        keep[k] = ok[k] && src_mask[c[k]] != 0;
-        row_src[k] = ok[k] && !is_last && src_mask[rows[k]] != 0;
-    }
+    for (int k0 = 0; k0 < kItems; k0 += kChunk) {
+        bool keep[kChunk];
 #pragma unroll
-    for (int k = 0; k < kCompactItems; ++k) {
-        if (row_src[k]) {
-            ngh_mask[rows[k]] = 1;
-            ngh_mask[c[k]] = 1;
+        for (int k = 0; k < kChunk; ++k) keep[k] = in_src(max(c[k0 + k], 0));
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            const uint64_t ballot = __ballot(keep[k] && c[k0 + k] >= 0);
+            if (lane == 0) s_kept[(k0 + k) * kMarkWaves + wave] = ballot;
         }
-        v[k] = keep[k] ? rows[k] : -1;
-        // kept slots per row: the lanes of a wave hold 64 consecutive slots of item k
-        const int row = rows[k];
-        const int prev_row = __shfl_up(row, 1, kWave);
-        const uint64_t heads = __ballot(lane == 0 || prev_row != row);
-        const uint64_t kept = __ballot(keep[k]);
-        if ((heads >> lane) & 1ull) {
-            const uint64_t above = lane == kWave - 1 ? 0ull : heads & ~((2ull << lane) - 1ull);
-            const int next = above ? __builtin_ctzll(above) : kWave;
-            const uint64_t upto = next == kWave ? ~0ull : (1ull << next) - 1ull;
-            const int n = __popcll(kept & upto & ~((1ull << lane) - 1ull));
-            if (n > 0) atomicAdd(node_degs + row, n);
+        if (!is_last) {
+            bool mark[kChunk];
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) mark[k] = c[k0 + k] >= 0 && (row_of(k0 + k) >> 31) != 0u;
+            // a vertex that already reads as marked is not stored again: hubs are neighbours of most rows
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) mark[k] = mark[k] && ngh_mask[c[k0 + k]] == 0;
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k)
+                if (mark[k]) ngh_mask[c[k0 + k]] = 1;
         }
-        if (lane == 0) s_count[k * (kCompactBlock / kWave) + wave] = __popcll(kept);
     }
     __syncthreads();
     if (wave == 0) {
-        const int cnt = s_count[lane];
-        const int incl = wave_inclusive_scan(cnt);
+        int n[kPerLane], sum = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) {
+            n[j] = __popcll(s_kept[lane * kPerLane + j]);
+            sum += n[j];
+        }
+        const int incl = wave_inclusive_scan(sum);
         const int total = __shfl(incl, kWave - 1, kWave);
-        s_count[lane] = incl - cnt;
+        int run = incl - sum;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) {
+            s_kept_before[lane * kPerLane + j] = run;
+            run += n[j];
+        }
         const uint64_t excl = tile_lookback(desc, st, tile, static_cast<uint64_t>(total), mode);
         if (lane == 0) {
+            s_kept_before[kWords] = total;
             s_prefix = static_cast<int>(excl);
             if (tile == num_tiles - 1) st->counts[0] = static_cast<int>(excl) + total;
         }
@@ -356,52 +446,142 @@ __global__ __launch_bounds__(kCompactBlock) void mark_compact_kernel(
     __syncthreads();
     const int prefix = s_prefix;
 #pragma unroll
-    for (int k = 0; k < kCompactItems; ++k) {
-        const bool pred = v[k] != -1;
-        const uint64_t ballot = __ballot(pred);
-        if (pred) {
-            const int dst = prefix + s_count[k * (kCompactBlock / kWave) + wave] + ballot_rank(ballot);
-            out_id[dst] = v[k];
+    for (int k = 0; k < kItems; ++k) {
+        const int word = k * kMarkWaves + wave;
+        const uint64_t ballot = s_kept[word];
+        if ((ballot >> lane) & 1ull) {
+            const int dst = prefix + s_kept_before[word] + ballot_rank(ballot);
+            const int row = static_cast<int>(row_of(k) & 0x7fffffffu);
+            out_id[dst] = row;
             out_edge[dst] = c[k];
+            if (self_kept && row == c[k]) self_kept[row] = 1;
         }
     }
+    // kept slots per row
+    auto kept_before = [&](long long p) {                 // kept slots of the tile before slot base + p
+        const int q = static_cast<int>(p < 0 ? 0 : p > kTile ? kTile : p);
+        const int word = q >> 6;
+        const int whole = s_kept_before[word];
+        return (q & 63) ? whole + __popcll(s_kept[word] & ((1ull << (q & 63)) - 1ull)) : whole;
+    };
+    for (int i0 = 0; i0 < g_cnt; i0 += kMarkBlock) {
+        const int i = i0 + static_cast<int>(threadIdx.x);
+        int row = -1, kept = 0;
+        if (i < g_cnt) {
+            row = staged ? static_cast<int>(s_row[i] & 0x7fffffffu) : part2node[g_lo + i];
+            kept = kept_before(part_ptr[g_lo + i + 1] - base) - kept_before(part_ptr[g_lo + i] - base);
+        }
+        const int prev_row = __shfl_up(row, 1, kWave);
+        const uint64_t heads = __ballot(lane == 0 || prev_row != row);
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const int other = __shfl_down(kept, off, kWave);
+            const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);   // run heads in lanes lane+1 .. lane+off
+            if (lane + off < kWave && between == 0) kept += other;
+        }
+        if (((heads >> lane) & 1ull) && kept > 0) atomicAdd(node_degs + row, kept);
+    }
+}
+
+// ---------------------------------------------------------------- the pass with everything a path needs around it
+// Before: the source mask packed into bits, the scan state, the tiles' first groups, no row seen with its self-loop.
+__global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __restrict__ src_mask, int num_nodes, int words,
+                                                             uint32_t* __restrict__ bits, uint32_t* __restrict__ self_kept,
+                                                             const int* __restrict__ part_ptr, int num_parts, int num_tiles,
+                                                             int tile_slots, int* __restrict__ first, ScanState* st,
+                                                             uint64_t* __restrict__ desc)
+{
+    const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    if (i0 == 0) *st = ScanState{};
+    for (int t = i0; t <= num_tiles; t += stride) {
+        if (t < num_tiles) desc[t] = kTileEmpty;
+        find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
+    }
+    // a thread packs 4 bytes into 4 bits of a word, 8 lanes a word (vertices past the end count as unmarked)
+    const bool quads = reinterpret_cast<uintptr_t>(src_mask) % 4 == 0;
+    for (int q0 = blockIdx.x * 256; q0 < words * 8; q0 += stride) {
+        const int q = q0 + static_cast<int>(threadIdx.x);
+        unsigned nibble = 0u;
+        if (q < words * 8) {
+            const int v = q * 4;
+            self_kept[q] = 0u;
+            if (quads && v + 4 <= num_nodes) {
+                nibble = nonzero_bytes(*reinterpret_cast<const uint32_t*>(src_mask + v));
+            } else {
+                for (int j = 0; j < 4; ++j)
+                    if (v + j < num_nodes && src_mask[v + j]) nibble |= 1u << j;
+            }
+        }
+        unsigned word = nibble << (4 * (threadIdx.x & 7));
+        word |= __shfl_xor(word, 1, kWave);
+        word |= __shfl_xor(word, 2, kWave);
+        word |= __shfl_xor(word, 4, kWave);
+        if ((threadIdx.x & 7) == 0 && q < words * 8) bits[q >> 3] = word;
+    }
+}
+
+// After: the rows the path gathers, the rows with kept slots, zeros behind the kept slots.
+// Every vertex of the source mask whose self-loop is a slot is gathered; when that is all of them (graphs with
+// self-loops, the usual case) the mask is the bitmap of the gathered rows and no pass over the kept slots is needed
+// (0.58 ms for 126 M of them).  st->pad: [0] vertices of the mask, [1] not all of them kept their self-loop, [2] rows with
+// kept slots.
+constexpr int kFinishCountBlocks = 256;
+__global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* __restrict__ bits, const uint4* __restrict__ self_kept,
+                                                               int words, uint32_t* __restrict__ gathered,
+                                                               const int* __restrict__ node_degs, int num_nodes,
+                                                               int* __restrict__ out_id, int* __restrict__ out_edge, int length,
+                                                               ScanState* st)
+{
+    const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    zero_from(out_id, st->counts[0], length, i0, stride);
+    zero_from(out_edge, st->counts[0], length, i0, stride);
+    // the first workgroups count: every workgroup that does ends in three atomics on one line (12 ns each, serial)
+    if (blockIdx.x >= kFinishCountBlocks) return;
+    const int count_stride = min(stride, kFinishCountBlocks * 256);
+    int marked = 0, missing = 0, rows = 0;
+    for (int w = i0; w < words; w += count_stride) {
+        const uint32_t b = bits[w];
+        const uint4 lo = self_kept[2 * static_cast<size_t>(w)], hi = self_kept[2 * static_cast<size_t>(w) + 1];
+        const uint32_t seen = nonzero_bytes(lo.x) | nonzero_bytes(lo.y) << 4 | nonzero_bytes(lo.z) << 8 |
+                              nonzero_bytes(lo.w) << 12 | nonzero_bytes(hi.x) << 16 | nonzero_bytes(hi.y) << 20 |
+                              nonzero_bytes(hi.z) << 24 | nonzero_bytes(hi.w) << 28;
+        gathered[w] = b;
+        marked += __popc(b);
+        missing |= seen != b;
+    }
+    if (reinterpret_cast<uintptr_t>(node_degs) % 16 == 0) {
+        const int4* quads = reinterpret_cast<const int4*>(node_degs);
+        for (int v = i0; v < num_nodes / 4; v += count_stride) {
+            const int4 d = quads[v];
+            rows += (d.x != 0) + (d.y != 0) + (d.z != 0) + (d.w != 0);
+        }
+        if (i0 < num_nodes % 4) rows += node_degs[num_nodes / 4 * 4 + i0] != 0;
+    } else {
+        for (int v = i0; v < num_nodes; v += count_stride) rows += node_degs[v] != 0;
+    }
+    add_block_count(marked, &st->pad[0]);
+    __syncthreads();
+    add_block_count(missing, &st->pad[1]);
+    __syncthreads();
+    add_block_count(rows, &st->pad[2]);
 }
 
 // Zero both outputs from the compacted length (read on the device) to the end.
 __global__ void zero_tail2_kernel(int* __restrict__ a, int* __restrict__ b, const int* __restrict__ d_start, int length)
 {
-    const long long start = *d_start;
+    const long long i0 = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
     const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-    for (long long i = start + static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < length; i += stride) {
-        a[i] = 0;
-        b[i] = 0;
-    }
+    zero_from(a, *d_start, length, i0, stride);
+    zero_from(b, *d_start, length, i0, stride);
 }
 
 __global__ void zero_tail1_kernel(int* __restrict__ a, const int* __restrict__ d_start, int offset, long long length)
 {
-    const long long start = static_cast<long long>(*d_start) + offset;
-    const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-    for (long long i = start + static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < length; i += stride)
-        a[i] = 0;
+    zero_from(a, static_cast<long long>(*d_start) + offset, length,
+              static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x, static_cast<long long>(gridDim.x) * blockDim.x);
 }
 
 // ================================================================ counting
-// Both counts below end in one atomic per workgroup.  Device-scope atomics on one address serialise at about 12 ns
-// each: with one per wave, a million vertices took 50 us of which 45 were the 4096 additions (now 5).
-__device__ __forceinline__ void add_block_count(int local, int* __restrict__ d_count)
-{
-    __shared__ int s_part[4];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
-    if ((threadIdx.x & (kWave - 1)) == 0) s_part[threadIdx.x / kWave] = local;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int sum = s_part[0] + s_part[1] + s_part[2] + s_part[3];
-        if (sum) atomicAdd(d_count, sum);
-    }
-}
-
 __global__ __launch_bounds__(256) void count_nonzero_kernel(const int* __restrict__ in, int length, int* __restrict__ d_count)
 {
     int local = 0;
@@ -440,13 +620,6 @@ __global__ __launch_bounds__(256) void mark_bytes_kernel(const int* __restrict__
         for (int j = 0; j < 4; ++j)
             if (!seen[j]) bytes[c[j]] = 1;
     }
-}
-
-// bit j of the result: byte j of x is not zero
-__device__ __forceinline__ unsigned nonzero_bytes(unsigned x)
-{
-    const unsigned top = (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u;
-    return ((top >> 7) * 0x01020408u) >> 24 & 0xfu;
 }
 
 // bitmap word w = bytes 32 w .. 32 w + 31 (the byte array is padded to whole words with zeros)
@@ -765,6 +938,13 @@ size_t scan_workspace_bytes(long long length, int tile)
 size_t compact_workspace_bytes(long long length) { return scan_workspace_bytes(length, kCompactTile); }
 size_t split_workspace_bytes(long long num_nodes) { return scan_workspace_bytes(num_nodes, kSplitTile); }
 
+// workgroups that write the zeros behind `length` words at most, four words per thread and step
+static unsigned tail_blocks(long long length)
+{
+    const long long blocks = (length + 1023) / 1024;
+    return static_cast<unsigned>(blocks > 2048 ? 2048 : blocks < 1 ? 1 : blocks);
+}
+
 static int init_scan(void* workspace, int num_tiles, hipStream_t stream)
 {
     ScanState* st = static_cast<ScanState*>(workspace);
@@ -801,10 +981,8 @@ int launch_compact_mask(const int* in_id, int* out_id, const int* in_edge, int* 
         hipLaunchKernelGGL(compact_mask_kernel, dim3(num_tiles), dim3(kCompactBlock), 0, stream, in_id, in_edge,
                            out_id, out_edge, static_cast<int>(length), num_tiles, st, desc, scan_mode());
         EPPGCN_HIP(hipGetLastError());
-        long long blocks = (length + 1023) / 1024;
-        if (blocks > 2048) blocks = 2048;
-        hipLaunchKernelGGL(zero_tail2_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, out_id,
-                           out_edge, st->counts, static_cast<int>(length));
+        hipLaunchKernelGGL(zero_tail2_kernel, dim3(tail_blocks(length)), dim3(256), 0, stream, out_id, out_edge, st->counts,
+                           static_cast<int>(length));
         EPPGCN_HIP(hipGetLastError());
     }
     return kOk;
@@ -865,6 +1043,21 @@ size_t mark_compact_workspace_bytes(long long length)
     return compact_workspace_bytes(length) + static_cast<size_t>(tiles + 2) * sizeof(int);
 }
 
+template <bool kBits>
+static void launch_mark_pass(const int* part2node, const int* part_ptr, const int* col, const uint8_t* src_bytes,
+                             const uint32_t* src_bits, uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge,
+                             uint8_t* self_kept, int num_parts, long long length, int num_tiles, int is_last,
+                             const int* tile_first, ScanState* st, uint64_t* desc, hipStream_t stream)
+{
+#define EPPGCN_MARK(ITEMS_)                                                                                              \
+    hipLaunchKernelGGL((mark_compact_kernel<ITEMS_, kBits>), dim3(num_tiles), dim3(kMarkBlock), 0, stream, part2node,     \
+                       part_ptr, col, src_bytes, src_bits, ngh_mask, node_degs, out_id, out_edge, self_kept, num_parts,    \
+                       static_cast<int>(length), num_tiles, is_last, tile_first, st, desc, scan_mode())
+    if (mark_tile_slots(length) == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge);
+    else EPPGCN_MARK(kMarkItemsSmall);
+#undef EPPGCN_MARK
+}
+
 // Results land in the ScanState at the head of the workspace: counts[0] = kept length.
 int launch_mark_compact(const int* part2node, const int* part_ptr, const int* col, const uint8_t* src_mask,
                         uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge, int num_parts,
@@ -872,7 +1065,8 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
 {
     ScanState* st = static_cast<ScanState*>(workspace);
     uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
-    const int num_tiles = num_parts > 0 ? static_cast<int>((length + kCompactTile - 1) / kCompactTile) : 0;
+    const int tile_slots = mark_tile_slots(length);
+    const int num_tiles = num_parts > 0 ? static_cast<int>((length + tile_slots - 1) / tile_slots) : 0;
     if (int rc = init_scan(workspace, num_tiles, stream)) return rc;
     if (num_tiles == 0) {
         if (length > 0) {
@@ -883,16 +1077,65 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
     }
     int* tile_first = reinterpret_cast<int*>(static_cast<char*>(workspace) + compact_workspace_bytes(length));
     hipLaunchKernelGGL(tile_groups_kernel, dim3((num_tiles + 1 + 255) / 256), dim3(256), 0, stream, part_ptr, num_parts,
-                       num_tiles, tile_first);
+                       num_tiles, tile_slots, tile_first);
     EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mark_compact_kernel, dim3(num_tiles), dim3(kCompactBlock), 0, stream, part2node, part_ptr, col,
-                       src_mask, ngh_mask, node_degs, out_id, out_edge, num_parts, static_cast<int>(length), num_tiles,
-                       is_last, tile_first, st, desc, scan_mode());
+    launch_mark_pass<false>(part2node, part_ptr, col, src_mask, nullptr, ngh_mask, node_degs, out_id, out_edge, nullptr,
+                            num_parts, length, num_tiles, is_last, tile_first, st, desc, stream);
     EPPGCN_HIP(hipGetLastError());
-    long long blocks = (length + 1023) / 1024;
-    if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(zero_tail2_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, out_id, out_edge,
-                       st->counts, static_cast<int>(length));
+    hipLaunchKernelGGL(zero_tail2_kernel, dim3(tail_blocks(length)), dim3(256), 0, stream, out_id, out_edge, st->counts,
+                       static_cast<int>(length));
+    EPPGCN_HIP(hipGetLastError());
+    return kOk;
+}
+
+// Workspace of launch_mark_path behind that of launch_mark_compact: the bit map of the source mask and one byte per
+// vertex (its self-loop was kept), both in whole words and 16-byte aligned.
+struct MarkPathLayout {
+    size_t bits, self_kept, total;
+    int words;
+};
+static MarkPathLayout mark_path_layout(long long length, long long num_nodes)
+{
+    MarkPathLayout l;
+    l.words = static_cast<int>((num_nodes + 31) / 32);
+    l.bits = (mark_compact_workspace_bytes(length) + 15) / 16 * 16;
+    l.self_kept = (l.bits + 4 * static_cast<size_t>(l.words) + 15) / 16 * 16;
+    l.total = l.self_kept + 32 * static_cast<size_t>(l.words);
+    return l;
+}
+size_t mark_path_workspace_bytes(long long length, long long num_nodes) { return mark_path_layout(length, num_nodes).total; }
+uint8_t* mark_path_scratch(void* workspace, long long length, long long num_nodes)
+{
+    return static_cast<uint8_t*>(workspace) + mark_path_layout(length, num_nodes).self_kept;
+}
+
+// launch_mark_compact with the rows of the path counted and its gathered rows marked; num_parts, length, num_nodes > 0.
+// Results land in the ScanState at the head of the workspace (16-byte aligned): counts[0] = kept length, pad as
+// mark_path_finish_kernel says.
+int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, const uint8_t* src_mask,
+                     uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge, uint32_t* gathered, int num_parts,
+                     long long length, int num_nodes, int is_last, void* workspace, hipStream_t stream)
+{
+    ScanState* st = static_cast<ScanState*>(workspace);
+    uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
+    const int tile_slots = mark_tile_slots(length);
+    const int num_tiles = static_cast<int>((length + tile_slots - 1) / tile_slots);
+    const MarkPathLayout l = mark_path_layout(length, num_nodes);
+    char* base = static_cast<char*>(workspace);
+    int* tile_first = reinterpret_cast<int*>(base + compact_workspace_bytes(length));
+    uint32_t* bits = reinterpret_cast<uint32_t*>(base + l.bits);
+    uint8_t* self_kept = reinterpret_cast<uint8_t*>(base + l.self_kept);
+    const int most = l.words * 8 > num_tiles + 1 ? l.words * 8 : num_tiles + 1;
+    const int init_blocks = most / 256 + 1 < 2048 ? most / 256 + 1 : 2048;
+    hipLaunchKernelGGL(mark_path_init_kernel, dim3(init_blocks), dim3(256), 0, stream, src_mask, num_nodes, l.words, bits,
+                       reinterpret_cast<uint32_t*>(self_kept), part_ptr, num_parts, num_tiles, tile_slots, tile_first, st, desc);
+    EPPGCN_HIP(hipGetLastError());
+    launch_mark_pass<true>(part2node, part_ptr, col, src_mask, bits, ngh_mask, node_degs, out_id, out_edge, self_kept,
+                           num_parts, length, num_tiles, is_last, tile_first, st, desc, stream);
+    EPPGCN_HIP(hipGetLastError());
+    hipLaunchKernelGGL(mark_path_finish_kernel, dim3(tail_blocks(length > num_nodes ? length : num_nodes)), dim3(256), 0,
+                       stream, bits, reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, out_id,
+                       out_edge, static_cast<int>(length), st);
     EPPGCN_HIP(hipGetLastError());
     return kOk;
 }
@@ -918,10 +1161,7 @@ int launch_split(bool from_row_ptr, const int* src, int num_nodes, int part_size
                            part_size, part_ptr_out, part2node_out, capacity, num_tiles, st, desc, scan_mode());
     EPPGCN_HIP(hipGetLastError());
     if (zero_tail) {
-        long long blocks = (capacity + 1023) / 1024;
-        if (blocks > 2048) blocks = 2048;
-        if (blocks < 1) blocks = 1;
-        hipLaunchKernelGGL(zero_tail1_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, part_ptr_out,
+        hipLaunchKernelGGL(zero_tail1_kernel, dim3(tail_blocks(capacity)), dim3(256), 0, stream, part_ptr_out,
                            st->counts, 1, capacity);
         EPPGCN_HIP(hipGetLastError());
     }

@@ -65,10 +65,9 @@ def choose_back_part_size(mode: str, constant: int, valid_node: int, valid_len: 
 def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, mask_seed: int = 2,
             part_size: int = None, backsize_mode: str = "constant", backsize: int = 32,
             train_mask: torch.Tensor = None, widths=(16, 22), plan=None, fused: bool = False) -> Workload:
-    """``fused``: mark and compact every layer in one pass (no E-entry edge masks) instead of the
-    reference's separate steps.  The results are identical; the one-pass form saves 4 bytes per edge and
-    layer of memory but is no faster (R-MAT scale 22, both layers: 7.0 ms either way), so the reference's
-    steps are the default."""
+    """Marking, compaction and the counts of a layer's path are one pass over the slots (``capi.mark_path``), for either
+    value of ``fused``: the reference's separate steps are ``capi.mask_forward``, ``compact_back_edge``,
+    ``count_nonzero`` and ``mark_gathered_rows``, with the same results."""
     g = graph
     dev = g.column_index.device
     n, e = g.num_nodes, g.num_edges
@@ -82,28 +81,21 @@ def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, 
 
     # per-run state, EPPGCN/dataset.py:135-156
     ngh_masks = [torch.zeros(n, dtype=torch.bool, device=dev) for _ in range(num_layers - 1)]
-    edge_masks = ([None] * num_layers if fused else
-                  [torch.full((e,), -1, dtype=torch.int32, device=dev) for _ in range(num_layers)])
     node_degs = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(num_layers)]
 
     # mask chain, EPPGCN/gcn_main.py:130-139: step i runs in the forward of conv i
+    marked = [None] * num_layers
     for i in range(num_layers):
         src = train_mask if i == 0 else ngh_masks[i - 1]
         last = i == num_layers - 1
-        dst = None if last else ngh_masks[i]
         k = num_layers - 1 - i
-        if fused:
-            edge_masks[k] = capi.mark_compact(part2node, part_ptr, g.column_index, src, dst, node_degs[k], last)
-        else:
-            capi.mask_forward(part2node, part_ptr, g.column_index, src, dst, edge_masks[k], node_degs[k], last)
+        marked[k] = capi.mark_path(part2node, part_ptr, g.column_index, src, None if last else ngh_masks[i],
+                                   node_degs[k], last)
 
     # buildBackPart, EPPGCN/gcn_main.py:151-168
     paths = []
     for k in range(num_layers):
-        ids, edge_list, valid_len = (edge_masks[k] if fused else
-                                     capi.compact_back_edge(edge_masks[k], g.column_index))
-        edge_masks[k] = None
-        valid_node = capi.count_nonzero(node_degs[k])
+        ids, edge_list, valid_len, valid_node, bitmap, distinct = marked[k]
         bps = choose_back_part_size(backsize_mode, backsize, valid_node, valid_len)
         part_pointer, num_parts, v2 = capi.split_back_part(node_degs[k], e, bps)
         assert v2 == valid_len
@@ -114,7 +106,6 @@ def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, 
                                      block_shift=0 if 2 * valid_len >= e else 31)
                      if plan and num_parts > 0 else None)
         # the pre-scaling pass of the gradient only has to cover the rows the path reads
-        bitmap, distinct = capi.mark_gathered_rows(edge_list, valid_len, n)
         paths.append(BackwardPath(k + 1, ids, edge_list, part_pointer, node_degs[k], bps, num_parts,
                                   valid_len, valid_node, path_plan, bitmap if 2 * distinct < n else None))
     # one plan of the forward groups serves every width (the column block is sized for the widest)

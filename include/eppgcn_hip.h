@@ -316,6 +316,16 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers,
                         int32_t* node_degs, int32_t* out_id, int32_t* out_edge, int num_parts,
                         int64_t num_edges, int is_last_layer, void* workspace, size_t workspace_bytes,
                         int32_t* d_valid_len, int64_t* h_valid_len, void* stream);
+/* eppgcn_mark_compact together with what is asked of a path afterwards: gathered_rows[(num_nodes + 31) / 32] as
+ * eppgcn_mark_gathered_rows fills it for the kept slots, and counts[3] (host) = kept slots, rows with node_degs != 0,
+ * gathered rows.  src_mask, ngh_mask and node_degs have num_nodes entries.  Synchronises the stream once (twice when a
+ * marked vertex has no self-loop among its slots).
+ * workspace: eppgcn_mark_path_workspace_bytes(num_edges, num_nodes) bytes, 16-byte aligned. */
+size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes);
+int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                     const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
+                     uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last,
+                     void* workspace, size_t workspace_bytes, int64_t* counts, void* stream);
 
 /* Number of entries != 0 (valid_node of the group-size heuristics).  Stands in for
  * compact_count (cuCompactor.cu:694-696 over :623-680).  d_count: one device int. */

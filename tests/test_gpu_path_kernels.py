@@ -42,3 +42,50 @@ def test_distinct_rows_with_and_without_scratch(api, n, length, shift):
 def test_count_of_rows_with_kept_edges(api, n):
     deg = (np.arange(n) % 3).astype(np.int32)
     assert api.count_nonzero(torch.from_numpy(deg).cuda()) == int(np.count_nonzero(deg))
+
+
+@pytest.mark.parametrize("n,slots_per_row,loops,ps", [
+    (1, 3, True, 2), (33, 5, True, 4), (500, 9, False, 1),          # a single small tile
+    (700, 0, True, 3),                                              # nothing but self-loops
+    (3000, 11, True, 8), (3001, 11, False, 64),                     # several small tiles, with and without self-loops
+    (9, 3000, True, 32),                                            # rows of several tiles
+    (300000, 15, True, 16), (9, 600000, False, 32),                 # large tiles
+    (4300000, 0, True, 1)])                                         # more groups in a large tile than are staged
+@pytest.mark.parametrize("is_last", [False, True])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shift):
+    """`shift`: the masks start one byte past a word boundary.  Vertex 0 is a neighbour of every third slot."""
+    rng = np.random.default_rng(n + slots_per_row)
+    deg = rng.integers(0, 2 * slots_per_row + 1, n) + (1 if loops else 0)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    e = int(indptr[-1])
+    row = np.repeat(np.arange(n, dtype=np.int32), deg)
+    col = rng.integers(0, n, e, dtype=np.int32)
+    col[::3] = 0
+    if loops:
+        col[indptr[:-1]] = np.arange(n)
+    src = rng.random(n) < 0.3
+    keep = src[col]
+    want_ngh = np.zeros(n, bool)
+    if not is_last:
+        want_ngh[row[src[row]]] = True
+        want_ngh[col[src[row]]] = True
+    degs_want = np.bincount(row[keep], minlength=n).astype(np.int32)
+    gathered = np.zeros((n + 31) // 32 * 32, np.uint8)
+    gathered[col[keep]] = 1
+
+    pp, p2n = api.build_part(ps, torch.from_numpy(indptr).cuda(), e)
+    hold = torch.zeros(2, n + 1, dtype=torch.bool, device="cuda")
+    d_src, ngh = hold[0][shift:shift + n], hold[1][shift:shift + n]
+    d_src.copy_(torch.from_numpy(src))
+    degs = torch.zeros(n, dtype=torch.int32, device="cuda")
+    ids, edges, kept, rows, bitmap, distinct = api.mark_path(p2n, pp, torch.from_numpy(col).cuda(), d_src,
+                                                             None if is_last else ngh, degs, is_last)
+    v = int(keep.sum())
+    assert (kept, rows, distinct) == (v, int(np.count_nonzero(degs_want)), int(gathered.sum()))
+    want = np.zeros((2, e), np.int32)
+    want[0, :v], want[1, :v] = row[keep], col[keep]
+    assert np.array_equal(ids.cpu().numpy(), want[0]) and np.array_equal(edges.cpu().numpy(), want[1])
+    assert np.array_equal(degs.cpu().numpy(), degs_want)
+    assert np.array_equal(ngh.cpu().numpy(), want_ngh)
+    assert np.array_equal(bitmap.cpu().numpy(), np.packbits(gathered, bitorder="little").view(np.int32))
