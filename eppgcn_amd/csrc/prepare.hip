@@ -246,26 +246,24 @@ __global__ __launch_bounds__(kCompactBlock) void compact_mask_kernel(
 }
 
 // ================================================================ marking + compaction in one pass
-// One pass over the slots does what mask_forward_kernel followed by compact_mask_kernel do, without the E-entry edge
-// mask between them.  A tile is kMarkBlock * kItems consecutive slots; slot k * kMarkBlock + t of the tile belongs to
-// thread t, so word k * (waves) + wave of every 64-slot bit map is one ballot and words are in slot order.
-//   - the column ids of a thread's slots are loaded first (kItems loads in flight), then their mask entries;
-//   - the row of a slot comes from a bit map of the group starts inside the tile (prefix population count; the tile's
-//     first group was found by mark_tiles_kernel) and the rows of the tile's groups, staged in LDS;
-//   - kept slots per group are differences of the prefix counts of the kept bit map, added over the groups of a row in a
-//     wave, one atomic per (wave, row): a hub of 600 thousand slots costs 40 tiles a few atomics each, where one per 64
-//     slots queued ten thousand on one address;
-//   - (row, col) of the kept slots go out at look-back prefix + word prefix + ballot rank.
-// What bounds it: the random reads of the source mask, one cache line per slot that misses the vector cache.  kBits: the
-// mask is read as a bit map (packed once per call), which lets eight times as many vertices share a line.
-// Tile ids come from one device counter at 12 ns each: 16384 slots per tile keep that below 0.1 ms for 132 M slots;
-// inputs of a few million slots take tiles of 4096 so that every CU has work.
-constexpr int kMarkBlock = 512;
+// What mask_forward_kernel followed by compact_mask_kernel do, without the E-entry edge mask between them, in two kernels
+// over tiles of kMarkBlock * kItems consecutive slots.  Slot k * kMarkBlock + t of a tile belongs to thread t, so word
+// k * kMarkWaves + wave of every 64-slot bit map is one ballot and words are in slot order.
+//   keep_slots_kernel    keep = the slot's column is in the source mask: one bit per slot and a count per tile.  Nothing but
+//                        column ids and mask entries is read, with kItems of each under way per thread.
+//   place_slots_kernel   rows and places of the kept slots.  The kept slots before a tile are the counts before its own,
+//                        added up by the tile's workgroup; the row of a slot comes from a bit map of the group starts inside
+//                        the tile (prefix population count; the tile's first group was found beforehand) and the rows of
+//                        the tile's groups, staged in LDS; kept slots per row are differences of the prefix counts, one
+//                        atomic per (wave, row): a hub of 600 thousand slots costs 40 tiles a few atomics each, where one
+//                        per 64 slots queued ten thousand on one address.
+// Inputs of a few million slots take tiles of 4096 so that every CU has work.
+constexpr int kMarkBlock = 1024;
 constexpr int kMarkWaves = kMarkBlock / kWave;
-constexpr int kMarkItemsLarge = 32, kMarkItemsSmall = 8;
+constexpr int kMarkItemsLarge = 16, kMarkItemsSmall = 4;
+constexpr int kMarkBatch = 4;             // groups a thread looks at together
 constexpr int kMarkStagedRows = 4096;     // groups of a tile whose rows are staged (more: read where they are needed)
-static_assert(kMarkBlock * kMarkItemsSmall >= kCompactTile, "the workspace is sized for tiles of kCompactTile slots");
-constexpr long long kMarkLargeLength = 4ll << 20;
+constexpr long long kMarkLargeLength = 32ll << 20;
 __host__ __device__ constexpr int mark_tile_slots(long long length)
 {
     return kMarkBlock * (length >= kMarkLargeLength ? kMarkItemsLarge : kMarkItemsSmall);
@@ -290,25 +288,86 @@ __device__ __forceinline__ void find_tile_groups(const int* __restrict__ part_pt
 }
 
 __global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_parts, int num_tiles, int tile_slots,
-                                   int* __restrict__ first)
+                                   int* __restrict__ first, ScanState* st)
 {
-    find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, blockIdx.x * blockDim.x + threadIdx.x);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) *st = ScanState{};
+    find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
+}
+
+// the 64-bit value of lane k (k the same in all lanes)
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int k)
+{
+    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(v), k);
+    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), k);
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
+
+// kBits: the source mask is read as bits (packed once per call): eight times as many vertices share a cache line
+template <bool kBits>
+__device__ __forceinline__ bool in_mask(const void* __restrict__ mask, int v)
+{
+    if constexpr (kBits) return ((static_cast<const uint32_t*>(mask)[static_cast<unsigned>(v) >> 5] >> (v & 31)) & 1u) != 0u;
+    else return static_cast<const uint8_t*>(mask)[v] != 0;
 }
 
 template <int kItems, bool kBits>
-__global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
-    const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
-    const uint8_t* __restrict__ src_bytes, const uint32_t* __restrict__ src_bits, uint8_t* __restrict__ ngh_mask,
-    int* __restrict__ node_degs, int* __restrict__ out_id, int* __restrict__ out_edge, uint8_t* __restrict__ self_kept,
-    int num_parts, int length, int num_tiles, int is_last, const int* __restrict__ tile_first, ScanState* st,
-    uint64_t* desc, unsigned mode)
+__global__ __launch_bounds__(kMarkBlock) void keep_slots_kernel(const int* __restrict__ part_ptr, const int* __restrict__ col,
+                                                                const void* __restrict__ src, int num_parts, int length,
+                                                                unsigned long long* __restrict__ kept, int* __restrict__ counts)
 {
     constexpr int kTile = kMarkBlock * kItems;
     constexpr int kWords = kTile / 64;
-    constexpr int kPerLane = (kWords + kWave - 1) / kWave;     // words a lane of the scanning wave adds up
-    constexpr int kChunk = kItems < 16 ? kItems : 16;
-    static_assert(kWords % kWave == 0, "the words of a tile are divided evenly over one wave");
-    __shared__ int s_tile;
+    __shared__ unsigned long long s_kept[kWords];
+    __shared__ int s_total;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x >> 6;
+    const long long base = static_cast<long long>(blockIdx.x) * kTile;
+    // slots outside [part_ptr[0], part_ptr[num_parts]) belong to no group and are never kept
+    const int owned_lo = part_ptr[0];
+    const int owned_hi = min(part_ptr[num_parts], length);
+    if (threadIdx.x == 0) s_total = 0;
+    int c[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const long long idx = base + k * kMarkBlock + threadIdx.x;
+        c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
+    }
+    bool keep[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) keep[k] = in_mask<kBits>(src, max(c[k], 0));
+    uint64_t mine = 0;                                       // lane k: the ballot of slot k
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const uint64_t ballot = __ballot(keep[k] && c[k] >= 0);
+        if (lane == k) mine = ballot;
+    }
+    if (lane < kItems) s_kept[lane * kMarkWaves + wave] = mine;
+    __syncthreads();
+    if (threadIdx.x < kWords) {
+        const unsigned long long word = s_kept[threadIdx.x];
+        kept[static_cast<long long>(blockIdx.x) * kWords + threadIdx.x] = word;
+        int n = __popcll(word);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
+        if (lane == 0) atomicAdd(&s_total, n);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = s_total;
+}
+
+template <int kItems, bool kBits>
+__global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
+    const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
+    const void* __restrict__ src, uint8_t* __restrict__ ngh_mask, int* __restrict__ node_degs, int* __restrict__ out_id,
+    int* __restrict__ out_edge, uint8_t* __restrict__ self_kept, int length, int num_tiles, int is_last,
+    const int* __restrict__ tile_first, const unsigned long long* __restrict__ kept, const int* __restrict__ counts,
+    ScanState* st)
+{
+    constexpr int kTile = kMarkBlock * kItems;
+    constexpr int kWords = kTile / 64;
+    constexpr int kPerLane = kWords / kWave;
+    static_assert(kWords % kWave == 0 && kItems <= kWave, "one wave scans the words; a wave's words fit its lanes");
     __shared__ int s_prefix;
     __shared__ int s_starts_in_tile;
     __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
@@ -316,44 +375,51 @@ __global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
     __shared__ int s_starts_before[kWords];            // group starts before each word
     __shared__ int s_kept_before[kWords + 1];          // kept slots before each word; [kWords] = all of the tile
     __shared__ unsigned s_row[kMarkStagedRows];        // rows of the tile's groups; bit 31: the row is in the source mask
-    for (int i = threadIdx.x; i < kWords; i += kMarkBlock) s_starts[i] = 0ull;
-    if (threadIdx.x == 0) s_starts_in_tile = 0;
-    const int tile = acquire_tile(st, &s_tile);        // contains the barrier that publishes the zeros
-    if (tile >= num_tiles) return;
+    const int tile = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
     const long long base = static_cast<long long>(tile) * kTile;
-    auto in_src = [&](int v) {
-        if constexpr (kBits) return ((src_bits[static_cast<unsigned>(v) >> 5] >> (v & 31)) & 1u) != 0u;
-        else return src_bytes[v] != 0;
-    };
-
-    // slots outside [part_ptr[0], part_ptr[num_parts]) belong to no group and are never kept
-    const int owned_lo = part_ptr[0];
-    const int owned_hi = min(part_ptr[num_parts], length);
-    int c[kItems];
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const long long idx = base + k * kMarkBlock + threadIdx.x;
-        c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
-    }
     const int g_lo = tile_first[tile];
     const int g_cnt = tile_first[tile + 1] - g_lo + 1;
     const bool staged = g_cnt <= kMarkStagedRows;
     const int before = part_ptr[g_lo] < base ? 1 : 0;    // g_lo itself starts before the tile
+    if (threadIdx.x < kWords) {
+        s_starts[threadIdx.x] = 0ull;
+        s_kept[threadIdx.x] = kept[static_cast<long long>(tile) * kWords + threadIdx.x];
+    }
+    if (threadIdx.x == 0) s_starts_in_tile = s_prefix = 0;
+    __syncthreads();
     {
+        int sum = 0;
+        for (int t = threadIdx.x; t < tile; t += kMarkBlock) sum += counts[t];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+        if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
         int mine = 0;
-        for (int i = threadIdx.x; i < g_cnt; i += kMarkBlock) {
-            const int start = part_ptr[g_lo + i];
-            const int row = part2node[g_lo + i];
-            const long long p = start - base;
-            if (p >= 0 && p < kTile) {
-                atomicOr(&s_starts[p >> 6], 1ull << (p & 63));
-                ++mine;
+        for (int i0 = threadIdx.x; i0 < g_cnt; i0 += kMarkBlock * kMarkBatch) {
+            int start[kMarkBatch], row[kMarkBatch];
+            bool some[kMarkBatch], marked[kMarkBatch];
+#pragma unroll
+            for (int j = 0; j < kMarkBatch; ++j) {
+                const int g = g_lo + min(i0 + j * kMarkBlock, g_cnt - 1);
+                start[j] = part_ptr[g];
+                some[j] = part_ptr[g + 1] > start[j];
+                row[j] = part2node[g];
             }
-            const bool marked = !is_last && in_src(row);
-            if (staged) s_row[i] = static_cast<unsigned>(row) | (marked ? 0x80000000u : 0u);
-            if (marked && part_ptr[g_lo + i + 1] > start) ngh_mask[row] = 1;
+#pragma unroll
+            for (int j = 0; j < kMarkBatch; ++j) marked[j] = !is_last && in_mask<kBits>(src, row[j]);
+#pragma unroll
+            for (int j = 0; j < kMarkBatch; ++j) {
+                const int i = i0 + j * kMarkBlock;
+                if (i >= g_cnt) continue;
+                const long long p = start[j] - base;
+                if (p >= 0 && p < kTile) {
+                    atomicOr(&s_starts[p >> 6], 1ull << (p & 63));
+                    ++mine;
+                }
+                if (staged) s_row[i] = static_cast<unsigned>(row[j]) | (marked[j] ? 0x80000000u : 0u);
+                if (marked[j] && some[j]) ngh_mask[row[j]] = 1;
+            }
         }
         if (mine) atomicAdd(&s_starts_in_tile, mine);
     }
@@ -361,30 +427,75 @@ __global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
     // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
     // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
     // population count over the map of group starts; otherwise every slot does a binary search over the group starts.
-    if (wave == 0) {
+    if (wave < 2) {
+        const unsigned long long* words = wave == 0 ? s_kept : s_starts;
+        int* out = wave == 0 ? s_kept_before : s_starts_before;
         int n[kPerLane], sum = 0;
 #pragma unroll
         for (int j = 0; j < kPerLane; ++j) {
-            n[j] = __popcll(s_starts[lane * kPerLane + j]);
+            n[j] = __popcll(words[lane * kPerLane + j]);
             sum += n[j];
         }
         const int incl = wave_inclusive_scan(sum);
         int run = incl - sum;
 #pragma unroll
         for (int j = 0; j < kPerLane; ++j) {
-            s_starts_before[lane * kPerLane + j] = run;
+            out[lane * kPerLane + j] = run;
             run += n[j];
         }
-        if (lane == kWave - 1 && incl != s_starts_in_tile) s_starts_in_tile = -1;   // duplicate starts
+        if (lane == kWave - 1) {
+            if (wave == 0) {
+                s_kept_before[kWords] = incl;
+                if (tile == num_tiles - 1) st->counts[0] = s_prefix + incl;
+            } else if (incl != s_starts_in_tile) {
+                s_starts_in_tile = -1;                       // duplicate starts
+            }
+        }
     }
     __syncthreads();
+    // kept slots per row
+    auto kept_before = [&](long long p) {                    // kept slots of the tile before slot base + p
+        const int q = static_cast<int>(p < 0 ? 0 : p > kTile ? kTile : p);
+        const int word = q >> 6;
+        const int whole = s_kept_before[word];
+        return (q & 63) ? whole + __popcll(s_kept[word] & ((1ull << (q & 63)) - 1ull)) : whole;
+    };
+    for (int i0 = 0; i0 < g_cnt; i0 += kMarkBlock * kMarkBatch) {
+        int from[kMarkBatch], to[kMarkBatch], row[kMarkBatch];
+#pragma unroll
+        for (int j = 0; j < kMarkBatch; ++j) {
+            const int i = i0 + j * kMarkBlock + static_cast<int>(threadIdx.x);
+            const int g = g_lo + min(i, g_cnt - 1);
+            from[j] = part_ptr[g];
+            to[j] = part_ptr[g + 1];
+            row[j] = i >= g_cnt ? -1 : staged ? static_cast<int>(s_row[i] & 0x7fffffffu) : part2node[g];
+        }
+#pragma unroll
+        for (int j = 0; j < kMarkBatch; ++j) {
+            if (i0 + j * kMarkBlock >= g_cnt) break;         // the same for the whole workgroup
+            int n = row[j] < 0 ? 0 : kept_before(to[j] - base) - kept_before(from[j] - base);
+            const int prev_row = __shfl_up(row[j], 1, kWave);
+            const uint64_t heads = __ballot(lane == 0 || prev_row != row[j]);
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+                const int other = __shfl_down(n, off, kWave);
+                const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);   // run heads in lanes lane+1 .. lane+off
+                if (lane + off < kWave && between == 0) n += other;
+            }
+            if (((heads >> lane) & 1ull) && n > 0) atomicAdd(node_degs + row[j], n);
+        }
+    }
     const bool by_bits = s_starts_in_tile >= 0;
-    auto row_of = [&](int k) {                            // row of this thread's slot k; bit 31 as in s_row
+    // lane k: word k of this wave
+    const int my_word = (lane < kItems ? lane : 0) * kMarkWaves + wave;
+    const uint64_t start_word = s_starts[my_word], kept_word = s_kept[my_word];
+    const int start_before = s_starts_before[my_word] + before - 1;
+    const int place = s_kept_before[my_word] + s_prefix;
+    auto row_of = [&](int k) {                               // row of this thread's slot k; bit 31 as in s_row
         int a = 0;
         if (by_bits) {
-            const int word = k * kMarkWaves + wave;
-            const unsigned long long upto = lane == 63 ? ~0ull : (2ull << lane) - 1ull;
-            a = before + s_starts_before[word] + __popcll(s_starts[word] & upto) - 1;
+            const uint64_t word = lane_value(start_word, k);
+            a = __builtin_amdgcn_readlane(start_before, k) + ballot_rank(word) + static_cast<int>((word >> lane) & 1ull);
         } else {
             const int e = static_cast<int>(base + k * kMarkBlock + threadIdx.x);
             int b = g_cnt;
@@ -393,93 +504,36 @@ __global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
                 if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
             }
         }
+        a = max(a, 0);                                       // a slot before the first group (it is never used)
         if (staged) return s_row[a];
         const int row = part2node[g_lo + a];
-        return static_cast<unsigned>(row) | (!is_last && in_src(row) ? 0x80000000u : 0u);
+        return static_cast<unsigned>(row) | (!is_last && in_mask<kBits>(src, row) ? 0x80000000u : 0u);
     };
-
+    const int owned_lo = part_ptr[0], owned_hi = min(part_ptr[g_lo + g_cnt], length);
+    constexpr int kChunk = kItems < 8 ? kItems : 8;
 #pragma unroll
     for (int k0 = 0; k0 < kItems; k0 += kChunk) {
-        bool keep[kChunk];
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) keep[k] = in_src(max(c[k0 + k], 0));
+        int c[kChunk];
 #pragma unroll
         for (int k = 0; k < kChunk; ++k) {
-            const uint64_t ballot = __ballot(keep[k] && c[k0 + k] >= 0);
-            if (lane == 0) s_kept[(k0 + k) * kMarkWaves + wave] = ballot;
+            const long long idx = base + (k0 + k) * kMarkBlock + threadIdx.x;
+            c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
         }
-        if (!is_last) {
-            bool mark[kChunk];
 #pragma unroll
-            for (int k = 0; k < kChunk; ++k) mark[k] = c[k0 + k] >= 0 && (row_of(k0 + k) >> 31) != 0u;
+        for (int k = 0; k < kChunk; ++k) {
+            const uint64_t ballot = lane_value(kept_word, k0 + k);
+            if (is_last && ballot == 0ull) continue;         // the same for the whole wave
+            const unsigned row = row_of(k0 + k);
+            if ((ballot >> lane) & 1ull) {
+                const int dst = __builtin_amdgcn_readlane(place, k0 + k) + ballot_rank(ballot);
+                const int r = static_cast<int>(row & 0x7fffffffu);
+                out_id[dst] = r;
+                out_edge[dst] = c[k];
+                if (self_kept && r == c[k]) self_kept[r] = 1;
+            }
             // a vertex that already reads as marked is not stored again: hubs are neighbours of most rows
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) mark[k] = mark[k] && ngh_mask[c[k0 + k]] == 0;
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k)
-                if (mark[k]) ngh_mask[c[k0 + k]] = 1;
+            if (!is_last && c[k] >= 0 && (row >> 31) != 0u && ngh_mask[c[k]] == 0) ngh_mask[c[k]] = 1;
         }
-    }
-    __syncthreads();
-    if (wave == 0) {
-        int n[kPerLane], sum = 0;
-#pragma unroll
-        for (int j = 0; j < kPerLane; ++j) {
-            n[j] = __popcll(s_kept[lane * kPerLane + j]);
-            sum += n[j];
-        }
-        const int incl = wave_inclusive_scan(sum);
-        const int total = __shfl(incl, kWave - 1, kWave);
-        int run = incl - sum;
-#pragma unroll
-        for (int j = 0; j < kPerLane; ++j) {
-            s_kept_before[lane * kPerLane + j] = run;
-            run += n[j];
-        }
-        const uint64_t excl = tile_lookback(desc, st, tile, static_cast<uint64_t>(total), mode);
-        if (lane == 0) {
-            s_kept_before[kWords] = total;
-            s_prefix = static_cast<int>(excl);
-            if (tile == num_tiles - 1) st->counts[0] = static_cast<int>(excl) + total;
-        }
-    }
-    __syncthreads();
-    const int prefix = s_prefix;
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int word = k * kMarkWaves + wave;
-        const uint64_t ballot = s_kept[word];
-        if ((ballot >> lane) & 1ull) {
-            const int dst = prefix + s_kept_before[word] + ballot_rank(ballot);
-            const int row = static_cast<int>(row_of(k) & 0x7fffffffu);
-            out_id[dst] = row;
-            out_edge[dst] = c[k];
-            if (self_kept && row == c[k]) self_kept[row] = 1;
-        }
-    }
-    // kept slots per row
-    auto kept_before = [&](long long p) {                 // kept slots of the tile before slot base + p
-        const int q = static_cast<int>(p < 0 ? 0 : p > kTile ? kTile : p);
-        const int word = q >> 6;
-        const int whole = s_kept_before[word];
-        return (q & 63) ? whole + __popcll(s_kept[word] & ((1ull << (q & 63)) - 1ull)) : whole;
-    };
-    for (int i0 = 0; i0 < g_cnt; i0 += kMarkBlock) {
-        const int i = i0 + static_cast<int>(threadIdx.x);
-        int row = -1, kept = 0;
-        if (i < g_cnt) {
-            row = staged ? static_cast<int>(s_row[i] & 0x7fffffffu) : part2node[g_lo + i];
-            kept = kept_before(part_ptr[g_lo + i + 1] - base) - kept_before(part_ptr[g_lo + i] - base);
-        }
-        const int prev_row = __shfl_up(row, 1, kWave);
-        const uint64_t heads = __ballot(lane == 0 || prev_row != row);
-#pragma unroll
-        for (int off = 1; off < kWave; off <<= 1) {
-            const int other = __shfl_down(kept, off, kWave);
-            const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);   // run heads in lanes lane+1 .. lane+off
-            if (lane + off < kWave && between == 0) kept += other;
-        }
-        if (((heads >> lane) & 1ull) && kept > 0) atomicAdd(node_degs + row, kept);
     }
 }
 
@@ -488,15 +542,11 @@ __global__ __launch_bounds__(kMarkBlock, 6) void mark_compact_kernel(
 __global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __restrict__ src_mask, int num_nodes, int words,
                                                              uint32_t* __restrict__ bits, uint32_t* __restrict__ self_kept,
                                                              const int* __restrict__ part_ptr, int num_parts, int num_tiles,
-                                                             int tile_slots, int* __restrict__ first, ScanState* st,
-                                                             uint64_t* __restrict__ desc)
+                                                             int tile_slots, int* __restrict__ first, ScanState* st)
 {
     const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
     if (i0 == 0) *st = ScanState{};
-    for (int t = i0; t <= num_tiles; t += stride) {
-        if (t < num_tiles) desc[t] = kTileEmpty;
-        find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
-    }
+    for (int t = i0; t <= num_tiles; t += stride) find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
     // a thread packs 4 bytes into 4 bits of a word, 8 lanes a word (vertices past the end count as unmarked)
     const bool quads = reinterpret_cast<uintptr_t>(src_mask) % 4 == 0;
     for (int q0 = blockIdx.x * 256; q0 < words * 8; q0 += stride) {
@@ -1037,25 +1087,58 @@ int launch_compact_mask_static(const int* in_id, int* out_id, const int* in_edge
     return launch_compact_mask(in_id, out_id, in_edge, out_edge, length, ws, stream);
 }
 
-size_t mark_compact_workspace_bytes(long long length)
+// Workspace of the marking pass behind its ScanState: one bit per slot, a count and the first group of every tile, and
+// for launch_mark_path the bit map of the source mask and one byte per vertex (its self-loop was kept), in whole words.
+struct MarkLayout {
+    size_t kept, counts, first, bits, self_kept, total;
+    int tile_slots, num_tiles, words;
+};
+static MarkLayout mark_layout(long long length, long long num_nodes)
 {
-    const long long tiles = (length + kCompactTile - 1) / kCompactTile;
-    return compact_workspace_bytes(length) + static_cast<size_t>(tiles + 2) * sizeof(int);
+    MarkLayout l;
+    l.tile_slots = mark_tile_slots(length);
+    l.num_tiles = static_cast<int>((length + l.tile_slots - 1) / l.tile_slots);
+    l.words = static_cast<int>((num_nodes + 31) / 32);
+    l.kept = sizeof(ScanState);
+    l.counts = l.kept + static_cast<size_t>(l.num_tiles) * (l.tile_slots / 8);
+    l.first = l.counts + 4 * static_cast<size_t>(l.num_tiles);
+    l.bits = (l.first + 4 * (static_cast<size_t>(l.num_tiles) + 1) + 15) / 16 * 16;
+    l.self_kept = (l.bits + 4 * static_cast<size_t>(l.words) + 15) / 16 * 16;
+    l.total = l.self_kept + 32 * static_cast<size_t>(l.words);
+    return l;
+}
+size_t mark_compact_workspace_bytes(long long length) { return mark_layout(length < 0 ? 0 : length, 0).total; }
+size_t mark_path_workspace_bytes(long long length, long long num_nodes) { return mark_layout(length, num_nodes).total; }
+uint8_t* mark_path_scratch(void* workspace, long long length, long long num_nodes)
+{
+    return static_cast<uint8_t*>(workspace) + mark_layout(length, num_nodes).self_kept;
 }
 
 template <bool kBits>
-static void launch_mark_pass(const int* part2node, const int* part_ptr, const int* col, const uint8_t* src_bytes,
-                             const uint32_t* src_bits, uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge,
-                             uint8_t* self_kept, int num_parts, long long length, int num_tiles, int is_last,
-                             const int* tile_first, ScanState* st, uint64_t* desc, hipStream_t stream)
+static int launch_mark_pass(const int* part2node, const int* part_ptr, const int* col, const void* src, uint8_t* ngh_mask,
+                            int* node_degs, int* out_id, int* out_edge, uint8_t* self_kept, int num_parts, long long length,
+                            int is_last, const MarkLayout& l, char* workspace, hipStream_t stream)
 {
+    ScanState* st = reinterpret_cast<ScanState*>(workspace);
+    unsigned long long* kept = reinterpret_cast<unsigned long long*>(workspace + l.kept);
+    int* counts = reinterpret_cast<int*>(workspace + l.counts);
+    const int* first = reinterpret_cast<const int*>(workspace + l.first);
+    const dim3 grid(l.num_tiles), block(kMarkBlock);
+    const int len = static_cast<int>(length);
 #define EPPGCN_MARK(ITEMS_)                                                                                              \
-    hipLaunchKernelGGL((mark_compact_kernel<ITEMS_, kBits>), dim3(num_tiles), dim3(kMarkBlock), 0, stream, part2node,     \
-                       part_ptr, col, src_bytes, src_bits, ngh_mask, node_degs, out_id, out_edge, self_kept, num_parts,    \
-                       static_cast<int>(length), num_tiles, is_last, tile_first, st, desc, scan_mode())
-    if (mark_tile_slots(length) == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge);
+    do {                                                                                                                \
+        hipLaunchKernelGGL((keep_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part_ptr, col, src, num_parts, len, \
+                           kept, counts);                                                                                 \
+        EPPGCN_HIP(hipGetLastError());                                                                                    \
+        hipLaunchKernelGGL((place_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part2node, part_ptr, col, src,     \
+                           ngh_mask, node_degs, out_id, out_edge, self_kept, len, l.num_tiles, is_last, first, kept,       \
+                           counts, st);                                                                                   \
+        EPPGCN_HIP(hipGetLastError());                                                                                    \
+    } while (0)
+    if (l.tile_slots == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge);
     else EPPGCN_MARK(kMarkItemsSmall);
 #undef EPPGCN_MARK
+    return kOk;
 }
 
 // Results land in the ScanState at the head of the workspace: counts[0] = kept length.
@@ -1063,50 +1146,27 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
                         uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge, int num_parts,
                         long long length, int is_last, void* workspace, hipStream_t stream)
 {
-    ScanState* st = static_cast<ScanState*>(workspace);
-    uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
-    const int tile_slots = mark_tile_slots(length);
-    const int num_tiles = num_parts > 0 ? static_cast<int>((length + tile_slots - 1) / tile_slots) : 0;
-    if (int rc = init_scan(workspace, num_tiles, stream)) return rc;
-    if (num_tiles == 0) {
+    const MarkLayout l = mark_layout(length, 0);
+    char* base = static_cast<char*>(workspace);
+    if (num_parts == 0 || l.num_tiles == 0) {
+        if (int rc = init_scan(workspace, 0, stream)) return rc;
         if (length > 0) {
             if (int rc = launch_zero_words(out_id, static_cast<size_t>(length), stream)) return rc;
             if (int rc = launch_zero_words(out_edge, static_cast<size_t>(length), stream)) return rc;
         }
         return kOk;
     }
-    int* tile_first = reinterpret_cast<int*>(static_cast<char*>(workspace) + compact_workspace_bytes(length));
-    hipLaunchKernelGGL(tile_groups_kernel, dim3((num_tiles + 1 + 255) / 256), dim3(256), 0, stream, part_ptr, num_parts,
-                       num_tiles, tile_slots, tile_first);
+    ScanState* st = static_cast<ScanState*>(workspace);
+    hipLaunchKernelGGL(tile_groups_kernel, dim3((l.num_tiles + 1 + 255) / 256), dim3(256), 0, stream, part_ptr, num_parts,
+                       l.num_tiles, l.tile_slots, reinterpret_cast<int*>(base + l.first), st);
     EPPGCN_HIP(hipGetLastError());
-    launch_mark_pass<false>(part2node, part_ptr, col, src_mask, nullptr, ngh_mask, node_degs, out_id, out_edge, nullptr,
-                            num_parts, length, num_tiles, is_last, tile_first, st, desc, stream);
-    EPPGCN_HIP(hipGetLastError());
+    if (int rc = launch_mark_pass<false>(part2node, part_ptr, col, src_mask, ngh_mask, node_degs, out_id, out_edge, nullptr,
+                                         num_parts, length, is_last, l, base, stream))
+        return rc;
     hipLaunchKernelGGL(zero_tail2_kernel, dim3(tail_blocks(length)), dim3(256), 0, stream, out_id, out_edge, st->counts,
                        static_cast<int>(length));
     EPPGCN_HIP(hipGetLastError());
     return kOk;
-}
-
-// Workspace of launch_mark_path behind that of launch_mark_compact: the bit map of the source mask and one byte per
-// vertex (its self-loop was kept), both in whole words and 16-byte aligned.
-struct MarkPathLayout {
-    size_t bits, self_kept, total;
-    int words;
-};
-static MarkPathLayout mark_path_layout(long long length, long long num_nodes)
-{
-    MarkPathLayout l;
-    l.words = static_cast<int>((num_nodes + 31) / 32);
-    l.bits = (mark_compact_workspace_bytes(length) + 15) / 16 * 16;
-    l.self_kept = (l.bits + 4 * static_cast<size_t>(l.words) + 15) / 16 * 16;
-    l.total = l.self_kept + 32 * static_cast<size_t>(l.words);
-    return l;
-}
-size_t mark_path_workspace_bytes(long long length, long long num_nodes) { return mark_path_layout(length, num_nodes).total; }
-uint8_t* mark_path_scratch(void* workspace, long long length, long long num_nodes)
-{
-    return static_cast<uint8_t*>(workspace) + mark_path_layout(length, num_nodes).self_kept;
 }
 
 // launch_mark_compact with the rows of the path counted and its gathered rows marked; num_parts, length, num_nodes > 0.
@@ -1116,23 +1176,20 @@ int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, 
                      uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge, uint32_t* gathered, int num_parts,
                      long long length, int num_nodes, int is_last, void* workspace, hipStream_t stream)
 {
-    ScanState* st = static_cast<ScanState*>(workspace);
-    uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
-    const int tile_slots = mark_tile_slots(length);
-    const int num_tiles = static_cast<int>((length + tile_slots - 1) / tile_slots);
-    const MarkPathLayout l = mark_path_layout(length, num_nodes);
+    const MarkLayout l = mark_layout(length, num_nodes);
     char* base = static_cast<char*>(workspace);
-    int* tile_first = reinterpret_cast<int*>(base + compact_workspace_bytes(length));
+    ScanState* st = static_cast<ScanState*>(workspace);
     uint32_t* bits = reinterpret_cast<uint32_t*>(base + l.bits);
     uint8_t* self_kept = reinterpret_cast<uint8_t*>(base + l.self_kept);
-    const int most = l.words * 8 > num_tiles + 1 ? l.words * 8 : num_tiles + 1;
+    const int most = l.words * 8 > l.num_tiles + 1 ? l.words * 8 : l.num_tiles + 1;
     const int init_blocks = most / 256 + 1 < 2048 ? most / 256 + 1 : 2048;
     hipLaunchKernelGGL(mark_path_init_kernel, dim3(init_blocks), dim3(256), 0, stream, src_mask, num_nodes, l.words, bits,
-                       reinterpret_cast<uint32_t*>(self_kept), part_ptr, num_parts, num_tiles, tile_slots, tile_first, st, desc);
+                       reinterpret_cast<uint32_t*>(self_kept), part_ptr, num_parts, l.num_tiles, l.tile_slots,
+                       reinterpret_cast<int*>(base + l.first), st);
     EPPGCN_HIP(hipGetLastError());
-    launch_mark_pass<true>(part2node, part_ptr, col, src_mask, bits, ngh_mask, node_degs, out_id, out_edge, self_kept,
-                           num_parts, length, num_tiles, is_last, tile_first, st, desc, stream);
-    EPPGCN_HIP(hipGetLastError());
+    if (int rc = launch_mark_pass<true>(part2node, part_ptr, col, bits, ngh_mask, node_degs, out_id, out_edge, self_kept,
+                                        num_parts, length, is_last, l, base, stream))
+        return rc;
     hipLaunchKernelGGL(mark_path_finish_kernel, dim3(tail_blocks(length > num_nodes ? length : num_nodes)), dim3(256), 0,
                        stream, bits, reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, out_id,
                        out_edge, static_cast<int>(length), st);
