@@ -738,16 +738,20 @@ __global__ __launch_bounds__(256) void ginfo_hist_kernel(const int* __restrict__
 // ================================================================ group splitting
 // Vertex i with g_i slots (g_i = kept degree, or CSR degree) yields q_i = ceil(g_i/ps)
 // groups; group j of vertex i starts at G_i + j*ps where G_i is the exclusive sum
-// of g.  One look-back scan carries (sum q, sum g) packed as q*2^31 + g.  The
-// tile's groups are then written in two ways: a vertex with at most kSmallGroups
-// groups by the thread that owns it, every other vertex - collected on a list in
-// LDS - by a whole wave, 64 groups per step with coalesced stores, so a hub vertex
-// with a hundred thousand groups costs its tile a longer loop, not one thread a
-// longer life.
-constexpr int kSplitBlock = 256;
-constexpr int kSplitItems = 8;
-constexpr int kSplitTile = kSplitBlock * kSplitItems;
+// of g.  One look-back scan carries (sum q, sum g) packed as q*2^31 + g over tiles of kSplitTile vertices; vertex
+// (round r, thread t) of a tile is r * kSplitBlock + t, so that degrees are read and groups written with neighbouring
+// lanes on neighbouring words; the (round, wave) sums are scanned by one wave.  The tile's groups are written in two ways:
+// a vertex with at most kSmallGroups groups by the thread that owns it, every other vertex - collected on a list in LDS -
+// by a whole wave, 64 groups per step, so a hub with a hundred thousand groups costs its tile a longer loop, not one
+// thread a longer life.  The tile with the hubs is the last to finish (the first 2048 vertices of an R-MAT graph of scale
+// 22 have 200 thousand groups): 16 waves write it.  4 waves, with 8 consecutive vertices per thread: 0.19 ms for the forward
+// groups of that graph against 0.07, and 84 against 31 us at scale 20.
+constexpr int kSplitBlock = 1024;
+constexpr int kSplitRounds = 2;
+constexpr int kSplitTile = kSplitBlock * kSplitRounds;
+constexpr int kSplitWaves = kSplitBlock / kWave;
 constexpr int kSmallGroups = 4;     // groups per vertex up to which the owning thread writes them itself
+static_assert(kSplitRounds * kSplitWaves <= kWave, "one wave scans the (round, wave) sums of a tile");
 
 template <bool kFromRowPtr>
 __global__ __launch_bounds__(kSplitBlock) void split_groups_kernel(
@@ -755,109 +759,80 @@ __global__ __launch_bounds__(kSplitBlock) void split_groups_kernel(
     int* __restrict__ part2node_out, long long capacity, int num_tiles, ScanState* st, uint64_t* desc, unsigned mode)
 {
     __shared__ int s_tile;
-    __shared__ int s_q[kSplitTile + 1];
-    __shared__ int s_g[kSplitTile];
-    __shared__ uint64_t s_wave[kSplitBlock / kWave];
-    __shared__ uint64_t s_tile_excl;
-    __shared__ int s_big[kSplitTile];
+    __shared__ uint64_t s_sum[kSplitRounds * kSplitWaves];
+    __shared__ int s_big_first[kSplitTile], s_big_start[kSplitTile], s_big_groups[kSplitTile], s_big_vertex[kSplitTile];
     __shared__ int s_big_count;
+    if (threadIdx.x == 0) s_big_count = 0;
     const int tile = acquire_tile(st, &s_tile);
     if (tile >= num_tiles) return;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
     const long long base = static_cast<long long>(tile) * kSplitTile;
 
-    int g[kSplitItems], q[kSplitItems];
-    int tq = 0, tg = 0;
+    int q[kSplitRounds];
+    uint64_t at[kSplitRounds];             // (groups, slots) before the vertex
 #pragma unroll
-    for (int j = 0; j < kSplitItems; ++j) {
-        const long long i = base + threadIdx.x * kSplitItems + j;
-        int gi = 0;
-        if (i < num_nodes) gi = kFromRowPtr ? src[i + 1] - src[i] : src[i];
-        gi = gi > 0 ? gi : 0;
-        g[j] = gi;
-        q[j] = (gi + part_size - 1) / part_size;
-        tq += q[j];
-        tg += gi;
+    for (int r = 0; r < kSplitRounds; ++r) {
+        const long long i = base + r * kSplitBlock + threadIdx.x;
+        int g = 0;
+        if (i < num_nodes) g = kFromRowPtr ? src[i + 1] - src[i] : src[i];
+        g = g > 0 ? g : 0;
+        q[r] = (g + part_size - 1) / part_size;
+        const uint64_t mine = (static_cast<uint64_t>(q[r]) << 31) | static_cast<uint64_t>(g);
+        const uint64_t incl = wave_inclusive_scan_u64(mine);
+        at[r] = incl - mine;
+        if (lane == kWave - 1) s_sum[r * kSplitWaves + wave] = incl;
     }
-    const uint64_t mine = (static_cast<uint64_t>(tq) << 31) | static_cast<uint64_t>(tg);
-    const uint64_t incl = wave_inclusive_scan_u64(mine);
-    if (lane == kWave - 1) s_wave[wave] = incl;
-    __syncthreads();
-    uint64_t wave_excl = 0, tile_total = 0;
-#pragma unroll
-    for (int w = 0; w < kSplitBlock / kWave; ++w) {
-        if (w < wave) wave_excl += s_wave[w];
-        tile_total += s_wave[w];
-    }
-    if (wave == 0) {
-        const uint64_t excl = tile_lookback(desc, st, tile, tile_total, mode);
-        if (lane == 0) s_tile_excl = excl;
-    }
-    // tile-relative q offsets and absolute g offsets of this thread's vertices
-    uint64_t run = wave_excl + incl - mine;
     const int g_first = kFromRowPtr ? src[0] : 0;
     __syncthreads();
-    const uint64_t tile_excl = s_tile_excl;
-    const int q_base = static_cast<int>(tile_excl >> 31);
-    const int g_base = static_cast<int>(tile_excl & 0x7fffffffull) + g_first;
-#pragma unroll
-    for (int j = 0; j < kSplitItems; ++j) {
-        const int slot = threadIdx.x * kSplitItems + j;
-        s_q[slot] = static_cast<int>(run >> 31);
-        s_g[slot] = g_base + static_cast<int>(run & 0x7fffffffull);
-        run += (static_cast<uint64_t>(q[j]) << 31) | static_cast<uint64_t>(g[j]);
-    }
-    const int tile_q = static_cast<int>(tile_total >> 31);
-    if (threadIdx.x == 0) {
-        s_q[kSplitTile] = tile_q;
-        s_big_count = 0;
+    if (wave == 0) {
+        const uint64_t mine = lane < kSplitRounds * kSplitWaves ? s_sum[lane] : 0ull;
+        const uint64_t incl = wave_inclusive_scan_u64(mine);
+        const uint64_t total = static_cast<uint64_t>(__shfl(static_cast<long long>(incl), kWave - 1, kWave));
+        const uint64_t excl = tile_lookback(desc, st, tile, total, mode);
+        if (lane < kSplitRounds * kSplitWaves) s_sum[lane] = excl + incl - mine;
+        if (tile == num_tiles - 1 && lane == 0) {
+            const uint64_t all = excl + total;
+            const int total_q = static_cast<int>(all >> 31);
+            const int total_g = static_cast<int>(all & 0x7fffffffull);
+            st->counts[0] = total_q;
+            st->counts[1] = total_g;
+            if (total_q < capacity) part_ptr_out[total_q] = total_g + g_first;
+            if (static_cast<long long>(total_q) + 1 > capacity) st->overflow = 1;
+        }
     }
     __syncthreads();
-
-    // A vertex with at most kSmallGroups groups is written by the thread that owns it; the others
-    // go on a list and are written by whole waves, 64 groups per step, so that a tile full of hubs
-    // (the first vertices of an R-MAT graph have 10^5 groups each) costs coalesced stores only.
+    auto write_group = [&](long long dst, int start, int vertex) {
+        if (dst < capacity) {
+            part_ptr_out[dst] = start;
+            if (part2node_out && dst + 1 < capacity) part2node_out[dst] = vertex;
+        }
+    };
 #pragma unroll
-    for (int j = 0; j < kSplitItems; ++j) {
-        const int slot = threadIdx.x * kSplitItems + j;
-        if (q[j] > kSmallGroups) {
-            s_big[atomicAdd(&s_big_count, 1)] = slot;
+    for (int r = 0; r < kSplitRounds; ++r) {
+        const uint64_t before = s_sum[r * kSplitWaves + wave] + at[r];
+        const int first = static_cast<int>(before >> 31);
+        const int start = static_cast<int>(before & 0x7fffffffull) + g_first;
+        const int vertex = static_cast<int>(base) + r * kSplitBlock + static_cast<int>(threadIdx.x);
+        if (q[r] > kSmallGroups) {
+            const int b = atomicAdd(&s_big_count, 1);
+            s_big_first[b] = first;
+            s_big_start[b] = start;
+            s_big_groups[b] = q[r];
+            s_big_vertex[b] = vertex;
         } else {
-            const int start = s_g[slot];
-            const long long first = static_cast<long long>(q_base) + s_q[slot];
-            for (int k = 0; k < q[j]; ++k) {
-                const long long dst = first + k;
-                if (dst < capacity) {
-                    part_ptr_out[dst] = start + k * part_size;
-                    if (part2node_out && dst + 1 < capacity) part2node_out[dst] = static_cast<int>(base) + slot;
-                }
-            }
+#pragma unroll
+            for (int k = 0; k < kSmallGroups; ++k)
+                if (k < q[r]) write_group(static_cast<long long>(first) + k, start + k * part_size, vertex);
         }
     }
     __syncthreads();
     const int big = s_big_count;
-    for (int b = wave; b < big; b += kSplitBlock / kWave) {
-        const int slot = s_big[b];
-        const int count = s_q[slot + 1] - s_q[slot];
-        const int start = s_g[slot];
-        const long long first = static_cast<long long>(q_base) + s_q[slot];
-        for (int k = lane; k < count; k += kWave) {
-            const long long dst = first + k;
-            if (dst < capacity) {
-                part_ptr_out[dst] = start + k * part_size;
-                if (part2node_out && dst + 1 < capacity) part2node_out[dst] = static_cast<int>(base) + slot;
-            }
-        }
-    }
-    if (tile == num_tiles - 1 && threadIdx.x == 0) {
-        const uint64_t total = tile_excl + tile_total;
-        const int total_q = static_cast<int>(total >> 31);
-        const int total_g = static_cast<int>(total & 0x7fffffffull);
-        st->counts[0] = total_q;
-        st->counts[1] = total_g;
-        if (total_q < capacity) part_ptr_out[total_q] = total_g + g_first;
-        if (static_cast<long long>(total_q) + 1 > capacity) st->overflow = 1;
+    for (int b = wave; b < big; b += kSplitWaves) {
+        const int groups = s_big_groups[b];
+        const long long first = s_big_first[b];
+        const int start = s_big_start[b], vertex = s_big_vertex[b];
+        for (int k = lane; k < groups; k += kWave) write_group(first + k, start + k * part_size, vertex);
     }
 }
 

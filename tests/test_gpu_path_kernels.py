@@ -89,3 +89,26 @@ def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shi
     assert np.array_equal(degs.cpu().numpy(), degs_want)
     assert np.array_equal(ngh.cpu().numpy(), want_ngh)
     assert np.array_equal(bitmap.cpu().numpy(), np.packbits(gathered, bitorder="little").view(np.int32))
+
+
+@pytest.mark.parametrize("n,top,ps", [(1, 3, 2), (1023, 9, 4), (2048, 7, 1), (2049, 7, 1), (4097, 40, 8), (5000, 0, 3),
+                                      (70000, 25, 4), (3, 200000, 5)])
+def test_group_split_at_the_ends_of_tiles(api, n, top, ps):
+    """Rows of 0 to `top` slots, a hub in the middle: both directions, with and without room to spare."""
+    rng = np.random.default_rng(n + top)
+    deg = rng.integers(0, top + 1, n).astype(np.int32)
+    deg[n // 2] = 40 * top
+    groups = (deg + ps - 1) // ps
+    inside = np.arange(groups.sum()) - np.repeat(np.cumsum(groups) - groups, groups)
+    first = np.cumsum(deg) - deg
+    e = int(deg.sum())
+    want = np.concatenate([np.repeat(first, groups) + inside * ps, [e]]).astype(np.int32)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    pp, p2n = api.build_part(ps, torch.from_numpy(indptr).cuda(), e)
+    assert np.array_equal(pp.cpu().numpy(), want)
+    assert np.array_equal(p2n.cpu().numpy(), np.repeat(np.arange(n, dtype=np.int32), groups))
+    for room in (e, e + 37):
+        got, parts, slots = api.split_back_part(torch.from_numpy(deg).cuda(), room, ps)
+        assert (parts, slots) == (int(groups.sum()), e)
+        got = got.cpu().numpy()
+        assert np.array_equal(got[:parts + 1], want) and not got[parts + 1:].any()
