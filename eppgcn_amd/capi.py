@@ -25,6 +25,7 @@ EXPORTS = [
     "eppgcn_feature_workspace_pitch", "eppgcn_update_forward", "eppgcn_update_backward_input",
     "eppgcn_update_workspace_bytes", "eppgcn_update_backward_weight", "eppgcn_update_supported", "eppgcn_update_backward",
     "eppgcn_mark_compact_workspace_bytes", "eppgcn_mark_compact", "eppgcn_mark_path_workspace_bytes", "eppgcn_mark_path",
+    "eppgcn_nll_workspace_bytes", "eppgcn_nll_forward", "eppgcn_nll_backward",
     "eppgcn_set_plan_length_classes",
     "eppgcn_mark_gathered_rows", "eppgcn_set_wide_index", "eppgcn_wave64_back_part_size",
     "eppgcn_compact_back_edge_static", "eppgcn_compact_back_edge_static_max_length",
@@ -138,6 +139,12 @@ def load():
     lib.eppgcn_mark_path_workspace_bytes.restype = sz
     lib.eppgcn_mark_path.argtypes = [p, p, p, p, p, p, p, p, p, i, i64, i, i, p, sz, C.POINTER(i64), p]
     lib.eppgcn_mark_path.restype = i
+    lib.eppgcn_nll_workspace_bytes.argtypes = []
+    lib.eppgcn_nll_workspace_bytes.restype = sz
+    lib.eppgcn_nll_forward.argtypes = [p, p, p, p, i64, i64, i, p, sz, p]
+    lib.eppgcn_nll_forward.restype = i
+    lib.eppgcn_nll_backward.argtypes = [p, p, p, p, i64, i64, i, p]
+    lib.eppgcn_nll_backward.restype = i
     lib.eppgcn_feature_workspace_pitch.argtypes = [i]
     lib.eppgcn_feature_workspace_pitch.restype = i
     lib.eppgcn_update_supported.argtypes = [i, i]

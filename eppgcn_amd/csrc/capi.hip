@@ -50,6 +50,9 @@ int static_compact_workspace(void**);
 int read_aggregation_status(hipStream_t);
 size_t mark_compact_workspace_bytes(long long);
 size_t mark_path_workspace_bytes(long long, long long);
+size_t nll_workspace_bytes();
+int launch_nll_forward(float*, const float*, const long long*, const int*, long long, long long, int, void*, hipStream_t);
+int launch_nll_backward(float*, const float*, const float*, const int*, long long, long long, int, hipStream_t);
 uint8_t* mark_path_scratch(void*, long long, long long);
 int launch_mark_path(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, uint32_t*, int,
                      long long, int, int, void*, hipStream_t);
@@ -328,6 +331,29 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers, 
         *h_valid_len = host.counts[0];
     }
     return kOk;
+}
+
+size_t eppgcn_nll_workspace_bytes(void) { return nll_workspace_bytes(); }
+
+int eppgcn_nll_forward(float* loss, const float* logits, const int64_t* rows, const int32_t* labels, int64_t num_rows,
+                       int64_t num_nodes, int num_classes, void* workspace, size_t workspace_bytes, void* stream)
+{
+    EPPGCN_REQUIRE(num_rows >= 0 && num_nodes >= 0 && num_classes > 0, "negative size");
+    EPPGCN_REQUIRE(num_rows == 0 || num_nodes > 0, "training rows of no vertices");
+    EPPGCN_REQUIRE(loss && (num_rows == 0 || (logits && rows && labels)), "null pointer");
+    EPPGCN_REQUIRE(workspace && aligned(workspace, 8) && workspace_bytes >= nll_workspace_bytes(), "workspace too small or not 8-byte aligned");
+    static_assert(sizeof(long long) == sizeof(int64_t), "row ids are passed through");
+    return launch_nll_forward(loss, logits, reinterpret_cast<const long long*>(rows), labels, num_rows, num_nodes, num_classes,
+                              workspace, static_cast<hipStream_t>(stream));
+}
+
+int eppgcn_nll_backward(float* d_logits, const float* d_loss, const float* logits, const int32_t* labels, int64_t num_rows,
+                        int64_t num_nodes, int num_classes, void* stream)
+{
+    EPPGCN_REQUIRE(num_rows >= 0 && num_nodes >= 0 && num_classes > 0, "negative size");
+    EPPGCN_REQUIRE(num_nodes == 0 || (d_logits && d_loss && logits && labels), "null pointer");
+    return launch_nll_backward(d_logits, d_loss, logits, labels, num_rows, num_nodes, num_classes,
+                               static_cast<hipStream_t>(stream));
 }
 
 size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes)

@@ -445,6 +445,35 @@ std::vector<Tensor> ours_backward(Tensor d_output, Tensor X, Tensor W, Tensor id
     return dense_backward(d_input_prime, X, W, need_dx, relu_input, written);
 }
 
+// ---------------------------------------------------------------- training loss
+// rows: int64 ids of the training rows; labels: class of every vertex, -1 outside the training rows
+Tensor nll_forward(Tensor logits, Tensor rows, Tensor labels)
+{
+    CHECK_F32(logits); CHECK_INPUT(rows); CHECK_I32(labels);
+    TORCH_CHECK(rows.scalar_type() == torch::kInt64, "rows must be int64");
+    TORCH_CHECK(logits.dim() == 2 && labels.numel() == logits.size(0), "labels must have one entry per row of logits");
+    auto loss = torch::empty({}, logits.options());
+    const size_t nbytes = eppgcn_nll_workspace_bytes();
+    auto ws = workspace(nbytes, logits);
+    check(eppgcn_nll_forward(loss.data_ptr<float>(), f32(logits), rows.numel() ? rows.data_ptr<int64_t>() : nullptr, i32(labels),
+                             rows.numel(), logits.size(0), static_cast<int>(logits.size(1)), ws.data_ptr(), nbytes,
+                             stream_of(logits)),
+          "nll_forward");
+    return loss;
+}
+
+Tensor nll_backward(Tensor d_loss, Tensor logits, Tensor labels, int64_t num_rows)
+{
+    CHECK_F32(d_loss); CHECK_F32(logits); CHECK_I32(labels);
+    TORCH_CHECK(d_loss.numel() == 1, "d_loss must be one number");
+    TORCH_CHECK(logits.dim() == 2 && labels.numel() == logits.size(0), "labels must have one entry per row of logits");
+    auto grad = torch::empty_like(logits);
+    check(eppgcn_nll_backward(grad.numel() ? grad.data_ptr<float>() : nullptr, d_loss.data_ptr<float>(), f32(logits), i32(labels),
+                              num_rows, logits.size(0), static_cast<int>(logits.size(1)), stream_of(logits)),
+          "nll_backward");
+    return grad;
+}
+
 // ---------------------------------------------------------------- path preparation
 std::vector<Tensor> build_part(int partSize, Tensor indptr)
 {
@@ -647,6 +676,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           "execution plans: 0 = where the feature table outgrows the caches (default), 1 = always, -1 = never");
     m.def("cached_plans", []() { return static_cast<int>(g_plans.size()); }, "number of execution plans held");
 
+    m.def("nll_forward", &nll_forward, "mean negative log-likelihood of the training rows (HIP)", py::arg("logits"),
+          py::arg("rows"), py::arg("labels"));
+    m.def("nll_backward", &nll_backward, "gradient of nll_forward (HIP)", py::arg("d_loss"), py::arg("logits"),
+          py::arg("labels"), py::arg("num_rows"));
     m.def("build_part", &build_part, "forward neighbour groups (HIP)");
     m.def("build_back_part", &build_back_part, "compaction + group split in one call (HIP)");
     m.def("compact_back_edge", &compact_back_edge, "compact the kept edges of one layer (HIP)");

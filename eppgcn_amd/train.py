@@ -42,6 +42,22 @@ class GraphDataset:
         self.node_degs = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(num_layers)]
 
 
+class _TrainingLoss(torch.autograd.Function):
+    """Mean negative log-likelihood of log_softmax over the training rows in two kernels each way."""
+
+    @staticmethod
+    def forward(ctx, logits, rows, labels):
+        ctx.save_for_backward(logits, labels)
+        ctx.num_rows = rows.numel()
+        return gnnadvisor().nll_forward(logits, rows, labels)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, d_loss):
+        logits, labels = ctx.saved_tensors
+        return gnnadvisor().nll_backward(d_loss.contiguous(), logits, labels, ctx.num_rows), None, None
+
+
 class Net(torch.nn.Module):
     """The reference's model (EPPGCN/gcn_main.py:190-208): conv -> relu -> ... -> conv.  With
     ``fuse_relu`` (default) the activation between two layers is applied by the consuming layer
@@ -118,6 +134,7 @@ class Trainer:
         self.for_time = self.loss_time = self.back_time = self.build_time = 0.0
         self.losses: List[float] = []
         self.train_idx = self.train_y = None
+        self.row_labels = None                     # int32 class of every training row, -1 for the other rows
         self.kept_edges = [None] * num_layers      # per conv layer, filled by build_back_part
 
     def build_back_part(self):
@@ -137,12 +154,20 @@ class Trainer:
             self.kept_edges[i] = valid_len
             ds.edge_masks[i] = None      # the marking buffer is not needed after compaction
 
+    def _select_training_rows(self):
+        """The training rows and their labels, worked out once (EPPGCN/gcn_main.py:252-253 selects them with the boolean
+        mask, a device-to-host round trip per epoch)."""
+        ds = self.dataset
+        self.train_idx = ds.train_mask.nonzero().squeeze(1)
+        self.train_y = ds.y[self.train_idx]
+        if self.train_y.numel() and not 0 <= int(self.train_y.min()) <= int(self.train_y.max()) < ds.num_classes:
+            raise ValueError("a label of the training rows lies outside the %d classes" % ds.num_classes)
+        self.row_labels = torch.full((ds.num_nodes,), -1, dtype=torch.int32, device=ds.x.device)
+        self.row_labels[self.train_idx] = self.train_y.int()
+
     def _loss(self, out):
-        """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax,
-        EPPGCN/gcn_main.py:252-253).  Written as a gather and a mean: torch's nll_loss kernels
-        reduce all rows in one workgroup (0.53 + 0.33 ms per epoch for 4.2e5 rows here)."""
-        logp = F.log_softmax(out.index_select(0, self.train_idx), dim=1)
-        return -logp.gather(1, self.train_y.unsqueeze(1)).mean()
+        """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax, EPPGCN/gcn_main.py:252-253)."""
+        return _TrainingLoss.apply(out, self.train_idx, self.row_labels)
 
     def train_step(self, is_first_iter: bool, record_loss: bool = False, phase_timers: bool = True):
         """One epoch.  ``phase_timers`` keeps the reference's three host synchronisations per epoch
@@ -162,12 +187,8 @@ class Trainer:
             torch.cuda.synchronize()
             self.build_time += time.perf_counter() - t
         t = time.perf_counter()
-        # EPPGCN/gcn_main.py:252-253 takes log_softmax of every row and then selects the training
-        # rows with the boolean mask (a device-to-host round trip per epoch); selecting the rows
-        # first, through indices computed once, is the same function of `out`
         if self.train_idx is None:
-            self.train_idx = ds.train_mask.nonzero().squeeze(1)
-            self.train_y = ds.y[self.train_idx]
+            self._select_training_rows()
         loss = self._loss(out)
         sync()
         self.loss_time += time.perf_counter() - t

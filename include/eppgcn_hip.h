@@ -239,6 +239,20 @@ int eppgcn_mark_gathered_rows_scratch(const int32_t* edge_list, int64_t valid_le
                                       void* stream);
 
 /* ---------------------------------------------------------------------------
+ * Training loss: *loss (device) = mean over the training rows r of -log_softmax(logits[r, :])[labels[r]].
+ * rows[num_rows] lists the training rows; labels[num_nodes] holds the class of a training row and -1 elsewhere
+ * (a class outside 0 .. num_classes - 1 makes the loss NaN).  Deterministic.
+ * Backward: d_logits[num_nodes, num_classes] = *d_loss times the gradient, zero outside the training rows.
+ * (EPPGCN/gcn_main.py:252-253 takes both from torch.)
+ * workspace: eppgcn_nll_workspace_bytes() bytes, 8-byte aligned.
+ * ------------------------------------------------------------------------- */
+size_t eppgcn_nll_workspace_bytes(void);
+int eppgcn_nll_forward(float* loss, const float* logits, const int64_t* rows, const int32_t* labels, int64_t num_rows,
+                       int64_t num_nodes, int num_classes, void* workspace, size_t workspace_bytes, void* stream);
+int eppgcn_nll_backward(float* d_logits, const float* d_loss, const float* logits, const int32_t* labels, int64_t num_rows,
+                        int64_t num_nodes, int num_classes, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Execution-path preparation.
  * ------------------------------------------------------------------------- */
 
