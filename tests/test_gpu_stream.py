@@ -516,3 +516,35 @@ def test_stream_kernel_with_64_bit_addressing_gives_the_same_bits(api, dim):
         api.set_stream_mode(True)
     assert torch.equal(out, narrow), "64-bit and 32-bit addressing must agree bit for bit"
     assert_close(out.cpu().numpy(), co.spmm_f64(x, indptr, col, s), cf.abs_sum_bound(indptr, col, s, x), f"D={dim}")
+
+
+@pytest.mark.parametrize("dim", [60, 64, 68, 124, 128, 132, 252, 256])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("n", [4096, 5000])
+def test_rows_gathered_from_the_callers_matrix(api, dim, wide, n):
+    """Wide rows of a sparse graph need no scaled table.  n = 4096: the padding's id is the first one past the matrix.
+    Row 0 holds infinities and NaN and is no neighbour of any row: neither the padding nor idle lanes may bring it in.
+    A source or a result that is not 16-byte aligned takes the table."""
+    indptr, col = random_symmetric_csr(n, 3 * n, 21)
+    s = scale_inv_sqrt(indptr)
+    rng = np.random.default_rng(dim + n)
+    x = rng.standard_normal((n, dim)).astype(np.float32)
+    keep = (col != 0)
+    row = np.repeat(np.arange(n), np.diff(indptr))
+    indptr = np.concatenate([[0], np.cumsum(np.bincount(row[keep], minlength=n))]).astype(np.int32)
+    col = col[keep]
+    assert col.size <= 10 * n
+    want = co.spmm_f64(np.where(np.arange(n)[:, None] == 0, 0, x).astype(np.float32), indptr, col, s)
+    bound = cf.abs_sum_bound(indptr, col, s, x)
+    x[0, ::2], x[0, 1::2] = np.inf, np.nan
+    pp, p2n = api.build_part(8, dev(indptr), col.size)
+    plan = api.build_plan(pp, dev(col), p2n.numel(), col.size, n, dim, part2node=p2n)
+    api.set_stream_mode(True, wide=wide)
+    hold_x, hold_y = torch.empty(n * dim + 4, device="cuda"), torch.empty(n * dim + 4, device="cuda")
+    for shift_x, shift_y in ((0, 0), (1, 0), (0, 1)):
+        src = hold_x[shift_x:shift_x + n * dim].view(n, dim)
+        out = hold_y[shift_y:shift_y + n * dim].view(n, dim)
+        src.copy_(dev(x))
+        out.fill_(float("nan"))
+        api.spmm_forward(src, dev(col), dev(s), pp, p2n, part_size=8, out=out, plan=plan)
+        assert_close(out.cpu().numpy(), want, bound, f"dim {dim}, shifts {shift_x} {shift_y}")
