@@ -25,6 +25,7 @@ EXPORTS = [
     "eppgcn_feature_workspace_pitch", "eppgcn_update_forward", "eppgcn_update_backward_input",
     "eppgcn_update_workspace_bytes", "eppgcn_update_backward_weight", "eppgcn_update_supported", "eppgcn_update_backward",
     "eppgcn_mark_compact_workspace_bytes", "eppgcn_mark_compact", "eppgcn_mark_path_workspace_bytes", "eppgcn_mark_path",
+    "eppgcn_mark_path_counts", "eppgcn_split_counts",
     "eppgcn_nll_workspace_bytes", "eppgcn_nll_forward", "eppgcn_nll_backward",
     "eppgcn_set_plan_length_classes",
     "eppgcn_mark_gathered_rows", "eppgcn_set_wide_index", "eppgcn_wave64_back_part_size",
@@ -139,6 +140,10 @@ def load():
     lib.eppgcn_mark_path_workspace_bytes.restype = sz
     lib.eppgcn_mark_path.argtypes = [p, p, p, p, p, p, p, p, p, i, i64, i, i, p, sz, C.POINTER(i64), p]
     lib.eppgcn_mark_path.restype = i
+    lib.eppgcn_mark_path_counts.argtypes = [p, p, i64, i, p, C.POINTER(i64), p]
+    lib.eppgcn_mark_path_counts.restype = i
+    lib.eppgcn_split_counts.argtypes = [p, C.POINTER(i64), C.POINTER(i64), p]
+    lib.eppgcn_split_counts.restype = i
     lib.eppgcn_nll_workspace_bytes.argtypes = []
     lib.eppgcn_nll_workspace_bytes.restype = sz
     lib.eppgcn_nll_forward.argtypes = [p, p, p, p, i64, i64, i, p, sz, p]
@@ -463,6 +468,12 @@ def build_plan(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes
     """Column-blocked execution plan of the groups; build once per graph and group array and pass it
     as ``plan=`` to the aggregation calls.  Forward groups: give part2node; backward path: give ids.
     ``block_shift``: 0 = blocks sized for the width, n = blocks of 2^n vertices (31: one block)."""
+    return build_plan_begin(part_ptr, column_index, num_parts, num_slots, num_nodes, dim, part2node, ids, block_shift)()
+
+
+def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes: int, dim: int,
+                     part2node=None, ids=None, block_shift: int = 0):
+    """Issues ``build_plan``; the returned call waits for it and gives the plan."""
     lib = load()
     _dev(part_ptr, torch.int32, "part_ptr"); _dev(column_index, torch.int32, "column_index")
     if (part2node is None) == (ids is None):
@@ -478,12 +489,18 @@ def build_plan(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes
     _check(lib.eppgcn_build_plan(_ptr(part_ptr), _ptr(column_index), _ptr(part2node), _ptr(ids), int(num_parts),
                                  int(num_slots), int(num_nodes), int(dim), int(block_shift), C.c_void_p(base), nbytes,
                                  C.c_void_p(wbase), wbytes, _stream()))
-    # synchronises (the workspace is released on return), refuses a plan whose scan stalled and lets the
-    # library know the plan's stream form
-    partial = C.c_int64(0)
-    _check(lib.eppgcn_plan_status(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes), C.byref(partial),
-                                  _stream()))
-    return Plan(buf, base, int(num_parts), int(num_slots), int(num_nodes), int(partial.value))
+
+    def finish():
+        # synchronises (the workspace is released with this function), refuses a plan whose scan stalled and lets the
+        # library know the plan's stream form
+        partial = C.c_int64(0)
+        _check(lib.eppgcn_plan_status(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes), C.byref(partial),
+                                      _stream()))
+        del keep[:]
+        return Plan(buf, base, int(num_parts), int(num_slots), int(num_nodes), int(partial.value))
+
+    keep = [ws]
+    return finish
 
 
 def plan_recommended(num_nodes: int, dim: int) -> bool:
@@ -677,6 +694,12 @@ def mark_compact(part2node, part_ptr, column_index, src_mask, ngh_mask, node_deg
 def mark_path(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool):
     """``mark_compact`` with what ``count_nonzero`` and ``mark_gathered_rows`` say about the path ->
     (id int32[E], edge_list int32[E], valid_len, valid_nodes, gathered rows bitmap int32[(N+31)//32], gathered rows)."""
+    return mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer)()
+
+
+def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool):
+    """Issues ``mark_path``; the result is what the returned call gives, which waits for it (the same stream must be
+    current)."""
     lib = load()
     _dev(part2node, torch.int32, "part2node"); _dev(part_ptr, torch.int32, "part_ptr")
     _dev(column_index, torch.int32, "column_index"); _dev(node_degs, torch.int32, "node_degs")
@@ -694,11 +717,16 @@ def mark_path(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, 
     bitmap = torch.empty((n + 31) // 32, dtype=torch.int32, device=dev)
     nbytes = lib.eppgcn_mark_path_workspace_bytes(length, n)
     ws = _workspace(nbytes, dev)
-    counts = (C.c_int64 * 3)()
     _check(lib.eppgcn_mark_path(_ptr(part2node), _ptr(part_ptr), _ptr(column_index), _ptr(src), _ptr(ngh), _ptr(node_degs),
                                 _ptr(out_id), _ptr(out_edge), _ptr(bitmap), part2node.numel(), length, n,
-                                int(bool(is_last_layer)), _ptr(ws), nbytes, counts, _stream()))
-    return out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
+                                int(bool(is_last_layer)), _ptr(ws), nbytes, None, _stream()))
+
+    def finish():
+        counts = (C.c_int64 * 3)()
+        _check(lib.eppgcn_mark_path_counts(_ptr(out_edge), _ptr(bitmap), length, n, _ptr(ws), counts, _stream()))
+        return out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
+
+    return finish
 
 
 def count_nonzero(node_deg) -> int:
@@ -748,6 +776,11 @@ def aggregation_status() -> None:
 
 def split_back_part(node_deg, num_edges: int, part_size: int):
     """-> (part_pointer int32[num_edges + 1], num_parts int, valid_len int)"""
+    return split_back_part_begin(node_deg, num_edges, part_size)()
+
+
+def split_back_part_begin(node_deg, num_edges: int, part_size: int):
+    """Issues ``split_back_part``; the returned call waits for it and gives its result."""
     lib = load()
     _dev(node_deg, torch.int32, "node_deg")
     n = node_deg.numel()
@@ -755,10 +788,15 @@ def split_back_part(node_deg, num_edges: int, part_size: int):
     part_pointer = torch.empty(capacity, dtype=torch.int32, device=node_deg.device)
     nbytes = lib.eppgcn_split_workspace_bytes(n)
     ws = _workspace(nbytes, node_deg.device)
-    p, v = C.c_int64(0), C.c_int64(0)
     _check(lib.eppgcn_split_back_part(_ptr(node_deg), n, int(part_size), _ptr(part_pointer), capacity, _ptr(ws),
-                                      nbytes, None, C.byref(p), C.byref(v), _stream()))
-    return part_pointer, int(p.value), int(v.value)
+                                      nbytes, None, None, None, _stream()))
+
+    def finish():
+        p, v = C.c_int64(0), C.c_int64(0)
+        _check(lib.eppgcn_split_counts(_ptr(ws), C.byref(p), C.byref(v), _stream()))
+        return part_pointer, int(p.value), int(v.value)
+
+    return finish
 
 
 def build_part(part_size: int, row_pointers, num_edges: int = None):

@@ -368,7 +368,6 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
 {
     EPPGCN_REQUIRE(num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
                    "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
-    EPPGCN_REQUIRE(counts, "null pointer");
     EPPGCN_REQUIRE(workspace && aligned(workspace, 16), "workspace must be 16-byte aligned");
     EPPGCN_REQUIRE(workspace_bytes >= mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
     EPPGCN_REQUIRE(num_edges == 0 || (out_id && out_edge), "null output pointer");
@@ -376,7 +375,6 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
     EPPGCN_REQUIRE(num_parts == 0 || (part2node && part_pointers && column_index && src_mask && node_degs), "null pointer");
     EPPGCN_REQUIRE(is_last || num_parts == 0 || ngh_mask, "ngh_mask is required unless this is the last layer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    counts[0] = counts[1] = counts[2] = 0;
     if (num_parts == 0 || num_edges == 0 || num_nodes == 0) {
         if (num_nodes > 0)
             if (int rc = launch_zero_words(gathered_rows, (static_cast<size_t>(num_nodes) + 31) / 32, s)) return rc;
@@ -384,15 +382,24 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
             if (int rc = launch_zero_words(out_id, static_cast<size_t>(num_edges), s)) return rc;
             if (int rc = launch_zero_words(out_edge, static_cast<size_t>(num_edges), s)) return rc;
         }
-        EPPGCN_HIP(hipStreamSynchronize(s));
-        return kOk;
-    }
-    {
+        if (int rc = launch_zero_words(workspace, sizeof(ScanState) / 4, s)) return rc;
+    } else {
         KernelTimer timer(s, &g_mask_ms);
         if (int rc = launch_mark_path(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
                                       gathered_rows, num_parts, num_edges, num_nodes, is_last ? 1 : 0, workspace, s))
             return rc;
     }
+    return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
+}
+
+int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
+                            void* workspace, int64_t* counts, void* stream)
+{
+    EPPGCN_REQUIRE(num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31), "num_nodes >= 0 and 0 <= num_edges < 2^31 required");
+    EPPGCN_REQUIRE(workspace && aligned(workspace, 16) && counts, "workspace (16-byte aligned) and counts required");
+    EPPGCN_REQUIRE((num_edges == 0 || out_edge) && (num_nodes == 0 || gathered_rows), "null pointer");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    counts[0] = counts[1] = counts[2] = 0;
     ScanState host;
     if (int rc = read_state(workspace, s, &host)) return rc;
     counts[0] = host.counts[0];
@@ -588,6 +595,12 @@ int eppgcn_split_back_part(const int32_t* node_deg, int num_nodes, int part_size
     if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, nullptr, capacity, true, workspace, s))
         return rc;
     return finish_split(workspace, s, d_counts, h_num_parts, h_valid_len);
+}
+
+int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_valid_len, void* stream)
+{
+    EPPGCN_REQUIRE(workspace && aligned(workspace, 8), "workspace must be 8-byte aligned");
+    return finish_split(const_cast<void*>(workspace), static_cast<hipStream_t>(stream), nullptr, h_num_parts, h_valid_len);
 }
 
 int eppgcn_build_part(const int32_t* row_pointers, int num_nodes, int part_size, int32_t* part_pointers,

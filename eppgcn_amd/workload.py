@@ -83,35 +83,49 @@ def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, 
     ngh_masks = [torch.zeros(n, dtype=torch.bool, device=dev) for _ in range(num_layers - 1)]
     node_degs = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(num_layers)]
 
+    # Every stage is issued for all layers before the host waits for its counts, so the GPU has work while the host
+    # sizes the next stage.
+    # one plan of the forward groups serves every width (the column block is sized for the widest)
+    forward_plan = None
+    if plan and part2node.numel() > 0:
+        forward_plan = capi.build_plan_begin(part_ptr, g.column_index, part2node.numel(), e, n, max(widths),
+                                             part2node=part2node)
+
     # mask chain, EPPGCN/gcn_main.py:130-139: step i runs in the forward of conv i
     marked = [None] * num_layers
     for i in range(num_layers):
         src = train_mask if i == 0 else ngh_masks[i - 1]
         last = i == num_layers - 1
         k = num_layers - 1 - i
-        marked[k] = capi.mark_path(part2node, part_ptr, g.column_index, src, None if last else ngh_masks[i],
-                                   node_degs[k], last)
+        marked[k] = capi.mark_path_begin(part2node, part_ptr, g.column_index, src, None if last else ngh_masks[i],
+                                         node_degs[k], last)
+    marked = [finish() for finish in marked]
 
     # buildBackPart, EPPGCN/gcn_main.py:151-168
+    sizes = [choose_back_part_size(backsize_mode, backsize, valid_node, valid_len)
+             for _, _, valid_len, valid_node, _, _ in marked]
+    split = [capi.split_back_part_begin(node_degs[k], e, sizes[k]) for k in range(num_layers)]
+    split = [finish() for finish in split]
+    path_plans = [None] * num_layers
+    for k, (part_pointer, num_parts, covered) in enumerate(split):
+        ids, edge_list, valid_len = marked[k][:3]
+        assert covered == valid_len
+        # a heavily pruned path gathers from few distinct rows, which stay cached in any order: its
+        # plan keeps the groups in one block
+        if plan and num_parts > 0:
+            path_plans[k] = capi.build_plan_begin(part_pointer, edge_list, num_parts, valid_len, n,
+                                                  widths[min(k, len(widths) - 1)], ids=ids,
+                                                  block_shift=0 if 2 * valid_len >= e else 31)
     paths = []
     for k in range(num_layers):
         ids, edge_list, valid_len, valid_node, bitmap, distinct = marked[k]
-        bps = choose_back_part_size(backsize_mode, backsize, valid_node, valid_len)
-        part_pointer, num_parts, v2 = capi.split_back_part(node_degs[k], e, bps)
-        assert v2 == valid_len
-        width = widths[min(k, len(widths) - 1)]
-        # a heavily pruned path gathers from few distinct rows, which stay cached in any order: its
-        # plan keeps the groups in one block
-        path_plan = (capi.build_plan(part_pointer, edge_list, num_parts, valid_len, n, width, ids=ids,
-                                     block_shift=0 if 2 * valid_len >= e else 31)
-                     if plan and num_parts > 0 else None)
         # the pre-scaling pass of the gradient only has to cover the rows the path reads
-        paths.append(BackwardPath(k + 1, ids, edge_list, part_pointer, node_degs[k], bps, num_parts,
-                                  valid_len, valid_node, path_plan, bitmap if 2 * distinct < n else None))
-    # one plan of the forward groups serves every width (the column block is sized for the widest)
+        paths.append(BackwardPath(k + 1, ids, edge_list, split[k][0], node_degs[k], sizes[k], split[k][1],
+                                  valid_len, valid_node, path_plans[k] and path_plans[k](),
+                                  bitmap if 2 * distinct < n else None))
     plans = {}
-    if plan and part2node.numel() > 0:
-        shared = capi.build_plan(part_ptr, g.column_index, part2node.numel(), e, n, max(widths), part2node=part2node)
+    if forward_plan:
+        shared = forward_plan()
         plans = {w: shared for w in set(widths)}
     return Workload(g, ps, part_ptr, part2node, train_mask, ngh_masks, paths, plans)
 

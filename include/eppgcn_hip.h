@@ -333,13 +333,17 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers,
 /* eppgcn_mark_compact together with what is asked of a path afterwards: gathered_rows[(num_nodes + 31) / 32] as
  * eppgcn_mark_gathered_rows fills it for the kept slots, and counts[3] (host) = kept slots, rows with node_degs != 0,
  * gathered rows.  src_mask, ngh_mask and node_degs have num_nodes entries.  Synchronises the stream once (twice when a
- * marked vertex has no self-loop among its slots).
+ * marked vertex has no self-loop among its slots).  counts == NULL: nothing waits, and the outputs are complete once
+ * eppgcn_mark_path_counts has been called with the same buffers and sizes - with several layers in flight one wait serves
+ * them all.
  * workspace: eppgcn_mark_path_workspace_bytes(num_edges, num_nodes) bytes, 16-byte aligned. */
 size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes);
 int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
                      const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
                      uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last,
                      void* workspace, size_t workspace_bytes, int64_t* counts, void* stream);
+int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
+                            void* workspace, int64_t* counts, void* stream);
 
 /* Number of entries != 0 (valid_node of the group-size heuristics).  Stands in for
  * compact_count (cuCompactor.cu:694-696 over :623-680).  d_count: one device int. */
@@ -380,6 +384,10 @@ int eppgcn_split_back_part(const int32_t* node_deg, int num_nodes, int part_size
                            int32_t* part_pointer, int64_t capacity,
                            void* workspace, size_t workspace_bytes, int32_t* d_counts,
                            int64_t* h_num_parts, int64_t* h_valid_len, void* stream);
+
+/* Counts of an eppgcn_split_back_part call that was made without host pointers, from its workspace: synchronises the
+ * stream and reports what that call would have (a stalled scan, groups that did not fit). */
+int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_valid_len, void* stream);
 
 /* Forward neighbour groups from the CSR row pointers (device): part_pointers[0..P]
  * (terminator = row_pointers[num_nodes]) and part2node[0..P-1]; `capacity` is the
