@@ -64,8 +64,7 @@ def parse():
     ap.add_argument("--length_classes", action="store_true",
                     help="plans with the length-class key (the group kernel's optimum; off by default)")
     ap.add_argument("--fused_prep", action="store_true",
-                    help="prepare the backward paths with the one-pass marking + compaction instead of the "
-                         "reference's separate steps (same results, same time, no edge masks)")
+                    help="kept for old command lines: the backward paths are always marked and compacted in one pass")
     ap.add_argument("--no_plan", action="store_true",
                     help="process the groups in CSR order instead of the column-blocked execution plan")
     ap.add_argument("--no_stream", action="store_true",

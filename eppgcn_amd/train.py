@@ -161,10 +161,11 @@ class Trainer:
         ds = self.dataset
         self.train_idx = ds.train_mask.nonzero().squeeze(1)
         self.train_y = ds.y[self.train_idx]
-        if self.train_y.numel() and not 0 <= int(self.train_y.min()) <= int(self.train_y.max()) < ds.num_classes:
-            raise ValueError("a label of the training rows lies outside the %d classes" % ds.num_classes)
-        self.row_labels = torch.full((ds.num_nodes,), -1, dtype=torch.int32, device=ds.x.device)
-        self.row_labels[self.train_idx] = self.train_y.int()
+        if self.train_y.numel():
+            lo, hi = torch.stack(torch.aminmax(self.train_y)).tolist()
+            if not 0 <= lo <= hi < ds.num_classes:
+                raise ValueError("a label of the training rows lies outside the %d classes" % ds.num_classes)
+        self.row_labels = torch.where(ds.train_mask.bool(), ds.y, -1).int()
 
     def _loss(self, out):
         """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax, EPPGCN/gcn_main.py:252-253)."""
