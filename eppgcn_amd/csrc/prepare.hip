@@ -859,8 +859,9 @@ int launch_zero_words(void* p, size_t words, hipStream_t stream)
     size_t head = ((16 - a % 16) % 16) / 4;
     if (head > words) head = words;
     const size_t vecs = (words - head) / 4;
+    // one vector per thread: 528 MB at 6.8 TB/s, against 5.5 with 2^14 workgroups that stride over it
     size_t blocks = (vecs + 255) / 256;
-    if (blocks > 256 * 64) blocks = 256 * 64;
+    if (blocks > (1u << 23)) blocks = 1u << 23;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(zero_words_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
                        static_cast<uint32_t*>(p), head, vecs, words);
@@ -964,10 +965,15 @@ size_t compact_workspace_bytes(long long length) { return scan_workspace_bytes(l
 size_t split_workspace_bytes(long long num_nodes) { return scan_workspace_bytes(num_nodes, kSplitTile); }
 
 // workgroups that write the zeros behind `length` words at most, four words per thread and step
+// Workgroups that clear what lies behind a length that only the device knows: two per CU.  A strided fill of 528 MB runs at
+// 5.9 TB/s with 512 workgroups and at 4.3 with 2048; a workgroup per 4 KB, as where the length is known, reaches 6.8 but may
+// find most of them with nothing to do.  In a path's preparation at R-MAT scale 22: zero_tail1_kernel 165 -> 127 us,
+// mark_path_finish_kernel 164 -> 139 us.
+constexpr int kTailBlocks = 512;
 static unsigned tail_blocks(long long length)
 {
     const long long blocks = (length + 1023) / 1024;
-    return static_cast<unsigned>(blocks > 2048 ? 2048 : blocks < 1 ? 1 : blocks);
+    return static_cast<unsigned>(blocks > kTailBlocks ? kTailBlocks : blocks < 1 ? 1 : blocks);
 }
 
 static int init_scan(void* workspace, int num_tiles, hipStream_t stream)
