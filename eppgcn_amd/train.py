@@ -130,8 +130,7 @@ class Trainer:
             self.back_props.append(backInputProperty(degrees=ds.degrees, dim=width, layer=i + 1))
             self.back_props[-1].unpruned = not self.prune
         self.model = Net(ds, hidden, num_layers, weight_seed, fuse_relu).to(ds.x.device)
-        # one kernel for all weights: a dozen launches per step otherwise, a fifth of an epoch on small graphs
-        self.optimizer = torch.optim.Adam(self.model.parameters(), lr=lr, fused=ds.x.is_cuda)
+        self.optimizer = torch.optim.Adam(self.model.parameters(), lr=lr)
         self.for_time = self.loss_time = self.back_time = self.build_time = 0.0
         self.losses: List[float] = []
         self.train_idx = self.train_y = None
