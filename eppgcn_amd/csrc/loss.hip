@@ -5,7 +5,9 @@
 // reductions, the columns are read again from the vector cache instead of being kept (any number of classes).
 //   forward    one team per training row; sums per workgroup in double, added in a fixed order by a second kernel
 //   backward   one team per row of the gradient: softmax minus the label's one, times d_loss / rows, in training rows,
-//              zeros in the others - each element is written once
+//              zeros in the others - each element is written once.  The label's element is p * s - s in one fused
+//              multiply-add, as torch rounds it: (p - 1) * s rounds twice, a 2-norm error against 64 bits of 5.11e-8 instead
+//              of 4.82e-8 (5826 rows of 22 classes), which the first Adam steps, close to a sign, pass on enlarged
 // As torch operations the two were 14 launches of 2 to 5 us (log-softmax, gather, mean and negation of the selected rows;
 // backward three fills, a scatter and an index_add), most of an epoch on graphs of a few thousand vertices.  What bounds
 // them: launches for small graphs, the write of the gradient for large ones.
@@ -31,16 +33,31 @@ __device__ __forceinline__ float team_sum(float v)
     return v;
 }
 
-// maximum of a row and logarithm of the sum of its exponentials relative to that maximum
+// Logarithm as torch rounds it.  Under hipcc's default (contract = fast) logf() expands to a form with 6.3e-8 of relative
+// error (2-norm, arguments 1 to 31); without contraction, which has to be said where the builtin is called, it is 5.7e-8.
+__device__ __forceinline__ float log_uncontracted(float v)
+{
+#pragma clang fp contract(off)
+    return __builtin_logf(v);
+}
+
+// Maximum of a row and logarithm of the sum of its exponentials relative to that maximum.  The sum is the one of 64 lanes
+// with a column each (more columns: each lane its own, ascending, first), added in halves - four of them per lane of the
+// team.  That keeps the longest chain of additions at dim / 64 + 6 (one running sum per lane of the team: dim / 16 + 4, which
+// at 1000 classes gave the gradient a third more error than torch's), and up to 1024 classes it has torch's rounding.
 __device__ __forceinline__ void row_norm(const float* __restrict__ x, int dim, int tl, float* top, float* log_sum)
 {
     float m = -INFINITY;
     for (int d = tl; d < dim; d += kTeam) m = fmaxf(m, x[d]);
     m = team_max(m);
-    float s = 0.f;
-    for (int d = tl; d < dim; d += kTeam) s += expf(x[d] - m);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int d0 = tl; d0 < dim; d0 += 4 * kTeam) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (d0 + j * kTeam < dim) s[j] += expf(x[d0 + j * kTeam] - m);
+    }
     *top = m;
-    *log_sum = logf(team_sum(s));
+    *log_sum = log_uncontracted(team_sum((s[0] + s[2]) + (s[1] + s[3])));
 }
 
 __global__ __launch_bounds__(kLossBlock) void nll_rows_kernel(const float* __restrict__ logits, const long long* __restrict__ rows,
@@ -102,7 +119,7 @@ __global__ __launch_bounds__(kLossBlock) void nll_gradient_kernel(float* __restr
         if (r >= num_nodes) continue;
         float* g = grad + r * dim;
         for (int d = tl; d < dim; d += kTeam)
-            g[d] = label < 0 ? 0.f : (expf(x[d] - top - log_sum) - (d == label ? 1.f : 0.f)) * scale;
+            g[d] = label < 0 ? 0.f : fmaf(expf(x[d] - top - log_sum), scale, d == label ? -scale : 0.f);
     }
 }
 

@@ -39,6 +39,66 @@ def test_loss_and_gradient(ops, n, classes, share):
     assert not grad[~mask].any()
 
 
+def _torch_loss(x, rows, y):
+    """The loss as torch operations on the selected rows, what the kernels took the place of."""
+    logp = torch.log_softmax(x.index_select(0, rows), dim=1)
+    return -logp.gather(1, y.unsqueeze(1)).mean()
+
+
+def _error(got, want):
+    return float((got.double() - want.double()).norm() / want.double().norm())
+
+
+@pytest.mark.parametrize("n,classes,share", [(19717, 22, 0.3), (2708, 22, 0.1), (5000, 3, 0.7), (3001, 16, 0.5), (3001, 17, 0.5),
+                                             (3001, 33, 0.5), (3001, 64, 0.5), (3001, 65, 0.5), (1001, 129, 0.5), (501, 1000, 0.5)])
+def test_gradient_rounds_as_torch_does(ops, n, classes, share):
+    """The error against 64 bits is not larger than that of torch's own fp32 loss.  (Up to 1024 classes the kernel's gradient
+    had the same bits: a sum of exponentials in halves, an uncontracted logarithm, the label's element in one fused
+    multiply-add.  Without them the error was 3 to 30 % larger; the half percent is for another build of torch.)"""
+    logits, mask, y, labels = _case(n, classes, share, 3 * n + classes)
+    rows = mask.nonzero().squeeze(1)
+    x64 = logits.double().requires_grad_()
+    _torch_loss(x64, rows, y[mask]).backward()
+    x = logits.cuda().requires_grad_()
+    _torch_loss(x, rows.cuda(), y[mask].cuda()).backward()
+    grad = ops.nll_backward(torch.ones((), device="cuda"), x.detach(), labels.cuda(), rows.numel())
+    assert _error(grad.cpu(), x64.grad) <= 1.005 * _error(x.grad.cpu(), x64.grad)
+    # p has at most 2^-24 of relative error per rounding of its exponent's argument (below 32) and of its own
+    assert float((grad.cpu().double() - x64.grad).abs().max()) <= 40 * 2.0 ** -24 / rows.numel()
+
+
+@pytest.mark.parametrize("seed", range(1, 11))
+def test_deep_model_follows_the_torch_loss(ops, seed):
+    """Three epochs of a four-layer model from the same start, with the loss in torch operations and in the kernels.  Adam's
+    first steps divide a gradient by its own size, so a weight whose gradient is near zero moves by what rounding made of
+    it, and the loss must not add to that.  With execution plans for every layer the aggregations add in a fixed order and
+    two runs have the same bits, so what is left between the two is the loss: 1.2e-5 in the 2-norm and 6e-5 of the largest
+    element are what the sums of another order would be allowed."""
+    from eppgcn_amd import graphs, train
+
+    def epochs(torch_loss):
+        g = graphs.chung_lu_graph(19717, 44363, seed=seed, device="cuda")
+        mask = graphs.bernoulli_mask(g.num_nodes, 0.3, seed + 1, "cuda")
+        ds = train.GraphDataset(g, 96, 22, 4, train_mask=mask, labels="uniform", feature_seed=seed + 2, label_seed=seed + 3)
+        tr = train.Trainer(g, hidden=32, weight_seed=seed + 4, dataset=ds)
+        if torch_loss:
+            tr._loss = lambda out: _torch_loss(out, tr.train_idx, tr.train_y)
+        for epoch in range(3):
+            tr.train_step(epoch == 0, phase_timers=False)
+        return [w.detach() for w in tr.model.parameters()]
+
+    ops.set_plan_policy(1)
+    try:
+        want, again, got = epochs(True), epochs(True), epochs(False)
+    finally:
+        ops.set_plan_policy(0)
+        ops.clear_plans()
+    assert all(torch.equal(a, b) for a, b in zip(want, again)), "the comparison needs runs that repeat bit for bit"
+    for a, b in zip(got, want):
+        assert _error(a, b) <= 1.2e-5
+        assert float(((a - b).abs() / torch.maximum(b.abs(), b.square().mean().sqrt())).max()) <= 6e-5
+
+
 def test_loss_of_no_rows_infinities_and_nan(ops):
     x = torch.randn(40, 7)
     none = torch.full((40,), -1, dtype=torch.int32)
