@@ -760,10 +760,8 @@ static int vector_width(int pitch, int width, const void* p)
 // or a separate buffer of feature_workspace_floats() floats (padded pitch).
 bool stream_covers(int num_nodes, int dim, int ld_in, const float* table);                     // stream.hip
 int launch_aggregate_stream(float* out, float* partial, const float* table, const int* scol, const StreamView& sv,
-                            const StreamInfo& info, const float* scale, int num_nodes, int dim, int ld_in, bool direct,
+                            const StreamInfo& info, const float* scale, int num_nodes, int dim, int ld_in,
                             hipStream_t stream);
-bool stream_direct(int dim, const float* in, const float* out, long long num_slots, long long num_nodes,
-                   const uint32_t* gathered_rows);
 
 // The stream form of the plan is used when the host knows it (eppgcn_plan_status has read its header), the
 // rows are gathered from a separate pre-scaled workspace, the shape fits the stream kernel and the workspace has
@@ -805,17 +803,13 @@ static int aggregate_stream_call(float* out, const float* in, const int* scol, c
             if (int rc = launch_zero_words(out, static_cast<size_t>(num_nodes) * dim, stream)) return rc;
         }
     }
-    float* partial = workspace + static_cast<size_t>(swizzle_padded_rows(num_nodes)) * ld;
-    if (in && stream_direct(dim, in, out, info.num_slots, num_nodes, gathered_rows)) {
-        KernelTimer timer(stream, sink, sink2);
-        return launch_aggregate_stream(out, partial, in, scol, sv, info, scale, num_nodes, dim, dim, true, stream);
-    }
     if (in) {
         KernelTimer timer(stream, phase_sink(1));
         if (int rc = launch_scale_rows(workspace, in, scale, gathered_rows, num_nodes, dim, ld, kRowSwizzleMask, stream)) return rc;
     }
     KernelTimer timer(stream, sink, sink2);
-    return launch_aggregate_stream(out, partial, workspace, scol, sv, info, scale, num_nodes, dim, ld, false, stream);
+    return launch_aggregate_stream(out, workspace + static_cast<size_t>(swizzle_padded_rows(num_nodes)) * ld, workspace, scol, sv, info, scale,
+                                   num_nodes, dim, ld, stream);
 }
 
 template <class Groups>

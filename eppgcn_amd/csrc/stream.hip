@@ -39,7 +39,6 @@ constexpr int kStreamWaves = kStreamBlock / kWave;
 constexpr int kStreamShiftTeams = 8;   // teams up to this size address rows with a shift (power-of-two row pitch)
 constexpr int kStreamEvents = kStreamWave;       // pieces that can end in a wave's slots
 constexpr unsigned kNoRowOffset = 0xffffffffu;
-constexpr int kStreamDirectWidth = 64;           // narrowest rows gathered from the caller's matrix
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -85,7 +84,6 @@ __device__ __forceinline__ void store_row_floats(float* p, const float (&v)[4], 
 template <int U> struct StreamBatch {
     u32x4 v[U];
     unsigned c[U];
-    float f[U];        // kDirect: scale of the slot's vertex
 };
 
 // Is the header in memory the one the host remembers for this plan address?  (num_events < 0: not compared)
@@ -105,14 +103,10 @@ __device__ __forceinline__ void report_mismatch(int* __restrict__ fault, int whi
     __hip_atomic_store(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// kDirect: the rows are gathered from the caller's matrix itself (vertex order, pitch = width) and each is multiplied by
-// its vertex's scale on the way into the sum (one fused multiply-add per element, so a product is not rounded before it is
-// added), instead of from a table that a separate pass scaled.  A lane fetches the scales of its own 8 slots, and they are
-// handed out with the ids.  stream_direct() says when.
 // kWide: the table is addressed with 64-bit global loads instead of 32-bit offsets into a buffer resource (tables of
 // 4 GB and more, wide rows of 2^24 vertices and more); the lanes a buffer load would have sent out of range load row 0
 // instead and their values are replaced by zeros when they are added.
-template <int MODE, int TS, int U, bool kWide, bool kDirect>
+template <int MODE, int TS, int U, bool kWide>
 __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     float* __restrict__ out, float* __restrict__ partial, const float* __restrict__ table,
     const int* __restrict__ scol, const int* __restrict__ erow, const int* __restrict__ cev,
@@ -167,14 +161,6 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     const u32x4 id_lo = __builtin_nontemporal_load(idp);
     const u32x4 id_hi = __builtin_nontemporal_load(idp + 1);
     const unsigned ids[8] = {id_lo.x, id_lo.y, id_lo.z, id_lo.w, id_hi.x, id_hi.y, id_hi.z, id_hi.w};
-    float factor[8];
-    if constexpr (kDirect) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const unsigned id = ids[u] & 0x7fffffffu;
-            factor[u] = id < static_cast<unsigned>(num_nodes) ? scale[id] : 0.f;      // the padding gathers nothing
-        }
-    }
     const int c0 = w * (kStreamWave / 32);
     const int ce_team = cev[c0 + team * kCevPerTeam];
     const int ce_first = cev[c0];
@@ -186,23 +172,15 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     const unsigned lane_off = tl < chunks ? static_cast<unsigned>(tl) * 16u : kNoRowOffset;
     const unsigned row_step = static_cast<unsigned>(__builtin_ctz(ld_bytes));       // wave-uniform
 
-    // a separate table has its own row order (common.hpp), the caller's matrix is in vertex order
-    auto row_at = [](unsigned c) {
-        const unsigned id = c & 0x7fffffffu;
-        return kDirect ? id : swizzled_row(id);
-    };
     // batch (s, part): the ids come from lane s of the team, registers part * U ...
     auto issue = [&](StreamBatch<U>& b, int s, auto part) {
         constexpr int kPart = decltype(part)::value;
         const int src = team * TS + s;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            b.c[u] = static_cast<unsigned>(__shfl(static_cast<int>(ids[kPart * U + u]), src, kWave));
-            if constexpr (kDirect) b.f[u] = __shfl(factor[kPart * U + u], src, kWave);
-        }
+        for (int u = 0; u < U; ++u) b.c[u] = static_cast<unsigned>(__shfl(static_cast<int>(ids[kPart * U + u]), src, kWave));
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const unsigned id = row_at(b.c[u]);
+            const unsigned id = swizzled_row(b.c[u] & 0x7fffffffu);      // the table's row order (common.hpp)
             // rows of a narrow team are a power of two bytes apart (row_step = log2): a shift serves any row count
             // of a table below 4 GB; wider rows use the 24-bit multiply (the host checks the row count)
             if constexpr (kWide) {
@@ -266,20 +244,13 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
         for (int u = 0; u < U; ++u) {
             u32x4 v = b.v[u];
             if constexpr (kWide) {          // what a buffer load would have returned as zeros
-                const bool ok = lane_off != kNoRowOffset && row_at(b.c[u]) < pad_row;
+                const bool ok = lane_off != kNoRowOffset && swizzled_row(b.c[u] & 0x7fffffffu) < pad_row;
                 if (!ok) v = u32x4{0u, 0u, 0u, 0u};
             }
-            if constexpr (kDirect) {
-                acc[0] = fmaf(b.f[u], __uint_as_float(v.x), acc[0]);
-                acc[1] = fmaf(b.f[u], __uint_as_float(v.y), acc[1]);
-                acc[2] = fmaf(b.f[u], __uint_as_float(v.z), acc[2]);
-                acc[3] = fmaf(b.f[u], __uint_as_float(v.w), acc[3]);
-            } else {
-                acc[0] += __uint_as_float(v.x);
-                acc[1] += __uint_as_float(v.y);
-                acc[2] += __uint_as_float(v.z);
-                acc[3] += __uint_as_float(v.w);
-            }
+            acc[0] += __uint_as_float(v.x);
+            acc[1] += __uint_as_float(v.y);
+            acc[2] += __uint_as_float(v.z);
+            acc[3] += __uint_as_float(v.w);
             if (static_cast<int>(b.c[u]) < 0) {            // the slot ends a piece
                 if (head_pending) {
 #pragma unroll
@@ -491,41 +462,18 @@ bool stream_covers(int num_nodes, int dim, int ld_in, const float* table)
     return swizzle_padded_rows(num_nodes) < (1ll << 31);
 }
 
-// Can (and should) the rows be gathered from the caller's matrix?  It saves the pass that writes the scaled table (8 bytes
-// per element of the matrix) and costs a scale per slot and the spread of the table's row order over the memory channels.
-// R-MAT scale 20, 8.4 slots per row: 64 floats, kernel 148 -> 181 us and no pass of 82 us; 256 floats, kernel 968 -> 1176
-// us and no pass of 400 us.  The gain goes with the rows and the cost with the slots, so it is even at 11 (64 floats) to 17
-// slots per row.  A path with few gathered rows (its bitmap is given) scales only those: 5 us, the table stays.  Rows below
-// 64 floats would read more scales than they save.
-constexpr int kStreamDirectSlots = 10;
-bool stream_direct(int dim, const float* in, const float* out, long long num_slots, long long num_nodes,
-                   const uint32_t* gathered_rows)
-{
-    const uintptr_t a = reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out);
-    const uintptr_t bytes = static_cast<uintptr_t>(num_nodes) * dim * 4;
-    // a call may write over its own input: the table is a copy of it
-    if (reinterpret_cast<uintptr_t>(in) < reinterpret_cast<uintptr_t>(out) + bytes &&
-        reinterpret_cast<uintptr_t>(out) < reinterpret_cast<uintptr_t>(in) + bytes)
-        return false;
-    return dim >= kStreamDirectWidth && dim <= 256 && dim % 4 == 0 && a % 16 == 0 && !gathered_rows &&
-           num_slots <= kStreamDirectSlots * num_nodes;
-}
-
-// Stream kernel + fix-up kernel over a pre-scaled table in swizzled row order (stream_covers() holds) or, `direct`, over
-// the caller's matrix of pitch ld_in = dim (stream_direct() holds).  `partial` holds
+// Stream kernel + fix-up kernel over a pre-scaled table in swizzled row order (stream_covers() holds).  `partial` holds
 // info.header.num_partials rows of ld_in floats.  Rows without slots are not written (the caller clears them).
 int launch_aggregate_stream(float* out, float* partial, const float* table, const int* scol, const StreamView& sv,
-                            const StreamInfo& info, const float* scale, int num_nodes, int dim, int ld_in, bool direct,
+                            const StreamInfo& info, const float* scale, int num_nodes, int dim, int ld_in,
                             hipStream_t stream)
 {
     const int chunks = (dim + 3) / 4;
     const int ts = stream_team(chunks);
     const long long padded = stream_padded_slots(info.num_slots);
     const bool wide = stream_needs_wide(num_nodes, dim, ld_in) || g_force_wide_stream.load();
-    // rows that may be read: a separate table holds whole blocks, the caller's matrix its vertices
-    const long long table_rows = direct ? num_nodes : swizzle_padded_rows(num_nodes);
-    const unsigned long long bytes = wide ? 0ull : static_cast<unsigned long long>(table_rows) * ld_in * 4ull;
-    const unsigned pad_row = static_cast<unsigned>(table_rows);
+    const unsigned long long bytes = wide ? 0ull : static_cast<unsigned long long>(swizzle_padded_rows(num_nodes)) * ld_in * 4ull;
+    const unsigned pad_row = static_cast<unsigned>(swizzle_padded_rows(num_nodes));
     const int num_wave_chunks = static_cast<int>(padded / kStreamWave);
     if (num_wave_chunks == 0) return kOk;
     const dim3 grid((num_wave_chunks + kStreamWaves - 1) / kStreamWaves), block(kStreamBlock);
@@ -537,20 +485,16 @@ int launch_aggregate_stream(float* out, float* partial, const float* table, cons
     const dim3 fgrid(static_cast<unsigned>(fix_blocks < 1 ? 1 : fix_blocks));
     int* fault = nullptr;
     if (int rc = plan_fault_address(&fault)) return rc;
-#define EPPGCN_STREAM_KERNEL(MODE_, TS_, WIDE_, DIRECT_)                                                               \
-    hipLaunchKernelGGL((aggregate_stream_kernel<MODE_, TS_, 8, WIDE_, DIRECT_>), grid, block, 0, stream, out, partial, table,   \
+#define EPPGCN_STREAM_KERNEL(MODE_, TS_, WIDE_)                                                                        \
+    hipLaunchKernelGGL((aggregate_stream_kernel<MODE_, TS_, 8, WIDE_>), grid, block, 0, stream, out, partial, table,   \
                        scol, sv.erow, sv.cev, sv.wtail, scale, sv.header, fault, info.header.generation,              \
                        num_wave_chunks, info.header.num_events,                                                       \
                        num_nodes, info.header.num_partials, chunks, static_cast<unsigned>(ld_in) * 4u, dim, dim,      \
                        static_cast<unsigned>(bytes), pad_row)
 #define EPPGCN_STREAM(MODE_, TS_)                                                                                      \
     do {                                                                                                              \
-        constexpr bool kCanDirect = MODE_ != kStorePlain && TS_ * 4 >= kStreamDirectWidth;                             \
-        if (kCanDirect && direct) {                                                                                    \
-            if (wide) EPPGCN_STREAM_KERNEL(MODE_, TS_, true, kCanDirect);                                              \
-            else EPPGCN_STREAM_KERNEL(MODE_, TS_, false, kCanDirect);                                                  \
-        } else if (wide) EPPGCN_STREAM_KERNEL(MODE_, TS_, true, false);                                                \
-        else EPPGCN_STREAM_KERNEL(MODE_, TS_, false, false);                                                           \
+        if (wide) EPPGCN_STREAM_KERNEL(MODE_, TS_, true);                                                              \
+        else EPPGCN_STREAM_KERNEL(MODE_, TS_, false);                                                                  \
         if (num_fix > 0)                                                                                              \
             hipLaunchKernelGGL((stream_fixup_kernel<MODE_, TS_>), fgrid, dim3(256), 0, stream, out, partial, sv.frow,  \
                                sv.fptr, scale, sv.header, fault, info.header.generation,                              \

@@ -521,10 +521,10 @@ def test_stream_kernel_with_64_bit_addressing_gives_the_same_bits(api, dim):
 @pytest.mark.parametrize("dim", [60, 64, 68, 124, 128, 132, 252, 256])
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("n", [4096, 5000])
-def test_rows_gathered_from_the_callers_matrix(api, dim, wide, n):
-    """Wide rows of a sparse graph need no scaled table.  n = 4096: the padding's id is the first one past the matrix.
-    Row 0 holds infinities and NaN and is no neighbour of any row: neither the padding nor idle lanes may bring it in.
-    A source or a result that is not 16-byte aligned takes the table."""
+def test_wide_rows_of_any_alignment_and_an_unread_row_of_infinities(api, dim, wide, n):
+    """Wide rows of a sparse graph, from and to buffers that are 16-byte aligned or not.  n = 4096: the padding's id is the
+    first one past the table.  Row 0 holds infinities and NaN and is no neighbour of any row: neither the padding nor idle
+    lanes may bring it in."""
     indptr, col = random_symmetric_csr(n, 3 * n, 21)
     s = scale_inv_sqrt(indptr)
     rng = np.random.default_rng(dim + n)
@@ -548,3 +548,42 @@ def test_rows_gathered_from_the_callers_matrix(api, dim, wide, n):
         out.fill_(float("nan"))
         api.spmm_forward(src, dev(col), dev(s), pp, p2n, part_size=8, out=out, plan=plan)
         assert_close(out.cpu().numpy(), want, bound, f"dim {dim}, shifts {shift_x} {shift_y}")
+
+
+@pytest.mark.parametrize("dim", [16, 60, 64, 100, 128, 256, 260])
+@pytest.mark.parametrize("planned", [False, True])
+def test_a_separate_workspace_holds_the_table_after_a_call(api, dim, planned):
+    """A call with an input leaves the scaled rows in a separate workspace, in its row order and padded with zeros; a call
+    without an input then gathers them again.  (An aggregation that gathers the caller's matrix itself would leave the
+    workspace as it was, and the second call would return what that happened to hold.)"""
+    from eppgcn_amd import graphs
+    indptr, col = random_symmetric_csr(5000, 15000, 33)         # 7 slots per row
+    n = indptr.size - 1
+    s = scale_inv_sqrt(indptr)
+    x = graphs.normal32(5, (n, dim), "cuda")
+    pp, p2n = api.build_part(8, dev(indptr), col.size)
+    src = torch.ones(n, dtype=torch.bool, device="cuda")
+    degs = torch.zeros(n, dtype=torch.int32, device="cuda")
+    ids, edge_list, valid = api.mark_compact(p2n, pp, dev(col), src, None, degs, True)
+    part_pointer, num_parts, _ = api.split_back_part(degs, col.size, 8)
+    plan = path_plan = None
+    if planned:
+        plan = api.build_plan(pp, dev(col), p2n.numel(), col.size, n, dim, part2node=p2n)
+        path_plan = api.build_plan(part_pointer, edge_list, num_parts, valid, n, dim, ids=ids)
+    rows, pitch = api.feature_workspace_rows(n, "cuda"), api.feature_workspace_pitch(dim)
+    args = (dev(col), dev(s), pp, p2n)
+    ws = api.feature_workspace(n, dim, "cuda", [plan, path_plan])
+    calls = {
+        "forward": lambda: api.spmm_forward(x, *args, part_size=8, workspace=ws, plan=plan),
+        "backward": lambda: api.spmm_forward(x, *args, part_size=8, workspace=ws, plan=plan, backward=True),
+        "pruned backward": lambda: api.ours_backward(x, ids, part_pointer, edge_list, dev(s), num_parts, 8, workspace=ws,
+                                                     plan=path_plan),
+    }
+    for name, call in calls.items():
+        ws.fill_(float("nan"))
+        first = call()
+        table = ws[:api.feature_workspace(n, dim, "cuda").numel()].view(-1, pitch)[rows]
+        assert torch.equal(table[:, :dim], dev(s)[:, None] * x) and not table[:, dim:].any(), name
+        again = api.spmm_forward(None, *args, part_size=8, workspace=ws, plan=plan, prescaled_dim=dim)
+        bound = cf.abs_sum_bound(indptr, col, s, x.cpu().numpy())
+        assert_close(again.cpu().numpy(), first.cpu().numpy(), bound, name)
