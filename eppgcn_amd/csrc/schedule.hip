@@ -434,7 +434,7 @@ __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
             const uint64_t all = excl + total;
             plan.ptr[num_parts] = static_cast<int>(all & 0x7fffffffull);
             sv.header->num_events = min(static_cast<int>(all >> 31), num_parts);
-            const int fill_tiles = (num_slots + kFillTile - 1) / kFillTile;
+            const int fill_tiles = static_cast<int>((static_cast<long long>(num_slots) + kFillTile - 1) / kFillTile);
             for (int t = static_cast<int>(((all & 0x7fffffffull) + kFillTile - 1) / kFillTile); t < fill_tiles; ++t)
                 tile_q[t] = num_parts - 1;              // slots the caller counted and no group covers
         }
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ 
     const bool closing = static_cast<int>(blockIdx.x) + 1 == num_fill_tiles;       // writes the entry behind the last slot too
     if (threadIdx.x <= kFillTile / kStreamChunk) {
         const int i = static_cast<int>(threadIdx.x) * kStreamChunk;
-        const int pos = base + i;
+        const long long pos = static_cast<long long>(base) + i;      // one tile past 2^31 - 1 for the last tile of the largest plan
         const bool mine = i < kFillTile ? pos < padded_slots || (closing && pos == padded_slots) : closing && pos == padded_slots;
         if (mine) {
             int e = sv.header->num_events;
@@ -810,7 +810,7 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
         set_error("build_plan: plan buffer smaller than eppgcn_plan_bytes(num_parts, num_slots, num_nodes)");
         return kErrInvalidArgument;
     }
-    if (num_slots >= (1ll << 31) - kFillTile) {
+    if (num_slots >= (1ll << 31) - kStreamWave) {            // the padded slots are counted in 32 bits too
         set_error("build_plan: slot count beyond 32-bit offsets");
         return kErrInvalidArgument;
     }

@@ -71,3 +71,32 @@ def test_slots_no_group_covers_gather_nothing(api):
     out = api.spmm_forward(dev(x), dev(longer), dev(ones), dev(pp), dev(p2n), part_size=16, plan=plan)
     assert api.last_call_used_stream()
     assert np.array_equal(out.cpu().numpy(), co.spmm_f64(x, indptr, col, ones).astype(np.float32))
+
+
+@pytest.mark.parametrize("num_slots", [2 ** 31 - 2049, 2 ** 31 - 1025, 2 ** 31 - 513])
+def test_the_largest_plans(api, num_slots):
+    """Up to the slot counts that 32-bit offsets hold (every count below 2^31 - 1024 is promised, the padding to whole waves
+    ends at 2^31 - 512): the last fill tile ends past 2^31 - 1.  Copied ids, padding, and the aggregation over them, whose
+    sums are whole numbers below 2^24."""
+    n, per_row = 4096, 1 << 19
+    ptr = torch.arange(n + 1, device="cuda").mul_(per_row).clamp_(max=num_slots).int()
+    col = torch.arange(num_slots, dtype=torch.int32, device="cuda").remainder_(4099).remainder_(n)
+    rows = torch.arange(n, dtype=torch.int32, device="cuda")
+    plan = api.build_plan(ptr, col, n, num_slots, n, 4, part2node=rows, block_shift=8)
+    got = plan.stream_view()
+    at, row, _, ids = plan.view(raw_col=True)
+    assert got["header"][0] == 1 and int(got["header"][4]) == 0 and int(at[n]) == num_slots
+    for q, (a, b, r) in enumerate(zip(at[:-1].tolist(), at[1:].tolist(), row.tolist())):
+        want = col[int(ptr[r]):int(ptr[r]) + b - a]
+        assert torch.equal(ids[a:b] & 0x7fffffff, want), (q, r)
+        assert int(ids[b - 1]) < 0 and not (ids[a:b - 1] < 0).any()
+    assert (got["col"][num_slots:] == n).all() and got["col"].numel() == (num_slots + 511) // 512 * 512
+    chunk = torch.arange(0, num_slots, 1 << 20, device="cuda") // 32
+    ends = torch.searchsorted((at[1:] - 1).long(), chunk * 32)
+    assert torch.equal((got["cev"][chunk] & 0x7fffffff).long(), ends)
+    x = torch.randint(-4, 5, (n, 4), device="cuda", generator=torch.Generator("cuda").manual_seed(1)).float()
+    out = api.spmm_forward(x, col, torch.ones(n, device="cuda"), ptr, rows, part_size=per_row, plan=plan)
+    assert api.last_call_used_stream()
+    for r in list(range(0, n, 97)) + [n - 2, n - 1]:
+        count = torch.bincount(col[int(ptr[r]):int(ptr[r + 1])].long(), minlength=n).double()
+        assert torch.equal(out[r].double(), count @ x.double()), r
