@@ -37,7 +37,7 @@ EXPORTS = [
     "eppgcn_mark_gathered_rows_scratch", "eppgcn_mark_gathered_rows_scratch_bytes",
 ]
 
-ABI_VERSION = 16      # what eppgcn_abi_version() of a matching library returns
+ABI_VERSION = 17      # what eppgcn_abi_version() of a matching library returns
 
 _lib = None
 

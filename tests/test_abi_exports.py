@@ -44,6 +44,21 @@ def test_library_exports_every_declared_symbol():
     assert capi.load().eppgcn_abi_version() == capi.ABI_VERSION
 
 
+def test_a_library_from_before_the_last_exports_is_refused_by_its_version(tmp_path, monkeypatch):
+    """The marking of whole paths, the split counts and the training loss came with ABI 17: a library of ABI 16 has to fail
+    the version check and not later, on the first symbol it lacks."""
+    import pytest
+    import subprocess
+    from eppgcn_amd import capi
+    old = tmp_path / "libold.so"
+    source = "int eppgcn_abi_version(void) { return 16; }\nconst char* eppgcn_last_error(void) { return \"\"; }\n"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", "-", "-o", str(old)], input=source, text=True, check=True)
+    monkeypatch.setattr(capi, "_lib", None)
+    monkeypatch.setattr(capi, "LIB_PATH", str(old))
+    with pytest.raises(capi.EppgcnError, match="ABI version 16"):
+        capi.load()
+
+
 def test_host_only_heuristics_match_the_checker():
     """These two entry points are pure host code, so they can be compared without a GPU."""
     from eppgcn_amd import capi
