@@ -473,7 +473,8 @@ def build_plan(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes
 
 def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes: int, dim: int,
                      part2node=None, ids=None, block_shift: int = 0):
-    """Issues ``build_plan``; the returned call waits for it and gives the plan."""
+    """Issues ``build_plan``; the returned call waits for it and gives the plan.  The build's workspace goes back to torch's
+    allocator at once, which hands it to later work on the same stream only: builds issued one after the other share it."""
     lib = load()
     _dev(part_ptr, torch.int32, "part_ptr"); _dev(column_index, torch.int32, "column_index")
     if (part2node is None) == (ids is None):
@@ -485,21 +486,18 @@ def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num
     nbytes = lib.eppgcn_plan_bytes(int(num_parts), int(num_slots), int(num_nodes))
     buf, base = _aligned_buffer(nbytes, part_ptr.device)
     wbytes = lib.eppgcn_plan_workspace_bytes(int(num_parts), int(num_slots))
-    ws, wbase = _aligned_buffer(wbytes, part_ptr.device)
+    ws, wbase = _aligned_buffer(wbytes, part_ptr.device)        # held until every kernel of the build is issued
     _check(lib.eppgcn_build_plan(_ptr(part_ptr), _ptr(column_index), _ptr(part2node), _ptr(ids), int(num_parts),
                                  int(num_slots), int(num_nodes), int(dim), int(block_shift), C.c_void_p(base), nbytes,
                                  C.c_void_p(wbase), wbytes, _stream()))
 
     def finish():
-        # synchronises (the workspace is released with this function), refuses a plan whose scan stalled and lets the
-        # library know the plan's stream form
+        # synchronises, refuses a plan whose scan stalled and lets the library know the plan's stream form
         partial = C.c_int64(0)
         _check(lib.eppgcn_plan_status(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes), C.byref(partial),
                                       _stream()))
-        del keep[:]
         return Plan(buf, base, int(num_parts), int(num_slots), int(num_nodes), int(partial.value))
 
-    keep = [ws]
     return finish
 
 

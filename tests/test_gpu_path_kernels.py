@@ -112,3 +112,26 @@ def test_group_split_at_the_ends_of_tiles(api, n, top, ps):
         assert (parts, slots) == (int(groups.sum()), e)
         got = got.cpu().numpy()
         assert np.array_equal(got[:parts + 1], want) and not got[parts + 1:].any()
+
+
+@pytest.mark.parametrize("layers", [2, 6])
+def test_preparing_several_layers_holds_one_build_workspace(api, layers):
+    """All plans of a run are under way before the host waits for the first one, but their builds follow one another on the
+    stream: beyond what stays, path preparation needs the workspace of the largest build and the marking of the layers (a
+    bit per slot and a little over a byte per vertex), not a build workspace per layer."""
+    from eppgcn_amd import graphs, workload
+    g = graphs.rmat_graph(17, 8, seed=3, device="cuda")
+    mask = graphs.bernoulli_mask(g.num_nodes, 0.9, 4, "cuda")
+    run = lambda: workload.prepare(g, layers, train_mask=mask, widths=(16,), plan=True, part_size=2, backsize=2)
+    run()                                            # whatever the first call loads and keeps
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    wl = run()
+    torch.cuda.synchronize()
+    over = torch.cuda.max_memory_allocated() - torch.cuda.memory_allocated()
+    lib = api.load()
+    build = max([lib.eppgcn_plan_workspace_bytes(wl.part2node.numel(), g.num_edges)] +
+                [lib.eppgcn_plan_workspace_bytes(p.num_parts, p.valid_len) for p in wl.paths])
+    marking = layers * lib.eppgcn_mark_path_workspace_bytes(g.num_edges, g.num_nodes)
+    assert over <= 1.05 * build + marking, (over, build, marking)
