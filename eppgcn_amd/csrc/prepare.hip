@@ -251,8 +251,11 @@ __global__ __launch_bounds__(kCompactBlock) void compact_mask_kernel(
 // k * kMarkWaves + wave of every 64-slot bit map is one ballot and words are in slot order.
 //   keep_slots_kernel    keep = the slot's column is in the source mask: one bit per slot and a count per tile.  Nothing but
 //                        column ids and mask entries is read, with kItems of each under way per thread.
-//   place_slots_kernel   rows and places of the kept slots.  The kept slots before a tile are the counts before its own,
-//                        added up by the tile's workgroup; the row of a slot comes from a bit map of the group starts inside
+//   scan_counts_kernel   (large tiles only) the kept slots before every tile, by one workgroup: 2^31 slots have 131 thousand
+//                        tiles, and a workgroup per tile that adds up the counts before its own reads 34 GB of them (the
+//                        whole pass 20.1 ms, with the scan 17.8; 2^30 slots 9.48 and 8.96; 2^27 1.23 either way).  The at most
+//                        8192 small tiles do add them up (0.13 GB, from L2): a launch costs more there.
+//   place_slots_kernel   rows and places of the kept slots; the row of a slot comes from a bit map of the group starts inside
 //                        the tile (prefix population count; the tile's first group was found beforehand) and the rows of
 //                        the tile's groups, staged in LDS; kept slots per row are differences of the prefix counts, one
 //                        atomic per (wave, row): a hub of 600 thousand slots costs 40 tiles a few atomics each, where one
@@ -356,6 +359,40 @@ __global__ __launch_bounds__(kMarkBlock) void keep_slots_kernel(const int* __res
     if (threadIdx.x == 0) counts[blockIdx.x] = s_total;
 }
 
+// counts[0 .. n) become their exclusive prefix sums
+__global__ __launch_bounds__(1024) void scan_counts_kernel(int* __restrict__ counts, int n)
+{
+    constexpr int kItems = 4, kWaves = 1024 / kWave;
+    __shared__ int s_wave[kWaves];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x >> 6;
+    int carry = 0;
+    for (int t0 = 0; t0 < n; t0 += 1024 * kItems) {
+        const int t = t0 + static_cast<int>(threadIdx.x) * kItems;
+        int c[kItems], sum = 0;
+#pragma unroll
+        for (int j = 0; j < kItems; ++j) {
+            c[j] = t + j < n ? counts[t + j] : 0;
+            sum += c[j];
+        }
+        const int incl = wave_inclusive_scan(sum);
+        if (lane == kWave - 1) s_wave[wave] = incl;
+        __syncthreads();
+        int run = carry + incl - sum;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            if (w < wave) run += s_wave[w];
+            carry += s_wave[w];
+        }
+#pragma unroll
+        for (int j = 0; j < kItems; ++j) {
+            if (t + j < n) counts[t + j] = run;
+            run += c[j];
+        }
+        __syncthreads();
+    }
+}
+
 template <int kItems, bool kBits>
 __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
@@ -368,6 +405,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     constexpr int kWords = kTile / 64;
     constexpr int kPerLane = kWords / kWave;
     static_assert(kWords % kWave == 0 && kItems <= kWave, "one wave scans the words; a wave's words fit its lanes");
+    constexpr bool kScanned = kItems == kMarkItemsLarge;       // counts[] holds the kept slots before every tile
     __shared__ int s_prefix;
     __shared__ int s_starts_in_tile;
     __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
@@ -387,14 +425,19 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
         s_starts[threadIdx.x] = 0ull;
         s_kept[threadIdx.x] = kept[static_cast<long long>(tile) * kWords + threadIdx.x];
     }
-    if (threadIdx.x == 0) s_starts_in_tile = s_prefix = 0;
+    if (threadIdx.x == 0) {
+        s_starts_in_tile = 0;
+        s_prefix = kScanned ? counts[tile] : 0;
+    }
     __syncthreads();
     {
-        int sum = 0;
-        for (int t = threadIdx.x; t < tile; t += kMarkBlock) sum += counts[t];
+        if constexpr (!kScanned) {
+            int sum = 0;
+            for (int t = threadIdx.x; t < tile; t += kMarkBlock) sum += counts[t];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
-        if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
+            for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+            if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
+        }
         int mine = 0;
         for (int i0 = threadIdx.x; i0 < g_cnt; i0 += kMarkBlock * kMarkBatch) {
             int start[kMarkBatch], row[kMarkBatch];
@@ -1110,6 +1153,9 @@ static int launch_mark_pass(const int* part2node, const int* part_ptr, const int
     do {                                                                                                                \
         hipLaunchKernelGGL((keep_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part_ptr, col, src, num_parts, len, \
                            kept, counts);                                                                                 \
+        EPPGCN_HIP(hipGetLastError());                                                                                    \
+        if (ITEMS_ == kMarkItemsLarge)                                                                                    \
+            hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, stream, counts, l.num_tiles);                  \
         EPPGCN_HIP(hipGetLastError());                                                                                    \
         hipLaunchKernelGGL((place_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part2node, part_ptr, col, src,     \
                            ngh_mask, node_degs, out_id, out_edge, self_kept, len, l.num_tiles, is_last, first, kept,       \

@@ -49,12 +49,24 @@ def test_count_of_rows_with_kept_edges(api, n):
     (700, 0, True, 3),                                              # nothing but self-loops
     (3000, 11, True, 8), (3001, 11, False, 64),                     # several small tiles, with and without self-loops
     (9, 3000, True, 32),                                            # rows of several tiles
-    (300000, 15, True, 16), (9, 600000, False, 32),                 # large tiles
-    (4300000, 0, True, 1)])                                         # more groups in a large tile than are staged
+    (300000, 15, True, 16), (9, 600000, False, 32),                 # a thousand tiles
+    (4300000, 0, True, 1)])                                         # as many groups in a tile as slots
 @pytest.mark.parametrize("is_last", [False, True])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shift):
-    """`shift`: the masks start one byte past a word boundary.  Vertex 0 is a neighbour of every third slot."""
+    _check_marking(api, n, slots_per_row, loops, ps, is_last, shift)
+
+
+@pytest.mark.parametrize("n,slots_per_row,loops,ps", [
+    (2300000, 15, True, 16), (9, 6000000, False, 32),               # two and three thousand large tiles (from 2^25 slots on)
+    (34000000, 0, True, 1)])                                        # more groups in a large tile than are staged
+@pytest.mark.parametrize("is_last", [False, True])
+def test_path_marking_in_large_tiles(api, n, slots_per_row, loops, ps, is_last):
+    assert _check_marking(api, n, slots_per_row, loops, ps, is_last, 1) >= 1 << 25
+
+
+def _check_marking(api, n, slots_per_row, loops, ps, is_last, shift):
+    """`shift`: the masks start one byte past a word boundary.  Vertex 0 is a neighbour of every third slot.  -> slots"""
     rng = np.random.default_rng(n + slots_per_row)
     deg = rng.integers(0, 2 * slots_per_row + 1, n) + (1 if loops else 0)
     indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
@@ -89,6 +101,7 @@ def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shi
     assert np.array_equal(degs.cpu().numpy(), degs_want)
     assert np.array_equal(ngh.cpu().numpy(), want_ngh)
     assert np.array_equal(bitmap.cpu().numpy(), np.packbits(gathered, bitorder="little").view(np.int32))
+    return e
 
 
 @pytest.mark.parametrize("n,top,ps", [(1, 3, 2), (1023, 9, 4), (2048, 7, 1), (2049, 7, 1), (4097, 40, 8), (5000, 0, 3),
