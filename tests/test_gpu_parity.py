@@ -831,18 +831,38 @@ def test_mark_compact_equals_marking_then_compaction(api, name, ratio, ps):
             assert np.array_equal(ngh.cpu().numpy(), want_ngh)
 
 
-def test_fused_and_stepwise_path_preparation_agree_at_scale(api):
-    """R-MAT scale 20: the whole mask chain and both layers' backward paths, fused versus the
-    reference's separate steps, bit for bit."""
+@pytest.mark.parametrize("ratio", [0.002, 0.1])
+def test_fused_and_stepwise_path_preparation_agree_at_scale(api, ratio):
+    """R-MAT scale 20: the whole mask chain and both layers' backward paths as ``workload.prepare`` makes them (one pass
+    per layer) against the reference's separate steps - marking into edge masks, compaction, counting, group split, the rows
+    a path gathers - bit for bit.  With the small mask both paths gather from less than half of the vertices."""
     from eppgcn_amd import graphs, workload
     g = graphs.make_graph("cfg3_rmat20", device="cuda")
-    a = workload.prepare(g, 2, 0.1, 2, fused=True, plan=False)
-    b = workload.prepare(g, 2, 0.1, 2, fused=False, plan=False)
-    assert torch.equal(a.ngh_masks[0], b.ngh_masks[0])
-    for pa, pb in zip(a.paths, b.paths):
-        assert (pa.valid_len, pa.num_parts, pa.valid_node) == (pb.valid_len, pb.num_parts, pb.valid_node)
-        assert torch.equal(pa.ids, pb.ids) and torch.equal(pa.edge_list, pb.edge_list)
-        assert torch.equal(pa.part_pointer, pb.part_pointer) and torch.equal(pa.node_degs, pb.node_degs)
+    n, e, layers = g.num_nodes, g.num_edges, 2
+    a = workload.prepare(g, layers, ratio, 2, plan=False)
+    ngh = [torch.zeros(n, dtype=torch.bool, device="cuda") for _ in range(layers - 1)]
+    masks = [torch.full((e,), -1, dtype=torch.int32, device="cuda") for _ in range(layers)]
+    degs = [torch.zeros(n, dtype=torch.int32, device="cuda") for _ in range(layers)]
+    for i in range(layers):
+        last, k = i == layers - 1, layers - 1 - i
+        api.mask_forward(a.part2node, a.part_ptr, g.column_index, a.train_mask if i == 0 else ngh[i - 1],
+                         None if last else ngh[i], masks[k], degs[k], last)
+    assert all(torch.equal(x, y) for x, y in zip(a.ngh_masks, ngh))
+    few = []
+    for k, path in enumerate(a.paths):
+        ids, edge_list, valid = api.compact_back_edge(masks[k], g.column_index)
+        part_pointer, parts, covered = api.split_back_part(degs[k], e, path.part_size)
+        bitmap, distinct = api.mark_gathered_rows(edge_list, valid, n)
+        assert (path.valid_len, path.num_parts, path.valid_node) == (valid, parts, api.count_nonzero(degs[k])) and covered == valid
+        assert torch.equal(path.ids, ids) and torch.equal(path.edge_list, edge_list)
+        assert torch.equal(path.part_pointer, part_pointer) and torch.equal(path.node_degs, degs[k])
+        few.append(2 * distinct < n)
+        assert torch.equal(path.gathered_rows, bitmap) if few[-1] else path.gathered_rows is None
+        src = a.train_mask if k == layers - 1 else ngh[layers - 2 - k]
+        again = torch.zeros(n, dtype=torch.int32, device="cuda")
+        marked = api.mark_path(a.part2node, a.part_ptr, g.column_index, src, torch.zeros_like(src), again, k == 0)
+        assert marked[2:4] == (valid, path.valid_node) and marked[5] == distinct and torch.equal(marked[4], bitmap)
+    assert any(few)
 
 
 # ----------------------------------------------------------------------------- HIP graph capture

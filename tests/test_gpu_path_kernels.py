@@ -101,6 +101,11 @@ def _check_marking(api, n, slots_per_row, loops, ps, is_last, shift):
     assert np.array_equal(degs.cpu().numpy(), degs_want)
     assert np.array_equal(ngh.cpu().numpy(), want_ngh)
     assert np.array_equal(bitmap.cpu().numpy(), np.packbits(gathered, bitorder="little").view(np.int32))
+    # the entry point without the path's counts (it reads the mask byte by byte)
+    again, ngh2 = torch.zeros_like(degs), torch.zeros_like(ngh)
+    ids2, edges2, kept2 = api.mark_compact(p2n, pp, torch.from_numpy(col).cuda(), d_src, None if is_last else ngh2, again, is_last)
+    assert kept2 == v and torch.equal(ids2, ids) and torch.equal(edges2, edges)
+    assert torch.equal(again, degs) and torch.equal(ngh2, ngh)
     return e
 
 
