@@ -154,21 +154,26 @@ class Trainer:
             self.kept_edges[i] = valid_len
             ds.edge_masks[i] = None      # the marking buffer is not needed after compaction
 
-    def _select_training_rows(self):
-        """The training rows and their labels, worked out once (EPPGCN/gcn_main.py:252-253 selects them with the boolean
-        mask, a device-to-host round trip per epoch)."""
+    def _select_training_rows(self, classes):
+        """The training rows and their labels (`classes`: columns of the model's output), worked out once
+        (EPPGCN/gcn_main.py:252-253 selects them with the boolean mask, a device-to-host round trip per epoch)."""
         ds = self.dataset
         self.train_idx = ds.train_mask.nonzero().squeeze(1)
         self.train_y = ds.y[self.train_idx]
         if self.train_y.numel():
             lo, hi = torch.stack(torch.aminmax(self.train_y)).tolist()
-            if not 0 <= lo <= hi < ds.num_classes:
-                raise ValueError("a label of the training rows lies outside the %d classes" % ds.num_classes)
+            if not 0 <= lo <= hi < classes:
+                raise ValueError("a label of the training rows lies outside the %d classes" % classes)
         self.row_labels = torch.where(ds.train_mask.bool(), ds.y, -1).int()
 
     def _loss(self, out):
-        """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax, EPPGCN/gcn_main.py:252-253)."""
-        return _TrainingLoss.apply(out, self.train_idx, self.row_labels)
+        """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax, EPPGCN/gcn_main.py:252-253): in
+        the library's kernels for what ``Net`` returns, in torch operations for a model of the caller's whose output is of
+        another type, layout or row count."""
+        if out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous() and out.shape[0] == self.row_labels.numel():
+            return _TrainingLoss.apply(out, self.train_idx, self.row_labels)
+        logp = F.log_softmax(out.index_select(0, self.train_idx), dim=1)
+        return -logp.gather(1, self.train_y.unsqueeze(1)).mean()
 
     def train_step(self, is_first_iter: bool, record_loss: bool = False, phase_timers: bool = True):
         """One epoch.  ``phase_timers`` keeps the reference's three host synchronisations per epoch
@@ -189,7 +194,7 @@ class Trainer:
             self.build_time += time.perf_counter() - t
         t = time.perf_counter()
         if self.train_idx is None:
-            self._select_training_rows()
+            self._select_training_rows(out.shape[1])
         loss = self._loss(out)
         sync()
         self.loss_time += time.perf_counter() - t

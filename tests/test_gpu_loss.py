@@ -121,3 +121,45 @@ def test_trainer_refuses_labels_outside_the_classes():
     ds.y[ds.train_mask.nonzero()[0]] = 4
     with pytest.raises(ValueError, match="outside the 4 classes"):
         train.Trainer(g, hidden=8, dataset=ds).train_step(True)
+
+
+@pytest.mark.parametrize("change", ["double", "bfloat16", "transposed", "more rows", "more classes"])
+def test_trainer_takes_what_a_model_of_the_callers_returns(change):
+    """A model in the place of ``Net`` may return any type, layout and number of rows and columns that the torch loss takes;
+    the gradients are those of the same loss on the same values."""
+    from eppgcn_amd import graphs, train
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, net):
+            super().__init__()
+            self.net = net
+
+        def forward(self, *args):
+            out = self.net(*args)
+            if change == "transposed":
+                return torch.stack([out, out], 2)[:, :, 0]
+            if change == "more rows":
+                return torch.cat([out, out])
+            if change == "more classes":
+                return torch.cat([out, out], 1)
+            return out.to(getattr(torch, change))
+
+    def step(wrap, torch_loss):
+        g = graphs.uniform_graph(300, 600, seed=1, device="cuda")
+        ds = train.GraphDataset(g, 8, 4, 2, train_ratio=0.5, labels="uniform")
+        if change == "more classes":
+            ds.y[ds.train_mask.nonzero()[0]] = 6
+        tr = train.Trainer(g, hidden=8, dataset=ds)
+        if wrap:
+            tr.model = Wrapped(tr.model)
+        if torch_loss:
+            tr._loss = lambda out: _torch_loss(out, tr.train_idx, tr.train_y)
+        loss = tr.train_step(True)
+        return loss.detach().double(), [w.grad.double() for w in tr.model.parameters()]
+
+    got, want = step(True, False), step(True, True)
+    # the same operations but for the order of the aggregation's sums; bfloat16 rounds what they leave to 2^-9
+    rtol = 2.0 ** -6 if change == "bfloat16" else 1e-5
+    assert torch.allclose(got[0], want[0], rtol=rtol)
+    for a, b in zip(got[1], want[1]):
+        assert float((a - b).norm() / b.norm()) <= rtol
