@@ -133,8 +133,7 @@ class Trainer:
         self.optimizer = torch.optim.Adam(self.model.parameters(), lr=lr)
         self.for_time = self.loss_time = self.back_time = self.build_time = 0.0
         self.losses: List[float] = []
-        self.train_idx = self.train_y = None
-        self.row_labels = None                     # int32 class of every training row, -1 for the other rows
+        self.train_idx = self.train_y = None       # set by the first epoch, or by the caller
         self.kept_edges = [None] * num_layers      # per conv layer, filled by build_back_part
 
     def build_back_part(self):
@@ -154,6 +153,24 @@ class Trainer:
             self.kept_edges[i] = valid_len
             ds.edge_masks[i] = None      # the marking buffer is not needed after compaction
 
+    # Training rows and their labels.  The loss kernels read them from row_labels (int32 class of every training row, -1 for
+    # the other rows), made by _select_training_rows; rows or labels that the caller sets drop it.
+    @property
+    def train_idx(self):
+        return self._train_idx
+
+    @train_idx.setter
+    def train_idx(self, rows):
+        self._train_idx, self.row_labels = rows, None
+
+    @property
+    def train_y(self):
+        return self._train_y
+
+    @train_y.setter
+    def train_y(self, labels):
+        self._train_y, self.row_labels = labels, None
+
     def _select_training_rows(self, classes):
         """The training rows and their labels (`classes`: columns of the model's output), worked out once
         (EPPGCN/gcn_main.py:252-253 selects them with the boolean mask, a device-to-host round trip per epoch)."""
@@ -165,12 +182,15 @@ class Trainer:
             if not 0 <= lo <= hi < classes:
                 raise ValueError("a label of the training rows lies outside the %d classes" % classes)
         self.row_labels = torch.where(ds.train_mask.bool(), ds.y, -1).int()
+        self._row_versions = (self.train_idx._version, self.train_y._version)
 
     def _loss(self, out):
         """Mean negative log-likelihood of the training rows (F.nll_loss of F.log_softmax, EPPGCN/gcn_main.py:252-253): in
         the library's kernels for what ``Net`` returns, in torch operations for a model of the caller's whose output is of
-        another type, layout or row count."""
-        if out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous() and out.shape[0] == self.row_labels.numel():
+        another type, layout or row count, and for rows or labels that the caller has set or changed."""
+        selected = self.row_labels is not None and self._row_versions == (self.train_idx._version, self.train_y._version)
+        if (selected and out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous()
+                and out.shape[0] == self.row_labels.numel()):
             return _TrainingLoss.apply(out, self.train_idx, self.row_labels)
         logp = F.log_softmax(out.index_select(0, self.train_idx), dim=1)
         return -logp.gather(1, self.train_y.unsqueeze(1)).mean()

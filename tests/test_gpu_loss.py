@@ -163,3 +163,31 @@ def test_trainer_takes_what_a_model_of_the_callers_returns(change):
     assert torch.allclose(got[0], want[0], rtol=rtol)
     for a, b in zip(got[1], want[1]):
         assert float((a - b).norm() / b.norm()) <= rtol
+
+
+@pytest.mark.parametrize("when", ["before", "after", "in place"])
+def test_trainer_takes_the_callers_training_rows(when):
+    """Rows and labels that the caller sets - some rows twice - are what the loss is taken over, whenever they are set."""
+    from eppgcn_amd import graphs, train
+    g = graphs.uniform_graph(300, 600, seed=1, device="cuda")
+    gen = torch.Generator().manual_seed(2)
+    rows, labels = torch.randint(0, 300, (90,), generator=gen).cuda(), torch.randint(0, 4, (90,), generator=gen).cuda()
+
+    def step(torch_loss):
+        ds = train.GraphDataset(g, 8, 4, 2, train_ratio=0.5, labels="uniform")
+        tr = train.Trainer(g, hidden=8, dataset=ds)
+        if torch_loss:
+            tr._loss = lambda out: _torch_loss(out, tr.train_idx, tr.train_y)
+        if when != "before":
+            tr.train_step(True)
+        if when == "in place":
+            tr.train_y[::2] = 3 - tr.train_y[::2]
+        else:
+            tr.train_idx, tr.train_y = rows, labels
+        loss = tr.train_step(when == "before")
+        return loss.detach(), [w.grad for w in tr.model.parameters()]
+
+    got, want = step(False), step(True)
+    assert torch.allclose(got[0], want[0], rtol=1e-5)
+    for a, b in zip(got[1], want[1]):
+        assert _error(a, b) <= 1e-5
