@@ -191,3 +191,72 @@ def test_trainer_takes_the_callers_training_rows(when):
     assert torch.allclose(got[0], want[0], rtol=1e-5)
     for a, b in zip(got[1], want[1]):
         assert _error(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("n,classes,share", [
+    (65537, 22, 0.3), (262147, 20, 0.02), (600001, 17, 0.5), (600001, 22, 1.1),      # stretches of 8 to 64 rows, teams of 16
+    (300007, 1, 0.5), (300007, 4, 0.5), (1100003, 16, 0.1), (1100003, 2, 1.1),       # teams of 4
+    (20011, 65, 0.5), (70003, 256, 0.3), (33003, 257, 0.9), (40009, 1025, 0.05), (530017, 70, 0.01)])     # whole waves
+@pytest.mark.parametrize("shift", [0, 1])
+def test_loss_of_many_rows(n, classes, share, shift):
+    """Every team size, registers held and not, with more rows than a step of the waves takes; `shift`: logits and gradient
+    start 4 bytes past a 16-byte boundary.  Against torch's fp32 loss, whose rounding the gradient has (the half percent is
+    for another build of torch), and the mean against 64 bits."""
+    from eppgcn_amd import capi
+    lib = capi.load()
+    gen = torch.Generator("cuda").manual_seed(n + classes)
+    hold_x, hold_g = (torch.full((n * classes + 8,), 7.0, device="cuda") for _ in range(2))
+    x, grad = (h[shift:shift + n * classes].view(n, classes) for h in (hold_x, hold_g))
+    x.copy_(torch.randn(n, classes, device="cuda", generator=gen) * 3)
+    mask = torch.rand(n, device="cuda", generator=gen) < share
+    y = torch.randint(0, classes, (n,), device="cuda", generator=gen)
+    rows, labels = mask.nonzero().squeeze(1), torch.where(mask, y, -1).int()
+    leaf = x.clone().requires_grad_()
+    _torch_loss(leaf, rows, y[rows]).backward()
+    x64 = x.double().requires_grad_()
+    want = _torch_loss(x64, rows, y[rows])
+    want.backward()
+    loss, one = torch.empty((), device="cuda"), torch.ones((), device="cuda")
+    ws = torch.empty(lib.eppgcn_nll_workspace_bytes() // 8, dtype=torch.float64, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.eppgcn_nll_forward(loss.data_ptr(), x.data_ptr(), rows.data_ptr(), labels.data_ptr(), rows.numel(), n, classes,
+                                  ws.data_ptr(), 8 * ws.numel(), stream) == 0
+    assert lib.eppgcn_nll_backward(grad.data_ptr(), one.data_ptr(), x.data_ptr(), labels.data_ptr(), rows.numel(), n, classes,
+                                   stream) == 0
+    assert abs(float(loss) - float(want)) <= 1e-6 * abs(float(want)) + 1e-7          # terms rounded to fp32, summed in 64 bits
+    assert float((grad - x64.grad).norm()) <= 1.005 * float((leaf.grad - x64.grad).norm())
+    assert not grad[~mask].any()
+    assert (hold_g[:shift] == 7).all() and (hold_g[shift + n * classes:] == 7).all()
+
+
+@pytest.mark.parametrize("n,classes,share", [(1 << 22, 22, 0.1), (1 << 22, 2, 0.1), (1 << 20, 172, 0.01), (1 << 18, 1000, 0.1)])
+def test_loss_of_large_graphs_is_not_slower_than_in_torch(ops, n, classes, share):
+    """The kernels took the place of torch's for their launches on small graphs; where the rows are many the work counts.
+    (A third to nine tenths of torch's time; teams that waited for one row after another took 1.7 to 2 times torch's.)"""
+    x = torch.randn(n, classes, device="cuda")
+    mask = torch.rand(n, device="cuda") < share
+    y = torch.randint(0, classes, (n,), device="cuda")
+    rows, labels, one = mask.nonzero().squeeze(1), torch.where(mask, y, -1).int(), torch.ones((), device="cuda")
+    leaf, y_rows = x.clone().requires_grad_(), y[rows]
+
+    def in_torch():
+        leaf.grad = None
+        _torch_loss(leaf, rows, y_rows).backward()
+
+    def in_kernels():
+        ops.nll_forward(x, rows, labels)
+        ops.nll_backward(one, x, labels, rows.numel())
+
+    def best(f):
+        times = []
+        for _ in range(6):
+            ends = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            ends[0].record()
+            for _ in range(5):
+                f()
+            ends[1].record()
+            torch.cuda.synchronize()
+            times.append(ends[0].elapsed_time(ends[1]))
+        return min(times[1:])
+
+    assert best(in_kernels) <= 1.25 * best(in_torch)
