@@ -1007,7 +1007,6 @@ size_t scan_workspace_bytes(long long length, int tile)
 size_t compact_workspace_bytes(long long length) { return scan_workspace_bytes(length, kCompactTile); }
 size_t split_workspace_bytes(long long num_nodes) { return scan_workspace_bytes(num_nodes, kSplitTile); }
 
-// workgroups that write the zeros behind `length` words at most, four words per thread and step
 // Workgroups that clear what lies behind a length that only the device knows: two per CU.  A strided fill of 528 MB runs at
 // 5.9 TB/s with 512 workgroups and at 4.3 with 2048; a workgroup per 4 KB, as where the length is known, reaches 6.8 but may
 // find most of them with nothing to do.  In a path's preparation at R-MAT scale 22: zero_tail1_kernel 165 -> 127 us,

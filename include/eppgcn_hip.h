@@ -42,7 +42,8 @@
  *     degrees[r]*in[r,:] in that row order at a pitch of eppgcn_feature_workspace_pitch(dim) floats
  *     with zeros in the padding (eppgcn_update_forward_table writes exactly that) and
  *     the scaling pass is skipped.  A call with an input leaves its rows so in a separate
- *     workspace (with gathered_rows: those rows), so a call without one may follow it.
+ *     workspace (with gathered_rows: those rows; without any group: none), so a call
+ *     without one may follow it.
  *     Results of the modes agree to rounding (a few ulp per term).
  *   - Limits: vertices and slots (CSR entries, kept edges) are int32 as in the
  *     reference and must stay below 2^31 - 1024 (the kernels step through slot
