@@ -189,8 +189,8 @@ def _ptr(t):
     return None if t is None else C.c_void_p(t.data_ptr())
 
 
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _stream(stream=None):
+    return C.c_void_p((stream or torch.cuda.current_stream()).cuda_stream)
 
 
 def _dev(t, dtype, name):
@@ -473,8 +473,9 @@ def build_plan(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes
 
 def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes: int, dim: int,
                      part2node=None, ids=None, block_shift: int = 0):
-    """Issues ``build_plan``; the returned call waits for it and gives the plan.  The build's workspace goes back to torch's
-    allocator at once, which hands it to later work on the same stream only: builds issued one after the other share it."""
+    """Issues ``build_plan``; the returned call waits for it, on the stream it was issued on, and gives the plan.  The
+    build's workspace goes back to torch's allocator at once, which hands it to later work on the same stream only: builds
+    issued one after the other share it."""
     lib = load()
     _dev(part_ptr, torch.int32, "part_ptr"); _dev(column_index, torch.int32, "column_index")
     if (part2node is None) == (ids is None):
@@ -483,19 +484,20 @@ def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num
         raise EppgcnError("part_ptr needs num_parts + 1 entries")
     if column_index.numel() < num_slots:
         raise EppgcnError("column_index is shorter than num_slots")
+    stream = torch.cuda.current_stream()
     nbytes = lib.eppgcn_plan_bytes(int(num_parts), int(num_slots), int(num_nodes))
     buf, base = _aligned_buffer(nbytes, part_ptr.device)
     wbytes = lib.eppgcn_plan_workspace_bytes(int(num_parts), int(num_slots))
     ws, wbase = _aligned_buffer(wbytes, part_ptr.device)        # held until every kernel of the build is issued
     _check(lib.eppgcn_build_plan(_ptr(part_ptr), _ptr(column_index), _ptr(part2node), _ptr(ids), int(num_parts),
                                  int(num_slots), int(num_nodes), int(dim), int(block_shift), C.c_void_p(base), nbytes,
-                                 C.c_void_p(wbase), wbytes, _stream()))
+                                 C.c_void_p(wbase), wbytes, _stream(stream)))
 
     def finish():
         # synchronises, refuses a plan whose scan stalled and lets the library know the plan's stream form
         partial = C.c_int64(0)
         _check(lib.eppgcn_plan_status(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes), C.byref(partial),
-                                      _stream()))
+                                      _stream(stream)))
         return Plan(buf, base, int(num_parts), int(num_slots), int(num_nodes), int(partial.value))
 
     return finish
@@ -696,9 +698,9 @@ def mark_path(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, 
 
 
 def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool):
-    """Issues ``mark_path``; the result is what the returned call gives, which waits for it (the same stream must be
-    current)."""
-    lib = load()
+    """Issues ``mark_path``; the result is what the returned call gives, which waits for it on the stream it was issued on,
+    whatever stream is current then."""
+    lib, stream = load(), torch.cuda.current_stream()
     _dev(part2node, torch.int32, "part2node"); _dev(part_ptr, torch.int32, "part_ptr")
     _dev(column_index, torch.int32, "column_index"); _dev(node_degs, torch.int32, "node_degs")
     src = _mask_bytes(src_mask, "src_mask")
@@ -717,11 +719,11 @@ def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_
     ws = _workspace(nbytes, dev)
     _check(lib.eppgcn_mark_path(_ptr(part2node), _ptr(part_ptr), _ptr(column_index), _ptr(src), _ptr(ngh), _ptr(node_degs),
                                 _ptr(out_id), _ptr(out_edge), _ptr(bitmap), part2node.numel(), length, n,
-                                int(bool(is_last_layer)), _ptr(ws), nbytes, None, _stream()))
+                                int(bool(is_last_layer)), _ptr(ws), nbytes, None, _stream(stream)))
 
     def finish():
         counts = (C.c_int64 * 3)()
-        _check(lib.eppgcn_mark_path_counts(_ptr(out_edge), _ptr(bitmap), length, n, _ptr(ws), counts, _stream()))
+        _check(lib.eppgcn_mark_path_counts(_ptr(out_edge), _ptr(bitmap), length, n, _ptr(ws), counts, _stream(stream)))
         return out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
 
     return finish
@@ -778,8 +780,8 @@ def split_back_part(node_deg, num_edges: int, part_size: int):
 
 
 def split_back_part_begin(node_deg, num_edges: int, part_size: int):
-    """Issues ``split_back_part``; the returned call waits for it and gives its result."""
-    lib = load()
+    """Issues ``split_back_part``; the returned call waits for it, on the stream it was issued on, and gives its result."""
+    lib, stream = load(), torch.cuda.current_stream()
     _dev(node_deg, torch.int32, "node_deg")
     n = node_deg.numel()
     capacity = int(num_edges) + 1
@@ -787,11 +789,11 @@ def split_back_part_begin(node_deg, num_edges: int, part_size: int):
     nbytes = lib.eppgcn_split_workspace_bytes(n)
     ws = _workspace(nbytes, node_deg.device)
     _check(lib.eppgcn_split_back_part(_ptr(node_deg), n, int(part_size), _ptr(part_pointer), capacity, _ptr(ws),
-                                      nbytes, None, None, None, _stream()))
+                                      nbytes, None, None, None, _stream(stream)))
 
     def finish():
         p, v = C.c_int64(0), C.c_int64(0)
-        _check(lib.eppgcn_split_counts(_ptr(ws), C.byref(p), C.byref(v), _stream()))
+        _check(lib.eppgcn_split_counts(_ptr(ws), C.byref(p), C.byref(v), _stream(stream)))
         return part_pointer, int(p.value), int(v.value)
 
     return finish

@@ -402,6 +402,13 @@ int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, in
     counts[0] = counts[1] = counts[2] = 0;
     ScanState host;
     if (int rc = read_state(workspace, s, &host)) return rc;
+    // the count sizes a launch below: a workspace that holds something else is told from it first
+    if (host.counts[0] < 0 || host.counts[0] > num_edges || host.pad[2] < 0 || host.pad[2] > num_nodes || host.pad[0] < 0 ||
+        host.pad[0] > num_nodes) {
+        set_error("mark_path_counts: the workspace does not hold a finished eppgcn_mark_path of these sizes (it has to be called "
+                  "with the same buffers and sizes, on the same stream)");
+        return kErrInvalidArgument;
+    }
     counts[0] = host.counts[0];
     counts[1] = host.pad[2];
     counts[2] = host.pad[0];

@@ -336,8 +336,8 @@ int eppgcn_mark_compact(const int32_t* part2node, const int32_t* part_pointers,
  * eppgcn_mark_gathered_rows fills it for the kept slots, and counts[3] (host) = kept slots, rows with node_degs != 0,
  * gathered rows.  src_mask, ngh_mask and node_degs have num_nodes entries.  Synchronises the stream once (twice when a
  * marked vertex has no self-loop among its slots).  counts == NULL: nothing waits, and the outputs are complete once
- * eppgcn_mark_path_counts has been called with the same buffers and sizes - with several layers in flight one wait serves
- * them all.
+ * eppgcn_mark_path_counts has been called with the same buffers, sizes and stream - with several layers in flight one wait
+ * serves them all.  Counts that cannot be those of these sizes are refused with EPPGCN_ERR_INVALID_ARGUMENT.
  * workspace: eppgcn_mark_path_workspace_bytes(num_edges, num_nodes) bytes, 16-byte aligned. */
 size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes);
 int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
@@ -387,8 +387,8 @@ int eppgcn_split_back_part(const int32_t* node_deg, int num_nodes, int part_size
                            void* workspace, size_t workspace_bytes, int32_t* d_counts,
                            int64_t* h_num_parts, int64_t* h_valid_len, void* stream);
 
-/* Counts of an eppgcn_split_back_part call that was made without host pointers, from its workspace: synchronises the
- * stream and reports what that call would have (a stalled scan, groups that did not fit). */
+/* Counts of an eppgcn_split_back_part call that was made without host pointers, from its workspace and on its stream:
+ * synchronises the stream and reports what that call would have (a stalled scan, groups that did not fit). */
 int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_valid_len, void* stream);
 
 /* Forward neighbour groups from the CSR row pointers (device): part_pointers[0..P]

@@ -153,3 +153,53 @@ def test_preparing_several_layers_holds_one_build_workspace(api, layers):
                 [lib.eppgcn_plan_workspace_bytes(p.num_parts, p.valid_len) for p in wl.paths])
     marking = layers * lib.eppgcn_mark_path_workspace_bytes(g.num_edges, g.num_nodes)
     assert over <= 1.05 * build + marking, (over, build, marking)
+
+
+def test_results_are_waited_for_on_the_stream_they_were_issued_on(api):
+    """The three calls that are issued first and waited for later, issued behind other work on a side stream and waited for
+    with the default stream current."""
+    from eppgcn_amd import graphs
+    g = graphs.rmat_graph(14, 8, seed=3, device="cuda")
+    n, e = g.num_nodes, g.num_edges
+    pp, p2n = api.build_part(16, g.row_pointers, e)
+    src = graphs.bernoulli_mask(n, 0.2, 4, "cuda")
+    degs, degs2 = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+    want = api.mark_path(p2n, pp, g.column_index, src, None, degs, True)
+    want_split = api.split_back_part(degs, e, 8)
+    want_plan = api.build_plan(pp, g.column_index, p2n.numel(), e, n, 16, part2node=p2n)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)                 # some milliseconds
+        marked = api.mark_path_begin(p2n, pp, g.column_index, src, None, degs2, True)
+        split = api.split_back_part_begin(degs, e, 8)
+        plan = api.build_plan_begin(pp, g.column_index, p2n.numel(), e, n, 16, part2node=p2n)
+    plan, split, marked = plan(), split(), marked()
+    assert marked[2:4] == want[2:4] and marked[5] == want[5]
+    assert all(torch.equal(marked[i], want[i]) for i in (0, 1, 4)) and torch.equal(degs2, degs)
+    assert split[1:] == want_split[1:] and torch.equal(split[0], want_split[0])
+    assert plan.partial_rows == want_plan.partial_rows
+    assert all(torch.equal(a, b) for a, b in zip(plan.view(), want_plan.view()))
+
+
+def test_path_counts_of_other_sizes_are_refused(api):
+    """The kept slots size a launch where a marked vertex has no self-loop: counts that cannot be those of the sizes given
+    are an error before anything is launched."""
+    from eppgcn_amd import graphs
+    g = graphs.rmat_graph(12, 8, seed=3, device="cuda")
+    n, e = g.num_nodes, g.num_edges
+    lib = api.load()
+    pp, p2n = api.build_part(16, g.row_pointers, e)
+    src, degs = torch.ones(n, dtype=torch.bool, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+    out = torch.empty(2, e, dtype=torch.int32, device="cuda")
+    bitmap = torch.empty((n + 31) // 32, dtype=torch.int32, device="cuda")
+    ws = torch.empty(lib.eppgcn_mark_path_workspace_bytes(e, n), dtype=torch.uint8, device="cuda")
+    stream, counts = torch.cuda.current_stream().cuda_stream, (ctypes.c_int64 * 3)()
+    assert lib.eppgcn_mark_path(p2n.data_ptr(), pp.data_ptr(), g.column_index.data_ptr(), src.data_ptr(), None, degs.data_ptr(),
+                                out[0].data_ptr(), out[1].data_ptr(), bitmap.data_ptr(), p2n.numel(), e, n, 1, ws.data_ptr(),
+                                ws.numel(), None, stream) == 0
+    ask = lambda edges, nodes: lib.eppgcn_mark_path_counts(out[1].data_ptr(), bitmap.data_ptr(), edges, nodes, ws.data_ptr(),
+                                                           counts, stream)
+    assert ask(e - 1, n) == -1 and b"finished eppgcn_mark_path" in lib.eppgcn_last_error()
+    assert ask(e, n - 1) == -1
+    assert ask(e, n) == 0 and list(counts) == [e, n, n]
