@@ -17,27 +17,37 @@
 //   wtail[S_pad / 512]    index of the partial sum of what wave w holds after its last slot, or -1
 //   frow, fptr    the rows that have partial sums and the range of each (numbered row by row)
 //
-// Mapping.  A wave takes kStreamWave = 512 consecutive slots with two 16-byte loads per lane: lane l
-// holds slots 8l .. 8l+7.  A team of TS lanes (TS * 16 bytes = one table row) owns the 8 * TS slots its
-// own lanes hold and walks them in TS steps of 8 row gathers; the ids of step s are broadcast from lane
-// s of the team, so no id goes through LDS or is loaded twice.  Every gather instruction of the wave is
-// full (64 / TS rows) whatever the lengths of the rows.  A team adds rows into its partial sum and, at a
-// slot that ends a piece, writes the sum to that piece's row (s[r] and r come from a per-wave list in LDS,
-// staged once with coalesced loads).  What a team holds at the ends of its slot range - the tail of a piece
-// that goes on in the next team, the head of one that began in an earlier team - is combined across the
-// teams of the wave once, at the end, with a segmented scan in registers.  Pieces that cross waves and rows cut
-// into several pieces leave unscaled partial sums in a scratch area, which a second small kernel adds up row by
-// row in a fixed order: no float atomics, no output clear for rows that have slots, and the same bits every run.
-#include <type_traits>
-
+// Mapping.  A workgroup of four waves takes a chunk of kStreamWave = 512 consecutive slots, a wave 128 of them: lane l
+// holds slots 2l and 2l + 1.  A team of TS lanes (TS * 16 bytes = one table row) owns the 2 * TS slots its own lanes hold
+// and walks them in batches of 8 row gathers; the ids of a batch are broadcast from four lanes of the team, so no id goes
+// through LDS or is loaded twice.  Every gather instruction of the wave is full (64 / TS rows) whatever the lengths of
+// the rows.  A team adds rows into its partial sum and, at a slot that ends a piece, writes the sum to that piece's row
+// (s[r] and r come from a per-wave list in LDS, staged once with coalesced loads).  What a team holds at the ends of its
+// slot range - the tail of a piece that goes on in the next team, the head of one that began in an earlier team - is
+// combined once, at the end: across the teams of a wave with a segmented scan in registers, across the four waves through
+// LDS.  Pieces that cross chunks and rows cut into several pieces leave unscaled partial sums in a scratch area, which a
+// second small kernel adds up row by row in a fixed order: no float atomics, no output clear for rows that have slots,
+// and the same bits every run.
+//
+// What bounds it: the line fills of the gathers (large tables) and, where a launch has few chunks, the serial chain of
+// batches a team walks.  One wave per chunk with two batches in flight (114 VGPRs, 4 waves per SIMD) walked four times as
+// many batches one after the other and filled the chip only from 4096 chunks (2 M slots) on.  Measured, us per call with
+// its table and fix-up, one wave per chunk -> four (66 VGPRs, 7 waves per SIMD, one batch in flight each):
+//   390 chunks, 256 floats 108.7 -> 48.0; 781 chunks, 47 floats 59.8 -> 33.8; 1953 chunks, 16 / 64 floats 28.6 -> 26.6 /
+//   57.0 -> 48.3; R-MAT 20 (18 014 chunks) 16 / 22 / 64 / 256 floats 134 -> 134 / 195 -> 181 / 368 -> 337 / 1680 -> 1553;
+//   R-MAT 22 (258 798 chunks) 16 / 22 / 48 floats 1073 -> 1070 / 1554 -> 1513 / 2770 -> 2716
+// Two waves per chunk are 1 % better at R-MAT 22 with 16 and 22 floats and 2 to 5 % worse elsewhere; eight are 2 % better
+// at 256 floats and up to 26 % worse at 22.  Two batches in flight with four waves per chunk: 1513 -> 1820 (22 floats,
+// 102 VGPRs, 4 waves per SIMD).  Eight waves per SIMD cost spills in the wide variants (1513 -> 2003).
 #include "common.hpp"
 
 namespace eppgcn {
 
-constexpr int kStreamBlock = 256;
-constexpr int kStreamWaves = kStreamBlock / kWave;
+constexpr int kStreamWaves = 4;                            // waves of a workgroup; they share a chunk of kStreamWave slots
+constexpr int kStreamBlock = kStreamWaves * kWave;
+constexpr int kStreamSlots = kStreamWave / kStreamWaves;   // slots of a wave
+constexpr int kStreamIds = kStreamSlots / kWave;           // slot ids of a lane
 constexpr int kStreamShiftTeams = 8;   // teams up to this size address rows with a shift (power-of-two row pitch)
-constexpr int kStreamEvents = kStreamWave;       // pieces that can end in a wave's slots
 constexpr unsigned kNoRowOffset = 0xffffffffu;
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -80,10 +90,11 @@ __device__ __forceinline__ void store_row_floats(float* p, const float (&v)[4], 
 // table rows: pitch ld_bytes (a multiple of 16), `chunks` 16-byte vectors of a row are read (chunks <= TS);
 // out rows: pitch ld_out floats, columns < width_out written as the store mode says;
 // partial rows: pitch ld_bytes, written whole (unscaled sums).
-// U: row gathers per batch (4 or 8); two batches are in flight.
-template <int U> struct StreamBatch {
-    u32x4 v[U];
-    unsigned c[U];
+// A batch is kStreamBatch row gathers of every team.
+constexpr int kStreamBatch = 8;
+struct StreamBatch {
+    u32x4 v[kStreamBatch];
+    unsigned c[kStreamBatch];
 };
 
 // Is the header in memory the one the host remembers for this plan address?  (num_events < 0: not compared)
@@ -106,7 +117,7 @@ __device__ __forceinline__ void report_mismatch(int* __restrict__ fault, int whi
 // kWide: the table is addressed with 64-bit global loads instead of 32-bit offsets into a buffer resource (tables of
 // 4 GB and more, wide rows of 2^24 vertices and more); the lanes a buffer load would have sent out of range load row 0
 // instead and their values are replaced by zeros when they are added.
-template <int MODE, int TS, int U, bool kWide>
+template <int MODE, int TS, bool kWide>
 __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     float* __restrict__ out, float* __restrict__ partial, const float* __restrict__ table,
     const int* __restrict__ scol, const int* __restrict__ erow, const int* __restrict__ cev,
@@ -116,24 +127,30 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     unsigned pad_row)
 {
     constexpr int TPW = kWave / TS;
-    constexpr int kParts = 8 / U;                  // batches per step
-    constexpr int kCevPerTeam = TS / 4;            // cev counts chunks of 32 slots; a team owns 8 * TS slots
+    constexpr int kIds = kStreamIds, kSlots = kStreamSlots;
+    constexpr int kLanes = kStreamBatch / kIds;    // lanes whose ids make one batch; a team owns kIds * TS slots
+    constexpr int kBatches = TS / kLanes;          // batches a team walks
+    constexpr int kEvents = kSlots;                // pieces that can end in a wave's slots
+    static_assert(kBatches >= 1 && kSlots % kStreamChunk == 0, "a team walks whole batches, cev counts at a wave's first slot");
     // per wave: where the sum of every piece that ends in its slots goes.  x, y: address of the target row's first
     // float (0: nowhere), z: the factor (the row's scale; 1 for a partial sum), w: floats the target row takes
     // (a partial sum is one table row wide) | bit 16 for a partial sum
-    __shared__ u32x4 ev_list[kStreamWaves][kStreamEvents + 1];
+    __shared__ u32x4 ev_list[kStreamWaves][kEvents + 1];
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int team = lane / TS;
     const int tl = lane % TS;
-    const int w = blockIdx.x * kStreamWaves + wave;
-    if (w >= num_wave_chunks) return;                       // wave-uniform; the LDS rows are wave-private
+    // four consecutive chunks go to workgroups of one XCD (workgroup b runs on XCD b mod 8): neighbouring rows share lines of
+    // the output (width 22 at R-MAT 22: 1522 -> 1514 us per call)
+    int w = blockIdx.x;
+    if ((w | 31) < num_wave_chunks) w = (w & ~31) | (w & 7) << 2 | (w >> 3 & 3);
+    
     // the counts the host remembers must be those of the plan in memory (they are unless the plan's bytes were
     // replaced behind the library's back): a mismatch ends the kernel instead of indexing with the wrong sizes,
     // and leaves a mark that eppgcn_aggregation_status reports (the output of this call is not written)
     if (header_mismatch(header, generation, num_events, num_partials)) {
-        if (w == 0 && lane == 0) report_mismatch(fault, 1, generation, header->generation);
+        if (blockIdx.x == 0 && threadIdx.x == 0) report_mismatch(fault, 1, generation, header->generation);
         return;
     }
     u32x4* my_list = ev_list[wave];
@@ -156,15 +173,33 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
         return u32x4{static_cast<unsigned>(a), static_cast<unsigned>(a >> 32), factor, floats};
     };
 
-    // the wave's 512 slot ids, 8 per lane (streamed once: non-temporal)
-    const u32x4* idp = reinterpret_cast<const u32x4*>(scol + static_cast<size_t>(w) * kStreamWave) + lane * 2;
-    const u32x4 id_lo = __builtin_nontemporal_load(idp);
-    const u32x4 id_hi = __builtin_nontemporal_load(idp + 1);
-    const unsigned ids[8] = {id_lo.x, id_lo.y, id_lo.z, id_lo.w, id_hi.x, id_hi.y, id_hi.z, id_hi.w};
-    const int c0 = w * (kStreamWave / 32);
-    const int ce_team = cev[c0 + team * kCevPerTeam];
+    // the wave's slot ids, kIds consecutive ones per lane (streamed once: non-temporal)
+    unsigned ids[kIds];
+    {
+        typedef unsigned ids_t __attribute__((ext_vector_type(kIds)));
+        const int* idp = scol + static_cast<size_t>(w) * kStreamWave + wave * kSlots + lane * kIds;
+        const ids_t q = __builtin_nontemporal_load(reinterpret_cast<const ids_t*>(idp));
+#pragma unroll
+        for (int j = 0; j < kIds; ++j) ids[j] = q[j];
+    }
+    const int c0 = w * (kStreamWave / kStreamChunk) + wave * (kSlots / kStreamChunk);
     const int ce_first = cev[c0];
-    const int ce_last = cev[c0 + kStreamWave / 32];
+    const int ce_last = cev[c0 + kSlots / kStreamChunk];
+    // pieces that end before the team's slots (cev at the wave's first slot and the flags of the lanes before the team),
+    // and whether its first slot is inside a piece (the slot before it does not end one)
+    bool head_pending;
+    int ends_before = 0;
+    {
+        const uint64_t below = (1ull << (team * TS)) - 1ull;
+        uint64_t closes = 0;
+#pragma unroll
+        for (int r = 0; r < kIds; ++r) {
+            closes = __ballot(static_cast<int>(ids[r]) < 0);
+            ends_before += __popcll(closes & below);
+        }
+        head_pending = team == 0 ? ce_first < 0 : ((closes >> (team > 0 ? team * TS - 1 : 0)) & 1ull) == 0;
+    }
+    const bool began_before = head_pending;      // the team's first piece end closes a piece from an earlier team
     const int tail_at = wtail[w];
 
     const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(table), 0,
@@ -172,14 +207,14 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     const unsigned lane_off = tl < chunks ? static_cast<unsigned>(tl) * 16u : kNoRowOffset;
     const unsigned row_step = static_cast<unsigned>(__builtin_ctz(ld_bytes));       // wave-uniform
 
-    // batch (s, part): the ids come from lane s of the team, registers part * U ...
-    auto issue = [&](StreamBatch<U>& b, int s, auto part) {
-        constexpr int kPart = decltype(part)::value;
-        const int src = team * TS + s;
+    // batch i: the ids of the team's lanes i * kLanes .. i * kLanes + kLanes - 1
+    auto issue = [&](StreamBatch& b, int i) {
+        const int src = team * TS + i * kLanes;
 #pragma unroll
-        for (int u = 0; u < U; ++u) b.c[u] = static_cast<unsigned>(__shfl(static_cast<int>(ids[kPart * U + u]), src, kWave));
+        for (int u = 0; u < kStreamBatch; ++u)
+            b.c[u] = static_cast<unsigned>(__shfl(static_cast<int>(ids[u % kIds]), src + u / kIds, kWave));
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < kStreamBatch; ++u) {
             const unsigned id = swizzled_row(b.c[u] & 0x7fffffffu);      // the table's row order (common.hpp)
             // rows of a narrow team are a power of two bytes apart (row_step = log2): a shift serves any row count
             // of a table below 4 GB; wider rows use the 24-bit multiply (the host checks the row count)
@@ -196,17 +231,15 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
             }
         }
     };
-    using P0 = std::integral_constant<int, 0>;
-    using P1 = std::integral_constant<int, kParts - 1>;
 
-    StreamBatch<U> ba, bb;
-    issue(ba, 0, P0{});            // the first gathers are under way while the piece list is staged
+    StreamBatch ba;
+    issue(ba, 0);                  // the first gathers are under way while the piece list is staged
 
     // pieces that end in the wave's slots: [ev0, ev1)
     const int ev0 = ce_first & 0x7fffffff;
     const int ev1 = ce_last & 0x7fffffff;
     {
-        const int staged = min(min(ev1, num_events) - ev0, kStreamEvents);
+        const int staged = min(min(ev1, num_events) - ev0, kEvents);
         for (int j = lane; j < staged; j += kWave) my_list[j] = target_of(erow[ev0 + j]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -231,17 +264,16 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
         }
     };
 
-    int ev = min(max((ce_team & 0x7fffffff) - ev0, 0), kStreamEvents);   // the team's next piece end in the staged list
-    bool head_pending = ce_team < 0;             // the first piece end of the team closes a piece from an earlier team
+    int ev = min(ends_before, kEvents);          // the team's next piece end in the staged list
     bool had_event = false;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     float head[4] = {0.f, 0.f, 0.f, 0.f};
     u32x4 head_to = {0u, 0u, 0u, 0u};
     u32x4 next_to = my_list[ev];
 
-    auto consume = [&](const StreamBatch<U>& b) {
+    auto consume = [&](const StreamBatch& b) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < kStreamBatch; ++u) {
             u32x4 v = b.v[u];
             if constexpr (kWide) {          // what a buffer load would have returned as zeros
                 const bool ok = lane_off != kNoRowOffset && swizzled_row(b.c[u] & 0x7fffffffu) < pad_row;
@@ -263,33 +295,18 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
                 had_event = true;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[j] = 0.f;
-                ev = min(ev + 1, kStreamEvents);
+                ev = min(ev + 1, kEvents);
                 next_to = my_list[ev];
             }
         }
     };
 
-    // two batches in flight; the loop bodies issue unconditionally so that the waits can count on the younger batch
-    if constexpr (kParts == 2) {
-        for (int s = 0; s + 1 < TS; ++s) {
-            issue(bb, s, P1{});
-            consume(ba);
-            issue(ba, s + 1, P0{});
-            consume(bb);
-        }
-        issue(bb, TS - 1, P1{});
+    // One batch in flight per wave: seven waves per SIMD keep more gathers under way than four with two batches each.
+    consume(ba);
+#pragma unroll 1
+    for (int i = 1; i < kBatches; ++i) {
+        issue(ba, i);
         consume(ba);
-        consume(bb);
-    } else {
-        for (int s = 0; s + 2 < TS; s += 2) {
-            issue(bb, s + 1, P0{});
-            consume(ba);
-            issue(ba, s + 2, P0{});
-            consume(bb);
-        }
-        issue(bb, TS - 1, P0{});
-        consume(ba);
-        consume(bb);
     }
 
     // ---- combine across the teams of the wave.  Inclusive segmented scan of the tails: a team in which a piece
@@ -316,13 +333,39 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
         const float o = TPW > 1 ? __shfl_up(run[j], TS, kWave) : 0.f;
         carry[j] = team > 0 ? o : 0.f;
     }
-    if (ce_team < 0 && had_event) {
+    {
+        // the same once more across the waves of the chunk: what the last team of each holds, and whether a piece ended
+        __shared__ f32x4 wave_run[kStreamWaves][TS];
+        __shared__ int wave_stop[kStreamWaves];
+        if (team == TPW - 1) {
+            wave_run[wave][tl] = f32x4{run[0], run[1], run[2], run[3]};
+            if (tl == 0) wave_stop[wave] = stop ? 1 : 0;
+        }
+        __syncthreads();
+        f32x4 in = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v + 1 < kStreamWaves; ++v) {
+            if (v >= wave) continue;
+            const f32x4 o = wave_run[v][tl];
+            const bool cut = wave_stop[v] != 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) in[j] = cut ? o[j] : in[j] + o[j];
+        }
+        const int left_stop = TPW > 1 ? __shfl_up(static_cast<int>(stop), TS, kWave) : 0;
+        const bool stop_before = team > 0 && left_stop != 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!stop_before) carry[j] += in[j];
+            if (!stop) run[j] += in[j];
+        }
+    }
+    if (began_before && had_event) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) head[j] += carry[j];
         flush(head, head_to);
     }
-    // the wave's last tail belongs to a piece that ends in a later wave: one more partial sum
-    if (team == TPW - 1 && tail_at >= 0) flush(run, target_of(tail_at | static_cast<int>(kStreamFlag)));
+    // the chunk's last tail belongs to a piece that ends in a later chunk: one more partial sum
+    if (wave == kStreamWaves - 1 && team == TPW - 1 && tail_at >= 0) flush(run, target_of(tail_at | static_cast<int>(kStreamFlag)));
 }
 
 // Rows with partial sums: out[frow[i], :] = s[frow[i]] * (sum of the partial rows fptr[i] .. fptr[i+1]), summed in
@@ -476,7 +519,7 @@ int launch_aggregate_stream(float* out, float* partial, const float* table, cons
     const unsigned pad_row = static_cast<unsigned>(swizzle_padded_rows(num_nodes));
     const int num_wave_chunks = static_cast<int>(padded / kStreamWave);
     if (num_wave_chunks == 0) return kOk;
-    const dim3 grid((num_wave_chunks + kStreamWaves - 1) / kStreamWaves), block(kStreamBlock);
+    const dim3 grid(num_wave_chunks), block(kStreamBlock);
     const uintptr_t a = reinterpret_cast<uintptr_t>(out);
     const int mode = (dim % 4 == 0 && a % 16 == 0) ? ((dim == ts * 4 && ld_in == ts * 4) ? kStoreExact : kStoreVec4) : kStorePlain;
     const int num_fix = info.header.num_fix;
@@ -486,7 +529,7 @@ int launch_aggregate_stream(float* out, float* partial, const float* table, cons
     int* fault = nullptr;
     if (int rc = plan_fault_address(&fault)) return rc;
 #define EPPGCN_STREAM_KERNEL(MODE_, TS_, WIDE_)                                                                        \
-    hipLaunchKernelGGL((aggregate_stream_kernel<MODE_, TS_, 8, WIDE_>), grid, block, 0, stream, out, partial, table,   \
+    hipLaunchKernelGGL((aggregate_stream_kernel<MODE_, TS_, WIDE_>), grid, block, 0, stream, out, partial, table,   \
                        scol, sv.erow, sv.cev, sv.wtail, scale, sv.header, fault, info.header.generation,              \
                        num_wave_chunks, info.header.num_events,                                                       \
                        num_nodes, info.header.num_partials, chunks, static_cast<unsigned>(ld_in) * 4u, dim, dim,      \

@@ -207,6 +207,31 @@ def test_stream_aggregation_exact_and_reproducible(api, name):
             assert torch.equal(a, b), "same bits on every run"
 
 
+@pytest.mark.parametrize("dim", [3, 16, 22, 47, 64, 100, 256])
+def test_pieces_ending_around_the_borders_of_teams_and_waves(api, dim):
+    """A chunk of 512 slots is walked by four waves of 128 slots, each cut into teams: rows that end on, just before and
+    just behind every such border, rows that span one, two, three waves and whole chunks without an end, a last chunk
+    with a single slot.  Integer features and unit scales: every sum is exact in fp32."""
+    spans = [127, 1, 1, 126, 2, 255, 128, 129, 384, 511, 1, 512, 513, 7, 1, 8, 9, 15, 16, 17, 31, 33, 1023, 1, 130, 640]
+    lengths = np.array(spans + [1] * 300 + [2, 3] * 40 + spans[::-1], np.int64)
+    lengths = np.append(lengths, 1 + (-int(lengths.sum())) % WAVE)        # the last chunk holds one slot
+    n = 6000
+    indptr = np.concatenate([[0], np.cumsum(np.concatenate([lengths, np.zeros(n - lengths.size, np.int64)]))]).astype(np.int32)
+    assert indptr[-1] % WAVE == 1
+    rng = np.random.default_rng(dim)
+    col = np.concatenate([np.sort(rng.choice(n, int(k), replace=False)) for k in lengths]).astype(np.int32)
+    x = rng.integers(-4, 5, (n, dim)).astype(np.float32)
+    ones = np.ones(n, np.float32)
+    for ps, shift in ((1024, 31), (16, 31), (32, 10)):        # whole rows, rows of several groups, column blocks
+        pp, p2n = co.build_part(ps, indptr)
+        api.set_plan_shift(shift)
+        plan = api.build_plan(dev(pp), dev(col), p2n.size, col.size, n, dim, part2node=dev(p2n))
+        out = torch.full((n, dim), float("nan"), device="cuda")
+        api.spmm_forward(dev(x), dev(col), dev(ones), dev(pp), dev(p2n), part_size=ps, plan=plan, out=out)
+        assert api.last_call_used_stream()
+        assert np.array_equal(out.cpu().numpy(), co.spmm_f64(x, indptr, col, ones).astype(np.float32)), f"groups of {ps}"
+
+
 def test_stream_path_selection_and_fallbacks(api):
     """The group kernel runs, with the same results, when the stream form cannot: stream mode off, a workspace
     without room for the partial sums, the input scaled in place, no workspace at all, a plan the library has not
