@@ -407,7 +407,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     static_assert(kWords % kWave == 0 && kItems <= kWave, "one wave scans the words; a wave's words fit its lanes");
     constexpr bool kScanned = kItems == kMarkItemsLarge;       // counts[] holds the kept slots before every tile
     __shared__ int s_prefix;
-    __shared__ int s_starts_in_tile;
+    __shared__ int s_starts_in_tile, s_kept_in_tile;
     __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
     __shared__ unsigned long long s_kept[kWords];      // bit p: slot base + p is kept
     __shared__ int s_starts_before[kWords];            // group starts before each word
@@ -467,6 +467,24 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
         if (mine) atomicAdd(&s_starts_in_tile, mine);
     }
     __syncthreads();
+    // Zeros behind the kept slots of the whole input, written here and not by a pass of their own because they cost what their
+    // bytes cost: 13 of 132 M slots kept, this kernel 384 -> 513 us and the pass behind it 195 -> 15.  As many words as this tile drops slots, counted from the end, behind
+    // those of the tiles before it (which dropped base - s_prefix slots).
+    if (wave == 0) {
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) n += __popcll(s_kept[lane * kPerLane + j]);
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
+        if (lane == 0) s_kept_in_tile = n;
+    }
+    __syncthreads();
+    {
+        const long long end = length - (base - s_prefix);
+        const long long from = end - (min(static_cast<long long>(kTile), length - base) - s_kept_in_tile);
+        zero_from(out_id, from, end, threadIdx.x, kMarkBlock);
+        zero_from(out_edge, from, end, threadIdx.x, kMarkBlock);
+    }
     // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
     // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
     // population count over the map of group starts; otherwise every slot does a binary search over the group starts.
@@ -613,24 +631,19 @@ __global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __re
     }
 }
 
-// After: the rows the path gathers, the rows with kept slots, zeros behind the kept slots.
+// After: the rows the path gathers, the rows with kept slots.
 // Every vertex of the source mask whose self-loop is a slot is gathered; when that is all of them (graphs with
 // self-loops, the usual case) the mask is the bitmap of the gathered rows and no pass over the kept slots is needed
 // (0.58 ms for 126 M of them).  st->pad: [0] vertices of the mask, [1] not all of them kept their self-loop, [2] rows with
 // kept slots.
+// Every workgroup ends in three atomics on one line (12 ns each, serial).
 constexpr int kFinishCountBlocks = 256;
 __global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* __restrict__ bits, const uint4* __restrict__ self_kept,
                                                                int words, uint32_t* __restrict__ gathered,
                                                                const int* __restrict__ node_degs, int num_nodes,
-                                                               int* __restrict__ out_id, int* __restrict__ out_edge, int length,
                                                                ScanState* st)
 {
-    const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
-    zero_from(out_id, st->counts[0], length, i0, stride);
-    zero_from(out_edge, st->counts[0], length, i0, stride);
-    // the first workgroups count: every workgroup that does ends in three atomics on one line (12 ns each, serial)
-    if (blockIdx.x >= kFinishCountBlocks) return;
-    const int count_stride = min(stride, kFinishCountBlocks * 256);
+    const int i0 = blockIdx.x * 256 + threadIdx.x, count_stride = gridDim.x * 256;
     int marked = 0, missing = 0, rows = 0;
     for (int w = i0; w < words; w += count_stride) {
         const uint32_t b = bits[w];
@@ -659,6 +672,8 @@ __global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* _
     add_block_count(rows, &st->pad[2]);
 }
 
+constexpr int kTailWords = 16384;
+
 // Zero both outputs from the compacted length (read on the device) to the end.
 __global__ void zero_tail2_kernel(int* __restrict__ a, int* __restrict__ b, const int* __restrict__ d_start, int length)
 {
@@ -668,10 +683,13 @@ __global__ void zero_tail2_kernel(int* __restrict__ a, int* __restrict__ b, cons
     zero_from(b, *d_start, length, i0, stride);
 }
 
-__global__ void zero_tail1_kernel(int* __restrict__ a, const int* __restrict__ d_start, int offset, long long length)
+// A workgroup per kTailWords consecutive words; those that lie before the start have nothing to do.  512 workgroups that
+// stride over the array took 123 / 91 us for the two paths of R-MAT scale 22 (530 MB each), this 105 / 92.
+__global__ __launch_bounds__(256) void zero_tail1_kernel(int* __restrict__ a, const int* __restrict__ d_start, int offset,
+                                                         long long length)
 {
-    zero_from(a, static_cast<long long>(*d_start) + offset, length,
-              static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x, static_cast<long long>(gridDim.x) * blockDim.x);
+    const long long first = static_cast<long long>(blockIdx.x) * kTailWords;
+    zero_from(a, max(first, static_cast<long long>(*d_start) + offset), min(first + kTailWords, length), threadIdx.x, 256);
 }
 
 // ================================================================ counting
@@ -1007,10 +1025,8 @@ size_t scan_workspace_bytes(long long length, int tile)
 size_t compact_workspace_bytes(long long length) { return scan_workspace_bytes(length, kCompactTile); }
 size_t split_workspace_bytes(long long num_nodes) { return scan_workspace_bytes(num_nodes, kSplitTile); }
 
-// Workgroups that clear what lies behind a length that only the device knows: two per CU.  A strided fill of 528 MB runs at
-// 5.9 TB/s with 512 workgroups and at 4.3 with 2048; a workgroup per 4 KB, as where the length is known, reaches 6.8 but may
-// find most of them with nothing to do.  In a path's preparation at R-MAT scale 22: zero_tail1_kernel 165 -> 127 us,
-// mark_path_finish_kernel 164 -> 139 us.
+// Workgroups of zero_tail2_kernel, which clears what lies behind a length that only the device knows: two per CU (528 MB at
+// 5.9 TB/s with 512 workgroups that stride over it, at 4.3 with 2048).
 constexpr int kTailBlocks = 512;
 static unsigned tail_blocks(long long length)
 {
@@ -1189,9 +1205,6 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
     if (int rc = launch_mark_pass<false>(part2node, part_ptr, col, src_mask, ngh_mask, node_degs, out_id, out_edge, nullptr,
                                          num_parts, length, is_last, l, base, stream))
         return rc;
-    hipLaunchKernelGGL(zero_tail2_kernel, dim3(tail_blocks(length)), dim3(256), 0, stream, out_id, out_edge, st->counts,
-                       static_cast<int>(length));
-    EPPGCN_HIP(hipGetLastError());
     return kOk;
 }
 
@@ -1216,9 +1229,9 @@ int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, 
     if (int rc = launch_mark_pass<true>(part2node, part_ptr, col, bits, ngh_mask, node_degs, out_id, out_edge, self_kept,
                                         num_parts, length, is_last, l, base, stream))
         return rc;
-    hipLaunchKernelGGL(mark_path_finish_kernel, dim3(tail_blocks(length > num_nodes ? length : num_nodes)), dim3(256), 0,
-                       stream, bits, reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, out_id,
-                       out_edge, static_cast<int>(length), st);
+    const int count_blocks = num_nodes / 1024 + 1 < kFinishCountBlocks ? num_nodes / 1024 + 1 : kFinishCountBlocks;
+    hipLaunchKernelGGL(mark_path_finish_kernel, dim3(count_blocks), dim3(256), 0, stream, bits,
+                       reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, st);
     EPPGCN_HIP(hipGetLastError());
     return kOk;
 }
@@ -1244,8 +1257,8 @@ int launch_split(bool from_row_ptr, const int* src, int num_nodes, int part_size
                            part_size, part_ptr_out, part2node_out, capacity, num_tiles, st, desc, scan_mode());
     EPPGCN_HIP(hipGetLastError());
     if (zero_tail) {
-        hipLaunchKernelGGL(zero_tail1_kernel, dim3(tail_blocks(capacity)), dim3(256), 0, stream, part_ptr_out,
-                           st->counts, 1, capacity);
+        hipLaunchKernelGGL(zero_tail1_kernel, dim3(static_cast<unsigned>((capacity + kTailWords - 1) / kTailWords)), dim3(256), 0,
+                           stream, part_ptr_out, st->counts, 1, capacity);
         EPPGCN_HIP(hipGetLastError());
     }
     return kOk;
