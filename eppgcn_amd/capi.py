@@ -25,7 +25,9 @@ EXPORTS = [
     "eppgcn_feature_workspace_pitch", "eppgcn_update_forward", "eppgcn_update_backward_input",
     "eppgcn_update_workspace_bytes", "eppgcn_update_backward_weight", "eppgcn_update_supported", "eppgcn_update_backward",
     "eppgcn_mark_compact_workspace_bytes", "eppgcn_mark_compact", "eppgcn_mark_path_workspace_bytes", "eppgcn_mark_path",
-    "eppgcn_mark_path_counts", "eppgcn_split_counts",
+    "eppgcn_mark_path_counts", "eppgcn_split_counts", "eppgcn_mark_path_groups", "eppgcn_mark_path_group_counts",
+    "eppgcn_state_bytes", "eppgcn_read_states", "eppgcn_plan_state", "eppgcn_plan_status_read", "eppgcn_split_counts_read",
+    "eppgcn_split_and_plan",
     "eppgcn_nll_workspace_bytes", "eppgcn_nll_forward", "eppgcn_nll_backward",
     "eppgcn_set_plan_length_classes",
     "eppgcn_mark_gathered_rows", "eppgcn_set_wide_index", "eppgcn_wave64_back_part_size",
@@ -37,7 +39,7 @@ EXPORTS = [
     "eppgcn_mark_gathered_rows_scratch", "eppgcn_mark_gathered_rows_scratch_bytes",
 ]
 
-ABI_VERSION = 17      # what eppgcn_abi_version() of a matching library returns
+ABI_VERSION = 18      # what eppgcn_abi_version() of a matching library returns
 
 _lib = None
 
@@ -142,6 +144,18 @@ def load():
     lib.eppgcn_mark_path.restype = i
     lib.eppgcn_mark_path_counts.argtypes = [p, p, i64, i, p, C.POINTER(i64), p]
     lib.eppgcn_mark_path_counts.restype = i
+    lib.eppgcn_mark_path_groups.argtypes = [p] * 9 + [i, i64, i, i, i, p, sz, p]
+    lib.eppgcn_mark_path_group_counts.argtypes = [p, p, i64, i, p, p, C.POINTER(i64), p]
+    lib.eppgcn_state_bytes.restype = sz
+    lib.eppgcn_read_states.argtypes = [C.POINTER(C.c_void_p), i, p, p]
+    lib.eppgcn_plan_state.argtypes = [p, i, i64, i]
+    lib.eppgcn_plan_state.restype = C.c_void_p
+    lib.eppgcn_plan_status_read.argtypes = [p, i, i64, i, p, C.POINTER(i64)]
+    lib.eppgcn_split_counts_read.argtypes = [p, C.POINTER(i64), C.POINTER(i64)]
+    lib.eppgcn_split_and_plan.argtypes = [p, p, i, i, p, i64, i, i64, i, i, p, sz, p, sz, p, sz, p]
+    for name in ("mark_path_groups", "mark_path_group_counts", "read_states", "plan_status_read", "split_counts_read",
+                 "split_and_plan"):
+        getattr(lib, "eppgcn_" + name).restype = i
     lib.eppgcn_split_counts.argtypes = [p, C.POINTER(i64), C.POINTER(i64), p]
     lib.eppgcn_split_counts.restype = i
     lib.eppgcn_nll_workspace_bytes.argtypes = []
@@ -473,7 +487,7 @@ def build_plan(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes
 
 def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num_nodes: int, dim: int,
                      part2node=None, ids=None, block_shift: int = 0):
-    """Issues ``build_plan``; the returned call waits for it, on the stream it was issued on, and gives the plan.  The
+    """Issues ``build_plan``; the returned call (a ``Pending``) waits for it, on the stream it was issued on, and gives the plan.  The
     build's workspace goes back to torch's allocator at once, which hands it to later work on the same stream only: builds
     issued one after the other share it."""
     lib = load()
@@ -493,14 +507,55 @@ def build_plan_begin(part_ptr, column_index, num_parts: int, num_slots: int, num
                                  int(num_slots), int(num_nodes), int(dim), int(block_shift), C.c_void_p(base), nbytes,
                                  C.c_void_p(wbase), wbytes, _stream(stream)))
 
-    def finish():
-        # synchronises, refuses a plan whose scan stalled and lets the library know the plan's stream form
-        partial = C.c_int64(0)
-        _check(lib.eppgcn_plan_status(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes), C.byref(partial),
-                                      _stream(stream)))
-        return Plan(buf, base, int(num_parts), int(num_slots), int(num_nodes), int(partial.value))
+    return _pending_plan(lib, buf, base, num_parts, num_slots, num_nodes, stream)
 
-    return finish
+
+def _pending_plan(lib, buf, base, num_parts, num_slots, num_nodes, stream):
+    def finish(states=None):
+        # (synchronises), refuses a plan whose scan stalled and lets the library know the plan's stream form
+        partial = C.c_int64(0)
+        sizes = int(num_parts), int(num_slots), int(num_nodes)
+        if states:
+            _check(lib.eppgcn_plan_status_read(C.c_void_p(base), *sizes, states[0], C.byref(partial)))
+        else:
+            _check(lib.eppgcn_plan_status(C.c_void_p(base), *sizes, C.byref(partial), _stream(stream)))
+        return Plan(buf, base, *sizes, int(partial.value))
+
+    # a plan without groups has no record
+    return Pending([lib.eppgcn_plan_state(C.c_void_p(base), int(num_parts), int(num_slots), int(num_nodes))], finish, stream)
+
+
+class Pending:
+    """The result of a call that was issued and not waited for: calling it waits, on the stream it was issued on, and gives
+    the result.  ``states``: addresses of the records on the device that hold its counts (``finish_all``)."""
+
+    def __init__(self, states, finish, stream):
+        self.states, self.finish, self.stream = states, finish, stream
+
+    def __call__(self):
+        return self.finish()
+
+
+def finish_all(pending):
+    """The results of several ``Pending`` calls with one wait for all that were issued on the same stream."""
+    lib, pending = load(), list(pending)
+    out = [None] * len(pending)
+    for stream in {p.stream.cuda_stream: p.stream for p in pending}.values():
+        mine = [k for k, p in enumerate(pending) if p.stream.cuda_stream == stream.cuda_stream]
+        addresses = [a for k in mine for a in pending[k].states]
+        if None in addresses:
+            for k in mine:
+                out[k] = pending[k]()
+            continue
+        size = lib.eppgcn_state_bytes()
+        host = torch.empty(size * len(addresses), dtype=torch.uint8, pin_memory=True)
+        _check(lib.eppgcn_read_states((C.c_void_p * len(addresses))(*addresses), len(addresses), _ptr(host), _stream(stream)))
+        at = host.data_ptr()
+        for k in mine:
+            count = len(pending[k].states)
+            out[k] = pending[k].finish([C.c_void_p(at + size * j) for j in range(count)])
+            at += size * count
+    return out
 
 
 def plan_recommended(num_nodes: int, dim: int) -> bool:
@@ -697,9 +752,10 @@ def mark_path(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, 
     return mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer)()
 
 
-def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool):
-    """Issues ``mark_path``; the result is what the returned call gives, which waits for it on the stream it was issued on,
-    whatever stream is current then."""
+def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_degs, is_last_layer: bool, part_size: int = 0):
+    """Issues ``mark_path``; the result is what the returned call (a ``Pending``) gives, which waits for it on the stream it was
+    issued on, whatever stream is current then.  ``part_size``: the result's last entry, behind those of ``mark_path``, is the
+    number of groups that ``split_back_part`` will make of the path."""
     lib, stream = load(), torch.cuda.current_stream()
     _dev(part2node, torch.int32, "part2node"); _dev(part_ptr, torch.int32, "part_ptr")
     _dev(column_index, torch.int32, "column_index"); _dev(node_degs, torch.int32, "node_degs")
@@ -717,16 +773,18 @@ def mark_path_begin(part2node, part_ptr, column_index, src_mask, ngh_mask, node_
     bitmap = torch.empty((n + 31) // 32, dtype=torch.int32, device=dev)
     nbytes = lib.eppgcn_mark_path_workspace_bytes(length, n)
     ws = _workspace(nbytes, dev)
-    _check(lib.eppgcn_mark_path(_ptr(part2node), _ptr(part_ptr), _ptr(column_index), _ptr(src), _ptr(ngh), _ptr(node_degs),
-                                _ptr(out_id), _ptr(out_edge), _ptr(bitmap), part2node.numel(), length, n,
-                                int(bool(is_last_layer)), _ptr(ws), nbytes, None, _stream(stream)))
+    _check(lib.eppgcn_mark_path_groups(_ptr(part2node), _ptr(part_ptr), _ptr(column_index), _ptr(src), _ptr(ngh),
+                                       _ptr(node_degs), _ptr(out_id), _ptr(out_edge), _ptr(bitmap), part2node.numel(), length,
+                                       n, int(bool(is_last_layer)), int(part_size), _ptr(ws), nbytes, _stream(stream)))
 
-    def finish():
-        counts = (C.c_int64 * 3)()
-        _check(lib.eppgcn_mark_path_counts(_ptr(out_edge), _ptr(bitmap), length, n, _ptr(ws), counts, _stream(stream)))
-        return out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
+    def finish(states=None):
+        counts = (C.c_int64 * 4)()
+        _check(lib.eppgcn_mark_path_group_counts(_ptr(out_edge), _ptr(bitmap), length, n, _ptr(ws),
+                                                 states[0] if states else None, counts, _stream(stream)))
+        out = out_id, out_edge, counts[0], counts[1], bitmap, counts[2]
+        return out + (counts[3],) if part_size else out
 
-    return finish
+    return Pending([ws.data_ptr()], finish, stream)
 
 
 def count_nonzero(node_deg) -> int:
@@ -791,12 +849,47 @@ def split_back_part_begin(node_deg, num_edges: int, part_size: int):
     _check(lib.eppgcn_split_back_part(_ptr(node_deg), n, int(part_size), _ptr(part_pointer), capacity, _ptr(ws),
                                       nbytes, None, None, None, _stream(stream)))
 
-    def finish():
+    def finish(states=None):
         p, v = C.c_int64(0), C.c_int64(0)
-        _check(lib.eppgcn_split_counts(_ptr(ws), C.byref(p), C.byref(v), _stream(stream)))
+        if states:
+            _check(lib.eppgcn_split_counts_read(states[0], C.byref(p), C.byref(v)))
+        else:
+            _check(lib.eppgcn_split_counts(_ptr(ws), C.byref(p), C.byref(v), _stream(stream)))
         return part_pointer, int(p.value), int(v.value)
 
-    return finish
+    return Pending([ws.data_ptr()], finish, stream)
+
+
+def split_and_plan_begin(node_deg, edge_list, num_edges: int, part_size: int, num_parts: int, num_slots: int, dim: int,
+                         block_shift: int = 0):
+    """``split_back_part_begin`` and ``build_plan_begin`` of the groups in one, for a path whose group count is known
+    (``mark_path_begin`` with ``part_size``); the ``Pending`` gives (part_pointer, num_parts, valid_len, plan)."""
+    lib, stream = load(), torch.cuda.current_stream()
+    _dev(node_deg, torch.int32, "node_deg"); _dev(edge_list, torch.int32, "edge_list")
+    if edge_list.numel() < num_slots or num_edges < num_parts:
+        raise EppgcnError("edge_list is shorter than num_slots, or num_edges than num_parts")
+    n, dev = node_deg.numel(), node_deg.device
+    part_pointer = torch.empty(int(num_edges) + 1, dtype=torch.int32, device=dev)
+    sbytes = lib.eppgcn_split_workspace_bytes(n)
+    sws = _workspace(sbytes, dev)
+    nbytes = lib.eppgcn_plan_bytes(int(num_parts), int(num_slots), n)
+    buf, base = _aligned_buffer(nbytes, dev)
+    wbytes = lib.eppgcn_plan_workspace_bytes(int(num_parts), int(num_slots))
+    ws, wbase = _aligned_buffer(wbytes, dev)                    # held until every kernel of the build is issued
+    _check(lib.eppgcn_split_and_plan(_ptr(node_deg), _ptr(edge_list), n, int(part_size), _ptr(part_pointer),
+                                     part_pointer.numel(), int(num_parts), int(num_slots), int(dim), int(block_shift),
+                                     C.c_void_p(base), nbytes, C.c_void_p(wbase), wbytes, _ptr(sws), sbytes, _stream(stream)))
+    plan = _pending_plan(lib, buf, base, num_parts, num_slots, n, stream)
+
+    def finish(states=None):
+        p, v = C.c_int64(0), C.c_int64(0)
+        if states:
+            _check(lib.eppgcn_split_counts_read(states[0], C.byref(p), C.byref(v)))
+        else:
+            _check(lib.eppgcn_split_counts(_ptr(sws), C.byref(p), C.byref(v), _stream(stream)))
+        return part_pointer, int(p.value), int(v.value), plan.finish(states and states[1:])
+
+    return Pending([sws.data_ptr()] + plan.states, finish, stream)
 
 
 def build_part(part_size: int, row_pointers, num_edges: int = None):

@@ -18,7 +18,7 @@ int aggregate_compacted_groups(float*, const float*, const int*, const int*, con
                                int, int, int, int, float*, size_t, const uint32_t*, hipStream_t, double*, double*,
                                const uint32_t** written = nullptr, long long* num_written = nullptr);
 size_t plan_workspace_bytes(long long, long long);
-int read_plan_status(const void*, long long, long long, long long, long long*, hipStream_t);
+int read_plan_status(const void*, long long, long long, long long, long long*, const void*, hipStream_t);
 void set_stream_mode(int);
 int last_call_used_stream();
 int schedule_shift(int);
@@ -26,7 +26,7 @@ void set_schedule_shift(int);
 void set_plan_keep_rows(int);
 void set_plan_length_classes(int);
 int launch_build_plan(const int*, const int*, const int*, const int*, int, long long, int, int, int, void*, size_t,
-                      void*, size_t, hipStream_t);
+                      void*, size_t, const ScanState*, hipStream_t);
 void set_agg_force_team(int);
 void set_agg_force_rounds(int);
 size_t feature_workspace_floats(long long, int);
@@ -55,10 +55,13 @@ int launch_nll_forward(float*, const float*, const long long*, const int*, long 
 int launch_nll_backward(float*, const float*, const float*, const int*, long long, long long, int, hipStream_t);
 uint8_t* mark_path_scratch(void*, long long, long long);
 int launch_mark_path(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, uint32_t*, int,
-                     long long, int, int, void*, hipStream_t);
+                     long long, int, int, int, void*, hipStream_t);
 int launch_mark_compact(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, int, long long,
                         int, void*, hipStream_t);
-int launch_split(bool, const int*, int, int, int*, int*, long long, bool, void*, hipStream_t);
+int launch_split(bool, const int*, int, int, int*, int*, long long, long long, bool, void*, hipStream_t);
+int launch_gather_states(const void* const*, int, void*, hipStream_t);
+int* plan_rows_in_workspace(void*, long long, long long);
+const void* plan_header_address(const void*, long long, long long, long long);
 int launch_count_nonzero(const int*, long long, int*, hipStream_t);
 int launch_ginfo_hist(const int*, long long, int*, hipStream_t);
 size_t mark_listed_rows_scratch_bytes(long long);
@@ -83,10 +86,15 @@ static double g_phase_ms[2] = {0.0, 0.0};       // output clears, pre-scaling pa
 bool timing_enabled() { return g_timing.load(); }
 double* phase_sink(int which) { return &g_phase_ms[which & 1]; }
 
-static int read_state(void* workspace, hipStream_t stream, ScanState* host)
+// (read: a complete copy of the state that the caller already has on the host)
+static int read_state(const void* workspace, hipStream_t stream, ScanState* host, const void* read = nullptr)
 {
-    EPPGCN_HIP(hipMemcpyAsync(host, workspace, sizeof(ScanState), hipMemcpyDeviceToHost, stream));
-    EPPGCN_HIP(hipStreamSynchronize(stream));
+    if (read) {
+        memcpy(host, read, sizeof(ScanState));
+    } else {
+        EPPGCN_HIP(hipMemcpyAsync(host, workspace, sizeof(ScanState), hipMemcpyDeviceToHost, stream));
+        EPPGCN_HIP(hipStreamSynchronize(stream));
+    }
     if (host->error) {
         set_error("look-back scan stalled: a tile waited past its spin limit; results are invalid");
         return kErrScanStalled;
@@ -103,7 +111,7 @@ using namespace eppgcn;
 extern "C" {
 
 const char* eppgcn_last_error(void) { return g_last_error.c_str(); }
-int eppgcn_abi_version(void) { return 17; }
+int eppgcn_abi_version(void) { return 18; }
 
 int eppgcn_spmm_forward(float* out, const float* in, const int32_t* row_pointers, const int32_t* column_index,
                         const float* degrees, const int32_t* part_pointers, const int32_t* part2node, int num_nodes,
@@ -234,9 +242,10 @@ size_t eppgcn_plan_workspace_bytes(int64_t num_parts, int64_t num_slots)
     return plan_workspace_bytes(num_parts, num_slots);
 }
 
-int eppgcn_build_plan(const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
-                      const int32_t* ids, int num_parts, int64_t num_slots, int num_nodes, int dim, int block_shift,
-                      void* plan, size_t plan_size, void* workspace, size_t workspace_bytes, void* stream)
+static int build_plan_call(const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
+                           const int32_t* ids, int num_parts, int64_t num_slots, int num_nodes, int dim, int block_shift,
+                           void* plan, size_t plan_size, void* workspace, size_t workspace_bytes, const ScanState* upstream,
+                           void* stream)
 {
     EPPGCN_REQUIRE(num_parts >= 0 && num_slots >= 0 && num_nodes >= 0 && dim > 0, "negative size");
     EPPGCN_REQUIRE(block_shift >= 0 && block_shift <= 31, "block_shift must be 0 (automatic) or 1..31");
@@ -246,7 +255,15 @@ int eppgcn_build_plan(const int32_t* part_pointers, const int32_t* column_index,
     EPPGCN_REQUIRE(aligned(plan, 256) && workspace && aligned(workspace, 256), "plan and workspace must be 256-byte aligned");
     return launch_build_plan(part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes,
                              block_shift > 0 ? block_shift : schedule_shift(dim), dim, plan, plan_size, workspace,
-                             workspace_bytes, static_cast<hipStream_t>(stream));
+                             workspace_bytes, upstream, static_cast<hipStream_t>(stream));
+}
+
+int eppgcn_build_plan(const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
+                      const int32_t* ids, int num_parts, int64_t num_slots, int num_nodes, int dim, int block_shift,
+                      void* plan, size_t plan_size, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return build_plan_call(part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes, dim, block_shift, plan,
+                           plan_size, workspace, workspace_bytes, nullptr, stream);
 }
 
 size_t eppgcn_compact_workspace_bytes(int64_t length) { return compact_workspace_bytes(length < 0 ? 0 : length); }
@@ -366,8 +383,21 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
                      uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, void* workspace,
                      size_t workspace_bytes, int64_t* counts, void* stream)
 {
+    if (int rc = eppgcn_mark_path_groups(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+                                         gathered_rows, num_parts, num_edges, num_nodes, is_last, 0, workspace,
+                                         workspace_bytes, stream))
+        return rc;
+    return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
+}
+
+int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                            const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id,
+                            int32_t* out_edge, uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes,
+                            int is_last, int part_size, void* workspace, size_t workspace_bytes, void* stream)
+{
     EPPGCN_REQUIRE(num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
                    "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
+    EPPGCN_REQUIRE(part_size >= 0, "part_size >= 0 required");
     EPPGCN_REQUIRE(workspace && aligned(workspace, 16), "workspace must be 16-byte aligned");
     EPPGCN_REQUIRE(workspace_bytes >= mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
     EPPGCN_REQUIRE(num_edges == 0 || (out_id && out_edge), "null output pointer");
@@ -382,29 +412,38 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
             if (int rc = launch_zero_words(out_id, static_cast<size_t>(num_edges), s)) return rc;
             if (int rc = launch_zero_words(out_edge, static_cast<size_t>(num_edges), s)) return rc;
         }
-        if (int rc = launch_zero_words(workspace, sizeof(ScanState) / 4, s)) return rc;
-    } else {
-        KernelTimer timer(s, &g_mask_ms);
-        if (int rc = launch_mark_path(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
-                                      gathered_rows, num_parts, num_edges, num_nodes, is_last ? 1 : 0, workspace, s))
-            return rc;
+        return launch_zero_words(workspace, sizeof(ScanState) / 4, s);
     }
-    return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
+    KernelTimer timer(s, &g_mask_ms);
+    return launch_mark_path(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+                            gathered_rows, num_parts, num_edges, num_nodes, is_last ? 1 : 0, part_size, workspace, s);
 }
 
 int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
                             void* workspace, int64_t* counts, void* stream)
 {
+    EPPGCN_REQUIRE(counts, "workspace (16-byte aligned) and counts required");
+    int64_t four[4];
+    counts[0] = counts[1] = counts[2] = 0;
+    if (int rc = eppgcn_mark_path_group_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, nullptr, four, stream))
+        return rc;
+    for (int i = 0; i < 3; ++i) counts[i] = four[i];
+    return kOk;
+}
+
+int eppgcn_mark_path_group_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
+                                  void* workspace, const void* state, int64_t* counts, void* stream)
+{
     EPPGCN_REQUIRE(num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31), "num_nodes >= 0 and 0 <= num_edges < 2^31 required");
     EPPGCN_REQUIRE(workspace && aligned(workspace, 16) && counts, "workspace (16-byte aligned) and counts required");
     EPPGCN_REQUIRE((num_edges == 0 || out_edge) && (num_nodes == 0 || gathered_rows), "null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    counts[0] = counts[1] = counts[2] = 0;
+    counts[0] = counts[1] = counts[2] = counts[3] = 0;
     ScanState host;
-    if (int rc = read_state(workspace, s, &host)) return rc;
+    if (int rc = read_state(workspace, s, &host, state)) return rc;
     // the count sizes a launch below: a workspace that holds something else is told from it first
     if (host.counts[0] < 0 || host.counts[0] > num_edges || host.pad[2] < 0 || host.pad[2] > num_nodes || host.pad[0] < 0 ||
-        host.pad[0] > num_nodes) {
+        host.pad[0] > num_nodes || host.counts[1] < 0 || host.counts[1] > host.counts[0]) {
         set_error("mark_path_counts: the workspace does not hold a finished eppgcn_mark_path of these sizes (it has to be called "
                   "with the same buffers and sizes, on the same stream)");
         return kErrInvalidArgument;
@@ -412,6 +451,7 @@ int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, in
     counts[0] = host.counts[0];
     counts[1] = host.pad[2];
     counts[2] = host.pad[0];
+    counts[3] = host.counts[1];
     if (host.pad[1]) {          // a marked vertex without a kept self-loop: the gathered rows have to be looked for
         ScanState* st = static_cast<ScanState*>(workspace);
         if (int rc = launch_mark_listed_rows(out_edge, counts[0], num_nodes, gathered_rows, &st->pad[0],
@@ -548,9 +588,39 @@ int eppgcn_plan_status(const void* plan, int num_parts, int64_t num_slots, int n
     if (num_parts == 0) return kOk;
     EPPGCN_REQUIRE(plan && aligned(plan, 256), "plan must be 256-byte aligned");
     long long partial = 0;
-    const int rc = read_plan_status(plan, num_parts, num_slots, num_nodes, &partial, static_cast<hipStream_t>(stream));
+    const int rc = read_plan_status(plan, num_parts, num_slots, num_nodes, &partial, nullptr, static_cast<hipStream_t>(stream));
     if (partial_rows) *partial_rows = partial;
     return rc;
+}
+
+const void* eppgcn_plan_state(const void* plan, int num_parts, int64_t num_slots, int num_nodes)
+{
+    return num_parts > 0 && num_slots >= 0 && num_nodes >= 0 && plan ? plan_header_address(plan, num_parts, num_slots, num_nodes)
+                                                                     : nullptr;
+}
+
+int eppgcn_plan_status_read(const void* plan, int num_parts, int64_t num_slots, int num_nodes, const void* state,
+                            int64_t* partial_rows)
+{
+    EPPGCN_REQUIRE(num_parts > 0 && num_slots >= 0 && num_nodes >= 0 && state, "num_parts > 0, sizes >= 0 and a state required");
+    EPPGCN_REQUIRE(plan && aligned(plan, 256), "plan must be 256-byte aligned");
+    long long partial = 0;
+    const int rc = read_plan_status(plan, num_parts, num_slots, num_nodes, &partial, state, nullptr);
+    if (partial_rows) *partial_rows = partial;
+    return rc;
+}
+
+size_t eppgcn_state_bytes(void) { return kStateBytes; }
+
+int eppgcn_read_states(const void* const* states, int count, void* host, void* stream)
+{
+    EPPGCN_REQUIRE(count >= 0 && (count == 0 || (states && host)), "null pointer");
+    for (int i = 0; i < count; ++i) EPPGCN_REQUIRE(states[i] && aligned(states[i], 4), "every record must be a 4-byte aligned address");
+    EPPGCN_REQUIRE(aligned(host, 4), "host memory must be 4-byte aligned");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int rc = launch_gather_states(states, count, host, s)) return rc;
+    EPPGCN_HIP(hipStreamSynchronize(s));
+    return kOk;
 }
 
 void eppgcn_plan_release(const void* plan)
@@ -571,13 +641,13 @@ size_t eppgcn_plan_workspace_floats(const void* plan, int64_t num_nodes, int dim
 void eppgcn_set_stream_mode(int on) { set_stream_mode(on); }
 int eppgcn_last_call_used_stream(void) { return last_call_used_stream(); }
 
-static int finish_split(void* workspace, hipStream_t s, int32_t* d_counts, int64_t* h_a, int64_t* h_b)
+static int finish_split(void* workspace, hipStream_t s, int32_t* d_counts, int64_t* h_a, int64_t* h_b, const void* read = nullptr)
 {
     ScanState* st = static_cast<ScanState*>(workspace);
     if (d_counts) EPPGCN_HIP(hipMemcpyAsync(d_counts, st->counts, 2 * sizeof(int), hipMemcpyDeviceToDevice, s));
     if (h_a || h_b) {
         ScanState host;
-        if (int rc = read_state(workspace, s, &host)) return rc;
+        if (int rc = read_state(workspace, s, &host, read)) return rc;
         if (h_a) *h_a = host.counts[0];
         if (h_b) *h_b = host.counts[1];
         if (host.overflow) {
@@ -599,7 +669,7 @@ int eppgcn_split_back_part(const int32_t* node_deg, int num_nodes, int part_size
     EPPGCN_REQUIRE(workspace_bytes >= split_workspace_bytes(num_nodes), "workspace too small");
     EPPGCN_REQUIRE(num_nodes == 0 || node_deg, "null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, nullptr, capacity, true, workspace, s))
+    if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, nullptr, capacity, 0, true, workspace, s))
         return rc;
     return finish_split(workspace, s, d_counts, h_num_parts, h_valid_len);
 }
@@ -608,6 +678,31 @@ int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_
 {
     EPPGCN_REQUIRE(workspace && aligned(workspace, 8), "workspace must be 8-byte aligned");
     return finish_split(const_cast<void*>(workspace), static_cast<hipStream_t>(stream), nullptr, h_num_parts, h_valid_len);
+}
+
+int eppgcn_split_counts_read(const void* state, int64_t* h_num_parts, int64_t* h_valid_len)
+{
+    EPPGCN_REQUIRE(state && h_num_parts && h_valid_len, "null pointer");
+    return finish_split(nullptr, nullptr, nullptr, h_num_parts, h_valid_len, state);
+}
+
+int eppgcn_split_and_plan(const int32_t* node_deg, const int32_t* edge_list, int num_nodes, int part_size,
+                          int32_t* part_pointer, int64_t capacity, int num_parts, int64_t num_slots, int dim, int block_shift,
+                          void* plan, size_t plan_bytes, void* workspace, size_t workspace_bytes, void* split_workspace,
+                          size_t split_workspace_bytes_, void* stream)
+{
+    EPPGCN_REQUIRE(num_nodes > 0 && part_size >= 1 && num_parts > 0 && dim > 0, "num_nodes, part_size, num_parts, dim > 0 required");
+    EPPGCN_REQUIRE(capacity > num_parts && part_pointer && node_deg, "part_pointer needs num_parts + 1 entries");
+    EPPGCN_REQUIRE(split_workspace && aligned(split_workspace, 8), "workspace must be 8-byte aligned");
+    EPPGCN_REQUIRE(split_workspace_bytes_ >= split_workspace_bytes(num_nodes), "workspace too small");
+    EPPGCN_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= plan_workspace_bytes(num_parts, num_slots),
+                   "workspace smaller than eppgcn_plan_workspace_bytes(num_parts, num_slots) or not 256-byte aligned");
+    int* rows = plan_rows_in_workspace(workspace, num_parts, num_slots);
+    if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, rows, capacity, num_parts, true,
+                              split_workspace, static_cast<hipStream_t>(stream)))
+        return rc;
+    return build_plan_call(part_pointer, edge_list, rows, nullptr, num_parts, num_slots, num_nodes, dim, block_shift, plan,
+                           plan_bytes, workspace, workspace_bytes, static_cast<const ScanState*>(split_workspace), stream);
 }
 
 int eppgcn_build_part(const int32_t* row_pointers, int num_nodes, int part_size, int32_t* part_pointers,
@@ -620,8 +715,8 @@ int eppgcn_build_part(const int32_t* row_pointers, int num_nodes, int part_size,
     EPPGCN_REQUIRE(workspace_bytes >= split_workspace_bytes(num_nodes), "workspace too small");
     EPPGCN_REQUIRE(row_pointers, "null pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (int rc = launch_split(true, row_pointers, num_nodes, part_size, part_pointers, part2node, capacity, false,
-                              workspace, s))
+    if (int rc = launch_split(true, row_pointers, num_nodes, part_size, part_pointers, part2node, capacity, capacity - 1,
+                              false, workspace, s))
         return rc;
     return finish_split(workspace, s, d_counts, h_num_parts, nullptr);
 }

@@ -636,15 +636,21 @@ __global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __re
 // self-loops, the usual case) the mask is the bitmap of the gathered rows and no pass over the kept slots is needed
 // (0.58 ms for 126 M of them).  st->pad: [0] vertices of the mask, [1] not all of them kept their self-loop, [2] rows with
 // kept slots.
-// Every workgroup ends in three atomics on one line (12 ns each, serial).
+// counts[1]: groups of at most group_size slots that the kept slots of the rows make (group_size 0: not counted).  Every
+// workgroup ends in three or four atomics on one line (12 ns each, serial).
 constexpr int kFinishCountBlocks = 256;
 __global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* __restrict__ bits, const uint4* __restrict__ self_kept,
                                                                int words, uint32_t* __restrict__ gathered,
                                                                const int* __restrict__ node_degs, int num_nodes,
-                                                               ScanState* st)
+                                                               int group_size, ScanState* st)
 {
     const int i0 = blockIdx.x * 256 + threadIdx.x, count_stride = gridDim.x * 256;
-    int marked = 0, missing = 0, rows = 0;
+    int marked = 0, missing = 0, rows = 0, groups = 0;
+    const unsigned gs = static_cast<unsigned>(max(group_size, 1));
+    auto count_row = [&](int d) {
+        rows += d != 0;
+        groups += d > 0 ? static_cast<int>((static_cast<unsigned>(d) + gs - 1u) / gs) : 0;
+    };
     for (int w = i0; w < words; w += count_stride) {
         const uint32_t b = bits[w];
         const uint4 lo = self_kept[2 * static_cast<size_t>(w)], hi = self_kept[2 * static_cast<size_t>(w) + 1];
@@ -659,17 +665,20 @@ __global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* _
         const int4* quads = reinterpret_cast<const int4*>(node_degs);
         for (int v = i0; v < num_nodes / 4; v += count_stride) {
             const int4 d = quads[v];
-            rows += (d.x != 0) + (d.y != 0) + (d.z != 0) + (d.w != 0);
+            count_row(d.x); count_row(d.y); count_row(d.z); count_row(d.w);
         }
-        if (i0 < num_nodes % 4) rows += node_degs[num_nodes / 4 * 4 + i0] != 0;
+        if (i0 < num_nodes % 4) count_row(node_degs[num_nodes / 4 * 4 + i0]);
     } else {
-        for (int v = i0; v < num_nodes; v += count_stride) rows += node_degs[v] != 0;
+        for (int v = i0; v < num_nodes; v += count_stride) count_row(node_degs[v]);
     }
     add_block_count(marked, &st->pad[0]);
     __syncthreads();
     add_block_count(missing, &st->pad[1]);
     __syncthreads();
     add_block_count(rows, &st->pad[2]);
+    if (group_size <= 0) return;
+    __syncthreads();
+    add_block_count(groups, &st->counts[1]);
 }
 
 constexpr int kTailWords = 16384;
@@ -817,7 +826,8 @@ static_assert(kSplitRounds * kSplitWaves <= kWave, "one wave scans the (round, w
 template <bool kFromRowPtr>
 __global__ __launch_bounds__(kSplitBlock) void split_groups_kernel(
     const int* __restrict__ src, int num_nodes, int part_size, int* __restrict__ part_ptr_out,
-    int* __restrict__ part2node_out, long long capacity, int num_tiles, ScanState* st, uint64_t* desc, unsigned mode)
+    int* __restrict__ part2node_out, long long capacity, long long rows_capacity, int num_tiles, ScanState* st, uint64_t* desc,
+    unsigned mode)
 {
     __shared__ int s_tile;
     __shared__ uint64_t s_sum[kSplitRounds * kSplitWaves];
@@ -859,14 +869,14 @@ __global__ __launch_bounds__(kSplitBlock) void split_groups_kernel(
             st->counts[0] = total_q;
             st->counts[1] = total_g;
             if (total_q < capacity) part_ptr_out[total_q] = total_g + g_first;
-            if (static_cast<long long>(total_q) + 1 > capacity) st->overflow = 1;
+            if (static_cast<long long>(total_q) + 1 > capacity || (part2node_out && total_q > rows_capacity)) st->overflow = 1;
         }
     }
     __syncthreads();
     auto write_group = [&](long long dst, int start, int vertex) {
         if (dst < capacity) {
             part_ptr_out[dst] = start;
-            if (part2node_out && dst + 1 < capacity) part2node_out[dst] = vertex;
+            if (part2node_out && dst < rows_capacity) part2node_out[dst] = vertex;
         }
     };
 #pragma unroll
@@ -1209,11 +1219,11 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
 }
 
 // launch_mark_compact with the rows of the path counted and its gathered rows marked; num_parts, length, num_nodes > 0.
-// Results land in the ScanState at the head of the workspace (16-byte aligned): counts[0] = kept length, pad as
+// Results land in the ScanState at the head of the workspace (16-byte aligned): counts[0] = kept length, counts[1] and pad as
 // mark_path_finish_kernel says.
 int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, const uint8_t* src_mask,
                      uint8_t* ngh_mask, int* node_degs, int* out_id, int* out_edge, uint32_t* gathered, int num_parts,
-                     long long length, int num_nodes, int is_last, void* workspace, hipStream_t stream)
+                     long long length, int num_nodes, int is_last, int group_size, void* workspace, hipStream_t stream)
 {
     const MarkLayout l = mark_layout(length, num_nodes);
     char* base = static_cast<char*>(workspace);
@@ -1231,14 +1241,17 @@ int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, 
         return rc;
     const int count_blocks = num_nodes / 1024 + 1 < kFinishCountBlocks ? num_nodes / 1024 + 1 : kFinishCountBlocks;
     hipLaunchKernelGGL(mark_path_finish_kernel, dim3(count_blocks), dim3(256), 0, stream, bits,
-                       reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, st);
+                       reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, group_size,
+                       st);
     EPPGCN_HIP(hipGetLastError());
     return kOk;
 }
 
 // counts[0] = number of groups, counts[1] = number of slots covered.
+// part2node_out (may be NULL for degrees): the vertex of every group, rows_capacity entries
 int launch_split(bool from_row_ptr, const int* src, int num_nodes, int part_size, int* part_ptr_out,
-                 int* part2node_out, long long capacity, bool zero_tail, void* workspace, hipStream_t stream)
+                 int* part2node_out, long long capacity, long long rows_capacity, bool zero_tail, void* workspace,
+                 hipStream_t stream)
 {
     ScanState* st = static_cast<ScanState*>(workspace);
     uint64_t* desc = reinterpret_cast<uint64_t*>(st + 1);
@@ -1251,14 +1264,37 @@ int launch_split(bool from_row_ptr, const int* src, int num_nodes, int part_size
     }
     if (from_row_ptr)
         hipLaunchKernelGGL((split_groups_kernel<true>), dim3(num_tiles), dim3(kSplitBlock), 0, stream, src, num_nodes,
-                           part_size, part_ptr_out, part2node_out, capacity, num_tiles, st, desc, scan_mode());
+                           part_size, part_ptr_out, part2node_out, capacity, rows_capacity, num_tiles, st, desc, scan_mode());
     else
         hipLaunchKernelGGL((split_groups_kernel<false>), dim3(num_tiles), dim3(kSplitBlock), 0, stream, src, num_nodes,
-                           part_size, part_ptr_out, part2node_out, capacity, num_tiles, st, desc, scan_mode());
+                           part_size, part_ptr_out, part2node_out, capacity, rows_capacity, num_tiles, st, desc, scan_mode());
     EPPGCN_HIP(hipGetLastError());
     if (zero_tail) {
         hipLaunchKernelGGL(zero_tail1_kernel, dim3(static_cast<unsigned>((capacity + kTailWords - 1) / kTailWords)), dim3(256), 0,
                            stream, part_ptr_out, st->counts, 1, capacity);
+        EPPGCN_HIP(hipGetLastError());
+    }
+    return kOk;
+}
+
+// The first bytes of up to kStateList records on the device, kStateBytes each, into host memory that the device can write:
+// one launch and one wait for all of them, where a copy and a wait for each took 20 to 25 us a record.
+struct StateList { const uint32_t* from[kStateList]; };
+__global__ __launch_bounds__(256) void gather_states_kernel(StateList list, int count, uint32_t* __restrict__ to)
+{
+    constexpr int kWords = kStateBytes / 4;
+    for (int i = threadIdx.x; i < count * kWords; i += 256) to[i] = list.from[i / kWords][i % kWords];
+}
+
+int launch_gather_states(const void* const* states, int count, void* host, hipStream_t stream)
+{
+    uint32_t* to = static_cast<uint32_t*>(host);
+    for (int at = 0; at < count; at += kStateList) {
+        StateList list = {};
+        const int some = count - at < kStateList ? count - at : kStateList;
+        for (int i = 0; i < some; ++i) list.from[i] = static_cast<const uint32_t*>(states[at + i]);
+        hipLaunchKernelGGL(gather_states_kernel, dim3(1), dim3(256), 0, stream, list, some,
+                           to + static_cast<size_t>(at) * (kStateBytes / 4));
         EPPGCN_HIP(hipGetLastError());
     }
     return kOk;

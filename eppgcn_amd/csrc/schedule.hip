@@ -208,7 +208,8 @@ struct PlanScans {            // states of the look-back scans of one build, ins
 // one launch clears everything a build counts on being clear
 __global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanScans sc, uint32_t* __restrict__ single,
                                                         uint32_t* __restrict__ touched, int words, int num_parts,
-                                                        int num_slots, int num_nodes, int generation)
+                                                        int num_slots, int num_nodes, int generation,
+                                                        const ScanState* upstream)
 {
     const int stride = gridDim.x * blockDim.x;
     const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
@@ -221,6 +222,9 @@ __global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanSca
     }
     if (i0 == 0) {
         *sc.sort = ScanState{};
+        // groups of a split that stalled are not to be read: every kernel that would ends at this flag
+        if (upstream && (upstream->error || upstream->overflow || upstream->counts[0] != num_parts || upstream->counts[1] > num_slots))
+            sc.sort->error = 1;
         *sc.order = ScanState{};
         *sc.partials = ScanState{};
         StreamHeader z = {};
@@ -253,7 +257,7 @@ __device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ map, int row,
     if (((heads >> lane) & 1ull) && bits) atomicOr(map + word, bits);
 }
 
-// Per group p: rowp[p] (0 for an empty group), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the
+// Per group p: rowp[p] (0 for an empty group; rowp == nullptr: part2node is that array), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the
 // group has slots; the row bitmaps; the sort key and the digit counts of the first radix pass (keys == nullptr: the plan
 // keeps the caller's order).
 // Sort key of group p: the column block of its first slot, except that all groups of a short row
@@ -265,15 +269,17 @@ __device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ map, int row,
 // to 2x at 256 columns).
 // The walk to the ends of a row stops as soon as the row cannot be short any more: with the usual group sizes that is
 // after two or three groups, where a hub's groups walked 64 neighbours each way before (0.55 -> 0.28 ms for the 7.8 M
-// forward groups of R-MAT scale 22).  What is left is one 64-byte sector of `col` (and of `ids`) per group.
+// forward groups of R-MAT scale 22).  What is left is one cache line of `col` per group, and one of `ids` where the rows are
+// looked up there: 5.9 M groups of a path 347 us with ids, 172 with the rows that the split left (eppgcn_split_and_plan).
 constexpr int kMaxRowWalk = 64;
 __global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
     const int* __restrict__ part_ptr, const int* __restrict__ col, const int* __restrict__ part2node,
     const int* __restrict__ ids, int num_parts, int num_nodes, int shift, int keep_slots, int classes, int digits,
     int num_tiles, unsigned* __restrict__ keys, int* __restrict__ hist, int* __restrict__ rowp, uint8_t* __restrict__ info,
-    uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h)
+    uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h, const ScanState* sort_state)
 {
     __shared__ int s_hist[kDigits];
+    if (sort_state->error) return;
     s_hist[threadIdx.x] = 0;
     __syncthreads();
     const long long base = static_cast<long long>(blockIdx.x) * kSortTile;
@@ -310,7 +316,7 @@ __global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
         const bool some = end[r] > beg[r];
         const bool prev = some && before[r] == row[r], next = some && after[r] == row[r];
         if (have) {
-            rowp[p] = row[r];
+            if (rowp) rowp[p] = row[r];
             info[p] = static_cast<uint8_t>((prev ? 1 : 0) | (next ? 2 : 0) | (some ? 4 : 0));
             if (!some) h->empty_groups = 1;
         }
@@ -375,10 +381,11 @@ __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
     const int* __restrict__ part_ptr, const int* __restrict__ order, const int* __restrict__ rowp,
     const uint8_t* __restrict__ info, int num_parts, int num_slots, int num_tiles, PlanView plan, StreamView sv,
     int* __restrict__ src, int* __restrict__ ends_before, int* __restrict__ first, int* __restrict__ last,
-    int* __restrict__ event_of, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode)
+    int* __restrict__ event_of, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode, const ScanState* sort_state)
 {
     __shared__ int s_tile;
     __shared__ uint64_t s_sum[kPlanItems * kPlanWaves];
+    if (sort_state->error) return;
     const int tile = acquire_tile(st, &s_tile);
     if (tile >= num_tiles) return;
     const int lane = threadIdx.x & (kWave - 1);
@@ -739,6 +746,13 @@ size_t plan_workspace_bytes(long long num_parts, long long num_slots)
     return plan_temp(nullptr, num_parts, num_slots).bytes;
 }
 
+// Where a build keeps the row of every group: a caller that already knows the rows leaves them there and passes the
+// address as part2node.
+int* plan_rows_in_workspace(void* workspace, long long num_parts, long long num_slots)
+{
+    return plan_temp(static_cast<char*>(workspace), num_parts, num_slots).rowp;
+}
+
 int workspace_pitch(int dim);   // aggregate.hip
 
 static std::atomic<int> g_force_shift{0};     // process-wide knobs (tuning header), atomics like the ones below
@@ -800,7 +814,7 @@ static int last_plan_generation() { return g_plan_generation.load(); }
 
 int launch_build_plan(const int* part_ptr, const int* col, const int* part2node, const int* ids, int num_parts,
                       long long num_slots, int num_nodes, int shift, int dim, void* plan, size_t plan_size,
-                      void* workspace, size_t workspace_bytes, hipStream_t stream)
+                      void* workspace, size_t workspace_bytes, const ScanState* upstream, hipStream_t stream)
 {
     forget_stream_info(plan);
     int keep_rows, length_classes;
@@ -837,14 +851,14 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
     if (init_blocks > 512) init_blocks = 512;
     if (init_blocks < 8) init_blocks = 8;
     hipLaunchKernelGGL(plan_init_kernel, dim3(init_blocks), dim3(256), 0, stream, sv.header, t.scans, v.single, sv.touched, words,
-                       num_parts, slots, num_nodes, next_plan_generation());
+                       num_parts, slots, num_nodes, next_plan_generation(), upstream);
     EPPGCN_HIP(hipGetLastError());
     unsigned* keys_in = reinterpret_cast<unsigned*>(t.keys_a);
     unsigned* keys_out = reinterpret_cast<unsigned*>(t.keys_b);
     hipLaunchKernelGGL(plan_keys_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, part_ptr, col, part2node, ids,
                        num_parts, num_nodes, shift > 31 ? 31 : shift, keep_rows * 32, length_classes,
-                       passes ? 1 << pass_bits(0) : 1, sort_tiles, passes ? keys_in : nullptr, t.hist, t.rowp, t.info, v.single,
-                       sv.touched, sv.header);
+                       passes ? 1 << pass_bits(0) : 1, sort_tiles, passes ? keys_in : nullptr, t.hist,
+                       part2node == t.rowp ? nullptr : t.rowp, t.info, v.single, sv.touched, sv.header, t.scans.sort);
     EPPGCN_HIP(hipGetLastError());
     int* order = nullptr;
     int* spare = t.order_b;
@@ -873,7 +887,7 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
     t.tails_at = spare;
     hipLaunchKernelGGL(plan_order_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, part_ptr, order, t.rowp, t.info,
                        num_parts, slots, t.scans.order_tiles, v, sv, t.src, t.ends_before, t.first, t.last, t.event_of,
-                       t.tile_q, t.scans.order, t.scans.order_desc, scan_mode());
+                       t.tile_q, t.scans.order, t.scans.order_desc, scan_mode(), t.scans.sort);
     EPPGCN_HIP(hipGetLastError());
     if (padded > 0) {
         const int fill_tiles = static_cast<int>(tiles_of(padded, kFillTile));
@@ -940,18 +954,27 @@ int read_aggregation_status(hipStream_t stream)
     return kErrPlanMismatch;
 }
 
-// Synchronises the stream, reads the plan's header and records it; the return code tells whether a look-back scan
-// of the build stalled.
+const void* plan_header_address(const void* plan, long long num_parts, long long num_slots, long long num_nodes)
+{
+    return stream_view(const_cast<void*>(plan), num_parts, num_slots, num_nodes).header;
+}
+
+// Records the plan's header, which is read from the device with a wait for the stream unless the caller has a copy of it
+// (`read`, complete); the return code tells whether a look-back scan of the build stalled.
 int read_plan_status(const void* plan, long long num_parts, long long num_slots, long long num_nodes,
-                     long long* partial_rows, hipStream_t stream)
+                     long long* partial_rows, const void* read, hipStream_t stream)
 {
     if (partial_rows) *partial_rows = 0;
     if (num_parts <= 0) return kOk;
     StreamInfo info;
     info.num_parts = num_parts; info.num_slots = num_slots; info.num_nodes = num_nodes;
-    const StreamView sv = stream_view(const_cast<void*>(plan), num_parts, num_slots, num_nodes);
-    EPPGCN_HIP(hipMemcpyAsync(&info.header, sv.header, sizeof(StreamHeader), hipMemcpyDeviceToHost, stream));
-    EPPGCN_HIP(hipStreamSynchronize(stream));
+    if (read) {
+        memcpy(&info.header, read, sizeof(StreamHeader));
+    } else {
+        EPPGCN_HIP(hipMemcpyAsync(&info.header, plan_header_address(plan, num_parts, num_slots, num_nodes), sizeof(StreamHeader),
+                                  hipMemcpyDeviceToHost, stream));
+        EPPGCN_HIP(hipStreamSynchronize(stream));
+    }
     {   // the address of the mismatch mark on this device is looked up here, outside any graph capture
         int* words = nullptr;
         if (int rc = plan_fault_address(&words)) return rc;

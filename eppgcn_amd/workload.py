@@ -93,40 +93,52 @@ def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, 
 
     # mask chain, EPPGCN/gcn_main.py:130-139: step i runs in the forward of conv i
     marked = [None] * num_layers
+    known = max(1, int(backsize)) if backsize_mode == "constant" else 0      # the group size, where no count decides it
     for i in range(num_layers):
         src = train_mask if i == 0 else ngh_masks[i - 1]
         last = i == num_layers - 1
         k = num_layers - 1 - i
         marked[k] = capi.mark_path_begin(part2node, part_ptr, g.column_index, src, None if last else ngh_masks[i],
-                                         node_degs[k], last)
-    marked = [finish() for finish in marked]
+                                         node_degs[k], last, part_size=known)
+    early = bool(known) and not plan             # nothing but the counts themselves waits for the marking
+    if early:
+        marked += [capi.split_back_part_begin(node_degs[k], e, known) for k in range(num_layers)]
+    marked = capi.finish_all(marked)
+    marked, split = marked[:num_layers], marked[num_layers:]
 
     # buildBackPart, EPPGCN/gcn_main.py:151-168
     sizes = [choose_back_part_size(backsize_mode, backsize, valid_node, valid_len)
-             for _, _, valid_len, valid_node, _, _ in marked]
-    split = [capi.split_back_part_begin(node_degs[k], e, sizes[k]) for k in range(num_layers)]
-    split = [finish() for finish in split]
-    path_plans = [None] * num_layers
-    for k, (part_pointer, num_parts, covered) in enumerate(split):
-        ids, edge_list, valid_len = marked[k][:3]
-        assert covered == valid_len
-        # a heavily pruned path gathers from few distinct rows, which stay cached in any order: its
-        # plan keeps the groups in one block
-        if plan and num_parts > 0:
-            path_plans[k] = capi.build_plan_begin(part_pointer, edge_list, num_parts, valid_len, n,
-                                                  widths[min(k, len(widths) - 1)], ids=ids,
-                                                  block_shift=0 if 2 * valid_len >= e else 31)
+             for _, _, valid_len, valid_node, *_ in marked]
+    # a heavily pruned path gathers from few distinct rows, which stay cached in any order: its plan keeps the groups in one
+    # block
+    widths_of = [widths[min(k, len(widths) - 1)] for k in range(num_layers)]
+    shifts = [0 if 2 * marked[k][2] >= e else 31 for k in range(num_layers)]
+    path_plans, shared = [None] * num_layers, None
+    if plan and known:           # the marking has counted the groups: split and plan follow one another on the GPU
+        work = [capi.split_and_plan_begin(node_degs[k], marked[k][1], e, known, marked[k][6], marked[k][2], widths_of[k],
+                                          shifts[k]) if marked[k][6] > 0
+                else capi.split_back_part_begin(node_degs[k], e, known) for k in range(num_layers)]
+        done = capi.finish_all(work + ([forward_plan] if forward_plan else []))
+        split, shared = done[:num_layers], done[-1] if forward_plan else None
+        path_plans = [s[3] if len(s) > 3 else None for s in split]
+    elif not early:
+        split = capi.finish_all(capi.split_back_part_begin(node_degs[k], e, sizes[k]) for k in range(num_layers))
+        built = [k for k in range(num_layers) if plan and split[k][1] > 0]
+        work = [capi.build_plan_begin(split[k][0], marked[k][1], split[k][1], marked[k][2], n, widths_of[k],
+                                      ids=marked[k][0], block_shift=shifts[k]) for k in built]
+        done = capi.finish_all(work + ([forward_plan] if forward_plan else []))
+        shared = done[-1] if forward_plan else None
+        for k, built_plan in zip(built, done):
+            path_plans[k] = built_plan
     paths = []
     for k in range(num_layers):
-        ids, edge_list, valid_len, valid_node, bitmap, distinct = marked[k]
+        ids, edge_list, valid_len, valid_node, bitmap, distinct = marked[k][:6]
+        assert split[k][2] == valid_len
         # the pre-scaling pass of the gradient only has to cover the rows the path reads
         paths.append(BackwardPath(k + 1, ids, edge_list, split[k][0], node_degs[k], sizes[k], split[k][1],
-                                  valid_len, valid_node, path_plans[k] and path_plans[k](),
+                                  valid_len, valid_node, path_plans[k],
                                   bitmap if 2 * distinct < n else None))
-    plans = {}
-    if forward_plan:
-        shared = forward_plan()
-        plans = {w: shared for w in set(widths)}
+    plans = {w: shared for w in set(widths)} if shared else {}
     return Workload(g, ps, part_ptr, part2node, train_mask, ngh_masks, paths, plans)
 
 

@@ -347,6 +347,29 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
 int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
                             void* workspace, int64_t* counts, void* stream);
 
+/* eppgcn_mark_path that also counts the groups of at most part_size slots into which eppgcn_split_back_part will split the
+ * path (part_size 0: it does not), and never waits.  eppgcn_mark_path_group_counts: counts[4] (host) = kept slots, rows
+ * with node_degs != 0, gathered rows, groups; `state` is NULL (the call waits and reads the workspace) or the workspace's
+ * record as eppgcn_read_states has read it. */
+int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                            const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id,
+                            int32_t* out_edge, uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes,
+                            int is_last, int part_size, void* workspace, size_t workspace_bytes, void* stream);
+int eppgcn_mark_path_group_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
+                                  void* workspace, const void* state, int64_t* counts, void* stream);
+
+/* Counts of several calls with one wait.  A call that leaves its results on the device (eppgcn_mark_path_groups,
+ * eppgcn_split_back_part and eppgcn_split_and_plan, eppgcn_build_plan) has a record: the head of the (split) workspace, or
+ * eppgcn_plan_state(plan, sizes).  eppgcn_read_states copies `count` of them to `host` - memory that the device can write,
+ * e.g. from hipHostMalloc, eppgcn_state_bytes() for each - and synchronises the stream.  The ..._read functions and
+ * eppgcn_mark_path_group_counts say of such a copy what the functions without it say after a wait of their own. */
+size_t eppgcn_state_bytes(void);
+int eppgcn_read_states(const void* const* states, int count, void* host, void* stream);
+const void* eppgcn_plan_state(const void* plan, int num_parts, int64_t num_slots, int num_nodes);
+int eppgcn_plan_status_read(const void* plan, int num_parts, int64_t num_slots, int num_nodes, const void* state,
+                            int64_t* partial_rows);
+int eppgcn_split_counts_read(const void* state, int64_t* h_num_parts, int64_t* h_valid_len);
+
 /* Number of entries != 0 (valid_node of the group-size heuristics).  Stands in for
  * compact_count (cuCompactor.cu:694-696 over :623-680).  d_count: one device int. */
 int eppgcn_count_nonzero(const int32_t* node_deg, int64_t length, int32_t* d_count,
@@ -390,6 +413,17 @@ int eppgcn_split_back_part(const int32_t* node_deg, int num_nodes, int part_size
 /* Counts of an eppgcn_split_back_part call that was made without host pointers, from its workspace and on its stream:
  * synchronises the stream and reports what that call would have (a stalled scan, groups that did not fit). */
 int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_valid_len, void* stream);
+
+/* eppgcn_split_back_part followed by eppgcn_build_plan of the groups, without a wait between them, for a caller that knows
+ * the number of groups (eppgcn_mark_path_groups counts them): the row of every group goes from the split to the plan, which
+ * does not look it up among the ids of the slots.  The same group pointers and the same plan.  edge_list: the kept slots'
+ * columns; num_slots: how many; capacity: entries of part_pointer (cleared behind the groups).  The counts are read from
+ * split_workspace's record (eppgcn_read_states), and both it and the plan's are to be looked at before the plan is used: a
+ * split that stalled or found other counts leaves a plan that is refused. */
+int eppgcn_split_and_plan(const int32_t* node_deg, const int32_t* edge_list, int num_nodes, int part_size,
+                          int32_t* part_pointer, int64_t capacity, int num_parts, int64_t num_slots, int dim,
+                          int block_shift, void* plan, size_t plan_bytes, void* workspace, size_t workspace_bytes,
+                          void* split_workspace, size_t split_workspace_bytes, void* stream);
 
 /* Forward neighbour groups from the CSR row pointers (device): part_pointers[0..P]
  * (terminator = row_pointers[num_nodes]) and part2node[0..P-1]; `capacity` is the

@@ -100,3 +100,66 @@ def test_the_largest_plans(api, num_slots):
     for r in list(range(0, n, 97)) + [n - 2, n - 1]:
         count = torch.bincount(col[int(ptr[r]):int(ptr[r + 1])].long(), minlength=n).double()
         assert torch.equal(out[r].double(), count @ x.double()), r
+
+
+@pytest.mark.parametrize("n,ps", [(1, 4), (2047, 1), (2048, 3), (2049, 32), (9000, 8)])
+def test_split_and_plan_in_one_gives_what_the_two_give(api, n, ps):
+    """Around the tiles of the split, an empty row next to a hub: the same group pointers, and in every array the plan that
+    the ids of the slots give; a group count that is not the path's is refused."""
+    rng = np.random.default_rng(n)
+    deg = rng.integers(0, 6, n)
+    deg[rng.random(n) < 0.4] = 0
+    deg[n // 2] = 700                                  # written by a whole wave
+    degs = dev(deg, torch.int32)
+    slots, e = int(deg.sum()), int(deg.sum()) + 5      # five slots dropped by the marking
+    ids, col = dev(np.repeat(np.arange(n), deg), torch.int32), dev(rng.integers(0, n, e), torch.int32)
+    pointer, parts, covered = api.split_back_part(degs, e, ps)
+    assert (parts, covered) == (int((-(-deg // ps)).sum()), slots)
+    for shift in (0, 5, 31):
+        a = api.build_plan(pointer, col, parts, covered, n, 16, ids=ids, block_shift=shift)
+        one = api.split_and_plan_begin(degs, col, e, ps, parts, slots, 16, shift)
+        got = one() if shift else api.finish_all([one])[0]
+        assert torch.equal(got[0], pointer) and got[1:3] == (parts, slots)
+        b = got[3]
+        for x, y in zip(a.view(raw_col=True), b.view(raw_col=True)):
+            assert torch.equal(x, y)
+        sa, sb = a.stream_view(), b.stream_view()
+        assert a.partial_rows == b.partial_rows and sa["header"][:4].tolist() == sb["header"][:4].tolist()
+        events, _, fix = sa["header"][1:4].tolist()
+        used = {"col": None, "erow": events, "cev": None, "wtail": None, "touched": None, "frow": fix, "fptr": fix + 1}
+        for name, count in used.items():
+            assert torch.equal(sa[name][:count], sb[name][:count]), name
+    for wrong in {max(parts - 1, 1), parts + 1} - {parts}:
+        for shift in (5, 31):
+            with pytest.raises(api.EppgcnError):
+                api.split_and_plan_begin(degs, col, e, ps, wrong, slots, 16, shift)()
+
+
+def test_several_results_with_one_wait(api):
+    """finish_all gives what the calls give one by one: marking, splits and plans of two streams, an empty plan among them."""
+    indptr, col = csr_of(degrees_of("mixed"), 5)
+    n = indptr.size - 1
+    pp, p2n = [dev(x) for x in co.build_part(16, indptr)]
+    cold, src = dev(col), dev(np.arange(n) % 3 == 0)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+
+    def issue():
+        degs = torch.zeros(n, dtype=torch.int32, device="cuda")
+        work = [api.mark_path_begin(p2n, pp, cold, src, None, degs, True, part_size=7), api.split_back_part_begin(degs, col.size, 7),
+                api.build_plan_begin(pp, cold, 0, 0, n, 16, part2node=p2n),
+                api.build_plan_begin(pp, cold, p2n.numel(), col.size, n, 16, part2node=p2n)]
+        with torch.cuda.stream(side):
+            sdegs = torch.zeros(n, dtype=torch.int32, device="cuda")
+            work += [api.mark_path_begin(p2n, pp, cold, src, None, sdegs, True), api.build_plan_begin(pp, cold, p2n.numel(), col.size, n, 64, part2node=p2n)]
+        return work
+
+    together, single = api.finish_all(issue()), [w() for w in issue()]
+    assert together[0][2:4] == single[0][2:4] and together[0][5:] == single[0][5:]
+    assert together[0][6] == together[1][1] == single[1][1] and together[1][2] == together[0][2]
+    for k in (0, 4):
+        assert all(torch.equal(x, y) for x, y in zip(together[k][:2], single[k][:2])) and len(together[k]) == 7 - k // 4
+    assert torch.equal(together[1][0], single[1][0])
+    for k in (2, 3, 5):
+        assert together[k].partial_rows == single[k].partial_rows and together[k].num_parts == single[k].num_parts
+        assert torch.equal(together[k].view(raw_col=True)[3], single[k].view(raw_col=True)[3])
