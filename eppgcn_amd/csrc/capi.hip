@@ -53,6 +53,8 @@ size_t mark_path_workspace_bytes(long long, long long);
 size_t nll_workspace_bytes();
 int launch_nll_forward(float*, const float*, const long long*, const int*, long long, long long, int, void*, hipStream_t);
 int launch_nll_backward(float*, const float*, const float*, const int*, long long, long long, int, hipStream_t);
+int launch_adam(int, float* const*, const float* const*, float* const*, float* const*, const long long*, const double*, double,
+                double, double, double, hipStream_t);
 uint8_t* mark_path_scratch(void*, long long, long long);
 int launch_mark_path(const int*, const int*, const int*, const uint8_t*, uint8_t*, int*, int*, int*, uint32_t*, int,
                      long long, int, int, int, void*, hipStream_t);
@@ -111,7 +113,7 @@ using namespace eppgcn;
 extern "C" {
 
 const char* eppgcn_last_error(void) { return g_last_error.c_str(); }
-int eppgcn_abi_version(void) { return 18; }
+int eppgcn_abi_version(void) { return 19; }
 
 int eppgcn_spmm_forward(float* out, const float* in, const int32_t* row_pointers, const int32_t* column_index,
                         const float* degrees, const int32_t* part_pointers, const int32_t* part2node, int num_nodes,
@@ -371,6 +373,23 @@ int eppgcn_nll_backward(float* d_logits, const float* d_loss, const float* logit
     EPPGCN_REQUIRE(num_nodes == 0 || (d_logits && d_loss && logits && labels), "null pointer");
     return launch_nll_backward(d_logits, d_loss, logits, labels, num_rows, num_nodes, num_classes,
                                static_cast<hipStream_t>(stream));
+}
+
+int eppgcn_adam_step(int count, float* const* params, const float* const* grads, float* const* exp_avg,
+                     float* const* exp_avg_sq, const int64_t* sizes, const double* steps, double lr, double beta1,
+                     double beta2, double eps, void* stream)
+{
+    EPPGCN_REQUIRE(count >= 0, "negative count");
+    EPPGCN_REQUIRE(count == 0 || (params && grads && exp_avg && exp_avg_sq && sizes && steps), "null list");
+    for (int k = 0; k < count; ++k) {
+        EPPGCN_REQUIRE(sizes[k] >= 0 && steps[k] >= 1.0, "sizes must be >= 0 and steps >= 1");
+        EPPGCN_REQUIRE(sizes[k] == 0 || (params[k] && grads[k] && exp_avg[k] && exp_avg_sq[k]), "null pointer");
+        EPPGCN_REQUIRE(aligned(params[k], 4) && aligned(grads[k], 4) && aligned(exp_avg[k], 4) && aligned(exp_avg_sq[k], 4),
+                       "pointers must be 4-byte aligned");
+    }
+    static_assert(sizeof(long long) == sizeof(int64_t), "sizes are passed through");
+    return launch_adam(count, params, grads, exp_avg, exp_avg_sq, reinterpret_cast<const long long*>(sizes), steps, lr, beta1,
+                       beta2, eps, static_cast<hipStream_t>(stream));
 }
 
 size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes)

@@ -23,6 +23,8 @@
 //     kept); it affects speed only.
 #include <torch/extension.h>
 
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstdint>
@@ -474,6 +476,57 @@ Tensor nll_backward(Tensor d_loss, Tensor logits, Tensor labels, int64_t num_row
     return grad;
 }
 
+// ---------------------------------------------------------------- optimizer
+// One Adam step of all weights in one launch, in the rounding of torch's grouped operations; `steps` are the optimizer's CPU
+// counters.  False, with nothing changed, for weights, gradients or state of another form than fp32, contiguous and on one
+// GPU, for beta1 <= 0.5 (torch then rounds its average another way) and under graph capture (where torch's Adam asks for its
+// capturable form): the caller then takes torch's step.
+bool adam_step(const std::vector<Tensor>& params, const std::vector<Tensor>& grads, const std::vector<Tensor>& exp_avg,
+               const std::vector<Tensor>& exp_avg_sq, const std::vector<Tensor>& steps, double lr, double beta1, double beta2,
+               double eps)
+{
+    const size_t count = params.size();
+    if (count == 0 || grads.size() != count || exp_avg.size() != count || exp_avg_sq.size() != count || steps.size() != count)
+        return false;
+    if (!(beta1 > 0.5 && beta1 < 1.0 && beta2 >= 0.0 && beta2 < 1.0)) return false;
+    const auto device = params[0].device();
+    const auto plain = [&](const Tensor& t, const Tensor& p) {
+        return t.defined() && t.layout() == torch::kStrided && t.is_cuda() && t.device() == device &&
+               t.scalar_type() == torch::kFloat32 && t.is_contiguous() && t.sizes() == p.sizes() && !t.is_inference();
+    };
+    for (size_t k = 0; k < count; ++k) {
+        const Tensor& s = steps[k];
+        if (!plain(params[k], params[k]) || !plain(grads[k], params[k]) || !plain(exp_avg[k], params[k]) ||
+            !plain(exp_avg_sq[k], params[k]))
+            return false;
+        if (!s.defined() || s.layout() != torch::kStrided || !s.is_cpu() || s.scalar_type() != torch::kFloat32 ||
+            s.numel() != 1 || s.is_inference())
+            return false;
+        if (!(s.data_ptr<float>()[0] >= 0.f && s.data_ptr<float>()[0] < 16777215.f)) return false;
+    }
+    if (device.index() != c10::hip::current_device()) return false;
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return false;
+    std::vector<float*> p(count), m(count), v(count);
+    std::vector<const float*> g(count);
+    std::vector<int64_t> sizes(count);
+    std::vector<double> at(count);
+    for (size_t k = 0; k < count; ++k) {
+        p[k] = params[k].data_ptr<float>(), m[k] = exp_avg[k].data_ptr<float>(), v[k] = exp_avg_sq[k].data_ptr<float>();
+        g[k] = grads[k].data_ptr<float>();
+        sizes[k] = params[k].numel();
+        at[k] = static_cast<double>(steps[k].data_ptr<float>()[0]) + 1.0;
+    }
+    check(eppgcn_adam_step(static_cast<int>(count), p.data(), g.data(), m.data(), v.data(), sizes.data(), at.data(), lr, beta1,
+                           beta2, eps, stream_of(params[0])),
+          "adam_step");
+    for (size_t k = 0; k < count; ++k) {
+        steps[k].data_ptr<float>()[0] = static_cast<float>(at[k]);
+        // written behind torch's back: a graph that saved one of them has to see that it changed
+        for (const Tensor* t : {&params[k], &exp_avg[k], &exp_avg_sq[k], &steps[k]}) t->unsafeGetTensorImpl()->bump_version();
+    }
+    return true;
+}
+
 // ---------------------------------------------------------------- path preparation
 std::vector<Tensor> build_part(int partSize, Tensor indptr)
 {
@@ -680,6 +733,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           py::arg("rows"), py::arg("labels"));
     m.def("nll_backward", &nll_backward, "gradient of nll_forward (HIP)", py::arg("d_loss"), py::arg("logits"),
           py::arg("labels"), py::arg("num_rows"));
+    m.def("adam_step", &adam_step, "one Adam step of all weights in one launch (HIP); False: not this form, nothing changed");
     m.def("build_part", &build_part, "forward neighbour groups (HIP)");
     m.def("build_back_part", &build_back_part, "compaction + group split in one call (HIP)");
     m.def("compact_back_edge", &compact_back_edge, "compact the kept edges of one layer (HIP)");

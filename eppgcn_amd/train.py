@@ -10,6 +10,7 @@ from typing import List
 
 import torch
 import torch.nn.functional as F
+import torch.optim.optimizer as torch_optimizer
 
 from . import gnnadvisor, graphs
 from .gcn_conv import GCNConv
@@ -86,6 +87,12 @@ class Net(torch.nn.Module):
             if i < self.num_layers - 1 and not self.fuse_relu:
                 x = F.relu(x)
         return x
+
+
+def _step_hooks(opt):
+    """Where torch keeps the callables that run around an optimizer's step."""
+    return ((opt, "_optimizer_step_pre_hooks"), (opt, "_optimizer_step_post_hooks"),
+            (torch_optimizer, "_global_optimizer_pre_hooks"), (torch_optimizer, "_global_optimizer_post_hooks"))
 
 
 class Trainer:
@@ -195,6 +202,36 @@ class Trainer:
         logp = F.log_softmax(out.index_select(0, self.train_idx), dim=1)
         return -logp.gather(1, self.train_y.unsqueeze(1)).mean()
 
+    def _adam_in_one_launch(self):
+        """The optimizer's step in the library's kernel, with the rounding and the state of torch's own; False, with nothing
+        changed, when it is torch's to take: another optimizer or form of Adam, options, hooks or a scheduler on its step, a
+        first step (it makes the state), weights of another type or layout (``GNNA.adam_step`` looks at those)."""
+        opt = self.optimizer
+        if type(opt) is not torch.optim.Adam or "step" in vars(opt):
+            return False
+        if any(getattr(owner, name, True) for owner, name in _step_hooks(opt)) or len(opt.param_groups) != 1:
+            return False
+        group = opt.param_groups[0]
+        if (group["weight_decay"] or group["amsgrad"] or group["maximize"] or group["capturable"] or group["differentiable"]
+                or group["fused"] or group["foreach"] is False or type(group["lr"]) is not float):
+            return False
+        weights, grads, averages, squares, steps = [], [], [], [], []
+        for w in group["params"]:
+            if w.grad is None:
+                continue
+            state = opt.state.get(w)
+            if not state:
+                return False
+            weights.append(w)
+            grads.append(w.grad)
+            averages.append(state["exp_avg"])
+            squares.append(state["exp_avg_sq"])
+            steps.append(state["step"])
+        beta1, beta2 = group["betas"]
+        if type(beta1) is not float or type(beta2) is not float:
+            return False
+        return self.GNNA.adam_step(weights, grads, averages, squares, steps, group["lr"], beta1, beta2, group["eps"])
+
     def train_step(self, is_first_iter: bool, record_loss: bool = False, phase_timers: bool = True):
         """One epoch.  ``phase_timers`` keeps the reference's three host synchronisations per epoch
         that split the time into forward / loss / backward (EPPGCN/gcn_main.py:242,254,260); without
@@ -222,7 +259,8 @@ class Trainer:
         loss.backward()
         sync()
         self.back_time += time.perf_counter() - t
-        self.optimizer.step()
+        if not self._adam_in_one_launch():
+            self.optimizer.step()
         if record_loss:
             self.losses.append(float(loss.item()))
         return loss

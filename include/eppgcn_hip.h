@@ -255,6 +255,17 @@ int eppgcn_nll_backward(float* d_logits, const float* d_loss, const float* logit
                         int64_t num_nodes, int num_classes, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * One Adam step of `count` weights (no weight decay; EPPGCN/gcn_main.py:209 takes it from torch.optim.Adam):
+ *   exp_avg += (1 - beta1) (grad - exp_avg);  exp_avg_sq = beta2 exp_avg_sq + (1 - beta2) grad^2;
+ *   param -= lr / (1 - beta1^step) * exp_avg / (sqrt(exp_avg_sq) / sqrt(1 - beta2^step) + eps)
+ * The lists are host arrays of device pointers (weight k has sizes[k] contiguous floats); steps[k] >= 1 counts this step.
+ * The lists are read before the call returns.  The weights of one call must not overlap.
+ * ------------------------------------------------------------------------- */
+int eppgcn_adam_step(int count, float* const* params, const float* const* grads, float* const* exp_avg,
+                     float* const* exp_avg_sq, const int64_t* sizes, const double* steps, double lr, double beta1,
+                     double beta2, double eps, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Execution-path preparation.
  * ------------------------------------------------------------------------- */
 

@@ -1,0 +1,120 @@
+"""Adam in one launch against torch's own step: the same bits in weights and state, and torch's step for every other form."""
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(shapes, lr=0.01, **options):
+    gen = torch.Generator().manual_seed(7)
+    start = [torch.randn(s, generator=gen) for s in shapes]
+    sides = []
+    for _ in range(2):
+        weights = [torch.nn.Parameter(w.clone().cuda()) for w in start]
+        sides.append((weights, torch.optim.Adam(weights, lr=lr, **options)))
+    return sides, gen
+
+
+def _call(opt, weights):
+    from eppgcn_amd import gnnadvisor
+    group, states = opt.param_groups[0], [opt.state[w] for w in weights]
+    return gnnadvisor().adam_step(list(weights), [w.grad for w in weights], [s["exp_avg"] for s in states],
+                                  [s["exp_avg_sq"] for s in states], [s["step"] for s in states], group["lr"],
+                                  *group["betas"], group["eps"])
+
+
+def _same(one, other):
+    for (a, oa), (b, ob) in [(x, y) for x, y in zip(one, other)]:
+        assert torch.equal(a, b)
+        for key in ("step", "exp_avg", "exp_avg_sq"):
+            assert torch.equal(oa[key], ob[key]), key
+
+
+def _states(side):
+    weights, opt = side
+    return [(w.detach(), opt.state[w]) for w in weights]
+
+
+@pytest.mark.parametrize("shapes", [[(1,)], [(96, 16), (16, 22)], [(255,), (256,), (257,)], [(3, 5)] * 33, [(0, 4), (4, 4)],
+                                    [(2048 * 256 + 1,)]], ids=["one", "model", "block", "two_launches", "empty", "strided"])
+@pytest.mark.parametrize("options", [{}, {"betas": (0.6, 0.9), "eps": 1e-4}], ids=["default", "betas"])
+def test_weights_and_state_have_the_bits_of_torch(shapes, options):
+    # gradients from 1e-25 (squares below the normal range) to 1e6, zeros, and one NaN and infinity
+    (ours, theirs), gen = _pair(shapes, **options)
+    for step in range(6):
+        for a, b in zip(ours[0], theirs[0]):
+            g = torch.randn(a.shape, generator=gen) * 10.0 ** torch.randint(-25, 7, a.shape, generator=gen)
+            g[torch.rand(a.shape, generator=gen) < 0.1] = 0.0
+            a.grad, b.grad = g.cuda(), g.cuda()
+        versions = [w._version for w in ours[0]]
+        if step == 0:
+            ours[1].step()
+        else:
+            assert _call(ours[1], ours[0])
+        theirs[1].step()
+        assert all(w._version > v for w, v in zip(ours[0], versions))
+        _same(_states(ours), _states(theirs))
+    if ours[0][0].numel() > 1:
+        for w in (ours[0][0], theirs[0][0]):
+            w.grad.view(-1)[0], w.grad.view(-1)[-1] = float("nan"), float("inf")
+        assert _call(ours[1], ours[0])
+        theirs[1].step()
+        for a, b in zip(ours[0], theirs[0]):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+
+
+@pytest.mark.parametrize("spoil", ["double", "strided", "beta1", "gpu_step", "count"])
+def test_other_forms_are_left_to_torch_unchanged(spoil):
+    (ours, _), gen = _pair([(8, 6), (5,)], betas=(0.5, 0.9) if spoil == "beta1" else (0.9, 0.999))
+    weights, opt = ours
+    for w in weights:
+        w.grad = torch.randn(w.shape, generator=gen).cuda()
+    opt.step()
+    if spoil == "double":
+        opt.state[weights[0]]["exp_avg"] = opt.state[weights[0]]["exp_avg"].double()
+    elif spoil == "strided":
+        weights[0].grad = torch.randn(6, 8, generator=gen).cuda().t()
+    elif spoil == "gpu_step":
+        opt.state[weights[1]]["step"] = opt.state[weights[1]]["step"].cuda()
+    elif spoil == "count":
+        from eppgcn_amd import gnnadvisor
+        assert not gnnadvisor().adam_step([], [], [], [], [], 0.01, 0.9, 0.999, 1e-8)
+        return
+    before = [(w.detach().clone(), {k: v.clone() for k, v in opt.state[w].items()}) for w in weights]
+    assert not _call(opt, weights)
+    _same(before, _states((weights, opt)))
+
+
+@pytest.mark.parametrize("option", ["plain", "hook", "scheduler", "decay", "sgd", "no_grad"])
+def test_trainer_takes_the_step_its_optimizer_says(option):
+    from eppgcn_amd import graphs, train
+    tr = train.Trainer(graphs.uniform_graph(300, 900, seed=1, device="cuda"), labels="uniform")
+    calls = []
+    if option == "decay":
+        tr.optimizer = torch.optim.Adam(tr.model.parameters(), lr=0.01, weight_decay=0.1)
+    elif option == "sgd":
+        tr.optimizer = torch.optim.SGD(tr.model.parameters(), lr=0.01)
+    elif option == "hook":
+        tr.optimizer.register_step_post_hook(lambda *a: calls.append(a))
+    elif option == "scheduler":
+        scheduler = torch.optim.lr_scheduler.ExponentialLR(tr.optimizer, 0.5)
+    tr.train_step(True)
+    if option == "scheduler":
+        scheduler.step()
+    weights = list(tr.model.parameters())
+    if option == "no_grad":
+        weights[0].requires_grad_(False)
+    copies = [torch.nn.Parameter(w.detach().clone()) for w in weights]
+    other = type(tr.optimizer)(copies, **{k: v for k, v in tr.optimizer.defaults.items()})
+    other.load_state_dict(copy.deepcopy(tr.optimizer.state_dict()))
+    tr.train_step(False)
+    for w, c in zip(weights, copies):
+        c.grad = None if w.grad is None else w.grad.clone()
+    other.step()
+    assert all(torch.equal(w, c) for w, c in zip(weights, copies))
+    assert len(calls) == (2 if option == "hook" else 0)
+    assert other.state_dict()["state"].keys() == tr.optimizer.state_dict()["state"].keys()
+    for k, s in tr.optimizer.state_dict()["state"].items():
+        assert all(torch.equal(s[n], other.state_dict()["state"][k][n]) for n in s if torch.is_tensor(s[n]))
