@@ -19,8 +19,8 @@
 //     (large paths) it returns the group size of the rule fitted for the wave64 kernels;
 //   - get_ginfo also accepts a CPU tensor, as the reference's host loop does;
 //   - the module keeps, per group array it has seen, a column-blocked execution plan for the
-//     aggregation kernels (built on first use, about 4 bytes per edge, the 8 most recently used
-//     kept); it affects speed only.
+//     aggregation kernels (built on first use, about 4 bytes per edge, the most recently used
+//     kept: eight, and more while they are small); it affects speed only.
 #include <torch/extension.h>
 
 #include <c10/hip/HIPFunctions.h>
@@ -28,6 +28,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <cstdint>
+#include <iterator>
 #include <list>
 #include <vector>
 
@@ -79,13 +80,25 @@ Tensor workspace(size_t bytes, const Tensor& like)
 // ---------------------------------------------------------------- plan cache
 // The column-blocked execution plan depends only on the groups and the column ids, which a
 // training run passes unchanged every epoch.  Entries are keyed by storage address, length,
-// tensor version and block-size class, and hold references to the key tensors so that an
-// address cannot be reused for other data while its entry lives.
+// tensor version and block-size class; an entry holds its key tensors, or (behind the eight used last) is valid only while
+// their storages live, so that an address cannot be reused for other data while its entry is valid.
 // Staleness rule: an entry is invalidated by writes that bump torch's version counter (ordinary
 // in-place tensor operations).  A writer that bypasses the counter - `.data` / detach() in-place
 // operations, a raw-pointer kernel of another extension, this library's own C ABI writing into the
 // same storage - leaves the cached plan describing the old groups; after such a write call
 // clear_plans() before the next layer operation.
+size_t held_bytes(const Tensor& t) { return t.defined() ? t.storage().nbytes() : 0; }
+
+// A key tensor of an entry.  As long as it is held, or its storage lives by somebody else's hand, the address the entry was
+// made for cannot hold other data.
+struct Key {
+    Tensor held;
+    c10::weak_intrusive_ptr<c10::StorageImpl> storage;
+    explicit Key(const Tensor& t) : held(t), storage(t.storage().getWeakStorageImpl()) {}
+    bool alive() const { return held.defined() || !storage.expired(); }
+    size_t bytes() const { return held_bytes(held); }
+};
+
 struct PlanEntry {
     const void* part_ptr;
     const void* col;
@@ -94,17 +107,41 @@ struct PlanEntry {
     int64_t num_nodes;          // the plan's layout depends on it
     int64_t version_part, version_col, version_rows;
     int dim_class;
-    Tensor keep_part, keep_col, keep_rows, plan;
+    Key keep_part, keep_col, keep_rows;
+    Tensor plan;
     const void* plan_ptr;
+    size_t bytes() const { return keep_part.bytes() + keep_col.bytes() + keep_rows.bytes() + held_bytes(plan); }
+    bool alive() const { return keep_part.alive() && keep_col.alive() && keep_rows.alive(); }
+    void let_go() { keep_part.held.reset(), keep_col.held.reset(), keep_rows.held.reset(); }
 };
 std::list<PlanEntry> g_plans;
-constexpr size_t kMaxPlans = 8;
+// What the two caches of this file keep: the eight entries used last, whatever their size, and behind them up to 56 more
+// whose key tensors live by their owner's hand, while all of a cache together hold at most 256 MB of device memory.  Eight
+// alone were less than the layers of a few live models: three models of four layers trained in turn looked every path over
+// again in every backward call, two host waits each - 628 us an epoch at 19 717 vertices instead of 369.
+constexpr size_t kAlwaysKept = 8, kMostKept = 64, kKeptBytes = size_t(256) << 20;
+template <class Cache, class Drop>
+void trim(Cache& cache, const Drop& drop)
+{
+    size_t bytes = 0, place = 0;
+    for (auto it = cache.begin(); it != cache.end();) {
+        if (place >= kAlwaysKept) it->let_go();
+        const size_t here = it->bytes();
+        if (place < kAlwaysKept || (place < kMostKept && bytes + here <= kKeptBytes && it->alive())) {
+            bytes += here;
+            ++place;
+            ++it;
+        } else {
+            drop(*it);
+            it = cache.erase(it);
+        }
+    }
+}
 // An entry that leaves the cache gives its plan's memory back to torch: the library is told first, so that it
 // forgets the header it read at that address.
-void drop_oldest_plan()
+void trim_plans()
 {
-    eppgcn_plan_release(g_plans.back().plan_ptr);
-    g_plans.pop_back();
+    trim(g_plans, [](const PlanEntry& e) { eppgcn_plan_release(e.plan_ptr); });
 }
 void drop_all_plans()
 {
@@ -136,15 +173,19 @@ const void* plan_for(const Tensor& part_ptr, const Tensor& col, const Tensor& ro
             it->num_parts == num_parts && it->num_nodes == num_nodes && it->dim_class == dc &&
             it->version_part == static_cast<int64_t>(part_ptr._version()) &&
             it->version_col == static_cast<int64_t>(col._version()) &&
-            it->version_rows == static_cast<int64_t>(rows._version())) {
-            g_plans.splice(g_plans.begin(), g_plans, it);   // most recently used first
+            it->version_rows == static_cast<int64_t>(rows._version()) && it->alive()) {
+            if (it != g_plans.begin()) {                    // most recently used first
+                it->keep_part.held = part_ptr, it->keep_col.held = col, it->keep_rows.held = rows;
+                g_plans.splice(g_plans.begin(), g_plans, it);
+                if (g_plans.size() > kAlwaysKept) std::next(g_plans.begin(), kAlwaysKept)->let_go();
+            }
             return g_plans.front().plan_ptr;
         }
     }
     if (num_slots < 0) num_slots = part_ptr[num_parts].item<int64_t>();   // slots the groups cover (one 4-byte read)
     PlanEntry e{part_ptr.data_ptr(), col.data_ptr(), rows.data_ptr(), num_parts, num_nodes,
                 static_cast<int64_t>(part_ptr._version()), static_cast<int64_t>(col._version()),
-                static_cast<int64_t>(rows._version()), dc, part_ptr, col, rows, Tensor(), nullptr};
+                static_cast<int64_t>(rows._version()), dc, Key(part_ptr), Key(col), Key(rows), Tensor(), nullptr};
     const size_t bytes = eppgcn_plan_bytes(num_parts, num_slots, num_nodes);
     void* base = nullptr;
     e.plan = aligned_bytes(bytes, part_ptr, &base);
@@ -162,7 +203,7 @@ const void* plan_for(const Tensor& part_ptr, const Tensor& col, const Tensor& ro
     check(eppgcn_plan_status(base, static_cast<int>(num_parts), num_slots, num_nodes, nullptr, stream_of(part_ptr)),
           "build_plan");
     g_plans.push_front(std::move(e));
-    if (g_plans.size() > kMaxPlans) drop_oldest_plan();
+    trim_plans();
     return g_plans.front().plan_ptr;
 }
 
@@ -172,14 +213,18 @@ const void* plan_for(const Tensor& part_ptr, const Tensor& col, const Tensor& ro
 //   - the bitmap of the rows it gathers, when they are fewer than half of the vertices: the
 //     pre-scaling pass of the gradient then touches those rows only.
 // An entry is valid for exactly the tensors it was made from (same storage, same version counters);
-// it holds references to them so that their memory cannot be handed to other tensors meanwhile.
+// see Key for why their memory cannot be handed to other tensors meanwhile.
 struct PathChoice {
     const void* part_ptr;
     const void* edge_ptr;
     int64_t num_parts, num_nodes;
     int64_t version_part, version_edge;
     bool use_plan;
-    Tensor keep_part, keep_edge, gathered;     // gathered: undefined when the path reads most rows
+    Key keep_part, keep_edge;
+    Tensor gathered;                           // undefined when the path reads most rows
+    size_t bytes() const { return keep_part.bytes() + keep_edge.bytes() + held_bytes(gathered); }
+    bool alive() const { return keep_part.alive() && keep_edge.alive(); }
+    void let_go() { keep_part.held.reset(), keep_edge.held.reset(); }
 };
 std::list<PathChoice> g_path_choices;
 
@@ -191,8 +236,12 @@ const PathChoice& path_choice(const Tensor& part_pointer, const Tensor& edge_lis
         if (it->part_ptr == part_pointer.data_ptr() && it->edge_ptr == edge_list.data_ptr() &&
             it->num_parts == num_parts && it->num_nodes == num_nodes &&
             it->version_part == static_cast<int64_t>(part_pointer._version()) &&
-            it->version_edge == static_cast<int64_t>(edge_list._version())) {
-            g_path_choices.splice(g_path_choices.begin(), g_path_choices, it);
+            it->version_edge == static_cast<int64_t>(edge_list._version()) && it->alive()) {
+            if (it != g_path_choices.begin()) {
+                it->keep_part.held = part_pointer, it->keep_edge.held = edge_list;
+                g_path_choices.splice(g_path_choices.begin(), g_path_choices, it);
+                if (g_path_choices.size() > kAlwaysKept) std::next(g_path_choices.begin(), kAlwaysKept)->let_go();
+            }
             return g_path_choices.front();
         }
     }
@@ -201,7 +250,7 @@ const PathChoice& path_choice(const Tensor& part_pointer, const Tensor& edge_lis
     TORCH_CHECK(valid_len >= 0 && valid_len <= edge_list.numel(), "partPointer[numParts] lies outside edgeList");
     PathChoice c{part_pointer.data_ptr(), edge_list.data_ptr(), num_parts, num_nodes,
                  static_cast<int64_t>(part_pointer._version()), static_cast<int64_t>(edge_list._version()),
-                 g_plan_policy > 0 || 2 * valid_len >= edge_list.numel(), part_pointer, edge_list, Tensor()};
+                 g_plan_policy > 0 || 2 * valid_len >= edge_list.numel(), Key(part_pointer), Key(edge_list), Tensor()};
     auto bitmap = torch::empty({(static_cast<int64_t>(num_nodes) + 31) / 32 + 1}, edge_list.options());
     int64_t distinct = 0;
     const size_t scratch_bytes = eppgcn_mark_gathered_rows_scratch_bytes(num_nodes);
@@ -213,7 +262,7 @@ const PathChoice& path_choice(const Tensor& part_pointer, const Tensor& edge_lis
           "mark_gathered_rows");
     if (2 * distinct < num_nodes) c.gathered = bitmap;
     g_path_choices.push_front(std::move(c));
-    if (g_path_choices.size() > 8) g_path_choices.pop_back();
+    trim(g_path_choices, [](const PathChoice&) {});
     return g_path_choices.front();
 }
 
@@ -728,6 +777,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("set_plan_policy", [](int policy) { g_plan_policy = policy; drop_all_plans(); g_path_choices.clear(); },
           "execution plans: 0 = where the feature table outgrows the caches (default), 1 = always, -1 = never");
     m.def("cached_plans", []() { return static_cast<int>(g_plans.size()); }, "number of execution plans held");
+    m.def("cached_paths", []() { return static_cast<int>(g_path_choices.size()); }, "number of backward paths remembered");
 
     m.def("nll_forward", &nll_forward, "mean negative log-likelihood of the training rows (HIP)", py::arg("logits"),
           py::arg("rows"), py::arg("labels"));

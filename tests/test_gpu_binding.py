@@ -2,6 +2,8 @@
 twelve reference exports with their positional signatures, error behaviour (raise, never abort),
 gradients against a dense float64 model, and the end-to-end loss trajectory against the host-CPU
 sparse trainer."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -596,3 +598,33 @@ def test_entry_point_smoke_runs():
     of the suite, so that a change of the library's contracts cannot leave it behind."""
     import __graft_entry__ as entry
     entry.smoke()
+
+
+def test_paths_of_several_live_models_are_all_remembered_and_large_ones_are_not():
+    """Twelve paths of three models are small enough to be kept together; of paths that hold 64 MB each eight are."""
+    from eppgcn_amd import gnnadvisor, graphs, train
+    GNNA = gnnadvisor()
+    GNNA.clear_plans()
+    trainers = [train.Trainer(graphs.uniform_graph(500, 1500, seed=s, device="cuda"), num_layers=4) for s in range(3)]
+    for first in (True, False):
+        for tr in trainers:
+            tr.train_step(first)
+    assert GNNA.cached_paths() == 12
+    # a fourth model: the paths of one that is gone leave, those of the three others stay
+    del trainers[0]
+    gc.collect()
+    trainers.append(train.Trainer(graphs.uniform_graph(500, 1500, seed=4, device="cuda"), num_layers=4))
+    trainers[-1].train_step(True)
+    assert GNNA.cached_paths() == 12
+    GNNA.clear_plans()
+    x, w = torch.ones(4, 8, device="cuda"), torch.ones(8, 8, device="cuda")
+    ones, ids = torch.ones(4, device="cuda"), torch.zeros(16, dtype=torch.int32, device="cuda")
+    bounds = [torch.tensor([0, 2], dtype=torch.int32, device="cuda") for _ in range(9)]
+    for k in range(9):
+        edges = torch.zeros(1 << 24, dtype=torch.int32, device="cuda")
+        edges[1] = k % 4
+        _, dw = GNNA.ours_backward(x * (k + 1), x, w, ids, bounds[k], edges, ones, 32, 1, 1, 1, 1)
+        assert torch.equal(dw, torch.full_like(dw, 2.0 * (k + 1)))
+        assert GNNA.cached_paths() == min(k + 1, 8)
+    GNNA.clear_plans()
+    assert GNNA.cached_paths() == 0
