@@ -35,7 +35,8 @@
 // How a plan is built (launch_build_plan), all on the device and without a host read-back:
 //   plan_init      clears the scan states, the two row bitmaps and the header
 //   plan_keys      per group, in the caller's order: row, adjacency, sort key, the digit counts of the first radix pass
-//   radix passes   stable least-significant-digit sort of (key, group index); none for a plan in one block
+//   radix passes   stable least-significant-digit sort of (key, group index), the last pass moves the groups' records; none
+//                  for a plan in one block
 //   plan_order     per plan entry: one look-back scan over (slots, piece ends) gives the slot offsets and the piece
 //                  numbers together; writes ptr / row / flags and the extent of every piece
 //   plan_fill      per 2048 slots: the column copy with the piece-end flags, cev, wtail preset
@@ -134,12 +135,18 @@ __global__ __launch_bounds__(kSortBlock) void radix_hist_kernel(const unsigned* 
         hist[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x] = s_hist[threadIdx.x];
 }
 
-// vals_in == nullptr: the value of element i is i (first pass); keys_out == nullptr: the last pass, whose keys nobody reads
+// vals_in == nullptr: the value of element i is i (first pass).  The last pass (rec_out) takes the records of the groups along
+// and leaves where each went in vals_out; nobody reads its keys.  A tile is 2048 groups in the caller's order, which go to one
+// run of neighbours per digit: this is the direction in which the records move in whole lines.  plan_order_kernel, which has
+// to take neighbours in sorted order, looked its groups up in four arrays before, each in lines of its own.  The builds of
+// R-MAT scale 22 (7.8 + 5.9 M groups sorted), us: plan_order 431 -> 191, this kernel 49 -> 118, plan_partials 215 -> 249 (it
+// reads the places); scale 20: 83 -> 53, 12 -> 23, 58 -> 64.
 __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigned* __restrict__ keys_in,
                                                                    const int* __restrict__ vals_in,
                                                                    unsigned* __restrict__ keys_out,
                                                                    int* __restrict__ vals_out, int n, int shift, int bits,
-                                                                   int num_tiles, const int* __restrict__ offsets)
+                                                                   int num_tiles, const int* __restrict__ offsets,
+                                                                   const int4* __restrict__ rec_in, int4* __restrict__ rec_out)
 {
     constexpr int kWaves = kSortBlock / kWave;
     __shared__ int s_count[kSortRounds * kWaves][kDigits];      // per (round, wave): elements of each digit
@@ -188,9 +195,15 @@ __global__ __launch_bounds__(kSortBlock) void radix_scatter_kernel(const unsigne
         if (i < n) {
             const unsigned d = (key[r] >> shift) & (digits - 1);
             const int dst = s_count[r * kWaves + wave][d] + rank[r];
-            if (dst >= 0 && dst < n) {                          // false only after a stalled scan
-                if (keys_out) keys_out[dst] = key[r];
-                vals_out[dst] = vals_in ? vals_in[i] : static_cast<int>(i);
+            const int val = vals_in ? vals_in[i] : static_cast<int>(i);
+            if (dst >= 0 && dst < n && val >= 0 && val < n) {   // false only after a stalled scan
+                if (rec_out) {
+                    rec_out[dst] = rec_in[val];
+                    vals_out[val] = dst;
+                } else {
+                    keys_out[dst] = key[r];
+                    vals_out[dst] = val;
+                }
             }
         }
     }
@@ -257,8 +270,15 @@ __device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ map, int row,
     if (((heads >> lane) & 1ull) && bits) atomicOr(map + word, bits);
 }
 
-// Per group p: rowp[p] (0 for an empty group; rowp == nullptr: part2node is that array), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the
-// group has slots; the row bitmaps; the sort key and the digit counts of the first radix pass (keys == nullptr: the plan
+// What plan_order_kernel needs of a group, 16 bytes that the sort moves: first slot, slots, row, number; bit 31 of the first two:
+// the row has groups before / after this one.
+__device__ __forceinline__ int4 pack_group(int beg, int size, int row, int p, bool before, bool after)
+{
+    return make_int4(beg | (before ? static_cast<int>(kStreamFlag) : 0), size | (after ? static_cast<int>(kStreamFlag) : 0), row, p);
+}
+
+// Per group p: rowp[p] (0 for an empty group; rowp == nullptr: part2node is that array), rec[p] (pack_group; nullptr: nothing is
+// sorted), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the group has slots; the row bitmaps; the sort key and the digit counts of the first radix pass (keys == nullptr: the plan
 // keeps the caller's order).
 // Sort key of group p: the column block of its first slot, except that all groups of a short row
 // (at most `keep_slots` slots in at most kMaxRowWalk groups) share the key of the row's first group:
@@ -276,7 +296,7 @@ __global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
     const int* __restrict__ part_ptr, const int* __restrict__ col, const int* __restrict__ part2node,
     const int* __restrict__ ids, int num_parts, int num_nodes, int shift, int keep_slots, int classes, int digits,
     int num_tiles, unsigned* __restrict__ keys, int* __restrict__ hist, int* __restrict__ rowp, uint8_t* __restrict__ info,
-    uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h, const ScanState* sort_state)
+    int4* __restrict__ rec, uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h, const ScanState* sort_state)
 {
     __shared__ int s_hist[kDigits];
     if (sort_state->error) return;
@@ -318,6 +338,7 @@ __global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
         if (have) {
             if (rowp) rowp[p] = row[r];
             info[p] = static_cast<uint8_t>((prev ? 1 : 0) | (next ? 2 : 0) | (some ? 4 : 0));
+            if (rec) rec[p] = pack_group(beg[r], some ? end[r] - beg[r] : 0, row[r], p, prev, next);
             if (!some) h->empty_groups = 1;
         }
         const bool in_range = some && row[r] >= 0 && row[r] < num_nodes;
@@ -373,15 +394,15 @@ static_assert(kPlanItems * kPlanWaves == kWave, "one wave scans the (round, wave
 constexpr int kFillTile = 2048;            // slots a workgroup of plan_fill_kernel writes
 static_assert(kFillTile % kStreamWave == 0 && kFillTile % kStreamChunk == 0, "cev and wtail entries belong to one fill tile");
 
-// Plan entry q holds group order[q] (order == nullptr: group q).  One scan carries (slots, piece ends) packed as
+// Plan entry q holds the group of rec[q] (rec == nullptr: group q).  One scan carries (slots, piece ends) packed as
 // ends * 2^31 + slots.  Piece e: first[e] = its first slot | bit 31 when the row has groups before it, last[e] = its last
-// slot, erow[e] = its row, event_of[p] = e for the group p that ends it and -1 for every other group.
+// slot, erow[e] = its row, event_at[q] = e for the entry q that ends it and -1 for every other entry.
 // tile_q[t] = the plan entry that holds slot t * kFillTile.
 __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
-    const int* __restrict__ part_ptr, const int* __restrict__ order, const int* __restrict__ rowp,
+    const int* __restrict__ part_ptr, const int4* __restrict__ rec, const int* __restrict__ rowp,
     const uint8_t* __restrict__ info, int num_parts, int num_slots, int num_tiles, PlanView plan, StreamView sv,
     int* __restrict__ src, int* __restrict__ ends_before, int* __restrict__ first, int* __restrict__ last,
-    int* __restrict__ event_of, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode, const ScanState* sort_state)
+    int* __restrict__ event_at, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode, const ScanState* sort_state)
 {
     __shared__ int s_tile;
     __shared__ uint64_t s_sum[kPlanItems * kPlanWaves];
@@ -391,36 +412,50 @@ __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
     const long long q0 = static_cast<long long>(tile) * kPlanTile + threadIdx.x;
-    int p[kPlanItems], left[kPlanItems], right[kPlanItems];      // group of the entry and of its neighbours (-1: none)
-    auto group_at = [&](long long q) {
-        if (q < 0 || q >= num_parts) return -1;
-        const int g = order ? order[q] : static_cast<int>(q);
-        return g >= 0 && g < num_parts ? g : 0;                   // out of range only after a stalled scan of the sort
-    };
-#pragma unroll
-    for (int r = 0; r < kPlanItems; ++r) {
-        const long long q = q0 + r * kPlanBlock;
-        p[r] = group_at(q);
-        left[r] = group_at(q - 1);
-        right[r] = group_at(q + 1);
-    }
+    int p[kPlanItems], side[kPlanItems];      // group of the entry; that of its neighbour in another wave (-1: none)
     int beg[kPlanItems], size[kPlanItems], row[kPlanItems];
-    unsigned f[kPlanItems];
+    unsigned f[kPlanItems];                   // bit 0: the row has groups before this one, 1: after it, 2: slots
+    auto side_of = [&](long long q) {         // entry of the neighbour in another wave
+        return lane == 0 ? q - 1 : lane == kWave - 1 ? q + 1 : -1;
+    };
+    if (rec) {
+        int4 g[kPlanItems];
 #pragma unroll
-    for (int r = 0; r < kPlanItems; ++r) {
-        const int g = p[r];
-        beg[r] = g >= 0 ? part_ptr[g] : 0;
-        size[r] = g >= 0 ? part_ptr[g + 1] : 0;
-        row[r] = g >= 0 ? rowp[g] : 0;
-        f[r] = g >= 0 ? info[g] : 0u;
+        for (int r = 0; r < kPlanItems; ++r) {
+            const long long q = q0 + r * kPlanBlock, n = side_of(q);
+            g[r] = q < num_parts ? rec[q] : make_int4(0, 0, 0, -1);
+            side[r] = n >= 0 && n < num_parts ? rec[n].w : -1;
+        }
+#pragma unroll
+        for (int r = 0; r < kPlanItems; ++r) {
+            p[r] = g[r].w;
+            beg[r] = g[r].x & kStreamIdMask;
+            size[r] = g[r].y & kStreamIdMask;
+            row[r] = g[r].z;
+            f[r] = (g[r].x < 0 ? 1u : 0u) | (g[r].y < 0 ? 2u : 0u) | (size[r] > 0 ? 4u : 0u);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kPlanItems; ++r) {
+            const long long q = q0 + r * kPlanBlock, n = side_of(q);
+            const bool have = q < num_parts;
+            const int g = static_cast<int>(have ? q : 0);
+            p[r] = have ? g : -1;
+            side[r] = n >= 0 && n < num_parts ? static_cast<int>(n) : -1;
+            beg[r] = have ? part_ptr[g] : 0;
+            size[r] = have ? max(part_ptr[g + 1] - beg[r], 0) : 0;
+            row[r] = have ? rowp[g] : 0;
+            f[r] = have ? info[g] : 0u;
+        }
     }
     int at[kPlanItems], eb[kPlanItems];
     unsigned is_end = 0u;
 #pragma unroll
     for (int r = 0; r < kPlanItems; ++r) {
-        size[r] = max(size[r] - beg[r], 0);
-        const bool joins_left = (f[r] & 1u) && left[r] >= 0 && left[r] == p[r] - 1;
-        const bool joins_right = (f[r] & 2u) && right[r] >= 0 && right[r] == p[r] + 1;
+        const int up = __shfl_up(p[r], 1, kWave), down = __shfl_down(p[r], 1, kWave);
+        const int left = lane == 0 ? side[r] : up, right = lane == kWave - 1 ? side[r] : down;
+        const bool joins_left = (f[r] & 1u) && left >= 0 && left == p[r] - 1;
+        const bool joins_right = (f[r] & 2u) && right >= 0 && right == p[r] + 1;
         const bool ends = (f[r] & 4u) && !joins_right;
         f[r] = (f[r] & 3u) | (joins_left ? 4u : 0u) | (joins_right ? 8u : 0u);
         is_end |= ends ? 1u << r : 0u;
@@ -460,7 +495,7 @@ __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
         plan.flags[q] = static_cast<uint8_t>(f[r]);
         src[q] = beg[r];
         ends_before[q] = e;
-        event_of[p[r]] = ends ? e : -1;
+        event_at[q] = ends ? e : -1;
         if (size[r] == 0) continue;
         if ((f[r] & 4u) == 0 && e < num_parts) first[e] = slot | ((f[r] & 1u) ? static_cast<int>(kStreamFlag) : 0);
         if (ends && e < num_parts) {
@@ -568,13 +603,15 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ 
 
 // Which pieces leave partial sums, and how many: a piece that is not all of its row, or that crosses from one wave's
 // slots into the next, leaves one at its end, and one more per wave boundary it crosses (what that wave still holds at
-// its last slot).  Group p (in the caller's order) speaks for the piece it ends.  Two scans run side by side, wave 0's
-// over (tails, ends) packed as tails * 2^31 + ends, wave 1's over (rows with slots, rows with partial sums).
+// its last slot).  Group p (in the caller's order; plan entry place[p], nullptr: p) speaks for the piece it ends.  Two scans
+// run side by side, wave 0's over (tails, ends) packed as tails * 2^31 + ends, wave 1's over (rows with slots, rows with
+// partial sums).
 // The partial sums of row j of the fix list are numbered ends first, then tails: its range starts at ends + tails before
 // its first group.  fix_of[p] = j or -1; ends_at / tails_at[p] the counts before p; ends0 / tails0[j] those before row j.
 __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
-    const int* __restrict__ rowp, const uint8_t* __restrict__ info, const int* __restrict__ event_of,
-    const int* __restrict__ first, const int* __restrict__ last, int num_parts, int num_nodes, int num_tiles,
+    const int* __restrict__ rowp, const uint8_t* __restrict__ info, const int* __restrict__ place,
+    const int* __restrict__ event_at, int* __restrict__ event_of, const int* __restrict__ first,
+    const int* __restrict__ last, int num_parts, int num_nodes, int num_tiles,
     StreamView sv, int* __restrict__ fix_of, int* __restrict__ ends_at, int* __restrict__ tails_at,
     int* __restrict__ ends0, int* __restrict__ tails0, int* __restrict__ ends_total, PlanScans sc, unsigned mode)
 {
@@ -591,7 +628,8 @@ __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
 #pragma unroll
     for (int r = 0; r < kPlanItems; ++r) {
         const long long p = p0 + r * kPlanBlock;
-        e[r] = p < num_parts ? event_of[p] : -1;
+        const int q = p < num_parts ? (place ? place[p] : static_cast<int>(p)) : -1;
+        e[r] = q >= 0 && q < num_parts ? event_at[q] : -1;
         more[r] = p < num_parts && (info[p] & 2u) != 0;
     }
 #pragma unroll
@@ -660,6 +698,7 @@ __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
             tails_at[p] = ta;
         }
         fix_of[p] = j;
+        if (place) event_of[p] = e[r];
     }
 }
 
@@ -700,10 +739,11 @@ static size_t scan_state_bytes(long long n, int tile)
 
 static long long tiles_of(long long n, int tile) { return (n + tile - 1) / tile; }
 
-// Workspace of a build: ten arrays of num_parts + 1 ints (some used twice, the later use in brackets), the adjacency
-// bytes, the fill tiles' first entries, the radix histogram and its offsets, the scan states.
+// Workspace of a build: ten arrays of num_parts + 1 ints (some used twice, the later use in brackets), the sorted records, the
+// adjacency bytes, the fill tiles' first entries, the radix histogram and its offsets, the scan states.
 struct PlanTemp {
-    int *keys_a, *keys_b, *order_a, *order_b, *rowp, *src, *ends_before, *first, *last, *event_of;
+    int *keys_a, *keys_b, *order_a, *order_b, *rowp, *src, *ends_before, *first, *last, *event_at;
+    int4 *rec_in, *rec_out;         // rec_in = src, ends_before, first, last (written after the sort)
     int *fix_of, *ends_at, *tails_at, *ends0, *tails0;      // = keys_a, keys_b, the spare order array, src, ends_before
     uint8_t* info;
     int *tile_q, *hist, *offsets, *ends_total;
@@ -716,7 +756,7 @@ static PlanTemp plan_temp(char* base, long long num_parts, long long num_slots)
     size_t at = 0;
     auto take = [&](size_t bytes) { char* p = base + at; at += align256(bytes); return p; };
     const size_t slab = sizeof(int) * (static_cast<size_t>(num_parts) + 1);
-    int** arrays[] = {&t.keys_a, &t.keys_b, &t.order_a, &t.order_b, &t.rowp, &t.src, &t.ends_before, &t.first, &t.last, &t.event_of};
+    int** arrays[] = {&t.keys_a, &t.keys_b, &t.order_a, &t.order_b, &t.rowp, &t.src, &t.ends_before, &t.first, &t.last, &t.event_at};
     for (int** a : arrays) *a = reinterpret_cast<int*>(take(slab));
     t.info = reinterpret_cast<uint8_t*>(take(static_cast<size_t>(num_parts)));
     t.tile_q = reinterpret_cast<int*>(take(sizeof(int) * static_cast<size_t>(tiles_of(stream_padded_slots(num_slots), kFillTile) + 1)));
@@ -733,6 +773,8 @@ static PlanTemp plan_temp(char* base, long long num_parts, long long num_slots)
     state(&t.scans.partials, &t.scans.ends_desc, num_parts, kPlanTile);
     t.scans.rows_desc = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * static_cast<size_t>(tiles_of(num_parts, kPlanTile))));
     t.ends_total = reinterpret_cast<int*>(take(sizeof(int)));
+    t.rec_in = reinterpret_cast<int4*>(t.src);                  // four slabs in a row
+    t.rec_out = reinterpret_cast<int4*>(take(4 * slab));
     t.scans.order_tiles = static_cast<int>(tiles_of(num_parts, kPlanTile));
     t.scans.sort_tiles = 0;
     t.fix_of = t.keys_a; t.ends_at = t.keys_b; t.tails_at = nullptr; t.ends0 = t.src; t.tails0 = t.ends_before;
@@ -858,12 +900,13 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
     hipLaunchKernelGGL(plan_keys_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, part_ptr, col, part2node, ids,
                        num_parts, num_nodes, shift > 31 ? 31 : shift, keep_rows * 32, length_classes,
                        passes ? 1 << pass_bits(0) : 1, sort_tiles, passes ? keys_in : nullptr, t.hist,
-                       part2node == t.rowp ? nullptr : t.rowp, t.info, v.single, sv.touched, sv.header, t.scans.sort);
+                       part2node == t.rowp ? nullptr : t.rowp, t.info, passes ? t.rec_in : nullptr, v.single, sv.touched, sv.header, t.scans.sort);
     EPPGCN_HIP(hipGetLastError());
-    int* order = nullptr;
+    int* order = nullptr;            // after the last pass: the plan entry of every group
     int* spare = t.order_b;
     for (int pass = 0; pass < passes; ++pass) {
         const int nb = pass_bits(pass), digits = 1 << nb;
+        const bool last_pass = pass + 1 == passes;
         const long long entries = static_cast<long long>(sort_tiles) * digits;
         const int scan_tiles = static_cast<int>(tiles_of(entries, kScanTile));
         if (pass > 0) {
@@ -877,29 +920,31 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
                            static_cast<int>(entries), scan_tiles, t.scans.sort, t.scans.sort_desc, scan_mode());
         EPPGCN_HIP(hipGetLastError());
         int* out = order == t.order_a ? t.order_b : t.order_a;
-        hipLaunchKernelGGL(radix_scatter_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, keys_in, order,
-                           pass + 1 < passes ? keys_out : nullptr, out, num_parts, 8 * pass, nb, sort_tiles, t.offsets);
+        hipLaunchKernelGGL(radix_scatter_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, keys_in, order, keys_out, out,
+                           num_parts, 8 * pass, nb, sort_tiles, t.offsets, t.rec_in, last_pass ? t.rec_out : nullptr);
         EPPGCN_HIP(hipGetLastError());
         unsigned* k = keys_in; keys_in = keys_out; keys_out = k;
         order = out;
         spare = out == t.order_a ? t.order_b : t.order_a;
     }
     t.tails_at = spare;
-    hipLaunchKernelGGL(plan_order_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, part_ptr, order, t.rowp, t.info,
-                       num_parts, slots, t.scans.order_tiles, v, sv, t.src, t.ends_before, t.first, t.last, t.event_of,
-                       t.tile_q, t.scans.order, t.scans.order_desc, scan_mode(), t.scans.sort);
+    hipLaunchKernelGGL(plan_order_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, part_ptr,
+                       passes ? t.rec_out : nullptr, t.rowp, t.info, num_parts, slots, t.scans.order_tiles, v, sv, t.src,
+                       t.ends_before, t.first, t.last, t.event_at, t.tile_q, t.scans.order, t.scans.order_desc, scan_mode(),
+                       t.scans.sort);
     EPPGCN_HIP(hipGetLastError());
+    int* event_of = passes ? reinterpret_cast<int*>(t.rec_out) : t.event_at;       // the records have been read
     if (padded > 0) {
         const int fill_tiles = static_cast<int>(tiles_of(padded, kFillTile));
         hipLaunchKernelGGL(plan_fill_kernel, dim3(fill_tiles), dim3(256), 0, stream, col, v, sv, t.src, t.ends_before, t.tile_q,
                            num_parts, slots, padded, num_nodes, fill_tiles, t.scans);
         EPPGCN_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(plan_partials_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, t.rowp, t.info, t.event_of,
-                       t.first, t.last, num_parts, num_nodes, t.scans.order_tiles, sv, t.fix_of, t.ends_at, t.tails_at,
+    hipLaunchKernelGGL(plan_partials_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, t.rowp, t.info, order, t.event_at,
+                       event_of, t.first, t.last, num_parts, num_nodes, t.scans.order_tiles, sv, t.fix_of, t.ends_at, t.tails_at,
                        t.ends0, t.tails0, t.ends_total, t.scans, scan_mode());
     EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(plan_targets_kernel, dim3((num_parts + 255) / 256), dim3(256), 0, stream, sv, t.event_of, t.first, t.last,
+    hipLaunchKernelGGL(plan_targets_kernel, dim3((num_parts + 255) / 256), dim3(256), 0, stream, sv, event_of, t.first, t.last,
                        t.fix_of, t.ends_at, t.tails_at, t.ends0, t.tails0, t.ends_total, num_parts, padded / kStreamWave, t.scans);
     EPPGCN_HIP(hipGetLastError());
     return kOk;
