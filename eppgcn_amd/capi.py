@@ -29,6 +29,7 @@ EXPORTS = [
     "eppgcn_state_bytes", "eppgcn_read_states", "eppgcn_plan_state", "eppgcn_plan_status_read", "eppgcn_split_counts_read",
     "eppgcn_split_and_plan",
     "eppgcn_nll_workspace_bytes", "eppgcn_nll_forward", "eppgcn_nll_backward", "eppgcn_adam_step",
+    "eppgcn_layer_forward",
     "eppgcn_set_plan_length_classes",
     "eppgcn_mark_gathered_rows", "eppgcn_set_wide_index", "eppgcn_wave64_back_part_size",
     "eppgcn_compact_back_edge_static", "eppgcn_compact_back_edge_static_max_length",
@@ -39,7 +40,7 @@ EXPORTS = [
     "eppgcn_mark_gathered_rows_scratch", "eppgcn_mark_gathered_rows_scratch_bytes",
 ]
 
-ABI_VERSION = 19      # what eppgcn_abi_version() of a matching library returns
+ABI_VERSION = 20      # what eppgcn_abi_version() of a matching library returns
 
 _lib = None
 
@@ -164,6 +165,8 @@ def load():
     lib.eppgcn_nll_forward.restype = i
     lib.eppgcn_nll_backward.argtypes = [p, p, p, p, i64, i64, i, p]
     lib.eppgcn_nll_backward.restype = i
+    lib.eppgcn_layer_forward.argtypes = [p, p, p, i, p, p, p, p, p, i, i, i, i, i, i, i, p, sz, p, p]
+    lib.eppgcn_layer_forward.restype = i
     lib.eppgcn_adam_step.argtypes = [i] + [C.POINTER(C.c_void_p)] * 4 + [C.POINTER(i64), C.POINTER(C.c_double)] + [C.c_double] * 4 + [p]
     lib.eppgcn_adam_step.restype = i
     lib.eppgcn_feature_workspace_pitch.argtypes = [i]

@@ -13,7 +13,7 @@ namespace eppgcn {
 
 // ---- implemented in aggregate.hip / prepare.hip
 int aggregate_forward_groups(float*, const float*, const int*, const float*, const int*, const int*, const void*, int,
-                             int, int, int, float*, size_t, hipStream_t, double*, double*);
+                             int, int, int, float*, size_t, hipStream_t, double*, double*, bool out_is_clear = false);
 int aggregate_compacted_groups(float*, const float*, const int*, const int*, const int*, const float*, const void*,
                                int, int, int, int, float*, size_t, const uint32_t*, hipStream_t, double*, double*,
                                const uint32_t** written = nullptr, long long* num_written = nullptr);
@@ -32,7 +32,8 @@ void set_agg_force_rounds(int);
 size_t feature_workspace_floats(long long, int);
 int workspace_pitch(int);
 int launch_dense_rows(float*, int, int, const float*, int, const float*, long long, long long, const float*,
-                      const float*, int, int, long long, int, int, hipStream_t, unsigned, const uint32_t* rows = nullptr);
+                      const float*, int, int, long long, int, int, hipStream_t, unsigned, const uint32_t* rows = nullptr,
+                      const RidingClear* clear = nullptr);
 size_t update_workspace_bytes(long long, int, int);
 int launch_dense_weight(float*, const float*, int, const float*, int, int, long long, int, int, void*, hipStream_t,
                         const uint32_t* rows = nullptr);
@@ -113,7 +114,7 @@ using namespace eppgcn;
 extern "C" {
 
 const char* eppgcn_last_error(void) { return g_last_error.c_str(); }
-int eppgcn_abi_version(void) { return 19; }
+int eppgcn_abi_version(void) { return 20; }
 
 int eppgcn_spmm_forward(float* out, const float* in, const int32_t* row_pointers, const int32_t* column_index,
                         const float* degrees, const int32_t* part_pointers, const int32_t* part2node, int num_nodes,
@@ -840,6 +841,37 @@ int eppgcn_update_forward_table(float* table, size_t table_floats, const float* 
     const int pitch = workspace_pitch(out_dim);
     return launch_dense_rows(table, pitch, pitch, x, in_dim, w, out_dim, 1, scale, nullptr, 0, relu_input ? 1 : 0,
                              num_nodes, in_dim, out_dim, static_cast<hipStream_t>(stream), kRowSwizzleMask);
+}
+
+int eppgcn_layer_forward(float* out, const float* x, const float* w, int relu_input, const int32_t* row_pointers,
+                         const int32_t* column_index, const float* degrees, const int32_t* part_pointers,
+                         const int32_t* part2node, int num_nodes, int in_dim, int out_dim, int num_parts, int part_size,
+                         int dim_worker, int warp_per_block, float* workspace, size_t workspace_floats, const void* plan,
+                         void* stream)
+{
+    const size_t words = static_cast<size_t>(num_nodes > 0 ? num_nodes : 0) * static_cast<size_t>(out_dim > 0 ? out_dim : 0);
+    // everything that either call refuses is refused before the first launch
+    const bool rides = !plan && num_nodes > 0 && in_dim > 0 && out_dim > 0 && num_parts > 0 && words <= kRidingClearWords &&
+                       !timing_enabled() && part_size > 0 && dim_worker > 0 && warp_per_block > 0 && out && aligned(out, 4) &&
+                       degrees && column_index && part_pointers && part2node && workspace && aligned(workspace, 16) &&
+                       workspace != out && x && w && aligned(x, 4) && aligned(w, 4) && x != out && w != out && workspace != x &&
+                       workspace_floats >= feature_workspace_floats(num_nodes, out_dim);
+    if (!rides) {
+        if (int rc = eppgcn_update_forward_table(workspace, workspace_floats, x, w, degrees, relu_input, num_nodes, in_dim,
+                                                 out_dim, stream))
+            return rc;
+        return eppgcn_spmm_forward(out, nullptr, row_pointers, column_index, degrees, part_pointers, part2node, num_nodes,
+                                   out_dim, num_parts, part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan,
+                                   stream);
+    }
+    const RidingClear clear = riding_clear(out, words);
+    const int pitch = workspace_pitch(out_dim);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int rc = launch_dense_rows(workspace, pitch, pitch, x, in_dim, w, out_dim, 1, degrees, nullptr, 0, relu_input ? 1 : 0,
+                                   num_nodes, in_dim, out_dim, s, kRowSwizzleMask, nullptr, &clear))
+        return rc;
+    return aggregate_forward_groups(out, nullptr, column_index, degrees, part_pointers, part2node, nullptr, num_nodes, out_dim,
+                                    num_parts, part_size, workspace, workspace_floats, s, &g_for_agg_ms, nullptr, true);
 }
 
 int64_t eppgcn_feature_workspace_row(int64_t vertex)

@@ -45,6 +45,35 @@ int hip_fail(hipError_t e, const char* what);
 // hipMemsetAsync everywhere so that every call of the library can be captured into a HIP graph
 // (memset nodes are the one node kind callers are told to avoid on this platform).
 int launch_zero_words(void* p, size_t words, hipStream_t stream);
+
+// The clear of a small output rides in the kernel that runs before the aggregation (it fills the table the aggregation reads):
+// workgroups behind those of that kernel's own work write the zeros.  For outputs of up to 16 MB, where the zeros cost about
+// what a launch costs; beyond, launch_zero_words writes them faster.  32 columns, one slot per row, us per call with a launch
+// of its own / riding: pruned backward 2.4 MB 15.5 / 12.5, 16 MB 16.5 / 12.4, 32 MB 20.9 / 20.7, 128 MB 71 / 87; forward of a
+// layer of 16 inputs 2.4 MB 11.4 / 8.2, 16 MB 16.4 / 13.5, 32 MB 22.0 / 20.3, 128 MB 69 / 84.
+struct RidingClear {
+    uint32_t* p = nullptr;      // 4-byte aligned
+    unsigned words = 0;
+    unsigned blocks = 0;        // workgroups that clear (0: nothing rides)
+};
+constexpr size_t kRidingClearWords = (16u << 20) / 4;
+inline RidingClear riding_clear(void* p, size_t words)
+{
+    const unsigned n = static_cast<unsigned>((words + 4095) / 4096);
+    return {static_cast<uint32_t*>(p), static_cast<unsigned>(words), n < 1 ? 1u : n > 1024 ? 1024u : n};
+}
+// workgroup `block` of c.blocks, any workgroup size
+__device__ __forceinline__ void clear_riding(const RidingClear& c, unsigned block)
+{
+    const unsigned misaligned = static_cast<unsigned>(reinterpret_cast<uintptr_t>(c.p) / 4 % 4);
+    const unsigned head = min(misaligned ? 4u - misaligned : 0u, c.words), vecs = (c.words - head) / 4;
+    const unsigned tid = block * blockDim.x + threadIdx.x, stride = c.blocks * blockDim.x;
+    uint4* v = reinterpret_cast<uint4*>(c.p + head);
+    for (unsigned i = tid; i < vecs; i += stride) v[i] = make_uint4(0u, 0u, 0u, 0u);
+    const unsigned tail = head + 4 * vecs;
+    if (tid < head) c.p[tid] = 0u;
+    if (tid < c.words - tail) c.p[tail + tid] = 0u;
+}
 // The streaming helper kernels index with 32 bits when the element count allows; true forces their
 // 64-bit instantiations at any size (so that tests reach them without 16 GB matrices).
 bool force_wide_index();

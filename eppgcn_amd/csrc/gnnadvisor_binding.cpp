@@ -284,20 +284,6 @@ int dense_support(const Tensor& X, const Tensor& W)
     return eppgcn_update_supported(static_cast<int>(X.size(1)), static_cast<int>(W.size(1)));
 }
 
-// scale[r] * act(X) * W as the padded, pre-scaled feature table the aggregation gathers from
-Tensor scaled_product(const Tensor& X, const Tensor& W, const Tensor& degrees, bool relu_input, const void* plan,
-                      size_t* ws_floats)
-{
-    const int64_t n = X.size(0);
-    const int dim = static_cast<int>(W.size(1));
-    *ws_floats = eppgcn_plan_workspace_floats(plan, n, dim);
-    auto scaled = torch::empty({static_cast<int64_t>(*ws_floats)}, X.options());
-    check(eppgcn_update_forward_table(scaled.data_ptr<float>(), *ws_floats, X.data_ptr<float>(), W.data_ptr<float>(), f32(degrees),
-                                      relu_input ? 1 : 0, n, static_cast<int>(X.size(1)), dim, stream_of(X)),
-          "update_forward_table");
-    return scaled;
-}
-
 // g_masked_update: 1 (default) lets the pruned backward hand the bitmap of the rows it wrote to the dense products
 // (rows outside the path are then neither cleared nor read); 0 clears and reads every row.
 int g_masked_update = 1;
@@ -376,12 +362,13 @@ std::vector<Tensor> forward(Tensor input, Tensor weight, Tensor row_pointers, Te
                                 static_cast<int>(n), dim);
     if (n > 0 && (dense_support(input, weight) & 1)) {
         // the product is written scaled and padded, ready to be gathered: no separate scaling pass
-        size_t ws_floats = 0;
-        auto scaled = scaled_product(input, weight, degrees, relu_input, plan, &ws_floats);
-        check(eppgcn_spmm_forward(output.data_ptr<float>(), nullptr, i32(row_pointers), i32(column_index),
-                                  f32(degrees), i32(part_pointers), i32(part2Node), static_cast<int>(n), dim,
-                                  static_cast<int>(part2Node.numel()), partSize, dimWorker, warpPerBlock,
-                                  scaled.data_ptr<float>(), ws_floats, plan, stream_of(input)),
+        const size_t ws_floats = eppgcn_plan_workspace_floats(plan, n, dim);
+        auto scaled = torch::empty({static_cast<int64_t>(ws_floats)}, input.options());
+        check(eppgcn_layer_forward(output.data_ptr<float>(), input.data_ptr<float>(), weight.data_ptr<float>(), relu_input ? 1 : 0,
+                                   i32(row_pointers), i32(column_index), f32(degrees), i32(part_pointers), i32(part2Node),
+                                   static_cast<int>(n), static_cast<int>(input.size(1)), dim,
+                                   static_cast<int>(part2Node.numel()), partSize, dimWorker, warpPerBlock,
+                                   scaled.data_ptr<float>(), ws_floats, plan, stream_of(input)),
               "forward");
         return {output};
     }

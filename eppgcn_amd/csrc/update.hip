@@ -93,12 +93,18 @@ struct RowsArgs {
                              // 16-byte aligned): they go through LDS and out as two 1 KB stores per wave
     unsigned swz_mask;       // row r of out lives at swizzled_row(r, swz_mask): 0 = vertex order (common.hpp)
     const uint32_t* rows;    // nullptr, or one bit per row of x: clear = the row counts as zeros and is not read
+    unsigned blocks;         // workgroups of the product; those behind them clear
+    RidingClear clear;
 };
 
 template <int VW, int MT, int CU, bool kRows>
 __global__ __launch_bounds__(kUpdateThreads) void dense_rows_kernel(RowsArgs a)
 {
     extern __shared__ __align__(16) float w_lds[];   // [MT][chunks_p][64 lanes][VW]
+    if (blockIdx.x >= a.blocks) {
+        clear_riding(a.clear, blockIdx.x - a.blocks);
+        return;
+    }
     const int chunks = (a.K + 4 * VW - 1) / (4 * VW);
     const int chunks_p = (chunks + CU - 1) / CU * CU;
     for (int idx = threadIdx.x; idx < MT * chunks_p * kWave * VW; idx += kUpdateThreads) {
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(kUpdateThreads) void dense_rows_kernel(RowsArgs a)
     const int i = lane % 16, j = lane / 16;
     const long long tiles = (a.n + kTileRows - 1) / kTileRows;
     for (long long tile = static_cast<long long>(blockIdx.x) * kUpdateWaves + wave; tile < tiles;
-         tile += static_cast<long long>(gridDim.x) * kUpdateWaves) {
+         tile += static_cast<long long>(a.blocks) * kUpdateWaves) {
         const long long r = tile * kTileRows + i;
         const bool row_ok = r < a.n;
         bool live = row_ok;
@@ -269,7 +275,8 @@ static hipError_t launch_rows_mt(const RowsArgs& a, int mt, int cu, unsigned blo
 // operand to fit the LDS (the caller then has to use a general GEMM).
 int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int ld_x, const float* w, long long sk,
                       long long sm, const float* scale, const float* relu_ref, int ld_ref, int relu_in,
-                      long long n, int K, int M, hipStream_t stream, unsigned swz_mask, const uint32_t* rows)
+                      long long n, int K, int M, hipStream_t stream, unsigned swz_mask, const uint32_t* rows,
+                      const RidingClear* clear)
 {
     if (n == 0 || out_cols == 0) return kOk;
     const uintptr_t xa = reinterpret_cast<uintptr_t>(x);
@@ -309,6 +316,9 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         a.relu_in = relu_in;
         a.swz_mask = swz_mask;
         a.rows = rows;
+        a.blocks = static_cast<unsigned>(blocks);
+        a.clear = clear && c0 == 0 ? *clear : RidingClear{};
+        const unsigned grid = a.blocks + a.clear.blocks;
         a.vec_store = (ld_out % 4 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0) ? 1 : 0;
         // measured at 4.2 M rows: a [N, 96] result 0.63 -> 0.47 ms with non-temporal stores, [N, 16] and
         // [N, 32] results unchanged or slower
@@ -316,9 +326,9 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         a.tile_store = (a.vec_store && ld_out == 32 && cols == 32 && c0 == 0 && n < (1ll << 32)) ? 1 : 0;
         const size_t lds = lds_per_tile * mt;
         hipError_t e;
-        if (vw == 4) e = launch_rows_mt<4>(a, mt, cu, static_cast<unsigned>(blocks), lds, stream);
-        else if (vw == 2) e = launch_rows_mt<2>(a, mt, cu, static_cast<unsigned>(blocks), lds, stream);
-        else e = launch_rows_mt<1>(a, mt, cu, static_cast<unsigned>(blocks), lds, stream);
+        if (vw == 4) e = launch_rows_mt<4>(a, mt, cu, grid, lds, stream);
+        else if (vw == 2) e = launch_rows_mt<2>(a, mt, cu, grid, lds, stream);
+        else e = launch_rows_mt<1>(a, mt, cu, grid, lds, stream);
         if (e != hipSuccess) return hip_fail(e, "dense rows kernel launch");
     }
     return kOk;

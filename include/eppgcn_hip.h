@@ -479,6 +479,15 @@ int eppgcn_update_forward_table(float* table, size_t table_floats, const float* 
                                 const float* scale, int relu_input, int64_t num_nodes, int in_dim,
                                 int out_dim, void* stream);
 
+/* Forward of a layer in one call: eppgcn_update_forward_table into `workspace`, then eppgcn_spmm_forward over it with a
+ * NULL input - the same results, with a launch less where no plan is given (the clear of a small `out` rides in the
+ * product's kernel).  Arguments as for the two; in_dim as far as eppgcn_update_supported allows. */
+int eppgcn_layer_forward(float* out, const float* x, const float* w, int relu_input, const int32_t* row_pointers,
+                         const int32_t* column_index, const float* degrees, const int32_t* part_pointers,
+                         const int32_t* part2node, int num_nodes, int in_dim, int out_dim, int num_parts, int part_size,
+                         int dim_worker, int warp_per_block, float* workspace, size_t workspace_floats, const void* plan,
+                         void* stream);
+
 /* d_x[num_nodes, in_dim] = g[num_nodes, out_dim] * w^T, w [in_dim, out_dim]; with relu_ref
  * ([num_nodes, in_dim], may be NULL) entries where relu_ref <= 0 are zeroed (gradient of a
  * ReLU applied to the layer input).

@@ -249,3 +249,82 @@ def test_update_products_on_random_shapes(api):
             assert_close(got, co.update_backward_weight(x, g, relu_input=relu), wb, "weight gradient")
 
     check()
+
+
+# ---------------------------------------------------------------- the clear that rides in the kernel before the aggregation
+def _whole_number_layer(n, k, m, seed):
+    """A graph with isolated vertices and a hub, and operands of small whole numbers: every sum is exact in any order."""
+    from tests.helpers import random_symmetric_csr
+    indptr, col = random_symmetric_csr(n, 2 * n, seed, isolated=0.3)
+    rng = np.random.default_rng(seed + 1)
+    x, w = rng.integers(-3, 4, (n, k)).astype(np.float32), rng.integers(-3, 4, (k, m)).astype(np.float32)
+    return indptr, col, x, w
+
+
+def _between_guards(words, offset):
+    """A view of `words` floats of NaN with guards of sevens around it, `offset` floats past a 16-byte boundary."""
+    whole = torch.full((words + 72,), 7.0, device="cuda")
+    view = whole[32 + offset:32 + offset + words]
+    view.fill_(float("nan"))
+    return whole, view
+
+
+@pytest.mark.parametrize("n,k,m,offset", [(1, 3, 1, 0), (2, 5, 3, 1), (65, 16, 22, 2), (300, 96, 16, 3), (1025, 33, 7, 1),
+                                          (131072, 4, 32, 0), (131073, 4, 32, 0)])
+@pytest.mark.parametrize("relu", [False, True])
+def test_layer_forward_gives_what_the_two_calls_give(api, n, k, m, offset, relu):
+    """Up to and past the 16 MB whose clear rides (131072 x 32 floats), any alignment of the output, nothing outside it."""
+    indptr, col, x, w = _whole_number_layer(n, k, m, n)
+    pp, p2n = co.build_part(32, indptr)
+    ones = dev(np.ones(n, np.float32))
+    args = dev(x), dev(w), dev(indptr), dev(col), dev(pp), dev(p2n)
+    lib, dx, dw, ip, cl, ppd, p2d = (api.load(), *args)
+    floats = lib.eppgcn_feature_workspace_floats(n, m)
+    stream = torch.cuda.current_stream().cuda_stream
+    table = torch.full((floats,), float("nan"), device="cuda")
+    whole, out = _between_guards(n * m, offset)
+    rc = lib.eppgcn_layer_forward(out.data_ptr(), dx.data_ptr(), dw.data_ptr(), int(relu), ip.data_ptr(), cl.data_ptr(),
+                                  ones.data_ptr(), ppd.data_ptr(), p2d.data_ptr(), n, k, m, p2n.size, 32, 32, 8,
+                                  table.data_ptr(), floats, None, stream)
+    assert rc == 0, lib.eppgcn_last_error()
+    act = np.maximum(x, 0) if relu else x
+    want = co.spmm_f64(act @ w, indptr, col, np.ones(n, np.float32))
+    assert np.array_equal(out.cpu().numpy().reshape(n, m), want.astype(np.float32))
+    assert (whole[:32 + offset] == 7).all() and (whole[32 + offset + n * m:] == 7).all()
+    for broken in ({"w": None}, {"table": table.data_ptr() + 4}, {"floats": floats - 1}):
+        out.fill_(5.0)
+        rc = lib.eppgcn_layer_forward(out.data_ptr(), dx.data_ptr(), broken.get("w", dw.data_ptr()), int(relu), ip.data_ptr(),
+                                      cl.data_ptr(), ones.data_ptr(), ppd.data_ptr(), p2d.data_ptr(), n, k, m, p2n.size, 32, 32,
+                                      8, broken.get("table", table.data_ptr()), broken.get("floats", floats), None, stream)
+        assert rc == -1 and (out == 5).all(), broken
+
+
+@pytest.mark.parametrize("n,m,offset", [(1, 1, 0), (3, 5, 1), (257, 16, 2), (2000, 22, 3), (1500, 47, 1), (131072, 32, 0),
+                                        (131073, 32, 0)])
+@pytest.mark.parametrize("listed", [False, True])
+def test_pruned_backward_clears_and_scales_in_one_launch(api, n, m, offset, listed):
+    """Rows outside the path are zero and the others exact, with the bitmap of the gathered rows (NaN outside it) and without."""
+    indptr, col, _, _ = _whole_number_layer(n, 1, 1, n + 7)
+    rng = np.random.default_rng(n)
+    mask = rng.random(n) < 0.3
+    keep = mask[col]
+    rows = np.repeat(np.arange(n), np.diff(indptr))
+    deg = np.bincount(rows[keep], minlength=n)
+    ids, edges = rows[keep].astype(np.int32), col[keep].astype(np.int32)
+    part_pointer = np.concatenate([[0], np.cumsum(deg[deg > 0])]).astype(np.int32)      # a group per row
+    parts = int((deg > 0).sum())
+    dy = rng.integers(-4, 5, (n, m)).astype(np.float32)
+    want = np.zeros((n, m), np.float64)
+    np.add.at(want, ids, dy[edges].astype(np.float64))
+    bitmap = None
+    if listed:
+        seen = np.zeros((n + 31) // 32 * 32, bool)
+        seen[edges] = True
+        bitmap = dev(np.packbits(seen, bitorder="little").view(np.int32))
+        dy[~seen[:n]] = np.nan
+    whole, out = _between_guards(n * m, offset)
+    pad = np.zeros(1, np.int32)
+    api.ours_backward(dev(dy), dev(np.concatenate([ids, pad])), dev(part_pointer), dev(np.concatenate([edges, pad])),
+                      dev(np.ones(n, np.float32)), parts, out=out.view(n, m), gathered_rows=bitmap)
+    assert np.array_equal(out.cpu().numpy().reshape(n, m), want.astype(np.float32))
+    assert (whole[:32 + offset] == 7).all() and (whole[32 + offset + n * m:] == 7).all()
