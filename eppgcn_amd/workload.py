@@ -81,7 +81,7 @@ def prepare(graph: graphs.Graph, num_layers: int = 2, train_ratio: float = 0.1, 
 
     # per-run state, EPPGCN/dataset.py:135-156
     ngh_masks = [torch.zeros(n, dtype=torch.bool, device=dev) for _ in range(num_layers - 1)]
-    node_degs = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(num_layers)]
+    node_degs = [d[:n] for d in torch.zeros((num_layers, (n + 63) // 64 * 64), dtype=torch.int32, device=dev).unbind()]
 
     # Every stage is issued for all layers before the host waits for its counts, so the GPU has work while the host
     # sizes the next stage.

@@ -163,3 +163,25 @@ def test_several_results_with_one_wait(api):
     for k in (2, 3, 5):
         assert together[k].partial_rows == single[k].partial_rows and together[k].num_parts == single[k].num_parts
         assert torch.equal(together[k].view(raw_col=True)[3], single[k].view(raw_col=True)[3])
+
+
+@pytest.mark.parametrize("capacity", [1, 2, 5, 1 << 20, (1 << 20) + 1, (1 << 20) + 3])
+@pytest.mark.parametrize("ps", [1, 3, 4])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+def test_the_entries_behind_the_groups_are_cleared(api, capacity, ps, offset):
+    """Either way of clearing (before the split, or behind it for tiny groups in large arrays), any alignment, nothing outside."""
+    deg = np.random.default_rng(3).integers(0, 9, 3000).astype(np.int32) if capacity > 5 else np.array([0, min(capacity - 1, 2)], np.int32)
+    lib = api.load()
+    whole = torch.full((capacity + 64,), 7, dtype=torch.int32, device="cuda")
+    out = whole[16 + offset:16 + offset + capacity]
+    nbytes = lib.eppgcn_split_workspace_bytes(deg.size)
+    ws = torch.empty(nbytes // 8 + 1, dtype=torch.int64, device="cuda")
+    rc = lib.eppgcn_split_back_part(dev(deg).data_ptr(), deg.size, ps, out.data_ptr(), capacity, ws.data_ptr(), nbytes, None,
+                                    None, None, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    at = np.cumsum(deg) - deg
+    starts = np.concatenate([np.arange(a, a + d, ps) for a, d in zip(at, deg)] + [[deg.sum()]])
+    want = np.zeros(capacity, np.int64)
+    want[:starts.size] = starts
+    assert np.array_equal(out.cpu().numpy(), want)
+    assert (whole[:16 + offset] == 7).all() and (whole[16 + offset + capacity:] == 7).all()
