@@ -393,19 +393,19 @@ __global__ __launch_bounds__(1024) void scan_counts_kernel(int* __restrict__ cou
     }
 }
 
-template <int kItems, bool kBits>
-__global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
+template <int kBlock, int kItems, bool kScanned, bool kBits>
+__global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
     const void* __restrict__ src, uint8_t* __restrict__ ngh_mask, int* __restrict__ node_degs, int* __restrict__ out_id,
     int* __restrict__ out_edge, uint8_t* __restrict__ self_kept, int length, int num_tiles, int is_last,
     const int* __restrict__ tile_first, const unsigned long long* __restrict__ kept, const int* __restrict__ counts,
     ScanState* st)
 {
-    constexpr int kTile = kMarkBlock * kItems;
+    constexpr int kTile = kBlock * kItems;
     constexpr int kWords = kTile / 64;
     constexpr int kPerLane = kWords / kWave;
     static_assert(kWords % kWave == 0 && kItems <= kWave, "one wave scans the words; a wave's words fit its lanes");
-    constexpr bool kScanned = kItems == kMarkItemsLarge;       // counts[] holds the kept slots before every tile
+    static_assert(kWords <= kBlock && kBlock >= 2 * kWave, "a thread per word, a wave for each of the two maps");
     __shared__ int s_prefix;
     __shared__ int s_starts_in_tile, s_kept_in_tile;
     __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
@@ -433,18 +433,23 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     {
         if constexpr (!kScanned) {
             int sum = 0;
-            for (int t = threadIdx.x; t < tile; t += kMarkBlock) sum += counts[t];
+            for (int t0 = threadIdx.x; t0 < tile; t0 += 4 * kBlock) {
+                int c[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) c[j] = t0 + j * kBlock < tile ? counts[t0 + j * kBlock] : 0;
+                sum += c[0] + c[1] + c[2] + c[3];
+            }
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
             if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
         }
         int mine = 0;
-        for (int i0 = threadIdx.x; i0 < g_cnt; i0 += kMarkBlock * kMarkBatch) {
+        for (int i0 = threadIdx.x; i0 < g_cnt; i0 += kBlock * kMarkBatch) {
             int start[kMarkBatch], row[kMarkBatch];
             bool some[kMarkBatch], marked[kMarkBatch];
 #pragma unroll
             for (int j = 0; j < kMarkBatch; ++j) {
-                const int g = g_lo + min(i0 + j * kMarkBlock, g_cnt - 1);
+                const int g = g_lo + min(i0 + j * kBlock, g_cnt - 1);
                 start[j] = part_ptr[g];
                 some[j] = part_ptr[g + 1] > start[j];
                 row[j] = part2node[g];
@@ -453,7 +458,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
             for (int j = 0; j < kMarkBatch; ++j) marked[j] = !is_last && in_mask<kBits>(src, row[j]);
 #pragma unroll
             for (int j = 0; j < kMarkBatch; ++j) {
-                const int i = i0 + j * kMarkBlock;
+                const int i = i0 + j * kBlock;
                 if (i >= g_cnt) continue;
                 const long long p = start[j] - base;
                 if (p >= 0 && p < kTile) {
@@ -482,8 +487,8 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     {
         const long long end = length - (base - s_prefix);
         const long long from = end - (min(static_cast<long long>(kTile), length - base) - s_kept_in_tile);
-        zero_from(out_id, from, end, threadIdx.x, kMarkBlock);
-        zero_from(out_edge, from, end, threadIdx.x, kMarkBlock);
+        zero_from(out_id, from, end, threadIdx.x, kBlock);
+        zero_from(out_edge, from, end, threadIdx.x, kBlock);
     }
     // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
     // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
@@ -521,11 +526,11 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
         const int whole = s_kept_before[word];
         return (q & 63) ? whole + __popcll(s_kept[word] & ((1ull << (q & 63)) - 1ull)) : whole;
     };
-    for (int i0 = 0; i0 < g_cnt; i0 += kMarkBlock * kMarkBatch) {
+    for (int i0 = 0; i0 < g_cnt; i0 += kBlock * kMarkBatch) {
         int from[kMarkBatch], to[kMarkBatch], row[kMarkBatch];
 #pragma unroll
         for (int j = 0; j < kMarkBatch; ++j) {
-            const int i = i0 + j * kMarkBlock + static_cast<int>(threadIdx.x);
+            const int i = i0 + j * kBlock + static_cast<int>(threadIdx.x);
             const int g = g_lo + min(i, g_cnt - 1);
             from[j] = part_ptr[g];
             to[j] = part_ptr[g + 1];
@@ -533,7 +538,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
         }
 #pragma unroll
         for (int j = 0; j < kMarkBatch; ++j) {
-            if (i0 + j * kMarkBlock >= g_cnt) break;         // the same for the whole workgroup
+            if (i0 + j * kBlock >= g_cnt) break;         // the same for the whole workgroup
             int n = row[j] < 0 ? 0 : kept_before(to[j] - base) - kept_before(from[j] - base);
             const int prev_row = __shfl_up(row[j], 1, kWave);
             const uint64_t heads = __ballot(lane == 0 || prev_row != row[j]);
@@ -548,7 +553,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     }
     const bool by_bits = s_starts_in_tile >= 0;
     // lane k: word k of this wave
-    const int my_word = (lane < kItems ? lane : 0) * kMarkWaves + wave;
+    const int my_word = (lane < kItems ? lane : 0) * (kBlock / kWave) + wave;
     const uint64_t start_word = s_starts[my_word], kept_word = s_kept[my_word];
     const int start_before = s_starts_before[my_word] + before - 1;
     const int place = s_kept_before[my_word] + s_prefix;
@@ -558,7 +563,7 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
             const uint64_t word = lane_value(start_word, k);
             a = __builtin_amdgcn_readlane(start_before, k) + ballot_rank(word) + static_cast<int>((word >> lane) & 1ull);
         } else {
-            const int e = static_cast<int>(base + k * kMarkBlock + threadIdx.x);
+            const int e = static_cast<int>(base + k * kBlock + threadIdx.x);
             int b = g_cnt;
             while (b - a > 1) {
                 const int mid = (a + b) >> 1;
@@ -572,12 +577,12 @@ __global__ __launch_bounds__(kMarkBlock, 8) void place_slots_kernel(
     };
     const int owned_lo = part_ptr[0], owned_hi = min(part_ptr[g_lo + g_cnt], length);
     constexpr int kChunk = kItems < 8 ? kItems : 8;
-#pragma unroll
+#pragma unroll(kItems <= 16 ? kItems / kChunk : 1)
     for (int k0 = 0; k0 < kItems; k0 += kChunk) {
         int c[kChunk];
 #pragma unroll
         for (int k = 0; k < kChunk; ++k) {
-            const long long idx = base + (k0 + k) * kMarkBlock + threadIdx.x;
+            const long long idx = base + (k0 + k) * kBlock + threadIdx.x;
             c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
         }
 #pragma unroll
@@ -1172,23 +1177,28 @@ static int launch_mark_pass(const int* part2node, const int* part_ptr, const int
     unsigned long long* kept = reinterpret_cast<unsigned long long*>(workspace + l.kept);
     int* counts = reinterpret_cast<int*>(workspace + l.counts);
     const int* first = reinterpret_cast<const int*>(workspace + l.first);
-    const dim3 grid(l.num_tiles), block(kMarkBlock);
+    const dim3 grid(l.num_tiles);
     const int len = static_cast<int>(length);
-#define EPPGCN_MARK(ITEMS_)                                                                                              \
+#define EPPGCN_MARK(ITEMS_, PLACE_BLOCK_, SCANNED_)                                                                       \
     do {                                                                                                                \
-        hipLaunchKernelGGL((keep_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part_ptr, col, src, num_parts, len, \
-                           kept, counts);                                                                                 \
+        hipLaunchKernelGGL((keep_slots_kernel<ITEMS_, kBits>), grid, dim3(kMarkBlock), 0, stream, part_ptr, col, src,      \
+                           num_parts, len, kept, counts);                                                                 \
         EPPGCN_HIP(hipGetLastError());                                                                                    \
-        if (ITEMS_ == kMarkItemsLarge)                                                                                    \
+        if (SCANNED_)                                                                                                     \
             hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, stream, counts, l.num_tiles);                  \
         EPPGCN_HIP(hipGetLastError());                                                                                    \
-        hipLaunchKernelGGL((place_slots_kernel<ITEMS_, kBits>), grid, block, 0, stream, part2node, part_ptr, col, src,     \
-                           ngh_mask, node_degs, out_id, out_edge, self_kept, len, l.num_tiles, is_last, first, kept,       \
-                           counts, st);                                                                                   \
+        hipLaunchKernelGGL((place_slots_kernel<PLACE_BLOCK_, kMarkBlock / PLACE_BLOCK_ * ITEMS_, SCANNED_, kBits>), grid, \
+                           dim3(PLACE_BLOCK_), 0, stream, part2node, part_ptr, col, src, ngh_mask, node_degs, out_id,     \
+                           out_edge, self_kept, len, l.num_tiles, is_last, first, kept, counts, st);                      \
         EPPGCN_HIP(hipGetLastError());                                                                                    \
     } while (0)
-    if (l.tile_slots == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge);
-    else EPPGCN_MARK(kMarkItemsSmall);
+    // place_slots walks a small tile from barrier to barrier.  1024 threads do that fastest as long as the chip holds all tiles
+    // at once (two workgroups on a CU: 512 tiles), beyond that four workgroups of 512 threads hide each other's waits better:
+    // 27 tiles 13.5 us with 1024 threads, 15.5 with 512, 21.5 with 256; 2250 tiles 63, 50, 54.  Tiles of 16 384 slots (scale
+    // 22, the mean of two layers): 450, 474, 522.
+    if (l.tile_slots == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge, 1024, true);
+    else if (l.num_tiles > 512) EPPGCN_MARK(kMarkItemsSmall, 512, false);
+    else EPPGCN_MARK(kMarkItemsSmall, 1024, false);
 #undef EPPGCN_MARK
     return kOk;
 }

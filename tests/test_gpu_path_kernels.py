@@ -65,6 +65,13 @@ def test_path_marking_in_large_tiles(api, n, slots_per_row, loops, ps, is_last):
     assert _check_marking(api, n, slots_per_row, loops, ps, is_last, 1) >= 1 << 25
 
 
+@pytest.mark.parametrize("n", [512 * 4096 - 1, 512 * 4096, 512 * 4096 + 1])
+@pytest.mark.parametrize("is_last", [False, True])
+def test_path_marking_where_the_workgroups_get_smaller(api, n, is_last):
+    """512 and 513 tiles of 4096 slots, the last one full, one slot short and one slot long."""
+    assert _check_marking(api, n, 0, True, 4, is_last, 0) == n
+
+
 def _check_marking(api, n, slots_per_row, loops, ps, is_last, shift):
     """`shift`: the masks start one byte past a word boundary.  Vertex 0 is a neighbour of every third slot.  -> slots"""
     rng = np.random.default_rng(n + slots_per_row)
