@@ -219,14 +219,12 @@ class Trainer:
         for w in group["params"]:
             if w.grad is None:
                 continue
-            state = opt.state.get(w)
-            if not state:
+            state = opt.state.get(w) or {}
+            tensors = w.grad, state.get("exp_avg"), state.get("exp_avg_sq"), state.get("step")
+            if type(w) is not torch.nn.Parameter or any(type(t) is not torch.Tensor for t in tensors):
                 return False
-            weights.append(w)
-            grads.append(w.grad)
-            averages.append(state["exp_avg"])
-            squares.append(state["exp_avg_sq"])
-            steps.append(state["step"])
+            for column, t in zip((weights, grads, averages, squares, steps), (w, *tensors)):
+                column.append(t)
         beta1, beta2 = group["betas"]
         if type(beta1) is not float or type(beta2) is not float:
             return False
