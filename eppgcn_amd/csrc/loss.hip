@@ -12,7 +12,7 @@
 //              rounds twice, a 2-norm error against 64 bits of 5.11e-8 instead of 4.82e-8 (5826 rows of 22 classes), which
 //              the first Adam steps, close to a sign, pass on enlarged
 // As torch operations the two were 14 launches of 2 to 5 us (log-softmax, gather, mean and negation of the selected rows;
-// backward three fills, a scatter and an index_add) out of 37 of a two-layer epoch; now 4 of 27 (12 us).  What bounds them:
+// backward three fills, a scatter and an index_add) of a two-layer epoch; now 4 of its 17 (12 us).  What bounds them:
 // launches for small graphs, the write of the gradient for large ones (4.1 to 4.8 TB/s).  2^22 rows of 22 classes, a tenth of
 // them in training: 31 + 124 us, with torch's operations 260; 2^20 rows of 172, a hundredth: 10 + 150 and 176; 2^20 rows of
 // 1000, a tenth: 91 + 1026 and 1721.  (A team per row, one row after another: 114 + 337, 11 + 286 and 667 + 2870.)
