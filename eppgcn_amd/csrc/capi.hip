@@ -105,6 +105,10 @@ static int read_state(const void* workspace, hipStream_t stream, ScanState* host
     return kOk;
 }
 
+// Bytes of a workspace whose head eppgcn_read_states copies: a whole record (kStateBytes), also where the call needs less (a
+// split of up to 6144 vertices needs 40 to 56).  The calls that are older than the records still take what they need.
+static size_t with_record(size_t bytes) { return bytes < kStateBytes ? kStateBytes : bytes; }
+
 static bool aligned(const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; }
 
 }  // namespace eppgcn
@@ -270,7 +274,7 @@ int eppgcn_build_plan(const int32_t* part_pointers, const int32_t* column_index,
 }
 
 size_t eppgcn_compact_workspace_bytes(int64_t length) { return compact_workspace_bytes(length < 0 ? 0 : length); }
-size_t eppgcn_split_workspace_bytes(int64_t num_nodes) { return split_workspace_bytes(num_nodes < 0 ? 0 : num_nodes); }
+size_t eppgcn_split_workspace_bytes(int64_t num_nodes) { return with_record(split_workspace_bytes(num_nodes < 0 ? 0 : num_nodes)); }
 
 int eppgcn_compact_back_edge(const int32_t* edge_mask, const int32_t* column_index, int32_t* out_id, int32_t* out_edge,
                              int64_t length, void* workspace, size_t workspace_bytes, int32_t* d_valid_len,
@@ -395,25 +399,13 @@ int eppgcn_adam_step(int count, float* const* params, const float* const* grads,
 
 size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes)
 {
-    return mark_path_workspace_bytes(num_edges < 0 ? 0 : num_edges, num_nodes < 0 ? 0 : num_nodes);
+    return with_record(mark_path_workspace_bytes(num_edges < 0 ? 0 : num_edges, num_nodes < 0 ? 0 : num_nodes));
 }
 
-int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
-                     const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
-                     uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, void* workspace,
-                     size_t workspace_bytes, int64_t* counts, void* stream)
-{
-    if (int rc = eppgcn_mark_path_groups(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
-                                         gathered_rows, num_parts, num_edges, num_nodes, is_last, 0, workspace,
-                                         workspace_bytes, stream))
-        return rc;
-    return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
-}
-
-int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
-                            const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id,
-                            int32_t* out_edge, uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes,
-                            int is_last, int part_size, void* workspace, size_t workspace_bytes, void* stream)
+static int mark_path_call(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                          const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
+                          uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, int part_size,
+                          void* workspace, size_t workspace_bytes, void* stream)
 {
     EPPGCN_REQUIRE(num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
                    "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
@@ -437,6 +429,27 @@ int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointe
     KernelTimer timer(s, &g_mask_ms);
     return launch_mark_path(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
                             gathered_rows, num_parts, num_edges, num_nodes, is_last ? 1 : 0, part_size, workspace, s);
+}
+
+int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                     const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
+                     uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, void* workspace,
+                     size_t workspace_bytes, int64_t* counts, void* stream)
+{
+    if (int rc = mark_path_call(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+                                gathered_rows, num_parts, num_edges, num_nodes, is_last, 0, workspace, workspace_bytes, stream))
+        return rc;
+    return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
+}
+
+int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+                            const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id,
+                            int32_t* out_edge, uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes,
+                            int is_last, int part_size, void* workspace, size_t workspace_bytes, void* stream)
+{
+    EPPGCN_REQUIRE(workspace_bytes >= eppgcn_mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
+    return mark_path_call(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge, gathered_rows,
+                          num_parts, num_edges, num_nodes, is_last, part_size, workspace, workspace_bytes, stream);
 }
 
 int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
@@ -714,7 +727,7 @@ int eppgcn_split_and_plan(const int32_t* node_deg, const int32_t* edge_list, int
     EPPGCN_REQUIRE(num_nodes > 0 && part_size >= 1 && num_parts > 0 && dim > 0, "num_nodes, part_size, num_parts, dim > 0 required");
     EPPGCN_REQUIRE(capacity > num_parts && part_pointer && node_deg, "part_pointer needs num_parts + 1 entries");
     EPPGCN_REQUIRE(split_workspace && aligned(split_workspace, 8), "workspace must be 8-byte aligned");
-    EPPGCN_REQUIRE(split_workspace_bytes_ >= split_workspace_bytes(num_nodes), "workspace too small");
+    EPPGCN_REQUIRE(split_workspace_bytes_ >= eppgcn_split_workspace_bytes(num_nodes), "workspace too small");
     EPPGCN_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= plan_workspace_bytes(num_parts, num_slots),
                    "workspace smaller than eppgcn_plan_workspace_bytes(num_parts, num_slots) or not 256-byte aligned");
     int* rows = plan_rows_in_workspace(workspace, num_parts, num_slots);

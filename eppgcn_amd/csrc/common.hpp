@@ -377,7 +377,8 @@ struct ScanState {
 unsigned scan_mode();
 void set_scan_test_mode(unsigned spin_limit, int mute_first_tile);
 static_assert(sizeof(ScanState) == 32, "descriptor array starts 32 bytes into the workspace");
-constexpr int kStateBytes = 64;     // what eppgcn_read_states copies of a record: a plan's header, or a ScanState and what follows
+// what eppgcn_read_states copies of a record: a plan's header, or a ScanState and what follows it in its workspace
+constexpr int kStateBytes = 64;
 constexpr int kStateList = 32;      // records per launch
 static_assert(sizeof(ScanState) <= kStateBytes && sizeof(StreamHeader) == kStateBytes, "records fit");
 

@@ -370,9 +370,10 @@ int eppgcn_mark_path_group_counts(const int32_t* out_edge, uint32_t* gathered_ro
                                   void* workspace, const void* state, int64_t* counts, void* stream);
 
 /* Counts of several calls with one wait.  A call that leaves its results on the device (eppgcn_mark_path_groups,
- * eppgcn_split_back_part and eppgcn_split_and_plan, eppgcn_build_plan) has a record: the head of the (split) workspace, or
- * eppgcn_plan_state(plan, sizes).  eppgcn_read_states copies `count` of them to `host` - memory that the device can write,
- * e.g. from hipHostMalloc, eppgcn_state_bytes() for each - and synchronises the stream.  The ..._read functions and
+ * eppgcn_split_back_part and eppgcn_split_and_plan, eppgcn_build_plan) has a record: the head of the (split) workspace, which
+ * has the size that its ..._workspace_bytes function says (at least eppgcn_state_bytes()), or eppgcn_plan_state(plan, sizes).
+ * eppgcn_read_states copies `count` of them, eppgcn_state_bytes() bytes each, to `host` - memory that the device can write,
+ * e.g. from hipHostMalloc - and synchronises the stream.  The ..._read functions and
  * eppgcn_mark_path_group_counts say of such a copy what the functions without it say after a wait of their own. */
 size_t eppgcn_state_bytes(void);
 int eppgcn_read_states(const void* const* states, int count, void* host, void* stream);

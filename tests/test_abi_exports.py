@@ -126,6 +126,26 @@ def test_argument_errors_are_reported_before_any_device_work():
     assert lib.eppgcn_mark_compact_workspace_bytes(4096 * 3 + 1) >= 32 + 8 * 4 + 4 * 5
 
 
+def test_workspaces_with_a_record_hold_a_whole_one():
+    """eppgcn_read_states copies eppgcn_state_bytes() from the head of a split or marking workspace: the advertised sizes
+    cover that, also for graphs whose scan needs less, and the calls made for it refuse a smaller workspace."""
+    from eppgcn_amd import capi
+    lib = capi.load()
+    record = lib.eppgcn_state_bytes()
+    sizes = [0, 1, 2047, 2048, 2049, 6144, 6145, 8193]
+    for n in [-1, *sizes]:
+        assert lib.eppgcn_split_workspace_bytes(n) >= record, n
+        for e in (-1, 0, 1, 4096):
+            assert lib.eppgcn_mark_path_workspace_bytes(e, n) >= record, (e, n)
+    # the scans' own need stays covered: a state of 32 bytes and 8 for each 2048 vertices
+    assert all(lib.eppgcn_split_workspace_bytes(n) >= 32 + 8 * ((n + 2047) // 2048) for n in sizes)
+    p0, one = ctypes.c_void_p(0), ctypes.c_void_p(256)
+    assert lib.eppgcn_mark_path_groups(p0, p0, p0, p0, p0, p0, p0, p0, p0, 0, 0, 0, 1, 4, one, record - 1, p0) == -1
+    assert b"workspace too small" in lib.eppgcn_last_error()
+    assert lib.eppgcn_split_and_plan(one, one, 100, 4, one, 9, 3, 9, 16, 5, one, 1 << 20, one, 1 << 20, one, record - 1, p0) == -1
+    assert b"workspace too small" in lib.eppgcn_last_error()
+
+
 def test_header_is_plain_c_and_a_c_program_links_against_the_library(tmp_path):
     """The boundary is a C ABI: the header must compile as C99 and as C++ without torch or HIP
     headers, and a C program must link against the library and call it.  Only host-side entry
