@@ -537,28 +537,36 @@ class Pending:
     def __init__(self, states, finish, stream):
         self.states, self.finish, self.stream = states, finish, stream
 
+    def result(self, states=None):
+        """``states``: where the records have been copied to, None to wait for them; the stream's GPU is current meanwhile."""
+        with torch.cuda.device(self.stream.device):
+            return self.finish(states)
+
     def __call__(self):
-        return self.finish()
+        return self.result()
 
 
 def finish_all(pending):
     """The results of several ``Pending`` calls with one wait for all that were issued on the same stream."""
     lib, pending = load(), list(pending)
-    out = [None] * len(pending)
-    for stream in {p.stream.cuda_stream: p.stream for p in pending}.values():
-        mine = [k for k, p in enumerate(pending) if p.stream.cuda_stream == stream.cuda_stream]
+    out, of_stream = [None] * len(pending), {}
+    for k, p in enumerate(pending):              # the default streams of all GPUs have the same handle
+        of_stream.setdefault((p.stream.device, p.stream.cuda_stream), []).append(k)
+    for mine in of_stream.values():
+        stream = pending[mine[0]].stream
         addresses = [a for k in mine for a in pending[k].states]
         if None in addresses:
             for k in mine:
                 out[k] = pending[k]()
             continue
         size = lib.eppgcn_state_bytes()
-        host = torch.empty(size * len(addresses), dtype=torch.uint8, pin_memory=True)
-        _check(lib.eppgcn_read_states((C.c_void_p * len(addresses))(*addresses), len(addresses), _ptr(host), _stream(stream)))
+        with torch.cuda.device(stream.device):
+            host = torch.empty(size * len(addresses), dtype=torch.uint8, pin_memory=True)
+            _check(lib.eppgcn_read_states((C.c_void_p * len(addresses))(*addresses), len(addresses), _ptr(host), _stream(stream)))
         at = host.data_ptr()
         for k in mine:
             count = len(pending[k].states)
-            out[k] = pending[k].finish([C.c_void_p(at + size * j) for j in range(count)])
+            out[k] = pending[k].result([C.c_void_p(at + size * j) for j in range(count)])
             at += size * count
     return out
 

@@ -1,10 +1,13 @@
 """CPU tests of the host-side pieces: benchmark graph generators, parameter records, byte
 accounting.  No GPU, no HIP calls."""
+import contextlib
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from eppgcn_amd import graphs, param, workload
+from eppgcn_amd import capi, graphs, param, workload
 
 
 def _check_graph(g):
@@ -217,3 +220,58 @@ def test_live_counter_attribution_and_guards(tmp_path, monkeypatch):
     monkeypatch.setenv("ROCPROFILER_LIBRARY_CTOR", "1")
     value, why = bench.live_traffic()
     assert value is None and "under a profiler" in why
+
+
+class _FakeStream:
+    """What ``capi.Pending`` looks at of a stream; the default stream of every GPU has the handle 0."""
+
+    def __init__(self, device, handle):
+        self.device, self.cuda_stream = device, handle
+
+
+class _FakeLibrary:
+    """Records what is read and with which GPU current; a record is the number at its address."""
+    eppgcn_state_bytes = staticmethod(lambda: 64)
+
+    def __init__(self):
+        self.current, self.reads = "cuda:0", []
+
+    def eppgcn_read_states(self, addresses, count, host, stream):
+        self.reads.append((self.current, stream.value or 0, list(addresses)))
+        for j in range(count):
+            ctypes.cast(host.value + 64 * j, ctypes.POINTER(ctypes.c_int64))[0] = addresses[j]
+        return 0
+
+    def device(self, device):
+        @contextlib.contextmanager
+        def made_current():
+            before, self.current = self.current, device
+            yield
+            self.current = before
+        return made_current()
+
+
+@pytest.fixture
+def fake(monkeypatch):
+    lib, empty = _FakeLibrary(), torch.empty
+    monkeypatch.setattr(capi, "load", lambda: lib)
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: empty(*a, **k))
+    monkeypatch.setattr(torch.cuda, "device", lib.device)
+    return lib
+
+
+def _pending(lib, records, stream):
+    """A result that is (records as read or None, the GPU that was current)."""
+    def finish(states=None):
+        return states and [ctypes.cast(s, ctypes.POINTER(ctypes.c_int64))[0] for s in states], lib.current
+    return capi.Pending(records, finish, stream)
+
+
+def test_results_of_two_gpus_are_read_by_a_call_each(fake):
+    """Streams of different GPUs with the same handle (0: the default streams) do not share a wait, streams that are the
+    same stream do, and everything happens with the stream's own GPU current."""
+    streams = [_FakeStream("cuda:0", 0), _FakeStream("cuda:1", 0), _FakeStream("cuda:0", 0), _FakeStream("cuda:1", 7)]
+    work = [_pending(fake, [100 + k, 200 + k], s) for k, s in enumerate(streams)]
+    assert capi.finish_all(work) == [([100 + k, 200 + k], s.device) for k, s in enumerate(streams)]
+    assert fake.reads == [("cuda:0", 0, [100, 200, 102, 202]), ("cuda:1", 0, [101, 201]), ("cuda:1", 7, [103, 203])]
+    assert work[1]() == (None, "cuda:1") and fake.current == "cuda:0"
