@@ -551,14 +551,13 @@ def finish_all(pending):
     lib, pending = load(), list(pending)
     out, of_stream = [None] * len(pending), {}
     for k, p in enumerate(pending):              # the default streams of all GPUs have the same handle
-        of_stream.setdefault((p.stream.device, p.stream.cuda_stream), []).append(k)
+        if None in p.states:                     # a plan without groups has no record and nothing to wait for
+            out[k] = p()
+        else:
+            of_stream.setdefault((p.stream.device, p.stream.cuda_stream), []).append(k)
     for mine in of_stream.values():
         stream = pending[mine[0]].stream
         addresses = [a for k in mine for a in pending[k].states]
-        if None in addresses:
-            for k in mine:
-                out[k] = pending[k]()
-            continue
         size = lib.eppgcn_state_bytes()
         with torch.cuda.device(stream.device):
             host = torch.empty(size * len(addresses), dtype=torch.uint8, pin_memory=True)

@@ -136,7 +136,8 @@ def test_split_and_plan_in_one_gives_what_the_two_give(api, n, ps):
 
 
 def test_several_results_with_one_wait(api):
-    """finish_all gives what the calls give one by one: marking, splits and plans of two streams, an empty plan among them."""
+    """finish_all gives what the calls give one by one: marking, splits and plans of two streams.  The empty plan among them
+    has no record and keeps none of the others from the common wait."""
     indptr, col = csr_of(degrees_of("mixed"), 5)
     n = indptr.size - 1
     pp, p2n = [dev(x) for x in co.build_part(16, indptr)]
@@ -163,6 +164,17 @@ def test_several_results_with_one_wait(api):
     for k in (2, 3, 5):
         assert together[k].partial_rows == single[k].partial_rows and together[k].num_parts == single[k].num_parts
         assert torch.equal(together[k].view(raw_col=True)[3], single[k].view(raw_col=True)[3])
+
+
+@pytest.mark.parametrize("count", [1, 31, 32, 33, 65])
+def test_more_records_than_one_launch_reads(api, count):
+    """32 records fit a launch: every split gets its own counts back, also from the second launch on."""
+    degs = [dev(np.arange(k + 1), torch.int32) for k in range(count)]
+    got = api.finish_all([api.split_back_part_begin(d, 5000, 3) for d in degs])
+    for k, (pointer, parts, covered) in enumerate(got):
+        want = -(-np.arange(k + 1) // 3)
+        assert (parts, covered) == (int(want.sum()), k * (k + 1) // 2)
+        assert pointer[parts] == covered and pointer.numel() == 5001
 
 
 @pytest.mark.parametrize("capacity", [1, 2, 5, 1 << 20, (1 << 20) + 1, (1 << 20) + 3])

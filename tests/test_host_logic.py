@@ -275,3 +275,11 @@ def test_results_of_two_gpus_are_read_by_a_call_each(fake):
     assert capi.finish_all(work) == [([100 + k, 200 + k], s.device) for k, s in enumerate(streams)]
     assert fake.reads == [("cuda:0", 0, [100, 200, 102, 202]), ("cuda:1", 0, [101, 201]), ("cuda:1", 7, [103, 203])]
     assert work[1]() == (None, "cuda:1") and fake.current == "cuda:0"
+
+
+def test_a_result_without_a_record_leaves_the_others_to_one_wait(fake):
+    stream = _FakeStream("cuda:0", 0)
+    work = [_pending(fake, r, stream) for r in ([101], [None], [102, 103])]
+    assert capi.finish_all(work) == [([101], "cuda:0"), (None, "cuda:0"), ([102, 103], "cuda:0")]
+    assert fake.reads == [("cuda:0", 0, [101, 102, 103])]
+    assert capi.finish_all([]) == []
