@@ -235,8 +235,9 @@ __global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanSca
     }
     if (i0 == 0) {
         *sc.sort = ScanState{};
-        // groups of a split that stalled are not to be read: every kernel that would ends at this flag
-        if (upstream && (upstream->error || upstream->overflow || upstream->counts[0] != num_parts || upstream->counts[1] > num_slots))
+        // groups of a split that stalled are not to be read, and groups that cover other slots than the caller's are not the
+        // path's: every kernel that would read them ends at this flag
+        if (upstream && (upstream->error || upstream->overflow || upstream->counts[0] != num_parts || upstream->counts[1] != num_slots))
             sc.sort->error = 1;
         *sc.order = ScanState{};
         *sc.partials = ScanState{};
@@ -1040,7 +1041,8 @@ int read_plan_status(const void* plan, long long num_parts, long long num_slots,
     }
     if (info.header.error) {
         forget_stream_info(plan);
-        set_error("look-back scan stalled: a tile waited past its spin limit; the plan is invalid");
+        set_error("look-back scan stalled: a tile waited past its spin limit, or the split before the plan found other counts "
+                  "than it was given; the plan is invalid");
         return kErrScanStalled;
     }
     remember_stream_info(plan, info);

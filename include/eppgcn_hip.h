@@ -431,7 +431,7 @@ int eppgcn_split_counts(const void* workspace, int64_t* h_num_parts, int64_t* h_
  * does not look it up among the ids of the slots.  The same group pointers and the same plan.  edge_list: the kept slots'
  * columns; num_slots: how many; capacity: entries of part_pointer (cleared behind the groups).  The counts are read from
  * split_workspace's record (eppgcn_read_states), and both it and the plan's are to be looked at before the plan is used: a
- * split that stalled or found other counts leaves a plan that is refused. */
+ * split that stalled, or found other counts than num_parts and num_slots, leaves a plan that is refused. */
 int eppgcn_split_and_plan(const int32_t* node_deg, const int32_t* edge_list, int num_nodes, int part_size,
                           int32_t* part_pointer, int64_t capacity, int num_parts, int64_t num_slots, int dim,
                           int block_shift, void* plan, size_t plan_bytes, void* workspace, size_t workspace_bytes,

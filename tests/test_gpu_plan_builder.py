@@ -105,7 +105,7 @@ def test_the_largest_plans(api, num_slots):
 @pytest.mark.parametrize("n,ps", [(1, 4), (2047, 1), (2048, 3), (2049, 32), (9000, 8)])
 def test_split_and_plan_in_one_gives_what_the_two_give(api, n, ps):
     """Around the tiles of the split, an empty row next to a hub: the same group pointers, and in every array the plan that
-    the ids of the slots give; a group count that is not the path's is refused."""
+    the ids of the slots give; a group count or a slot count that is not the path's is refused."""
     rng = np.random.default_rng(n)
     deg = rng.integers(0, 6, n)
     deg[rng.random(n) < 0.4] = 0
@@ -129,10 +129,11 @@ def test_split_and_plan_in_one_gives_what_the_two_give(api, n, ps):
         used = {"col": None, "erow": events, "cev": None, "wtail": None, "touched": None, "frow": fix, "fptr": fix + 1}
         for name, count in used.items():
             assert torch.equal(sa[name][:count], sb[name][:count]), name
-    for wrong in {max(parts - 1, 1), parts + 1} - {parts}:
+    wrong = {(max(parts - 1, 1), slots), (parts + 1, slots), (parts, slots - 1), (parts, slots + 1), (parts, e)} - {(parts, slots)}
+    for wrong_parts, wrong_slots in wrong:             # edge_list is long enough for all of them
         for shift in (5, 31):
-            with pytest.raises(api.EppgcnError):
-                api.split_and_plan_begin(degs, col, e, ps, wrong, slots, 16, shift)()
+            with pytest.raises(api.EppgcnError, match="other counts|do not fit"):   # the split says so of too few groups
+                api.split_and_plan_begin(degs, col, e, ps, wrong_parts, wrong_slots, 16, shift)()
 
 
 def test_several_results_with_one_wait(api):
