@@ -25,6 +25,7 @@ int schedule_shift(int);
 void set_schedule_shift(int);
 void set_plan_keep_rows(int);
 void set_plan_length_classes(int);
+int check_plan_sizes(long long, long long, long long, size_t, size_t);
 int launch_build_plan(const int*, const int*, const int*, const int*, int, long long, int, int, int, void*, size_t,
                       void*, size_t, const ScanState*, hipStream_t);
 void set_agg_force_team(int);
@@ -120,23 +121,36 @@ extern "C" {
 const char* eppgcn_last_error(void) { return g_last_error.c_str(); }
 int eppgcn_abi_version(void) { return 20; }
 
+// What the two unpruned aggregations refuse (`call` of them, or of a call that ends in one); reads nothing on the device.
+static int check_spmm(const char* call, const float* out, const float* in, const int32_t* column_index, const float* degrees,
+                      const int32_t* part_pointers, const int32_t* part2node, int num_nodes, int dim, int num_parts,
+                      int part_size, int dim_worker, int warp_per_block, const float* workspace, size_t workspace_floats,
+                      const void* plan)
+{
+    EPPGCN_REQUIRE_OF(call, num_nodes >= 0 && dim > 0 && num_parts >= 0, "num_nodes >= 0, dim > 0, num_parts >= 0 required");
+    EPPGCN_REQUIRE_OF(call, part_size > 0 && dim_worker > 0 && warp_per_block > 0, "launch hints must be positive");
+    if (num_nodes == 0) return kOk;
+    EPPGCN_REQUIRE_OF(call, out && (in || workspace) && degrees, "null feature or scale pointer");
+    EPPGCN_REQUIRE_OF(call, num_parts == 0 || (column_index && part_pointers && part2node), "null index pointer");
+    EPPGCN_REQUIRE_OF(call, aligned(out, 4) && aligned(in, 4), "feature pointers must be 4-byte aligned");
+    EPPGCN_REQUIRE_OF(call, !plan || aligned(plan, 256), "plan must be 256-byte aligned");
+    EPPGCN_REQUIRE_OF(call, !workspace || (aligned(workspace, 16) && workspace != out),
+                      "workspace must be 16-byte aligned and distinct from the output");
+    EPPGCN_REQUIRE_OF(call, !workspace || workspace == in || workspace_floats >= feature_workspace_floats(num_nodes, dim),
+                      "workspace smaller than eppgcn_feature_workspace_floats(num_nodes, dim)");
+    return kOk;
+}
+
 int eppgcn_spmm_forward(float* out, const float* in, const int32_t* row_pointers, const int32_t* column_index,
                         const float* degrees, const int32_t* part_pointers, const int32_t* part2node, int num_nodes,
                         int dim, int num_parts, int part_size, int dim_worker, int warp_per_block, float* workspace,
                         size_t workspace_floats, const void* plan, void* stream)
 {
     (void)row_pointers;
-    EPPGCN_REQUIRE(num_nodes >= 0 && dim > 0 && num_parts >= 0, "num_nodes >= 0, dim > 0, num_parts >= 0 required");
-    EPPGCN_REQUIRE(part_size > 0 && dim_worker > 0 && warp_per_block > 0, "launch hints must be positive");
+    if (int rc = check_spmm(__func__, out, in, column_index, degrees, part_pointers, part2node, num_nodes, dim, num_parts,
+                            part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan))
+        return rc;
     if (num_nodes == 0) return kOk;
-    EPPGCN_REQUIRE(out && (in || workspace) && degrees, "null feature or scale pointer");
-    EPPGCN_REQUIRE(num_parts == 0 || (column_index && part_pointers && part2node), "null index pointer");
-    EPPGCN_REQUIRE(aligned(out, 4) && aligned(in, 4), "feature pointers must be 4-byte aligned");
-    EPPGCN_REQUIRE(!plan || aligned(plan, 256), "plan must be 256-byte aligned");
-    EPPGCN_REQUIRE(!workspace || (aligned(workspace, 16) && workspace != out),
-                   "workspace must be 16-byte aligned and distinct from the output");
-    EPPGCN_REQUIRE(!workspace || workspace == in || workspace_floats >= feature_workspace_floats(num_nodes, dim),
-                   "workspace smaller than eppgcn_feature_workspace_floats(num_nodes, dim)");
     return aggregate_forward_groups(out, in, column_index, degrees, part_pointers, part2node, plan, num_nodes, dim,
                                     num_parts, part_size, workspace, workspace_floats, static_cast<hipStream_t>(stream),
                                     &g_for_agg_ms, nullptr);
@@ -148,17 +162,10 @@ int eppgcn_spmm_backward(float* d_input, const float* d_output, const int32_t* r
                          int warp_per_block, float* workspace, size_t workspace_floats, const void* plan, void* stream)
 {
     (void)row_pointers;
-    EPPGCN_REQUIRE(num_nodes >= 0 && dim > 0 && num_parts >= 0, "num_nodes >= 0, dim > 0, num_parts >= 0 required");
-    EPPGCN_REQUIRE(part_size > 0 && dim_worker > 0 && warp_per_block > 0, "launch hints must be positive");
+    if (int rc = check_spmm(__func__, d_input, d_output, column_index, degrees, part_pointers, part2node, num_nodes, dim,
+                            num_parts, part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan))
+        return rc;
     if (num_nodes == 0) return kOk;
-    EPPGCN_REQUIRE(d_input && (d_output || workspace) && degrees, "null feature or scale pointer");
-    EPPGCN_REQUIRE(num_parts == 0 || (column_index && part_pointers && part2node), "null index pointer");
-    EPPGCN_REQUIRE(aligned(d_input, 4) && aligned(d_output, 4), "feature pointers must be 4-byte aligned");
-    EPPGCN_REQUIRE(!plan || aligned(plan, 256), "plan must be 256-byte aligned");
-    EPPGCN_REQUIRE(!workspace || (aligned(workspace, 16) && workspace != d_input),
-                   "workspace must be 16-byte aligned and distinct from the output");
-    EPPGCN_REQUIRE(!workspace || workspace == d_output || workspace_floats >= feature_workspace_floats(num_nodes, dim),
-                   "workspace smaller than eppgcn_feature_workspace_floats(num_nodes, dim)");
     return aggregate_forward_groups(d_input, d_output, column_index, degrees, part_pointers, part2node, plan,
                                     num_nodes, dim, num_parts, part_size, workspace, workspace_floats,
                                     static_cast<hipStream_t>(stream), &g_back_agg_ms, nullptr);
@@ -249,28 +256,30 @@ size_t eppgcn_plan_workspace_bytes(int64_t num_parts, int64_t num_slots)
     return plan_workspace_bytes(num_parts, num_slots);
 }
 
-static int build_plan_call(const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
+static int check_plan_call(const char* call, const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
                            const int32_t* ids, int num_parts, int64_t num_slots, int num_nodes, int dim, int block_shift,
-                           void* plan, size_t plan_size, void* workspace, size_t workspace_bytes, const ScanState* upstream,
-                           void* stream)
+                           const void* plan, const void* workspace)
 {
-    EPPGCN_REQUIRE(num_parts >= 0 && num_slots >= 0 && num_nodes >= 0 && dim > 0, "negative size");
-    EPPGCN_REQUIRE(block_shift >= 0 && block_shift <= 31, "block_shift must be 0 (automatic) or 1..31");
+    EPPGCN_REQUIRE_OF(call, num_parts >= 0 && num_slots >= 0 && num_nodes >= 0 && dim > 0, "negative size");
+    EPPGCN_REQUIRE_OF(call, block_shift >= 0 && block_shift <= 31, "block_shift must be 0 (automatic) or 1..31");
     if (num_parts == 0) return kOk;
-    EPPGCN_REQUIRE(part_pointers && column_index && plan, "null pointer");
-    EPPGCN_REQUIRE((part2node != nullptr) != (ids != nullptr), "give exactly one of part2node (forward) and ids (backward)");
-    EPPGCN_REQUIRE(aligned(plan, 256) && workspace && aligned(workspace, 256), "plan and workspace must be 256-byte aligned");
-    return launch_build_plan(part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes,
-                             block_shift > 0 ? block_shift : schedule_shift(dim), dim, plan, plan_size, workspace,
-                             workspace_bytes, upstream, static_cast<hipStream_t>(stream));
+    EPPGCN_REQUIRE_OF(call, part_pointers && column_index && plan, "null pointer");
+    EPPGCN_REQUIRE_OF(call, (part2node != nullptr) != (ids != nullptr), "give exactly one of part2node (forward) and ids (backward)");
+    EPPGCN_REQUIRE_OF(call, aligned(plan, 256) && workspace && aligned(workspace, 256), "plan and workspace must be 256-byte aligned");
+    return kOk;
 }
 
 int eppgcn_build_plan(const int32_t* part_pointers, const int32_t* column_index, const int32_t* part2node,
                       const int32_t* ids, int num_parts, int64_t num_slots, int num_nodes, int dim, int block_shift,
                       void* plan, size_t plan_size, void* workspace, size_t workspace_bytes, void* stream)
 {
-    return build_plan_call(part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes, dim, block_shift, plan,
-                           plan_size, workspace, workspace_bytes, nullptr, stream);
+    if (int rc = check_plan_call(__func__, part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes, dim,
+                                 block_shift, plan, workspace))
+        return rc;
+    if (num_parts == 0) return kOk;
+    return launch_build_plan(part_pointers, column_index, part2node, ids, num_parts, num_slots, num_nodes,
+                             block_shift > 0 ? block_shift : schedule_shift(dim), dim, plan, plan_size, workspace,
+                             workspace_bytes, nullptr, static_cast<hipStream_t>(stream));
 }
 
 size_t eppgcn_compact_workspace_bytes(int64_t length) { return compact_workspace_bytes(length < 0 ? 0 : length); }
@@ -402,20 +411,20 @@ size_t eppgcn_mark_path_workspace_bytes(int64_t num_edges, int64_t num_nodes)
     return with_record(mark_path_workspace_bytes(num_edges < 0 ? 0 : num_edges, num_nodes < 0 ? 0 : num_nodes));
 }
 
-static int mark_path_call(const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
+static int mark_path_call(const char* call, const int32_t* part2node, const int32_t* part_pointers, const int32_t* column_index,
                           const uint8_t* src_mask, uint8_t* ngh_mask, int32_t* node_degs, int32_t* out_id, int32_t* out_edge,
                           uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, int part_size,
                           void* workspace, size_t workspace_bytes, void* stream)
 {
-    EPPGCN_REQUIRE(num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
-                   "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
-    EPPGCN_REQUIRE(part_size >= 0, "part_size >= 0 required");
-    EPPGCN_REQUIRE(workspace && aligned(workspace, 16), "workspace must be 16-byte aligned");
-    EPPGCN_REQUIRE(workspace_bytes >= mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
-    EPPGCN_REQUIRE(num_edges == 0 || (out_id && out_edge), "null output pointer");
-    EPPGCN_REQUIRE(num_nodes == 0 || gathered_rows, "null output pointer");
-    EPPGCN_REQUIRE(num_parts == 0 || (part2node && part_pointers && column_index && src_mask && node_degs), "null pointer");
-    EPPGCN_REQUIRE(is_last || num_parts == 0 || ngh_mask, "ngh_mask is required unless this is the last layer");
+    EPPGCN_REQUIRE_OF(call, num_parts >= 0 && num_nodes >= 0 && num_edges >= 0 && num_edges < (1ll << 31),
+                      "num_parts, num_nodes >= 0 and 0 <= num_edges < 2^31 required");
+    EPPGCN_REQUIRE_OF(call, part_size >= 0, "part_size >= 0 required");
+    EPPGCN_REQUIRE_OF(call, workspace && aligned(workspace, 16), "workspace must be 16-byte aligned");
+    EPPGCN_REQUIRE_OF(call, workspace_bytes >= mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
+    EPPGCN_REQUIRE_OF(call, num_edges == 0 || (out_id && out_edge), "null output pointer");
+    EPPGCN_REQUIRE_OF(call, num_nodes == 0 || gathered_rows, "null output pointer");
+    EPPGCN_REQUIRE_OF(call, num_parts == 0 || (part2node && part_pointers && column_index && src_mask && node_degs), "null pointer");
+    EPPGCN_REQUIRE_OF(call, is_last || num_parts == 0 || ngh_mask, "ngh_mask is required unless this is the last layer");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (num_parts == 0 || num_edges == 0 || num_nodes == 0) {
         if (num_nodes > 0)
@@ -436,7 +445,7 @@ int eppgcn_mark_path(const int32_t* part2node, const int32_t* part_pointers, con
                      uint32_t* gathered_rows, int num_parts, int64_t num_edges, int num_nodes, int is_last, void* workspace,
                      size_t workspace_bytes, int64_t* counts, void* stream)
 {
-    if (int rc = mark_path_call(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+    if (int rc = mark_path_call(__func__, part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
                                 gathered_rows, num_parts, num_edges, num_nodes, is_last, 0, workspace, workspace_bytes, stream))
         return rc;
     return counts ? eppgcn_mark_path_counts(out_edge, gathered_rows, num_edges, num_nodes, workspace, counts, stream) : kOk;
@@ -448,8 +457,8 @@ int eppgcn_mark_path_groups(const int32_t* part2node, const int32_t* part_pointe
                             int is_last, int part_size, void* workspace, size_t workspace_bytes, void* stream)
 {
     EPPGCN_REQUIRE(workspace_bytes >= eppgcn_mark_path_workspace_bytes(num_edges, num_nodes), "workspace too small");
-    return mark_path_call(part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge, gathered_rows,
-                          num_parts, num_edges, num_nodes, is_last, part_size, workspace, workspace_bytes, stream);
+    return mark_path_call(__func__, part2node, part_pointers, column_index, src_mask, ngh_mask, node_degs, out_id, out_edge,
+                          gathered_rows, num_parts, num_edges, num_nodes, is_last, part_size, workspace, workspace_bytes, stream);
 }
 
 int eppgcn_mark_path_counts(const int32_t* out_edge, uint32_t* gathered_rows, int64_t num_edges, int num_nodes,
@@ -728,14 +737,20 @@ int eppgcn_split_and_plan(const int32_t* node_deg, const int32_t* edge_list, int
     EPPGCN_REQUIRE(capacity > num_parts && part_pointer && node_deg, "part_pointer needs num_parts + 1 entries");
     EPPGCN_REQUIRE(split_workspace && aligned(split_workspace, 8), "workspace must be 8-byte aligned");
     EPPGCN_REQUIRE(split_workspace_bytes_ >= eppgcn_split_workspace_bytes(num_nodes), "workspace too small");
-    EPPGCN_REQUIRE(workspace && aligned(workspace, 256) && workspace_bytes >= plan_workspace_bytes(num_parts, num_slots),
-                   "workspace smaller than eppgcn_plan_workspace_bytes(num_parts, num_slots) or not 256-byte aligned");
-    int* rows = plan_rows_in_workspace(workspace, num_parts, num_slots);
-    if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, rows, capacity, num_parts, true,
-                              split_workspace, static_cast<hipStream_t>(stream)))
+    // everything that the plan's build refuses is refused before the split is launched; the build keeps the groups' rows in
+    // its workspace, where the split leaves them
+    int* rows = num_slots >= 0 ? plan_rows_in_workspace(workspace, num_parts, num_slots) : nullptr;
+    if (int rc = check_plan_call(__func__, part_pointer, edge_list, rows, nullptr, num_parts, num_slots, num_nodes, dim,
+                                 block_shift, plan, workspace))
         return rc;
-    return build_plan_call(part_pointer, edge_list, rows, nullptr, num_parts, num_slots, num_nodes, dim, block_shift, plan,
-                           plan_bytes, workspace, workspace_bytes, static_cast<const ScanState*>(split_workspace), stream);
+    if (int rc = check_plan_sizes(num_parts, num_slots, num_nodes, plan_bytes, workspace_bytes)) return rc;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (int rc = launch_split(false, node_deg, num_nodes, part_size, part_pointer, rows, capacity, num_parts, true,
+                              split_workspace, s))
+        return rc;
+    return launch_build_plan(part_pointer, edge_list, rows, nullptr, num_parts, num_slots, num_nodes,
+                             block_shift > 0 ? block_shift : schedule_shift(dim), dim, plan, plan_bytes, workspace,
+                             workspace_bytes, static_cast<const ScanState*>(split_workspace), s);
 }
 
 int eppgcn_build_part(const int32_t* row_pointers, int num_nodes, int part_size, int32_t* part_pointers,
@@ -840,17 +855,25 @@ int eppgcn_update_forward(float* out, int ld_out, const float* x, const float* w
                              num_nodes, in_dim, out_dim, static_cast<hipStream_t>(stream), 0u);
 }
 
+static int check_forward_table(const char* call, const float* table, size_t table_floats, const float* x, const float* w,
+                               const float* scale, int64_t num_nodes, int in_dim, int out_dim)
+{
+    EPPGCN_REQUIRE_OF(call, num_nodes >= 0 && in_dim > 0 && out_dim > 0, "num_nodes >= 0, in_dim > 0, out_dim > 0 required");
+    if (num_nodes == 0) return kOk;
+    EPPGCN_REQUIRE_OF(call, table && x && w && scale, "null pointer");
+    EPPGCN_REQUIRE_OF(call, aligned(table, 16) && aligned(x, 4) && aligned(w, 4), "table must be 16-byte, matrices 4-byte aligned");
+    EPPGCN_REQUIRE_OF(call, table != x, "the product cannot be written over its input");
+    EPPGCN_REQUIRE_OF(call, num_nodes < (1ll << 31), "too many rows");
+    EPPGCN_REQUIRE_OF(call, table_floats >= feature_workspace_floats(num_nodes, out_dim),
+                      "table smaller than eppgcn_feature_workspace_floats(num_nodes, out_dim)");
+    return kOk;
+}
+
 int eppgcn_update_forward_table(float* table, size_t table_floats, const float* x, const float* w, const float* scale,
                                 int relu_input, int64_t num_nodes, int in_dim, int out_dim, void* stream)
 {
-    EPPGCN_REQUIRE(num_nodes >= 0 && in_dim > 0 && out_dim > 0, "num_nodes >= 0, in_dim > 0, out_dim > 0 required");
+    if (int rc = check_forward_table(__func__, table, table_floats, x, w, scale, num_nodes, in_dim, out_dim)) return rc;
     if (num_nodes == 0) return kOk;
-    EPPGCN_REQUIRE(table && x && w && scale, "null pointer");
-    EPPGCN_REQUIRE(aligned(table, 16) && aligned(x, 4) && aligned(w, 4), "table must be 16-byte, matrices 4-byte aligned");
-    EPPGCN_REQUIRE(table != x, "the product cannot be written over its input");
-    EPPGCN_REQUIRE(num_nodes < (1ll << 31), "too many rows");
-    EPPGCN_REQUIRE(table_floats >= feature_workspace_floats(num_nodes, out_dim),
-                   "table smaller than eppgcn_feature_workspace_floats(num_nodes, out_dim)");
     const int pitch = workspace_pitch(out_dim);
     return launch_dense_rows(table, pitch, pitch, x, in_dim, w, out_dim, 1, scale, nullptr, 0, relu_input ? 1 : 0,
                              num_nodes, in_dim, out_dim, static_cast<hipStream_t>(stream), kRowSwizzleMask);
@@ -862,29 +885,23 @@ int eppgcn_layer_forward(float* out, const float* x, const float* w, int relu_in
                          int dim_worker, int warp_per_block, float* workspace, size_t workspace_floats, const void* plan,
                          void* stream)
 {
-    const size_t words = static_cast<size_t>(num_nodes > 0 ? num_nodes : 0) * static_cast<size_t>(out_dim > 0 ? out_dim : 0);
-    // everything that either call refuses is refused before the first launch
-    const bool rides = !plan && num_nodes > 0 && in_dim > 0 && out_dim > 0 && num_parts > 0 && words <= kRidingClearWords &&
-                       !timing_enabled() && part_size > 0 && dim_worker > 0 && warp_per_block > 0 && out && aligned(out, 4) &&
-                       degrees && column_index && part_pointers && part2node && workspace && aligned(workspace, 16) &&
-                       workspace != out && x && w && aligned(x, 4) && aligned(w, 4) && x != out && w != out && workspace != x &&
-                       workspace_floats >= feature_workspace_floats(num_nodes, out_dim);
-    if (!rides) {
-        if (int rc = eppgcn_update_forward_table(workspace, workspace_floats, x, w, degrees, relu_input, num_nodes, in_dim,
-                                                 out_dim, stream))
-            return rc;
-        return eppgcn_spmm_forward(out, nullptr, row_pointers, column_index, degrees, part_pointers, part2node, num_nodes,
-                                   out_dim, num_parts, part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan,
-                                   stream);
-    }
-    const RidingClear clear = riding_clear(out, words);
+    (void)row_pointers;
+    // everything that the product or the aggregation refuses is refused before the first launch
+    if (int rc = check_forward_table(__func__, workspace, workspace_floats, x, w, degrees, num_nodes, in_dim, out_dim)) return rc;
+    if (int rc = check_spmm(__func__, out, nullptr, column_index, degrees, part_pointers, part2node, num_nodes, out_dim,
+                            num_parts, part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan))
+        return rc;
+    if (num_nodes == 0) return kOk;
+    const size_t words = static_cast<size_t>(num_nodes) * out_dim;
+    const bool rides = !plan && num_parts > 0 && words <= kRidingClearWords && !timing_enabled() && x != out && w != out;
+    const RidingClear clear = rides ? riding_clear(out, words) : RidingClear{};
     const int pitch = workspace_pitch(out_dim);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (int rc = launch_dense_rows(workspace, pitch, pitch, x, in_dim, w, out_dim, 1, degrees, nullptr, 0, relu_input ? 1 : 0,
-                                   num_nodes, in_dim, out_dim, s, kRowSwizzleMask, nullptr, &clear))
+                                   num_nodes, in_dim, out_dim, s, kRowSwizzleMask, nullptr, rides ? &clear : nullptr))
         return rc;
-    return aggregate_forward_groups(out, nullptr, column_index, degrees, part_pointers, part2node, nullptr, num_nodes, out_dim,
-                                    num_parts, part_size, workspace, workspace_floats, s, &g_for_agg_ms, nullptr, true);
+    return aggregate_forward_groups(out, nullptr, column_index, degrees, part_pointers, part2node, plan, num_nodes, out_dim,
+                                    num_parts, part_size, workspace, workspace_floats, s, &g_for_agg_ms, nullptr, rides);
 }
 
 int64_t eppgcn_feature_workspace_row(int64_t vertex)

@@ -33,13 +33,15 @@ int hip_fail(hipError_t e, const char* what);
         if (_e != hipSuccess) return ::eppgcn::hip_fail(_e, #expr); \
     } while (0)
 
-#define EPPGCN_REQUIRE(cond, msg)                               \
+// the message names the entry point `call`, also from a helper that several of them share
+#define EPPGCN_REQUIRE_OF(call, cond, msg)                      \
     do {                                                        \
         if (!(cond)) {                                          \
-            ::eppgcn::set_error(std::string(__func__) + ": " + (msg)); \
+            ::eppgcn::set_error(std::string(call) + ": " + (msg)); \
             return ::eppgcn::kErrInvalidArgument;               \
         }                                                       \
     } while (0)
+#define EPPGCN_REQUIRE(cond, msg) EPPGCN_REQUIRE_OF(__func__, cond, msg)
 
 // Zeroes `words` 32-bit words at p (4-byte aligned) with a fill kernel.  Used instead of
 // hipMemsetAsync everywhere so that every call of the library can be captured into a HIP graph

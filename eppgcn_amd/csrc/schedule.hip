@@ -855,14 +855,9 @@ static int next_plan_generation()
 }
 static int last_plan_generation() { return g_plan_generation.load(); }
 
-int launch_build_plan(const int* part_ptr, const int* col, const int* part2node, const int* ids, int num_parts,
-                      long long num_slots, int num_nodes, int shift, int dim, void* plan, size_t plan_size,
-                      void* workspace, size_t workspace_bytes, const ScanState* upstream, hipStream_t stream)
+// num_parts > 0
+int check_plan_sizes(long long num_parts, long long num_slots, long long num_nodes, size_t plan_size, size_t workspace_bytes)
 {
-    forget_stream_info(plan);
-    int keep_rows, length_classes;
-    plan_policy(num_nodes, dim, &keep_rows, &length_classes);
-    if (num_parts <= 0) return kOk;
     if (plan_size < plan_bytes(num_parts, num_slots, num_nodes)) {
         set_error("build_plan: plan buffer smaller than eppgcn_plan_bytes(num_parts, num_slots, num_nodes)");
         return kErrInvalidArgument;
@@ -875,6 +870,18 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
         set_error("build_plan: workspace smaller than eppgcn_plan_workspace_bytes(num_parts, num_slots)");
         return kErrInvalidArgument;
     }
+    return kOk;
+}
+
+int launch_build_plan(const int* part_ptr, const int* col, const int* part2node, const int* ids, int num_parts,
+                      long long num_slots, int num_nodes, int shift, int dim, void* plan, size_t plan_size,
+                      void* workspace, size_t workspace_bytes, const ScanState* upstream, hipStream_t stream)
+{
+    forget_stream_info(plan);
+    int keep_rows, length_classes;
+    plan_policy(num_nodes, dim, &keep_rows, &length_classes);
+    if (num_parts <= 0) return kOk;
+    if (int rc = check_plan_sizes(num_parts, num_slots, num_nodes, plan_size, workspace_bytes)) return rc;
     PlanTemp t = plan_temp(static_cast<char*>(workspace), num_parts, num_slots);
     const PlanView v = plan_view(plan, num_parts, num_nodes);
     const StreamView sv = stream_view(plan, num_parts, num_slots, num_nodes);

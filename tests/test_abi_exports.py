@@ -146,6 +146,35 @@ def test_workspaces_with_a_record_hold_a_whole_one():
     assert b"workspace too small" in lib.eppgcn_last_error()
 
 
+def test_calls_made_of_two_refuse_what_the_second_refuses_before_the_first_runs():
+    """Layer forward (product, aggregation) and split with plan: -1 and not an error of a launch, which is what a box without
+    a GPU gives as soon as the first of the two has started."""
+    from eppgcn_amd import capi
+    lib = capi.load()
+    p0, one, two, odd = (ctypes.c_void_p(a) for a in (0, 1 << 20, 1 << 24, (1 << 24) + 16))
+    n, k, m = 8, 4, 4
+    floats = lib.eppgcn_feature_workspace_floats(n, m)
+    good = dict(out=one, x=two, w=two, relu=0, rows=one, col=one, degrees=one, parts=one, nodes=one, n=n, k=k, m=m, groups=3,
+                part_size=16, dim_worker=32, warps=8, table=ctypes.c_void_p(1 << 28), floats=floats, plan=p0, stream=p0)
+    for bad, message in ((dict(out=p0), "null feature"), (dict(col=p0), "null index"), (dict(parts=p0), "null index"),
+                         (dict(nodes=p0), "null index"), (dict(part_size=0), "launch hints"), (dict(dim_worker=-1), "launch hints"),
+                         (dict(warps=0), "launch hints"), (dict(groups=-1), "num_parts >= 0"), (dict(plan=odd), "256-byte aligned"),
+                         (dict(out=ctypes.c_void_p(1 << 28)), "distinct"), (dict(out=ctypes.c_void_p((1 << 20) + 2)), "4-byte"),
+                         (dict(n=0, warps=0), "launch hints"), (dict(k=0), "in_dim > 0"), (dict(w=p0), "null pointer"),
+                         (dict(floats=floats - 1), "table smaller")):
+        assert lib.eppgcn_layer_forward(*{**good, **bad}.values()) == -1, bad
+        assert lib.eppgcn_last_error().startswith(b"eppgcn_layer_forward: ") and message.encode() in lib.eppgcn_last_error(), bad
+    assert lib.eppgcn_layer_forward(*{**good, **dict(n=0, out=p0, x=p0, w=p0)}.values()) == 0
+    need = lib.eppgcn_plan_bytes(3, 9, 100)
+    good = dict(degs=one, edges=two, n=100, part_size=4, pointer=one, capacity=9, groups=3, slots=9, dim=16, shift=5, plan=two,
+                plan_bytes=need, ws=one, ws_bytes=1 << 40, split=one, split_bytes=1 << 20, stream=p0)
+    for bad, message in ((dict(edges=p0), "null pointer"), (dict(plan=p0), "null pointer"), (dict(plan=odd), "256-byte aligned"),
+                         (dict(shift=-1), "block_shift"), (dict(shift=32), "block_shift"), (dict(slots=-1), "negative"),
+                         (dict(slots=(1 << 31) - 512, plan_bytes=1 << 40), "32-bit"), (dict(plan_bytes=need - 1), "plan buffer smaller")):
+        assert lib.eppgcn_split_and_plan(*{**good, **bad}.values()) == -1, bad
+        assert message.encode() in lib.eppgcn_last_error(), bad
+
+
 def test_header_is_plain_c_and_a_c_program_links_against_the_library(tmp_path):
     """The boundary is a C ABI: the header must compile as C99 and as C++ without torch or HIP
     headers, and a C program must link against the library and call it.  Only host-side entry
