@@ -879,6 +879,12 @@ int eppgcn_update_forward_table(float* table, size_t table_floats, const float* 
                              num_nodes, in_dim, out_dim, static_cast<hipStream_t>(stream), kRowSwizzleMask);
 }
 
+static bool overlap(const float* a, size_t a_floats, const float* b, size_t b_floats)
+{
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + 4 * b_floats && q < p + 4 * a_floats;
+}
+
 int eppgcn_layer_forward(float* out, const float* x, const float* w, int relu_input, const int32_t* row_pointers,
                          const int32_t* column_index, const float* degrees, const int32_t* part_pointers,
                          const int32_t* part2node, int num_nodes, int in_dim, int out_dim, int num_parts, int part_size,
@@ -892,8 +898,10 @@ int eppgcn_layer_forward(float* out, const float* x, const float* w, int relu_in
                             num_parts, part_size, dim_worker, warp_per_block, workspace, workspace_floats, plan))
         return rc;
     if (num_nodes == 0) return kOk;
-    const size_t words = static_cast<size_t>(num_nodes) * out_dim;
-    const bool rides = !plan && num_parts > 0 && words <= kRidingClearWords && !timing_enabled() && x != out && w != out;
+    const size_t n = static_cast<size_t>(num_nodes), words = n * out_dim;
+    // an output that shares memory with an operand is cleared when the product has read it
+    const bool rides = !plan && num_parts > 0 && words <= kRidingClearWords && !timing_enabled() &&
+                       !overlap(out, words, x, n * in_dim) && !overlap(out, words, w, static_cast<size_t>(in_dim) * out_dim);
     const RidingClear clear = rides ? riding_clear(out, words) : RidingClear{};
     const int pitch = workspace_pitch(out_dim);
     hipStream_t s = static_cast<hipStream_t>(stream);

@@ -299,6 +299,28 @@ def test_layer_forward_gives_what_the_two_calls_give(api, n, k, m, offset, relu)
         assert rc == -1 and (out == 5).all(), broken
 
 
+@pytest.mark.parametrize("where", ["x", "x_tail", "w_head"])
+def test_layer_forward_over_the_memory_of_an_operand(api, where):
+    """The output may share memory with an operand, as in the two calls: it is cleared when the product has read them."""
+    n, k, m = 9000, 16, 16
+    indptr, col, x, w = _whole_number_layer(n, k, m, 5)
+    pp, p2n = co.build_part(32, indptr)
+    ones, cl, ip, ppd, p2d = dev(np.ones(n, np.float32)), dev(col), dev(indptr), dev(pp), dev(p2n)
+    lib = api.load()
+    floats = lib.eppgcn_feature_workspace_floats(n, m)
+    table = torch.empty(floats, device="cuda")
+    memory = torch.zeros(4 * n * m, device="cuda")
+    at = {"x": (0, 0, 2 * n * m), "x_tail": (0, n * m - 16 * m, 3 * n * m), "w_head": (2 * n * m, k * m // 2, 0)}[where]
+    dx, out, dw = (memory[a:a + size] for a, size in zip(at, (n * k, n * m, k * m)))
+    dx.copy_(dev(x).view(-1)), dw.copy_(dev(w).view(-1))
+    rc = lib.eppgcn_layer_forward(out.data_ptr(), dx.data_ptr(), dw.data_ptr(), 0, ip.data_ptr(), cl.data_ptr(), ones.data_ptr(),
+                                  ppd.data_ptr(), p2d.data_ptr(), n, k, m, p2n.size, 32, 32, 8, table.data_ptr(), floats, None,
+                                  torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.eppgcn_last_error()
+    want = co.spmm_f64(x @ w, indptr, col, np.ones(n, np.float32)).astype(np.float32)
+    assert np.array_equal(out.cpu().numpy().reshape(n, m), want)
+
+
 @pytest.mark.parametrize("n,m,offset", [(1, 1, 0), (3, 5, 1), (257, 16, 2), (2000, 22, 3), (1500, 47, 1), (131072, 32, 0),
                                         (131073, 32, 0)])
 @pytest.mark.parametrize("listed", [False, True])
