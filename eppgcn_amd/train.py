@@ -95,6 +95,15 @@ def _step_hooks(opt):
             (torch_optimizer, "_global_optimizer_pre_hooks"), (torch_optimizer, "_global_optimizer_post_hooks"))
 
 
+def _is_torchs(step):
+    """No function of another module's is ``step`` or one that it wraps (torch puts wrappers of its own around it)."""
+    while step is not None:
+        if not getattr(step, "__globals__", {}).get("__name__", "").startswith("torch."):
+            return False
+        step = getattr(step, "__wrapped__", None)
+    return True
+
+
 class Trainer:
     """Wiring of EPPGCN/gcn_main.py: decider -> build_part -> mask/back records -> Net -> Adam."""
 
@@ -204,10 +213,11 @@ class Trainer:
 
     def _adam_in_one_launch(self):
         """The optimizer's step in the library's kernel, with the rounding and the state of torch's own; False, with nothing
-        changed, when it is torch's to take: another optimizer or form of Adam, options, hooks or a scheduler on its step, a
-        first step (it makes the state), weights of another type or layout (``GNNA.adam_step`` looks at those)."""
+        changed, when it is torch's to take: another optimizer or form of Adam, options, hooks, a scheduler or a wrapper on its
+        step or its class's, a first step (it makes the state), weights of another type or layout (``GNNA.adam_step`` looks at
+        those)."""
         opt = self.optimizer
-        if type(opt) is not torch.optim.Adam or "step" in vars(opt):
+        if type(opt) is not torch.optim.Adam or "step" in vars(opt) or not _is_torchs(torch.optim.Adam.step):
             return False
         if any(getattr(owner, name, True) for owner, name in _step_hooks(opt)) or len(opt.param_groups) != 1:
             return False

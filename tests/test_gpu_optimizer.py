@@ -87,8 +87,8 @@ def test_other_forms_are_left_to_torch_unchanged(spoil):
     _same(before, _states((weights, opt)))
 
 
-@pytest.mark.parametrize("option", ["plain", "hook", "scheduler", "decay", "sgd", "no_grad"])
-def test_trainer_takes_the_step_its_optimizer_says(option):
+@pytest.mark.parametrize("option", ["plain", "hook", "scheduler", "decay", "sgd", "no_grad", "class"])
+def test_trainer_takes_the_step_its_optimizer_says(option, monkeypatch):
     from eppgcn_amd import graphs, train
     tr = train.Trainer(graphs.uniform_graph(300, 900, seed=1, device="cuda"), labels="uniform")
     calls = []
@@ -98,6 +98,9 @@ def test_trainer_takes_the_step_its_optimizer_says(option):
         tr.optimizer = torch.optim.SGD(tr.model.parameters(), lr=0.01)
     elif option == "hook":
         tr.optimizer.register_step_post_hook(lambda *a: calls.append(a))
+    elif option == "class":
+        inner = torch.optim.Adam.step
+        monkeypatch.setattr(torch.optim.Adam, "step", lambda self: calls.append(self) or inner(self))
     elif option == "scheduler":
         scheduler = torch.optim.lr_scheduler.ExponentialLR(tr.optimizer, 0.5)
     tr.train_step(True)
@@ -112,9 +115,10 @@ def test_trainer_takes_the_step_its_optimizer_says(option):
     tr.train_step(False)
     for w, c in zip(weights, copies):
         c.grad = None if w.grad is None else w.grad.clone()
+    monkeypatch.undo()
     other.step()
     assert all(torch.equal(w, c) for w, c in zip(weights, copies))
-    assert len(calls) == (2 if option == "hook" else 0)
+    assert len(calls) == (2 if option in ("hook", "class") else 0)
     assert other.state_dict()["state"].keys() == tr.optimizer.state_dict()["state"].keys()
     for k, s in tr.optimizer.state_dict()["state"].items():
         assert all(torch.equal(s[n], other.state_dict()["state"][k][n]) for n in s if torch.is_tensor(s[n]))

@@ -2,6 +2,7 @@
 accounting.  No GPU, no HIP calls."""
 import contextlib
 import ctypes
+import functools
 
 import numpy as np
 import pytest
@@ -283,3 +284,25 @@ def test_a_result_without_a_record_leaves_the_others_to_one_wait(fake):
     assert capi.finish_all(work) == [([101], "cuda:0"), (None, "cuda:0"), ([102, 103], "cuda:0")]
     assert fake.reads == [("cuda:0", 0, [101, 102, 103])]
     assert capi.finish_all([]) == []
+
+
+@pytest.mark.parametrize("wraps", [False, True])
+@pytest.mark.parametrize("hooked", [False, True])
+def test_a_wrapper_on_the_optimizer_class_is_seen(monkeypatch, wraps, hooked):
+    """A caller's wrapper around ``torch.optim.Adam.step``, with and without ``functools.wraps``, outside and inside of the
+    wrapper that torch puts there when an optimizer is made."""
+    from eppgcn_amd import train
+    weights = [torch.nn.Parameter(torch.ones(2))]
+    torch.optim.Adam(weights)
+    assert train._is_torchs(torch.optim.Adam.step)
+    inner = torch.optim.Adam.step
+
+    def step(self, *args):
+        return inner(self, *args)
+
+    monkeypatch.setattr(torch.optim.Adam, "step", functools.wraps(inner)(step) if wraps else step)
+    if hooked:
+        torch.optim.Adam(weights)
+    assert not train._is_torchs(torch.optim.Adam.step)
+    monkeypatch.setattr(torch.optim.Adam, "step", functools.partial(inner))
+    assert not train._is_torchs(torch.optim.Adam.step)
