@@ -23,6 +23,7 @@
 //     kept: eight, and more while they are small); it affects speed only.
 #include <torch/extension.h>
 
+#include <ATen/record_function.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
@@ -542,6 +543,7 @@ bool adam_step(const std::vector<Tensor>& params, const std::vector<Tensor>& gra
     }
     if (device.index() != c10::hip::current_device()) return false;
     if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return false;
+    RECORD_USER_SCOPE("Optimizer.step#Adam.step");      // the range a profile of torch's own step has
     std::vector<float*> p(count), m(count), v(count);
     std::vector<const float*> g(count);
     std::vector<int64_t> sizes(count);

@@ -122,3 +122,13 @@ def test_trainer_takes_the_step_its_optimizer_says(option, monkeypatch):
     assert other.state_dict()["state"].keys() == tr.optimizer.state_dict()["state"].keys()
     for k, s in tr.optimizer.state_dict()["state"].items():
         assert all(torch.equal(s[n], other.state_dict()["state"][k][n]) for n in s if torch.is_tensor(s[n]))
+
+
+def test_a_profile_has_the_range_of_the_optimizer():
+    """Torch's step and the one in one launch are the same range of a profile, once per epoch."""
+    from eppgcn_amd import graphs, train
+    tr = train.Trainer(graphs.uniform_graph(300, 900, seed=1, device="cuda"))
+    for epoch in range(3):                        # the first step is torch's
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+            tr.train_step(epoch == 0)
+        assert [e.count for e in profile.key_averages() if e.key == "Optimizer.step#Adam.step"] == [1], epoch
