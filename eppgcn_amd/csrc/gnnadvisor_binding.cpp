@@ -548,17 +548,17 @@ bool adam_step(const std::vector<Tensor>& params, const std::vector<Tensor>& gra
     std::vector<const float*> g(count);
     std::vector<int64_t> sizes(count);
     std::vector<double> at(count);
+    for (size_t k = 0; k < count; ++k) steps[k].data_ptr<float>()[0] += 1.f;      // before any is read: weights may share one
     for (size_t k = 0; k < count; ++k) {
         p[k] = params[k].data_ptr<float>(), m[k] = exp_avg[k].data_ptr<float>(), v[k] = exp_avg_sq[k].data_ptr<float>();
         g[k] = grads[k].data_ptr<float>();
         sizes[k] = params[k].numel();
-        at[k] = static_cast<double>(steps[k].data_ptr<float>()[0]) + 1.0;
+        at[k] = static_cast<double>(steps[k].data_ptr<float>()[0]);
     }
     check(eppgcn_adam_step(static_cast<int>(count), p.data(), g.data(), m.data(), v.data(), sizes.data(), at.data(), lr, beta1,
                            beta2, eps, stream_of(params[0])),
           "adam_step");
     for (size_t k = 0; k < count; ++k) {
-        steps[k].data_ptr<float>()[0] = static_cast<float>(at[k]);
         // written behind torch's back: a graph that saved one of them has to see that it changed
         for (const Tensor* t : {&params[k], &exp_avg[k], &exp_avg_sq[k], &steps[k]}) t->unsafeGetTensorImpl()->bump_version();
     }

@@ -87,6 +87,25 @@ def test_other_forms_are_left_to_torch_unchanged(spoil):
     _same(before, _states((weights, opt)))
 
 
+def test_weights_that_share_a_step_counter():
+    """The counter moves once for each of them before any of them reads it, as in torch's step."""
+    sides, gen = _pair([(4, 3), (5,), (7,)])
+    grads = [[torch.randn(w.shape, generator=gen) for w in sides[0][0]] for _ in range(3)]
+    for step in range(3):
+        for weights, opt in sides:
+            for w, g in zip(weights, grads[step]):
+                w.grad = g.cuda()
+        if step == 0:
+            for weights, opt in sides:
+                opt.step()
+                opt.state[weights[2]]["step"] = opt.state[weights[0]]["step"]
+        else:
+            assert _call(sides[0][1], sides[0][0])
+            sides[1][1].step()
+        _same(_states(sides[0]), _states(sides[1]))
+    assert [float(sides[0][1].state[w]["step"]) for w in sides[0][0]] == [5.0, 3.0, 5.0]
+
+
 @pytest.mark.parametrize("option", ["plain", "hook", "scheduler", "decay", "sgd", "no_grad", "class"])
 def test_trainer_takes_the_step_its_optimizer_says(option, monkeypatch):
     from eppgcn_amd import graphs, train
