@@ -90,13 +90,19 @@ Tensor workspace(size_t bytes, const Tensor& like)
 // clear_plans() before the next layer operation.
 size_t held_bytes(const Tensor& t) { return t.defined() ? t.storage().nbytes() : 0; }
 
-// A key tensor of an entry.  As long as it is held, or its storage lives by somebody else's hand, the address the entry was
-// made for cannot hold other data.
+// A key tensor of an entry.  As long as its storage lives, by the entry's hand or by somebody else's, and has the memory it
+// had, the address the entry was made for cannot hold other data.  A held tensor alone does not say so: its storage can be
+// resized, and it can be given another storage (`.data = ...`).
 struct Key {
     Tensor held;
     c10::weak_intrusive_ptr<c10::StorageImpl> storage;
-    explicit Key(const Tensor& t) : held(t), storage(t.storage().getWeakStorageImpl()) {}
-    bool alive() const { return held.defined() || !storage.expired(); }
+    const void* memory;
+    explicit Key(const Tensor& t) : held(t), storage(t.storage().getWeakStorageImpl()), memory(t.storage().data()) {}
+    bool alive() const
+    {
+        const auto s = storage.lock();
+        return s && s->data() == memory;
+    }
     size_t bytes() const { return held_bytes(held); }
 };
 
@@ -128,7 +134,7 @@ void trim(Cache& cache, const Drop& drop)
     for (auto it = cache.begin(); it != cache.end();) {
         if (place >= kAlwaysKept) it->let_go();
         const size_t here = it->bytes();
-        if (place < kAlwaysKept || (place < kMostKept && bytes + here <= kKeptBytes && it->alive())) {
+        if (it->alive() && (place < kAlwaysKept || (place < kMostKept && bytes + here <= kKeptBytes))) {
             bytes += here;
             ++place;
             ++it;

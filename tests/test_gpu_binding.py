@@ -628,3 +628,37 @@ def test_paths_of_several_live_models_are_all_remembered_and_large_ones_are_not(
         assert GNNA.cached_paths() == min(k + 1, 8)
     GNNA.clear_plans()
     assert GNNA.cached_paths() == 0
+
+
+@pytest.mark.parametrize("how", ["resized", "swapped"])
+def test_memory_that_a_remembered_path_has_lost_is_looked_over_again(how):
+    """A remembered tensor can lose its memory without dying (its storage resized, its data set to another tensor's): another
+    path in that memory, with the same version counters, is another path."""
+    from eppgcn_amd import gnnadvisor
+    GNNA = gnnadvisor()
+    GNNA.clear_plans()
+    n, size = 4096, 1 << 20                       # four megabytes: a block of its own in torch's allocator
+    x, w, ones = torch.ones(n, 8, device="cuda"), torch.ones(8, 8, device="cuda"), torch.ones(n, device="cuda")
+    grad = torch.arange(n, device="cuda").float()[:, None].expand(n, 8).contiguous()
+    ids, bounds = torch.zeros(size, dtype=torch.int32, device="cuda"), torch.tensor([0, 2], dtype=torch.int32, device="cuda")
+
+    def path(first):
+        return torch.tensor(np.arange(first, first + size, dtype=np.int32) % n).cuda()
+
+    def check(edges, first):
+        dx, _ = GNNA.ours_backward(grad, x, w, ids, bounds, edges, ones, 32, 1, 1, 1, 1)
+        assert torch.equal(dx[0], torch.full_like(dx[0], 8.0 * (2 * first + 1)))
+
+    edges = path(5)
+    check(edges, 5)
+    at = edges.data_ptr()
+    if how == "resized":
+        edges.untyped_storage().resize_(0)
+    else:
+        edges.data = torch.empty(1, dtype=torch.int32, device="cuda")
+    other = path(700)
+    if other.data_ptr() != at:
+        pytest.skip("torch's allocator put the other path elsewhere")
+    assert other._version == edges._version
+    check(other, 700)
+    GNNA.clear_plans()
