@@ -6,6 +6,7 @@ when the library has not been built - there is no fallback implementation.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 
@@ -537,13 +538,14 @@ class Pending:
     def __init__(self, states, finish, stream):
         self.states, self.finish, self.stream = states, finish, stream
 
-    def result(self, states=None):
-        """``states``: where the records have been copied to, None to wait for them; the stream's GPU is current meanwhile."""
-        with torch.cuda.device(self.stream.device):
-            return self.finish(states)
-
     def __call__(self):
-        return self.result()
+        with _current(self.stream.device):
+            return self.finish()
+
+
+def _current(device):
+    """``device`` made current; nothing to do where it is, which is almost always (a switch takes 2 us)."""
+    return contextlib.nullcontext() if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def finish_all(pending):
@@ -555,18 +557,18 @@ def finish_all(pending):
             out[k] = p()
         else:
             of_stream.setdefault((p.stream.device, p.stream.cuda_stream), []).append(k)
-    for mine in of_stream.values():
-        stream = pending[mine[0]].stream
+    for (device, _), mine in of_stream.items():
         addresses = [a for k in mine for a in pending[k].states]
         size = lib.eppgcn_state_bytes()
-        with torch.cuda.device(stream.device):
+        with _current(device):
             host = torch.empty(size * len(addresses), dtype=torch.uint8, pin_memory=True)
-            _check(lib.eppgcn_read_states((C.c_void_p * len(addresses))(*addresses), len(addresses), _ptr(host), _stream(stream)))
-        at = host.data_ptr()
-        for k in mine:
-            count = len(pending[k].states)
-            out[k] = pending[k].result([C.c_void_p(at + size * j) for j in range(count)])
-            at += size * count
+            _check(lib.eppgcn_read_states((C.c_void_p * len(addresses))(*addresses), len(addresses), _ptr(host),
+                                          _stream(pending[mine[0]].stream)))
+            at = host.data_ptr()
+            for k in mine:
+                count = len(pending[k].states)
+                out[k] = pending[k].finish([C.c_void_p(at + size * j) for j in range(count)])
+                at += size * count
     return out
 
 

@@ -227,7 +227,7 @@ class _FakeStream:
     """What ``capi.Pending`` looks at of a stream; the default stream of every GPU has the handle 0."""
 
     def __init__(self, device, handle):
-        self.device, self.cuda_stream = device, handle
+        self.device, self.cuda_stream = torch.device(device), handle
 
 
 class _FakeLibrary:
@@ -235,10 +235,10 @@ class _FakeLibrary:
     eppgcn_state_bytes = staticmethod(lambda: 64)
 
     def __init__(self):
-        self.current, self.reads = "cuda:0", []
+        self.current, self.reads, self.switches = torch.device("cuda:0"), [], 0
 
     def eppgcn_read_states(self, addresses, count, host, stream):
-        self.reads.append((self.current, stream.value or 0, list(addresses)))
+        self.reads.append((str(self.current), stream.value or 0, list(addresses)))
         for j in range(count):
             ctypes.cast(host.value + 64 * j, ctypes.POINTER(ctypes.c_int64))[0] = addresses[j]
         return 0
@@ -247,6 +247,7 @@ class _FakeLibrary:
         @contextlib.contextmanager
         def made_current():
             before, self.current = self.current, device
+            self.switches += 1
             yield
             self.current = before
         return made_current()
@@ -258,13 +259,14 @@ def fake(monkeypatch):
     monkeypatch.setattr(capi, "load", lambda: lib)
     monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **k: empty(*a, **k))
     monkeypatch.setattr(torch.cuda, "device", lib.device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: lib.current.index)
     return lib
 
 
 def _pending(lib, records, stream):
     """A result that is (records as read or None, the GPU that was current)."""
     def finish(states=None):
-        return states and [ctypes.cast(s, ctypes.POINTER(ctypes.c_int64))[0] for s in states], lib.current
+        return states and [ctypes.cast(s, ctypes.POINTER(ctypes.c_int64))[0] for s in states], str(lib.current)
     return capi.Pending(records, finish, stream)
 
 
@@ -273,9 +275,11 @@ def test_results_of_two_gpus_are_read_by_a_call_each(fake):
     same stream do, and everything happens with the stream's own GPU current."""
     streams = [_FakeStream("cuda:0", 0), _FakeStream("cuda:1", 0), _FakeStream("cuda:0", 0), _FakeStream("cuda:1", 7)]
     work = [_pending(fake, [100 + k, 200 + k], s) for k, s in enumerate(streams)]
-    assert capi.finish_all(work) == [([100 + k, 200 + k], s.device) for k, s in enumerate(streams)]
+    assert capi.finish_all(work) == [([100 + k, 200 + k], str(s.device)) for k, s in enumerate(streams)]
     assert fake.reads == [("cuda:0", 0, [100, 200, 102, 202]), ("cuda:1", 0, [101, 201]), ("cuda:1", 7, [103, 203])]
-    assert work[1]() == (None, "cuda:1") and fake.current == "cuda:0"
+    assert fake.switches == 2                    # none for the GPU that is current
+    assert work[1]() == (None, "cuda:1") and work[0]() == (None, "cuda:0")
+    assert fake.current == torch.device("cuda:0") and fake.switches == 3
 
 
 def test_a_result_without_a_record_leaves_the_others_to_one_wait(fake):
