@@ -97,7 +97,7 @@ struct PlanView {
 
 // Stream form of a plan (read by stream.hip, built by schedule.hip).  A "piece" is a maximal stretch of
 // plan entries that continue one another, i.e. consecutive slots of one row.
-constexpr int kStreamWave = 512;     // slots a wave of the stream kernel takes
+constexpr int kStreamWave = 512;     // slots of a chunk: what a workgroup of the stream kernel takes
 constexpr int kStreamChunk = 32;     // piece ends are counted per chunk of this many slots
 constexpr unsigned kStreamFlag = 0x80000000u;
 constexpr int kStreamIdMask = 0x7fffffff;
@@ -122,7 +122,7 @@ struct StreamView {
     StreamHeader* header;
     int* erow;          // [P]  per piece: its row, or kStreamFlag | index of its partial sum
     int* cev;           // [S_pad / 32 + 1]  pieces that end before slot 32 c; bit 31: slot 32 c continues a piece
-    int* wtail;         // [S_pad / 512]  index of the partial sum of what wave w holds at its end, or -1
+    int* wtail;         // [S_pad / 512]  index of the partial sum of what chunk w holds at its end, or -1
     uint32_t* touched;  // [ceil(N/32)]  bit r: row r has at least one slot
     int* frow;          // [N]  rows with partial sums ...
     int* fptr;          // [N+1] ... and where their partial sums start

@@ -473,8 +473,8 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     }
     __syncthreads();
     // Zeros behind the kept slots of the whole input, written here and not by a pass of their own because they cost what their
-    // bytes cost: 13 of 132 M slots kept, this kernel 384 -> 513 us and the pass behind it 195 -> 15.  As many words as this tile drops slots, counted from the end, behind
-    // those of the tiles before it (which dropped base - s_prefix slots).
+    // bytes cost: 13 of 132 M slots kept, this kernel 384 -> 513 us and the pass behind it 195 -> 15.  As many words as this
+    // tile drops slots, counted from the end, behind those of the tiles before it (which dropped base - s_prefix slots).
     if (wave == 0) {
         int n = 0;
 #pragma unroll
@@ -1195,7 +1195,9 @@ static int launch_mark_pass(const int* part2node, const int* part_ptr, const int
     // place_slots walks a small tile from barrier to barrier.  1024 threads do that fastest as long as the chip holds all tiles
     // at once (two workgroups on a CU: 512 tiles), beyond that four workgroups of 512 threads hide each other's waits better:
     // 27 tiles 13.5 us with 1024 threads, 15.5 with 512, 21.5 with 256; 2250 tiles 63, 50, 54.  Tiles of 16 384 slots (scale
-    // 22, the mean of two layers): 450, 474, 522.
+    // 22, the mean of two layers): 450, 474, 522.  At the line, a whole marking with 1024 / 512 threads, us: 256 tiles 25.7 /
+    // 27.9, 500 tiles 32.8 / 33.5, 520 tiles 42.4 / 36.4, 1024 tiles 55.7 / 45.9 (a tenth kept: 24.0 / 24.8, 30.6 / 29.8,
+    // 36.4 / 32.1, 49.2 / 40.2).
     if (l.tile_slots == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge, 1024, true);
     else if (l.num_tiles > 512) EPPGCN_MARK(kMarkItemsSmall, 512, false);
     else EPPGCN_MARK(kMarkItemsSmall, 1024, false);
@@ -1257,12 +1259,16 @@ int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, 
     return kOk;
 }
 
-// counts[0] = number of groups, counts[1] = number of slots covered.
-// part2node_out (may be NULL for degrees): the vertex of every group, rows_capacity entries
 // Before a split of kept degrees: the scan state, and the whole array of group pointers cleared.  With groups of the usual
 // size they are a few hundredths of the entries, so clearing what they overwrite costs less than a launch behind the split
 // that first has to know their end: path preparation at R-MAT scale 22 3954 -> 3908 us, at 19 717 vertices 1.5 % less.  Groups
 // of one to three slots can fill most of a large array: there the tail is cleared afterwards (zero_tail1_kernel).
+// A split, us, cleared before / behind, with every slot kept (groups of 1 / 2 / 3 fill 78 / 42 / 29 % of the entries):
+//   0.6 M entries  groups of 1, 3, 4 slots: 27.2 / 29.1, 13.3 / 15.4, 7.9 / 10.1      1.3 M  28.3 / 29.9, 14.3 / 16.1, 9.1 / 10.9
+//   5 M            35.7 / 34.9, 20.8 / 21.7, 14.7 / 15.7      161 M  608 / 546, 355 / 349, 272 / 279, of 32 slots 224 / 243
+// and with a tenth of the slots kept, 161 M: 262 / 287, 238 / 269, 227 / 260.  So both lines are on the cautious side: groups
+// of one slot are even at 4 M entries, and below that, and with few slots kept, clearing before is up to 2 us (a tenth) faster
+// also for groups of less than four slots, which clear behind from 1 M entries on.
 constexpr int kClearFirstPartSize = 4;
 constexpr long long kClearFirstEntries = 1 << 20;
 __global__ __launch_bounds__(256) void split_init_kernel(ScanState* st, uint64_t* desc, int num_tiles, int* __restrict__ p,
@@ -1286,6 +1292,8 @@ __global__ __launch_bounds__(256) void split_init_kernel(ScanState* st, uint64_t
     if (tid < words - tail) p[tail + tid] = 0;
 }
 
+// counts[0] = number of groups, counts[1] = number of slots covered.
+// part2node_out (may be NULL for degrees): the vertex of every group, rows_capacity entries
 int launch_split(bool from_row_ptr, const int* src, int num_nodes, int part_size, int* part_ptr_out,
                  int* part2node_out, long long capacity, long long rows_capacity, bool zero_tail, void* workspace,
                  hipStream_t stream)

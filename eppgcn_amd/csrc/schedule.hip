@@ -19,12 +19,13 @@
 // of slots of one row); the last slot of every piece carries bit 31 in col[], col[] is padded to a multiple
 // of 512 slots with an id behind every table row (N rounded up to a multiple of 4096), and
 //     erow[e]    row of piece e when the stream kernel can write it with one store (the piece is all of its row
-//                and lies inside one wave's 512 slots), otherwise bit 31 | index of the partial sum it leaves
+//                and lies inside one chunk, the 512 slots of a workgroup), otherwise bit 31 | index of the partial
+//                sum it leaves
 //     cev[c]     pieces that end before slot 32 c; bit 31 when slot 32 c continues a piece
-//     wtail[w]   index of the partial sum for what wave w still holds at its last slot, or -1
+//     wtail[w]   index of the partial sum for what chunk w still holds at its last slot, or -1
 //     touched    one bit per vertex: the row has at least one slot
 //     frow/fptr  rows that have partial sums and the range of each; the partial sums are numbered row by row,
-//                inside a row those of its piece ends, then those of the waves' tails, each in the caller's group order
+//                inside a row those of its piece ends, then those of the chunks' tails, each in the caller's group order
 //                (the stream's too when the columns of a row ascend), so that summing a range in order gives the
 //                same bits every run
 // and a header with the counts.  A plan with empty groups gets no stream form (header.valid = 0).
@@ -279,8 +280,8 @@ __device__ __forceinline__ int4 pack_group(int beg, int size, int row, int p, bo
 }
 
 // Per group p: rowp[p] (0 for an empty group; rowp == nullptr: part2node is that array), rec[p] (pack_group; nullptr: nothing is
-// sorted), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the group has slots; the row bitmaps; the sort key and the digit counts of the first radix pass (keys == nullptr: the plan
-// keeps the caller's order).
+// sorted), info[p] = bit0 the row has groups before this one, bit1 after it, bit2 the group has slots; the row bitmaps; the sort
+// key and the digit counts of the first radix pass (keys == nullptr: the plan keeps the caller's order).
 // Sort key of group p: the column block of its first slot, except that all groups of a short row
 // (at most `keep_slots` slots in at most kMaxRowWalk groups) share the key of the row's first group:
 // such a row stays together in the plan, is summed in registers and written once with plain stores,
@@ -602,9 +603,9 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ 
     }
 }
 
-// Which pieces leave partial sums, and how many: a piece that is not all of its row, or that crosses from one wave's
-// slots into the next, leaves one at its end, and one more per wave boundary it crosses (what that wave still holds at
-// its last slot).  Group p (in the caller's order; plan entry place[p], nullptr: p) speaks for the piece it ends.  Two scans
+// Which pieces leave partial sums, and how many: a piece that is not all of its row, or that crosses from one chunk of
+// 512 slots into the next, leaves one at its end, and one more per chunk boundary it crosses (what that chunk still holds
+// at its last slot).  Group p (in the caller's order; plan entry place[p], nullptr: p) speaks for the piece it ends.  Two scans
 // run side by side, wave 0's over (tails, ends) packed as tails * 2^31 + ends, wave 1's over (rows with slots, rows with
 // partial sums).
 // The partial sums of row j of the fix list are numbered ends first, then tails: its range starts at ends + tails before
@@ -703,7 +704,7 @@ __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
     }
 }
 
-// The number of every partial sum into erow (a piece's end) and wtail (a wave's tail); the header is completed.
+// The number of every partial sum into erow (a piece's end) and wtail (a chunk's tail); the header is completed.
 __global__ __launch_bounds__(256) void plan_targets_kernel(StreamView sv, const int* __restrict__ event_of,
                                                           const int* __restrict__ first, const int* __restrict__ last,
                                                           const int* __restrict__ fix_of, const int* __restrict__ ends_at,

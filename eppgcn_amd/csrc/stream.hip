@@ -1,5 +1,5 @@
 // Slot-stream aggregation for gfx950 (wave64): the aggregation of a planned launch as a segmented sum
-// over one stream of slots, every wave taking the same number of slots.
+// over one stream of slots, every workgroup taking a chunk of the same number of slots.
 //
 // Same contract as aggregate_kernel (EPPGCN/GCNConv/EPPGCN_kernel.cu:204-295, :626-670):
 //
@@ -11,10 +11,10 @@
 //   scol[S_pad]   column id of every slot in processing order; bit 31 set on the last slot of a piece;
 //                 padded to a multiple of kStreamWave slots with an id behind the table ("gathers nothing")
 //   erow[NE]      one entry per piece, in stream order: its row when one store writes it (the piece is all of
-//                 its row and lies inside one wave's slots), else bit 31 | the index of its partial sum
+//                 its row and lies inside one chunk), else bit 31 | the index of its partial sum
 //   cev[S_pad / 32 + 1]   number of pieces that end before slot 32 c; bit 31 set when slot 32 c lies inside
 //                 a piece that started earlier
-//   wtail[S_pad / 512]    index of the partial sum of what wave w holds after its last slot, or -1
+//   wtail[S_pad / 512]    index of the partial sum of what chunk w holds after its last slot, or -1
 //   frow, fptr    the rows that have partial sums and the range of each (numbered row by row)
 //
 // Mapping.  A workgroup of four waves takes a chunk of kStreamWave = 512 consecutive slots, a wave 128 of them: lane l
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kStreamBlock) void aggregate_stream_kernel(
     // the output (width 22 at R-MAT 22: 1522 -> 1514 us per call)
     int w = blockIdx.x;
     if ((w | 31) < num_wave_chunks) w = (w & ~31) | (w & 7) << 2 | (w >> 3 & 3);
-    
+
     // the counts the host remembers must be those of the plan in memory (they are unless the plan's bytes were
     // replaced behind the library's back): a mismatch ends the kernel instead of indexing with the wrong sizes,
     // and leaves a mark that eppgcn_aggregation_status reports (the output of this call is not written)

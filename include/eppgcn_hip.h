@@ -106,8 +106,8 @@ int64_t eppgcn_feature_workspace_row(int64_t vertex);
  *
  * Stream form.  The plan also holds its slots as one stream with the ends of the rows' pieces marked
  * (a piece = consecutive plan entries that continue one another), for a second kernel in which every
- * wave takes the same number of slots, every gather instruction is full whatever the row lengths,
- * and no float atomics are used: pieces that are all of their row and lie inside one wave's 512 slots
+ * workgroup takes a chunk of 512 slots, every gather instruction is full whatever the row lengths,
+ * and no float atomics are used: pieces that are all of their row and lie inside one chunk
  * are stored directly, the others leave partial sums in a scratch area behind the feature table,
  * which a small second kernel adds up row by row in a fixed order.  Results are then the same bits
  * on every run.  An aggregation call takes this path when

@@ -381,7 +381,7 @@ def test_stream_from_a_table_written_by_the_dense_update(api):
 
 def _ragged_csr(rng, n):
     """Rows of very different lengths: a share of empty rows, mostly short ones, a few hubs of up to thousands of
-    slots (longer than a wave's 512 slots, cut into many column blocks)."""
+    slots (longer than a chunk of 512 slots, cut into many column blocks)."""
     deg = rng.geometric(rng.uniform(0.05, 0.6), n).astype(np.int64)
     deg[rng.random(n) < rng.uniform(0.0, 0.5)] = 0
     hubs = rng.integers(0, n, rng.integers(0, 4))
