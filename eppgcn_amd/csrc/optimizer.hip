@@ -2,7 +2,8 @@
 //
 // A weight matrix of this model holds 96 x 16 or 16 x 22 floats, so a step is launches and host work.  As torch's grouped
 // operations a step was eleven launches of 2 to 3 us and 90 to 104 us of host time; an epoch without a wait at its end takes, us,
-// before -> with this kernel: 2708 vertices 338 -> 225, 19 717 vertices 337 -> 228, there with four layers of 32 771 -> 628.
+// before -> with this kernel: 2708 vertices 338 -> 225, 19 717 vertices 337 -> 228, there with four layers of 32 (three live
+// models) 771 -> 628.
 // Every element is rounded as torch's grouped operations round it (a fused multiply-add where one of them multiplies and
 // adds), which is needed: the first steps divide a gradient by its own size, so a weight whose gradient is near zero moves by
 // what rounding made of it.  What bounds it: the launch; large weights are streamed (28 bytes per element).
