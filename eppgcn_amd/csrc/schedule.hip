@@ -253,23 +253,29 @@ __global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanSca
     }
 }
 
-// Sets bit (row & 31) of map[row >> 5] for the lanes with `set`: the lanes of a wave whose rows share a word (rows ascend
-// along the groups, so they are neighbours) combine their bits first, one atomic per run.  One atomic per group, as before,
-// was most of the old classification kernel (0.7 ms per run at R-MAT scale 22).
-__device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ map, int row, bool set)
+// Sets bit (row & 31) of touched[row >> 5] for the lanes with `set`, and of single[row >> 5] for those with `alone` too: the
+// lanes of a wave whose rows share a word (rows ascend along the groups, so they are neighbours) combine their bits first,
+// one atomic per run.  One atomic per group was most of the classification kernel before (0.7 ms per run at R-MAT scale 22);
+// combining the bits in six shuffle steps per map cost plan_keys 22 of 401 us more than these sums.  A row's bit is counted in its first lane, so the bits of a run are distinct and their sum is their union;
+// rows that do not ascend are set one by one.
+__device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ touched, uint32_t* __restrict__ single, int row, bool set,
+                                            bool alone)
 {
-    const int lane = lane_id();
-    const int word = set ? row >> 5 : -1;
-    uint32_t bits = set ? 1u << (row & 31) : 0u;
-    const int prev = __shfl_up(word, 1, kWave);
-    const uint64_t heads = __ballot(lane == 0 || prev != word);
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t other = static_cast<uint32_t>(__shfl_down(static_cast<int>(bits), off, kWave));
-        const uint64_t between = (heads >> 1 >> lane) & ((1ull << off) - 1ull);      // run heads in lanes lane+1 .. lane+off
-        if (lane + off < kWave && between == 0) bits |= other;
+    const int mine = set ? row : -1;
+    const int left = __builtin_amdgcn_update_dpp(-1, mine, kDppWaveShr1, 0xF, 0xF, false);
+    const int bit = static_cast<int>(1u << (row & 31));
+    if (__any(set && left > row)) {
+        if (set) atomicOr(touched + (row >> 5), static_cast<uint32_t>(bit));
+        if (set && alone) atomicOr(single + (row >> 5), static_cast<uint32_t>(bit));
+        return;
     }
-    if (((heads >> lane) & 1ull) && bits) atomicOr(map + word, bits);
+    const uint64_t heads = __ballot(left >> 5 != mine >> 5) | 1ull;
+    const uint32_t all = static_cast<uint32_t>(wave_run_sum(set && left != row ? bit : 0, heads));
+    const uint32_t some = static_cast<uint32_t>(wave_run_sum(set && left != row && alone ? bit : 0, heads));
+    if ((heads >> lane_id()) & 1ull) {
+        if (all) atomicOr(touched + (row >> 5), all);
+        if (some) atomicOr(single + (row >> 5), some);
+    }
 }
 
 // What plan_order_kernel needs of a group, 16 bytes that the sort moves: first slot, slots, row, number; bit 31 of the first two:
@@ -344,8 +350,7 @@ __global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
             if (!some) h->empty_groups = 1;
         }
         const bool in_range = some && row[r] >= 0 && row[r] < num_nodes;
-        or_row_bits(touched, row[r], in_range);
-        or_row_bits(single, row[r], in_range && !prev && !next);
+        or_row_bits(touched, single, row[r], in_range, !prev && !next);
         if (!keys || !have) continue;
         unsigned key = 0u;
         if (some) {

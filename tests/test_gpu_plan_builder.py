@@ -198,3 +198,36 @@ def test_the_entries_behind_the_groups_are_cleared(api, capacity, ps, offset):
     want[:starts.size] = starts
     assert np.array_equal(out.cpu().numpy(), want)
     assert (whole[:16 + offset] == 7).all() and (whole[16 + offset + capacity:] == 7).all()
+
+
+@pytest.mark.parametrize("order", ["ascending", "descending", "mixed"])
+@pytest.mark.parametrize("ps", [1, 7, 32])
+def test_rows_in_any_order(api, order, ps):
+    """The bitmaps of the rows are put together from runs of neighbouring groups whose rows ascend, and row by row where they
+    do not: rows in another order than the groups' give the plan they give in order, for both kernels that run over it."""
+    indptr, col = csr_of(degrees_of("mixed"), 9)
+    n = indptr.size - 1
+    name = np.arange(n, dtype=np.int32)
+    if order == "descending":
+        name = name[::-1].copy()
+    elif order == "mixed":                             # blocks of 96 rows in a random order: ascending and not inside a wave
+        blocks = np.random.default_rng(2).permutation((n + 95) // 96)
+        name = np.concatenate([np.arange(b * 96, min(n, b * 96 + 96), dtype=np.int32) for b in blocks])
+    pp, p2n = co.build_part(ps, indptr)
+    rows = dev(name[p2n])
+    plan = api.build_plan(dev(pp), dev(col), p2n.size, col.size, n, 16, part2node=rows)
+    touched = plan.stream_view()["touched"].cpu().numpy().view(np.uint8)
+    want = np.zeros(touched.size * 8, np.uint8)
+    want[name[np.diff(indptr) > 0]] = 1
+    assert np.array_equal(np.unpackbits(touched, bitorder="little"), want)
+    x = np.random.default_rng(1).integers(-4, 5, (n, 16)).astype(np.float32)
+    sums = np.zeros((n, 16), np.float32)
+    sums[name] = co.spmm_f64(x, indptr, col, np.ones(n, np.float32)).astype(np.float32)
+    try:
+        for stream in (True, False):                   # the group kernel reads the rows of a single group (stored, not cleared)
+            api.set_stream_mode(stream)
+            out = torch.full((n, 16), float("nan"), device="cuda")
+            api.spmm_forward(dev(x), dev(col), torch.ones(n, device="cuda"), dev(pp), rows, part_size=ps, plan=plan, out=out)
+            assert api.last_call_used_stream() == stream and np.array_equal(out.cpu().numpy(), sums)
+    finally:
+        api.set_stream_mode(True)
