@@ -47,7 +47,7 @@
 //   plan_targets   writes erow / wtail from those numbers and completes the header
 // Every kernel streams its arrays once; what used to be 46 launches, four of them radix passes over 8 M keys, is 9.  R-MAT
 // scale 22, both paths and the forward groups of a two-layer run (7.8 + 5.9 + 1.7 M groups, 132 + 126 + 13 M slots):
-// 6.0 -> 2.2 ms for the three plans; scale 20 (8.8 + 7.3 + 0.9 M slots): 1.3 -> 0.35 ms.
+// 6.0 -> 1.65 ms for the three plans; scale 20 (8.8 + 7.3 + 0.9 M slots): 1.3 -> 0.30 ms.
 #include <atomic>
 #include <cstring>
 
@@ -296,93 +296,107 @@ __device__ __forceinline__ int4 pack_group(int beg, int size, int row, int p, bo
 // groups, are what a block can speed up: with groups of 4-8 slots a bound in groups spread rows of 40 slots and lost up
 // to 2x at 256 columns).
 // The walk to the ends of a row stops as soon as the row cannot be short any more: with the usual group sizes that is
-// after two or three groups, where a hub's groups walked 64 neighbours each way before (0.55 -> 0.28 ms for the 7.8 M
-// forward groups of R-MAT scale 22).  What is left is one cache line of `col` per group, and one of `ids` where the rows are
-// looked up there: 5.9 M groups of a path 347 us with ids, 172 with the rows that the split left (eppgcn_split_and_plan).
+// after two or three groups.  It runs over pointers and rows in LDS, those of the tile and of the 64 groups on either side of it
+// (a step was a round trip to memory, one round of groups after the other: 48 us for the 705 tiles of R-MAT scale 20, all of
+// which run at once; with the sorted path of that scale 81 -> 52 us, with 256 threads 69, with 1024 48 but 6 % slower at scale
+// 22), and the columns that decide the keys are loaded together.  What is left at scale 22 (7.8 M groups 202 -> 190 us) is one cache line
+// of `col` per group, and one of `ids` where the rows are looked up there: 5.9 M groups of a path 347 us with ids, 172 with the
+// rows that the split left (eppgcn_split_and_plan).
 constexpr int kMaxRowWalk = 64;
-__global__ __launch_bounds__(kSortBlock) void plan_keys_kernel(
+constexpr int kKeysBlock = 512;
+constexpr int kKeysRounds = kSortTile / kKeysBlock;
+static_assert(kSortTile % kKeysBlock == 0 && kKeysBlock >= kDigits, "group (round r, thread t) of a tile is r * 512 + t; a thread per digit");
+__global__ __launch_bounds__(kKeysBlock) void plan_keys_kernel(
     const int* __restrict__ part_ptr, const int* __restrict__ col, const int* __restrict__ part2node,
     const int* __restrict__ ids, int num_parts, int num_nodes, int shift, int keep_slots, int classes, int digits,
     int num_tiles, unsigned* __restrict__ keys, int* __restrict__ hist, int* __restrict__ rowp, uint8_t* __restrict__ info,
     int4* __restrict__ rec, uint32_t* __restrict__ single, uint32_t* __restrict__ touched, StreamHeader* __restrict__ h, const ScanState* sort_state)
 {
+    constexpr int kHalo = kMaxRowWalk;                  // groups of the neighbouring tiles that a walk can reach
+    constexpr int kStaged = kSortTile + 2 * kHalo;
+    __shared__ int s_ptr[kStaged + 1];                  // [i]: group base - kHalo + i
+    __shared__ int s_row[kStaged];
     __shared__ int s_hist[kDigits];
     if (sort_state->error) return;
-    s_hist[threadIdx.x] = 0;
+    if (threadIdx.x < kDigits) s_hist[threadIdx.x] = 0;
+    const int base = static_cast<int>(static_cast<long long>(blockIdx.x) * kSortTile);      // < num_parts
+    const long long origin = static_cast<long long>(base) - kHalo;
+    for (int i = threadIdx.x; i <= kStaged; i += kKeysBlock) {
+        const long long g = min(max(origin + i, 0ll), static_cast<long long>(num_parts));
+        s_ptr[i] = part_ptr[g];
+        if (part2node && i < kStaged) s_row[i] = part2node[min(g, static_cast<long long>(num_parts) - 1)];
+    }
     __syncthreads();
-    const long long base = static_cast<long long>(blockIdx.x) * kSortTile;
-    int beg[kSortRounds], end[kSortRounds], row[kSortRounds], before[kSortRounds], after[kSortRounds];
-#pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
-        const long long p = base + r * kSortBlock + threadIdx.x;
-        beg[r] = p < num_parts ? part_ptr[p] : 0;
-        end[r] = p < num_parts ? part_ptr[p + 1] : 0;
+    if (!part2node) {
+        for (int i = threadIdx.x; i < kStaged; i += kKeysBlock)
+            s_row[i] = s_ptr[i + 1] > s_ptr[i] ? ids[s_ptr[i]] : 0;
+        __syncthreads();
     }
+    int at[kKeysRounds], cls[kKeysRounds];              // slot whose column decides the key (-1: an empty group's), length class
 #pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
-        const int p = static_cast<int>(base) + r * kSortBlock + static_cast<int>(threadIdx.x);
-        const bool some = end[r] > beg[r];
-        row[r] = 0;
-        before[r] = after[r] = -1;
-        if (some) {
-            if (part2node) {
-                row[r] = part2node[p];
-                if (p > 0) before[r] = part2node[p - 1];
-                if (p + 1 < num_parts) after[r] = part2node[p + 1];
-            } else {
-                row[r] = ids[beg[r]];
-                if (beg[r] > 0) before[r] = ids[beg[r] - 1];
-                if (p + 1 < num_parts) after[r] = ids[end[r]];
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kSortRounds; ++r) {
-        const long long pl = base + r * kSortBlock + threadIdx.x;
+    for (int r = 0; r < kKeysRounds; ++r) {
+        const int i = kHalo + r * kKeysBlock + static_cast<int>(threadIdx.x);
+        const long long pl = origin + i;
         const int p = static_cast<int>(pl);
         const bool have = pl < num_parts;
-        const bool some = end[r] > beg[r];
-        const bool prev = some && before[r] == row[r], next = some && after[r] == row[r];
+        const int beg = s_ptr[i], end = s_ptr[i + 1];
+        const bool some = have && end > beg;
+        const int row = some ? s_row[i] : 0;
+        int before = -1, after = -1;
+        if (some) {
+            if (part2node) {
+                if (p > 0) before = s_row[i - 1];
+                if (p + 1 < num_parts) after = s_row[i + 1];
+            } else {
+                if (beg > 0) before = ids[beg - 1];
+                if (p + 1 < num_parts) after = ids[end];
+            }
+        }
+        const bool prev = some && before == row, next = some && after == row;
         if (have) {
-            if (rowp) rowp[p] = row[r];
+            if (rowp) rowp[p] = row;
             info[p] = static_cast<uint8_t>((prev ? 1 : 0) | (next ? 2 : 0) | (some ? 4 : 0));
-            if (rec) rec[p] = pack_group(beg[r], some ? end[r] - beg[r] : 0, row[r], p, prev, next);
+            if (rec) rec[p] = pack_group(beg, some ? end - beg : 0, row, p, prev, next);
             if (!some) h->empty_groups = 1;
         }
-        const bool in_range = some && row[r] >= 0 && row[r] < num_nodes;
-        or_row_bits(touched, single, row[r], in_range, !prev && !next);
-        if (!keys || !have) continue;
-        unsigned key = 0u;
-        if (some) {
-            auto same_row = [&](int j) {
-                const int b = part_ptr[j];
-                if (part_ptr[j + 1] <= b) return false;
-                return (part2node ? part2node[j] : ids[b]) == row[r];
-            };
-            int start = p, last = p;
-            bool short_row = keep_slots > 0 && end[r] - beg[r] <= keep_slots;
-            int first_slot = beg[r], past = end[r];
-            while (short_row && start > 0 && same_row(start - 1)) {
-                first_slot = part_ptr[--start];
-                short_row = past - first_slot <= keep_slots && p - start < kMaxRowWalk;
-            }
-            while (short_row && last + 1 < num_parts && same_row(last + 1)) {
-                past = part_ptr[++last + 1];
-                short_row = past - first_slot <= keep_slots && last - start < kMaxRowWalk;
-            }
-            key = static_cast<unsigned>(col[short_row ? first_slot : beg[r]]) >> shift;
-            if (classes) {
-                // second key: length class of a row that is a single group (a class = one gather step of 8
-                // slots), so that the groups a wave works on in one round take the same number of steps;
-                // rows of several groups consist of full groups but for the last one: class 3
-                const int cls = (short_row && start == last) ? min(3, (end[r] - beg[r] - 1) >> 3) : 3;
-                key = (key << 2) | static_cast<unsigned>(cls);
-            }
+        const bool in_range = some && row >= 0 && row < num_nodes;
+        or_row_bits(touched, single, row, in_range, !prev && !next);
+        at[r] = -1;
+        cls[r] = 0;
+        if (!keys || !some) continue;
+        auto same_row = [&](int j) { return s_ptr[j + 1] > s_ptr[j] && s_row[j] == row; };
+        const int lo = base < kHalo ? kHalo - base : 0;                                         // group 0
+        const int hi = static_cast<int>(min(static_cast<long long>(kStaged), num_parts - origin));      // behind the last group
+        int start = i, last = i;
+        bool short_row = keep_slots > 0 && end - beg <= keep_slots;
+        int first_slot = beg, past = end;
+        while (short_row && start > lo && same_row(start - 1)) {
+            first_slot = s_ptr[--start];
+            short_row = past - first_slot <= keep_slots && i - start < kMaxRowWalk;
         }
+        while (short_row && last + 1 < hi && same_row(last + 1)) {
+            past = s_ptr[++last + 1];
+            short_row = past - first_slot <= keep_slots && last - start < kMaxRowWalk;
+        }
+        at[r] = short_row ? first_slot : beg;
+        // second key: length class of a row that is a single group (a class = one gather step of 8
+        // slots), so that the groups a wave works on in one round take the same number of steps;
+        // rows of several groups consist of full groups but for the last one: class 3
+        cls[r] = (short_row && start == last) ? min(3, (end - beg - 1) >> 3) : 3;
+    }
+    if (!keys) return;
+    int first_col[kKeysRounds];
+#pragma unroll
+    for (int r = 0; r < kKeysRounds; ++r) first_col[r] = at[r] >= 0 ? col[at[r]] : 0;
+#pragma unroll
+    for (int r = 0; r < kKeysRounds; ++r) {
+        const long long p = static_cast<long long>(base) + r * kKeysBlock + threadIdx.x;
+        if (p >= num_parts) continue;
+        unsigned key = static_cast<unsigned>(first_col[r]) >> shift;
+        if (classes) key = (key << 2) | static_cast<unsigned>(cls[r]);
         keys[p] = key;
         atomicAdd(&s_hist[key & (digits - 1)], 1);
     }
-    if (!keys) return;
     __syncthreads();
     if (static_cast<int>(threadIdx.x) < digits)
         hist[static_cast<long long>(threadIdx.x) * num_tiles + blockIdx.x] = s_hist[threadIdx.x];
@@ -402,13 +416,13 @@ constexpr int kFillTile = 2048;            // slots a workgroup of plan_fill_ker
 static_assert(kFillTile % kStreamWave == 0 && kFillTile % kStreamChunk == 0, "cev and wtail entries belong to one fill tile");
 
 // Plan entry q holds the group of rec[q] (rec == nullptr: group q).  One scan carries (slots, piece ends) packed as
-// ends * 2^31 + slots.  Piece e: first[e] = its first slot | bit 31 when the row has groups before it, last[e] = its last
-// slot, erow[e] = its row, event_at[q] = e for the entry q that ends it and -1 for every other entry.
+// ends * 2^31 + slots.  Piece e: extent[e] = its first slot | bit 31 when the row has groups before it, and its last
+// slot; erow[e] = its row, event_at[q] = e for the entry q that ends it and -1 for every other entry.
 // tile_q[t] = the plan entry that holds slot t * kFillTile.
 __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
     const int* __restrict__ part_ptr, const int4* __restrict__ rec, const int* __restrict__ rowp,
     const uint8_t* __restrict__ info, int num_parts, int num_slots, int num_tiles, PlanView plan, StreamView sv,
-    int* __restrict__ src, int* __restrict__ ends_before, int* __restrict__ first, int* __restrict__ last,
+    int* __restrict__ src, int* __restrict__ ends_before, int2* __restrict__ extent,
     int* __restrict__ event_at, int* __restrict__ tile_q, ScanState* st, uint64_t* desc, unsigned mode, const ScanState* sort_state)
 {
     __shared__ int s_tile;
@@ -504,9 +518,9 @@ __global__ __launch_bounds__(kPlanBlock) void plan_order_kernel(
         ends_before[q] = e;
         event_at[q] = ends ? e : -1;
         if (size[r] == 0) continue;
-        if ((f[r] & 4u) == 0 && e < num_parts) first[e] = slot | ((f[r] & 1u) ? static_cast<int>(kStreamFlag) : 0);
+        if ((f[r] & 4u) == 0 && e < num_parts) extent[e].x = slot | ((f[r] & 1u) ? static_cast<int>(kStreamFlag) : 0);
         if (ends && e < num_parts) {
-            last[e] = slot + size[r] - 1;
+            extent[e].y = slot + size[r] - 1;
             sv.erow[e] = row[r];
         }
         for (long long t = (static_cast<long long>(slot) + kFillTile - 1) / kFillTile;
@@ -584,7 +598,8 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ 
     for (int k = 0; k < kItems; ++k) {
         const int i = k * 256 + static_cast<int>(threadIdx.x);
         const bool flagged = (s_last[i >> 6] >> (i & 63)) & 1ull;
-        if (base + i < padded_slots) plan.col[base + i] = v[k] | (flagged ? static_cast<int>(kStreamFlag) : 0);
+        if (base + i < padded_slots)
+            __builtin_nontemporal_store(v[k] | (flagged ? static_cast<int>(kStreamFlag) : 0), plan.col + base + i);
     }
     if (threadIdx.x < kFillTile / kStreamWave) {
         const int w = base / kStreamWave + threadIdx.x;
@@ -617,8 +632,8 @@ __global__ __launch_bounds__(256) void plan_fill_kernel(const int* __restrict__ 
 // its first group.  fix_of[p] = j or -1; ends_at / tails_at[p] the counts before p; ends0 / tails0[j] those before row j.
 __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
     const int* __restrict__ rowp, const uint8_t* __restrict__ info, const int* __restrict__ place,
-    const int* __restrict__ event_at, int* __restrict__ event_of, const int* __restrict__ first,
-    const int* __restrict__ last, int num_parts, int num_nodes, int num_tiles,
+    const int* __restrict__ event_at, int* __restrict__ event_of, const int2* __restrict__ extent,
+    int num_parts, int num_nodes, int num_tiles,
     StreamView sv, int* __restrict__ fix_of, int* __restrict__ ends_at, int* __restrict__ tails_at,
     int* __restrict__ ends0, int* __restrict__ tails0, int* __restrict__ ends_total, PlanScans sc, unsigned mode)
 {
@@ -641,8 +656,9 @@ __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
     }
 #pragma unroll
     for (int r = 0; r < kPlanItems; ++r) {
-        a[r] = e[r] >= 0 ? first[e[r]] : -1;
-        b[r] = e[r] >= 0 ? last[e[r]] : 0;
+        const int2 x = e[r] >= 0 ? extent[e[r]] : make_int2(-1, 0);
+        a[r] = x.x;
+        b[r] = x.y;
     }
     unsigned partial = 0u, head = 0u;
     int ends_before[kPlanItems], rows_before[kPlanItems];
@@ -711,7 +727,7 @@ __global__ __launch_bounds__(kPlanBlock) void plan_partials_kernel(
 
 // The number of every partial sum into erow (a piece's end) and wtail (a chunk's tail); the header is completed.
 __global__ __launch_bounds__(256) void plan_targets_kernel(StreamView sv, const int* __restrict__ event_of,
-                                                          const int* __restrict__ first, const int* __restrict__ last,
+                                                          const int2* __restrict__ extent,
                                                           const int* __restrict__ fix_of, const int* __restrict__ ends_at,
                                                           const int* __restrict__ tails_at, const int* __restrict__ ends0,
                                                           const int* __restrict__ tails0, const int* __restrict__ ends_total,
@@ -730,7 +746,8 @@ __global__ __launch_bounds__(256) void plan_targets_kernel(StreamView sv, const 
     if (j < 0) return;
     const int e = event_of[p];
     sv.erow[e] = static_cast<int>(kStreamFlag) | (ends_at[p] + tails0[j]);
-    const int w0 = (first[e] & kStreamIdMask) / kStreamWave, tails = last[e] / kStreamWave - w0;
+    const int2 x = extent[e];
+    const int w0 = (x.x & kStreamIdMask) / kStreamWave, tails = x.y / kStreamWave - w0;
     if (tails > 0) {
         const int at = (j + 1 < sv.header->num_fix ? ends0[j + 1] : *ends_total) + tails_at[p];
         for (int k = 0; k < tails && w0 + k < num_waves; ++k) sv.wtail[w0 + k] = at + k;
@@ -749,8 +766,9 @@ static long long tiles_of(long long n, int tile) { return (n + tile - 1) / tile;
 // Workspace of a build: ten arrays of num_parts + 1 ints (some used twice, the later use in brackets), the sorted records, the
 // adjacency bytes, the fill tiles' first entries, the radix histogram and its offsets, the scan states.
 struct PlanTemp {
-    int *keys_a, *keys_b, *order_a, *order_b, *rowp, *src, *ends_before, *first, *last, *event_at;
-    int4 *rec_in, *rec_out;         // rec_in = src, ends_before, first, last (written after the sort)
+    int *keys_a, *keys_b, *order_a, *order_b, *rowp, *src, *ends_before, *event_at;
+    int2* extent;                   // two slabs
+    int4 *rec_in, *rec_out;         // rec_in = src, ends_before, extent (written after the sort)
     int *fix_of, *ends_at, *tails_at, *ends0, *tails0;      // = keys_a, keys_b, the spare order array, src, ends_before
     uint8_t* info;
     int *tile_q, *hist, *offsets, *ends_total;
@@ -763,8 +781,10 @@ static PlanTemp plan_temp(char* base, long long num_parts, long long num_slots)
     size_t at = 0;
     auto take = [&](size_t bytes) { char* p = base + at; at += align256(bytes); return p; };
     const size_t slab = sizeof(int) * (static_cast<size_t>(num_parts) + 1);
-    int** arrays[] = {&t.keys_a, &t.keys_b, &t.order_a, &t.order_b, &t.rowp, &t.src, &t.ends_before, &t.first, &t.last, &t.event_at};
+    int** arrays[] = {&t.keys_a, &t.keys_b, &t.order_a, &t.order_b, &t.rowp, &t.src, &t.ends_before};
     for (int** a : arrays) *a = reinterpret_cast<int*>(take(slab));
+    t.extent = reinterpret_cast<int2*>(take(2 * slab));
+    t.event_at = reinterpret_cast<int*>(take(slab));
     t.info = reinterpret_cast<uint8_t*>(take(static_cast<size_t>(num_parts)));
     t.tile_q = reinterpret_cast<int*>(take(sizeof(int) * static_cast<size_t>(tiles_of(stream_padded_slots(num_slots), kFillTile) + 1)));
     const long long entries = tiles_of(num_parts, kSortTile) * kDigits;
@@ -911,7 +931,7 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
     EPPGCN_HIP(hipGetLastError());
     unsigned* keys_in = reinterpret_cast<unsigned*>(t.keys_a);
     unsigned* keys_out = reinterpret_cast<unsigned*>(t.keys_b);
-    hipLaunchKernelGGL(plan_keys_kernel, dim3(sort_tiles), dim3(kSortBlock), 0, stream, part_ptr, col, part2node, ids,
+    hipLaunchKernelGGL(plan_keys_kernel, dim3(sort_tiles), dim3(kKeysBlock), 0, stream, part_ptr, col, part2node, ids,
                        num_parts, num_nodes, shift > 31 ? 31 : shift, keep_rows * 32, length_classes,
                        passes ? 1 << pass_bits(0) : 1, sort_tiles, passes ? keys_in : nullptr, t.hist,
                        part2node == t.rowp ? nullptr : t.rowp, t.info, passes ? t.rec_in : nullptr, v.single, sv.touched, sv.header, t.scans.sort);
@@ -944,7 +964,7 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
     t.tails_at = spare;
     hipLaunchKernelGGL(plan_order_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, part_ptr,
                        passes ? t.rec_out : nullptr, t.rowp, t.info, num_parts, slots, t.scans.order_tiles, v, sv, t.src,
-                       t.ends_before, t.first, t.last, t.event_at, t.tile_q, t.scans.order, t.scans.order_desc, scan_mode(),
+                       t.ends_before, t.extent, t.event_at, t.tile_q, t.scans.order, t.scans.order_desc, scan_mode(),
                        t.scans.sort);
     EPPGCN_HIP(hipGetLastError());
     int* event_of = passes ? reinterpret_cast<int*>(t.rec_out) : t.event_at;       // the records have been read
@@ -955,10 +975,10 @@ int launch_build_plan(const int* part_ptr, const int* col, const int* part2node,
         EPPGCN_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(plan_partials_kernel, dim3(t.scans.order_tiles), dim3(kPlanBlock), 0, stream, t.rowp, t.info, order, t.event_at,
-                       event_of, t.first, t.last, num_parts, num_nodes, t.scans.order_tiles, sv, t.fix_of, t.ends_at, t.tails_at,
+                       event_of, t.extent, num_parts, num_nodes, t.scans.order_tiles, sv, t.fix_of, t.ends_at, t.tails_at,
                        t.ends0, t.tails0, t.ends_total, t.scans, scan_mode());
     EPPGCN_HIP(hipGetLastError());
-    hipLaunchKernelGGL(plan_targets_kernel, dim3((num_parts + 255) / 256), dim3(256), 0, stream, sv, event_of, t.first, t.last,
+    hipLaunchKernelGGL(plan_targets_kernel, dim3((num_parts + 255) / 256), dim3(256), 0, stream, sv, event_of, t.extent,
                        t.fix_of, t.ends_at, t.tails_at, t.ends0, t.tails0, t.ends_total, num_parts, padded / kStreamWave, t.scans);
     EPPGCN_HIP(hipGetLastError());
     return kOk;

@@ -231,3 +231,29 @@ def test_rows_in_any_order(api, order, ps):
             assert api.last_call_used_stream() == stream and np.array_equal(out.cpu().numpy(), sums)
     finally:
         api.set_stream_mode(True)
+
+
+@pytest.mark.parametrize("ps", [1, 3, 32])
+@pytest.mark.parametrize("shift", [3, 6])
+def test_sort_keys_of_rows_that_cross_a_tile(api, ps, shift):
+    """Rows of up to 64 slots share a key.  Rows of 60 to 68 slots in groups of one slot reach 64 groups into the next tile of
+    2048 groups, at many places relative to it; from the rows of the groups and from the ids of the slots."""
+    from tests.test_gpu_parity import _check_plan_order_with
+    rng = np.random.default_rng(7)
+    n = 700
+    deg = np.tile([64, 65, 1, 63, 68, 2, 60], n // 7)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, d, replace=False)) for d in deg]).astype(np.int32)
+    for keep, classes in ((2, False), (8, True)):
+        api.set_plan_keep_rows(keep)
+        api.set_plan_length_classes(classes)
+        try:
+            _check_plan_order_with(api, indptr, col, ps, ((16, shift),), 32 * keep, classes)
+            pp, p2n = co.build_part(ps, indptr)
+            args = (dev(pp), dev(col), p2n.size, col.size, n, 16)
+            a = api.build_plan(*args, part2node=dev(p2n), block_shift=shift)
+            b = api.build_plan(*args, ids=dev(np.repeat(np.arange(n, dtype=np.int32), deg)), block_shift=shift)
+            assert all(torch.equal(x, y) for x, y in zip(a.view(raw_col=True), b.view(raw_col=True)))
+        finally:
+            api.set_plan_keep_rows(None)
+            api.set_plan_length_classes(None)
