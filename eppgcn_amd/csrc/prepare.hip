@@ -241,55 +241,54 @@ __global__ __launch_bounds__(kCompactBlock) void compact_mask_kernel(
 
 // ================================================================ marking + compaction in one pass
 // What mask_forward_kernel followed by compact_mask_kernel do, without the E-entry edge mask between them, in two kernels
-// over tiles of kMarkBlock * kItems consecutive slots.  Slot k * kMarkBlock + t of a tile belongs to thread t, so word
-// k * kMarkWaves + wave of every 64-slot bit map is one ballot and words are in slot order.
+// over tiles of kMarkTile consecutive slots.
 //   keep_slots_kernel    keep = the slot's column is in the source mask: one bit per slot and a count per tile.  Nothing but
-//                        column ids and mask entries is read, with kItems of each under way per thread.
-//   scan_counts_kernel   (large tiles only) the kept slots before every tile, by one workgroup: 2^31 slots have 131 thousand
-//                        tiles, and a workgroup per tile that adds up the counts before its own reads 34 GB of them (the
-//                        whole pass 20.1 ms, with the scan 17.8; 2^30 slots 9.48 and 8.96; 2^27 1.23 either way).  The at most
-//                        8192 small tiles do add them up (0.13 GB, from L2): a launch costs more there.
+//                        column ids and mask entries is read.  The lookups are what it takes (64 lines an instruction), and
+//                        they run best with few of them under way per thread: 16, 8, 4 of each 312, 265, 254 us for 132 M slots.
+//   scan_counts_kernel   (kMarkScannedTiles tiles and more) the kept slots before every tile, by one workgroup: 5.7 us for 32
+//                        thousand tiles.  A workgroup per tile that adds up the counts before its own reads 2 tiles^2 bytes:
+//                        0.13 GB, from L2, at the line, where either way takes the same time (7 thousand tiles 142 / 139 us
+//                        with and without the scan, 16 thousand 374 / 353; 4 thousand 112 / 113, 900 36 / 39).
 //   place_slots_kernel   rows and places of the kept slots; the row of a slot comes from a bit map of the group starts inside
 //                        the tile (prefix population count; the tile's first group was found beforehand) and the rows of
 //                        the tile's groups, staged in LDS; kept slots per row are differences of the prefix counts, one
-//                        atomic per (wave, row): a hub of 600 thousand slots costs 40 tiles a few atomics each, where one
+//                        atomic per (wave, row): a hub of 600 thousand slots costs 150 tiles a few atomics each, where one
 //                        per 64 slots queued ten thousand on one address.
-// Inputs of a few million slots take tiles of 4096 so that every CU has work.
-constexpr int kMarkBlock = 1024;
-constexpr int kMarkWaves = kMarkBlock / kWave;
-constexpr int kMarkItemsLarge = 16, kMarkItemsSmall = 4;
-constexpr int kMarkBatch = 4;             // groups a thread looks at together
-constexpr int kMarkStagedRows = 4096;     // groups of a tile whose rows are staged (more: read where they are needed)
-constexpr long long kMarkLargeLength = 32ll << 20;
-__host__ __device__ constexpr int mark_tile_slots(long long length)
+constexpr int kMarkTile = 4096;           // slots of a tile
+constexpr int kKeepBlock = 1024;
+constexpr int kMarkStagedRows = kMarkTile;     // groups of a tile whose rows are staged (more: read where they are needed)
+constexpr int kMarkScannedTiles = 8192;   // tiles from which on their counts are scanned by a launch of its own
+
+// first[t] = last group starting at or before slot t * kMarkTile (group 0 for slots before all groups); first[num_tiles] = last
+// group.  Every group says so for the tiles whose first slot it holds: the pointers are read once, in order (a search per tile is
+// a chain of 20 loads).  A thread takes four groups at a time.
+__device__ __forceinline__ void mark_tile_groups(const int* __restrict__ part_ptr, int num_parts, int num_tiles,
+                                                 int* __restrict__ first, int thread, int threads)
 {
-    return kMarkBlock * (length >= kMarkLargeLength ? kMarkItemsLarge : kMarkItemsSmall);
+    constexpr int kGroups = 4;
+    for (long long g0 = static_cast<long long>(thread) * kGroups; g0 < num_parts; g0 += static_cast<long long>(threads) * kGroups) {
+        int start[kGroups + 1];
+#pragma unroll
+        for (int j = 0; j <= kGroups; ++j) start[j] = part_ptr[min(g0 + j, static_cast<long long>(num_parts))];
+#pragma unroll
+        for (int j = 0; j < kGroups; ++j) {
+            const long long g = g0 + j;
+            if (g >= num_parts) break;
+            const bool last = g == num_parts - 1;
+            const int t0 = g == 0 ? 0 : static_cast<int>((static_cast<unsigned>(max(start[j], 0)) + (kMarkTile - 1u)) / kMarkTile);
+            const int t1 = last ? num_tiles : min(num_tiles, static_cast<int>((static_cast<unsigned>(max(start[j + 1], 0)) + (kMarkTile - 1u)) / kMarkTile));
+            for (int t = t0; t < t1; ++t) first[t] = static_cast<int>(g);
+            if (last) first[num_tiles] = static_cast<int>(g);
+        }
+    }
 }
 
-// first[t] = last group starting at or before slot t * tile_slots; first[num_tiles] = last group
-__device__ __forceinline__ void find_tile_groups(const int* __restrict__ part_ptr, int num_parts, int num_tiles,
-                                                 int tile_slots, int* __restrict__ first, int t)
+__global__ __launch_bounds__(256) void tile_groups_kernel(const int* __restrict__ part_ptr, int num_parts, int num_tiles,
+                                                          int* __restrict__ first, ScanState* st)
 {
-    if (t > num_tiles) return;
-    if (t == num_tiles) {
-        first[t] = num_parts - 1;
-        return;
-    }
-    const long long slot = static_cast<long long>(t) * tile_slots;
-    int a = 0, b = num_parts;                 // part_ptr[a] <= slot is assumed for a = 0
-    while (b - a > 1) {
-        const int mid = a + (b - a) / 2;
-        if (part_ptr[mid] <= slot) a = mid; else b = mid;
-    }
-    first[t] = a;
-}
-
-__global__ void tile_groups_kernel(const int* __restrict__ part_ptr, int num_parts, int num_tiles, int tile_slots,
-                                   int* __restrict__ first, ScanState* st)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) *st = ScanState{};
-    find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
+    const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
+    if (i0 == 0) *st = ScanState{};
+    mark_tile_groups(part_ptr, num_parts, num_tiles, first, i0, stride);
 }
 
 // kBits: the source mask is read as bits (packed once per call): eight times as many vertices share a cache line
@@ -300,26 +299,25 @@ __device__ __forceinline__ bool in_mask(const void* __restrict__ mask, int v)
     else return static_cast<const uint8_t*>(mask)[v] != 0;
 }
 
-template <int kItems, bool kBits>
-__global__ __launch_bounds__(kMarkBlock) void keep_slots_kernel(const int* __restrict__ part_ptr, const int* __restrict__ col,
+template <bool kBits>
+__global__ __launch_bounds__(kKeepBlock) void keep_slots_kernel(const int* __restrict__ part_ptr, const int* __restrict__ col,
                                                                 const void* __restrict__ src, int num_parts, int length,
                                                                 unsigned long long* __restrict__ kept, int* __restrict__ counts)
 {
-    constexpr int kTile = kMarkBlock * kItems;
-    constexpr int kWords = kTile / 64;
+    constexpr int kItems = kMarkTile / kKeepBlock;
+    constexpr int kWaves = kKeepBlock / kWave;
+    constexpr int kWords = kMarkTile / 64;
     __shared__ unsigned long long s_kept[kWords];
-    __shared__ int s_total;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
-    const long long base = static_cast<long long>(blockIdx.x) * kTile;
+    const long long base = static_cast<long long>(blockIdx.x) * kMarkTile;
     // slots outside [part_ptr[0], part_ptr[num_parts]) belong to no group and are never kept
     const int owned_lo = part_ptr[0];
     const int owned_hi = min(part_ptr[num_parts], length);
-    if (threadIdx.x == 0) s_total = 0;
     int c[kItems];
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
-        const long long idx = base + k * kMarkBlock + threadIdx.x;
+        const long long idx = base + k * kKeepBlock + threadIdx.x;
         c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
     }
     bool keep[kItems];
@@ -331,69 +329,88 @@ __global__ __launch_bounds__(kMarkBlock) void keep_slots_kernel(const int* __res
         const uint64_t ballot = __ballot(keep[k] && c[k] >= 0);
         if (lane == k) mine = ballot;
     }
-    if (lane < kItems) s_kept[lane * kMarkWaves + wave] = mine;
+    if (lane < kItems) s_kept[lane * kWaves + wave] = mine;
     __syncthreads();
-    if (threadIdx.x < kWords) {
-        const unsigned long long word = s_kept[threadIdx.x];
-        kept[static_cast<long long>(blockIdx.x) * kWords + threadIdx.x] = word;
-        int n = __popcll(word);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
-        if (lane == 0) atomicAdd(&s_total, n);
+    static_assert(kWords == kWave, "one wave takes the words of a tile");
+    if (wave == 0) {
+        const unsigned long long word = s_kept[lane];
+        kept[static_cast<long long>(blockIdx.x) * kWords + lane] = word;
+        const int n = wave_inclusive_scan(__popcll(word));
+        if (lane == kWave - 1) counts[blockIdx.x] = n;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) counts[blockIdx.x] = s_total;
 }
 
 // counts[0 .. n) become their exclusive prefix sums
 __global__ __launch_bounds__(1024) void scan_counts_kernel(int* __restrict__ counts, int n)
 {
-    constexpr int kItems = 4, kWaves = 1024 / kWave;
-    __shared__ int s_wave[kWaves];
+    typedef int int4u __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int kVecs = 4, kWaves = 1024 / kWave;          // vector (v, thread) of a step: 4 counts at (v * 1024 + thread) * 4
+    __shared__ int s_wave[kVecs * kWaves];
+    static_assert(kVecs * kWaves == kWave, "one wave scans the (vector, wave) sums");
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
     int carry = 0;
-    for (int t0 = 0; t0 < n; t0 += 1024 * kItems) {
-        const int t = t0 + static_cast<int>(threadIdx.x) * kItems;
-        int c[kItems], sum = 0;
+    for (int t0 = 0; t0 < n; t0 += 4096 * kVecs) {
+        int4u c[kVecs];
+        int before[kVecs];
 #pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            c[j] = t + j < n ? counts[t + j] : 0;
-            sum += c[j];
+        for (int v = 0; v < kVecs; ++v) {
+            const int t = t0 + (v * 1024 + static_cast<int>(threadIdx.x)) * 4;
+            c[v] = int4u{0, 0, 0, 0};
+            if (t + 4 <= n) c[v] = *reinterpret_cast<const int4u*>(counts + t);
+            else
+                for (int j = 0; j < 4; ++j) c[v][j] = t + j < n ? counts[t + j] : 0;
         }
-        const int incl = wave_inclusive_scan(sum);
-        if (lane == kWave - 1) s_wave[wave] = incl;
+#pragma unroll
+        for (int v = 0; v < kVecs; ++v) {
+            const int sum = c[v][0] + c[v][1] + c[v][2] + c[v][3];
+            const int incl = wave_inclusive_scan(sum);
+            before[v] = incl - sum;
+            if (lane == kWave - 1) s_wave[v * kWaves + wave] = incl;
+        }
         __syncthreads();
-        int run = carry + incl - sum;
+        const int mine = s_wave[lane], incl = wave_inclusive_scan(mine);
+        const int excl = carry + incl - mine;                // lane v * kWaves + w: before wave w's vector v
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-            if (w < wave) run += s_wave[w];
-            carry += s_wave[w];
+        for (int v = 0; v < kVecs; ++v) {
+            const int t = t0 + (v * 1024 + static_cast<int>(threadIdx.x)) * 4;
+            int4u out;
+            out[0] = __shfl(excl, v * kWaves + wave, kWave) + before[v];
+            out[1] = out[0] + c[v][0];
+            out[2] = out[1] + c[v][1];
+            out[3] = out[2] + c[v][2];
+            if (t + 4 <= n) *reinterpret_cast<int4u*>(counts + t) = out;
+            else
+                for (int j = 0; j < 4; ++j)
+                    if (t + j < n) counts[t + j] = out[j];
         }
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            if (t + j < n) counts[t + j] = run;
-            run += c[j];
-        }
+        carry += __builtin_amdgcn_readlane(incl, kWave - 1);
         __syncthreads();
     }
 }
 
-template <int kBlock, int kItems, bool kScanned, bool kBits>
+// Vector loads and stores of a wave are counted together and in order: a wait for a load waits for every store before it.  So a
+// workgroup loads first - the columns of all its slots, then the groups - and stores last: neighbour marks, kept slots, counts
+// per row, zeros.  A wave has consecutive slots, so that its stores share lines with its own next ones.  Slot by slot, each
+// waiting for the stores of the one before it (and all of them for the zeros), in tiles of 16 384 slots, a layer of R-MAT scale
+// 22 took 519 / 372 us (a tenth / 95 % of 132 M slots kept); now 454 / 331.  2253 tiles 52 / 44 -> 43 / 38, 27 tiles
+// 13.5 -> 12.
+template <int kBlock, bool kScanned, bool kBits>
 __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     const int* __restrict__ part2node, const int* __restrict__ part_ptr, const int* __restrict__ col,
     const void* __restrict__ src, uint8_t* __restrict__ ngh_mask, int* __restrict__ node_degs, int* __restrict__ out_id,
-    int* __restrict__ out_edge, uint8_t* __restrict__ self_kept, int length, int num_tiles, int is_last,
+    int* __restrict__ out_edge, uint8_t* __restrict__ self_kept, int num_parts, int length, int num_tiles, int is_last,
     const int* __restrict__ tile_first, const unsigned long long* __restrict__ kept, const int* __restrict__ counts,
     ScanState* st)
 {
-    constexpr int kTile = kBlock * kItems;
+    constexpr int kTile = kMarkTile, kItems = kTile / kBlock;
     constexpr int kWords = kTile / 64;
     constexpr int kPerLane = kWords / kWave;
+    constexpr int kBatch = kItems > 8 ? 1 : 2;           // groups a thread looks at together
     static_assert(kWords % kWave == 0 && kItems <= kWave, "one wave scans the words; a wave's words fit its lanes");
     static_assert(kWords <= kBlock && kBlock >= 2 * kWave, "a thread per word, a wave for each of the two maps");
     __shared__ int s_prefix;
-    __shared__ int s_starts_in_tile, s_kept_in_tile;
+    __shared__ int s_starts_in_tile;
     __shared__ unsigned long long s_starts[kWords];    // bit p: a group starts at slot base + p
     __shared__ unsigned long long s_kept[kWords];      // bit p: slot base + p is kept
     __shared__ int s_starts_before[kWords];            // group starts before each word
@@ -402,11 +419,23 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     const int tile = blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x >> 6;
-    const long long base = static_cast<long long>(tile) * kTile;
-    const int g_lo = tile_first[tile];
-    const int g_cnt = tile_first[tile + 1] - g_lo + 1;
+    const long long base = static_cast<long long>(tile) * kTile;       // < length
+    const int inside = static_cast<int>(min(static_cast<long long>(kTile), length - base));
+    const int mine = wave * (kItems * kWave) + lane;      // this thread's first slot of the tile; the others are 64 apart
+    int c[kItems];
+    {
+        const int* __restrict__ tile_col = col + base;
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) c[k] = tile_col[min(mine + k * kWave, inside - 1)];
+    }
+    // in range for any pointers: a table of tiles whose groups do not ascend is left incomplete
+    const int g_lo = min(max(tile_first[tile], 0), num_parts - 1);
+    const int g_cnt = min(max(tile_first[tile + 1], g_lo), num_parts - 1) - g_lo + 1;
     const bool staged = g_cnt <= kMarkStagedRows;
     const int before = part_ptr[g_lo] < base ? 1 : 0;    // g_lo itself starts before the tile
+    // slots of the tile that belong to groups: [owned_first, owned_first + owned_slots)
+    const int owned_first = static_cast<int>(min(max(part_ptr[0] - base, 0ll), static_cast<long long>(kTile)));
+    const unsigned owned_slots = static_cast<unsigned>(max(min(static_cast<int>(part_ptr[g_lo + g_cnt] - base), inside) - owned_first, 0));
     if (threadIdx.x < kWords) {
         s_starts[threadIdx.x] = 0ull;
         s_kept[threadIdx.x] = kept[static_cast<long long>(tile) * kWords + threadIdx.x];
@@ -416,66 +445,66 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
         s_prefix = kScanned ? counts[tile] : 0;
     }
     __syncthreads();
-    {
-        if constexpr (!kScanned) {
-            int sum = 0;
-            for (int t0 = threadIdx.x; t0 < tile; t0 += 4 * kBlock) {
-                int c[4];
+    if constexpr (!kScanned) {
+        int sum = 0;
+        for (int t0 = threadIdx.x; t0 < tile; t0 += 4 * kBlock) {
+            int n[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) c[j] = t0 + j * kBlock < tile ? counts[t0 + j * kBlock] : 0;
-                sum += c[0] + c[1] + c[2] + c[3];
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
-            if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
+            for (int j = 0; j < 4; ++j) n[j] = t0 + j * kBlock < tile ? counts[t0 + j * kBlock] : 0;
+            sum += n[0] + n[1] + n[2] + n[3];
         }
-        int mine = 0;
-        for (int i0 = threadIdx.x; i0 < g_cnt; i0 += kBlock * kMarkBatch) {
-            int start[kMarkBatch], row[kMarkBatch];
-            bool some[kMarkBatch], marked[kMarkBatch];
 #pragma unroll
-            for (int j = 0; j < kMarkBatch; ++j) {
-                const int g = g_lo + min(i0 + j * kBlock, g_cnt - 1);
-                start[j] = part_ptr[g];
-                some[j] = part_ptr[g + 1] > start[j];
-                row[j] = part2node[g];
-            }
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+        if (lane == 0 && sum) atomicAdd(&s_prefix, sum);
+    }
+    // the tile's groups, kBatch of them per thread at a time; the first of them (usually all) stay in registers
+    struct Groups { int from[kBatch], to[kBatch]; };
+    auto load_groups = [&](Groups& g, int i0) {
 #pragma unroll
-            for (int j = 0; j < kMarkBatch; ++j) marked[j] = !is_last && in_mask<kBits>(src, row[j]);
+        for (int j = 0; j < kBatch; ++j) {
+            const int at = g_lo + min(i0 + j * kBlock + static_cast<int>(threadIdx.x), g_cnt - 1);
+            g.from[j] = part_ptr[at];
+            g.to[j] = part_ptr[at + 1];
+        }
+    };
+    auto load_rows = [&](unsigned (&row)[kBatch], int i0) {        // bit 31: the row is in the source mask (never on the last layer)
 #pragma unroll
-            for (int j = 0; j < kMarkBatch; ++j) {
-                const int i = i0 + j * kBlock;
+        for (int j = 0; j < kBatch; ++j)
+            row[j] = static_cast<unsigned>(part2node[g_lo + min(i0 + j * kBlock + static_cast<int>(threadIdx.x), g_cnt - 1)]);
+        if (is_last) return;
+        bool marked[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) marked[j] = in_mask<kBits>(src, static_cast<int>(row[j]));
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) row[j] |= marked[j] ? 0x80000000u : 0u;
+    };
+    Groups first;
+    {
+        int starts = 0;
+        auto stage = [&](Groups& g, int i0) {
+            unsigned row[kBatch];
+            load_groups(g, i0);
+            if (staged) load_rows(row, i0);
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int i = i0 + j * kBlock + static_cast<int>(threadIdx.x);
                 if (i >= g_cnt) continue;
-                const long long p = start[j] - base;
+                const long long p = g.from[j] - base;
                 if (p >= 0 && p < kTile) {
                     atomicOr(&s_starts[p >> 6], 1ull << (p & 63));
-                    ++mine;
+                    ++starts;
                 }
-                if (staged) s_row[i] = static_cast<unsigned>(row[j]) | (marked[j] ? 0x80000000u : 0u);
-                if (marked[j] && some[j]) ngh_mask[row[j]] = 1;
+                if (staged) s_row[i] = row[j];
             }
+        };
+        stage(first, 0);
+        for (int i0 = kBlock * kBatch; i0 < g_cnt; i0 += kBlock * kBatch) {
+            Groups g;
+            stage(g, i0);
         }
-        if (mine) atomicAdd(&s_starts_in_tile, mine);
+        if (starts) atomicAdd(&s_starts_in_tile, starts);
     }
     __syncthreads();
-    // Zeros behind the kept slots of the whole input, written here and not by a pass of their own because they cost what their
-    // bytes cost: 13 of 132 M slots kept, this kernel 384 -> 513 us and the pass behind it 195 -> 15.  As many words as this
-    // tile drops slots, counted from the end, behind those of the tiles before it (which dropped base - s_prefix slots).
-    if (wave == 0) {
-        int n = 0;
-#pragma unroll
-        for (int j = 0; j < kPerLane; ++j) n += __popcll(s_kept[lane * kPerLane + j]);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, kWave);
-        if (lane == 0) s_kept_in_tile = n;
-    }
-    __syncthreads();
-    {
-        const long long end = length - (base - s_prefix);
-        const long long from = end - (min(static_cast<long long>(kTile), length - base) - s_kept_in_tile);
-        zero_from(out_id, from, end, threadIdx.x, kBlock);
-        zero_from(out_edge, from, end, threadIdx.x, kBlock);
-    }
     // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
     // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
     // population count over the map of group starts; otherwise every slot does a binary search over the group starts.
@@ -505,83 +534,109 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
         }
     }
     __syncthreads();
-    // kept slots per row
+    // ---- the row of every slot
+    const bool by_bits = s_starts_in_tile >= 0;
+    // lane k: word k of this wave
+    const int my_word = wave * kItems + (lane < kItems ? lane : 0);
+    const uint64_t start_word = s_starts[my_word], kept_word = s_kept[my_word];
+    const int start_before = s_starts_before[my_word] + before - 1;
+    const int place = s_kept_before[my_word] + s_prefix;
+    unsigned row[kItems];                                    // bit 31 as in s_row
+    if (by_bits && staged) {
+#pragma unroll
+        for (int k = 0; k < kItems; ++k) {
+            // starts at or before the lane: those below it in the word without its first bit, and the first bit
+            const uint64_t word = lane_value(start_word, k);
+            const int head = __builtin_amdgcn_readlane(start_before, k) + static_cast<int>(word & 1ull);
+            const int a = head + ballot_rank(word >> 1);
+            row[k] = s_row[max(a, 0)];                       // a slot before the first group is never used
+        }
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < kItems; ++k) {
+            const int e = static_cast<int>(base + mine + k * kWave);
+            int a = 0, b = g_cnt;
+            while (b - a > 1) {
+                const int mid = (a + b) >> 1;
+                if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
+            }
+            const int r = part2node[g_lo + a];
+            const unsigned found = static_cast<unsigned>(r) | (!is_last && in_mask<kBits>(src, r) ? 0x80000000u : 0u);
+#pragma unroll
+            for (int j = 0; j < kItems; ++j) row[j] = j == k ? found : row[j];
+        }
+    }
+    // ---- neighbours of marked rows
+    if (!is_last) {
+        // a vertex that already reads as marked is not stored again: hubs are neighbours of most rows
+        constexpr int kMarks = kItems < 8 ? kItems : 8;
+#pragma unroll
+        for (int k0 = 0; k0 < kItems; k0 += kMarks) {
+            bool want[kMarks];
+            uint8_t seen[kMarks];
+#pragma unroll
+            for (int k = 0; k < kMarks; ++k) {
+                const unsigned pos = static_cast<unsigned>(mine + (k0 + k) * kWave - owned_first);
+                want[k] = row[k0 + k] >> 31 && pos < owned_slots && c[k0 + k] >= 0;
+                seen[k] = ngh_mask[want[k] ? static_cast<unsigned>(c[k0 + k]) : 0u];      // no branch: all loads under way together
+            }
+#pragma unroll
+            for (int k = 0; k < kMarks; ++k)
+                if (want[k] && seen[k] == 0) ngh_mask[static_cast<unsigned>(c[k0 + k])] = 1;
+        }
+    }
+    // ---- kept slots
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const uint64_t ballot = lane_value(kept_word, k);
+        const unsigned to = __builtin_amdgcn_readlane(place, k), rank = static_cast<unsigned>(ballot_rank(ballot));
+        if (__builtin_amdgcn_inverse_ballot_w64(ballot)) {
+            const unsigned r = row[k] & 0x7fffffffu;
+            (out_id + to)[rank] = static_cast<int>(r);
+            (out_edge + to)[rank] = c[k];
+            if (self_kept && static_cast<int>(r) == c[k]) self_kept[r] = 1;
+        }
+    }
+    // ---- kept slots per row, and the marked rows themselves
     auto kept_before = [&](long long p) {                    // kept slots of the tile before slot base + p
         const int q = static_cast<int>(p < 0 ? 0 : p > kTile ? kTile : p);
         const int word = q >> 6;
         const int whole = s_kept_before[word];
         return (q & 63) ? whole + __popcll(s_kept[word] & ((1ull << (q & 63)) - 1ull)) : whole;
     };
-    for (int i0 = 0; i0 < g_cnt; i0 += kBlock * kMarkBatch) {
-        int from[kMarkBatch], to[kMarkBatch], row[kMarkBatch];
+    auto count_rows = [&](const Groups& g, int i0) {
+        unsigned row[kBatch];
+        if (staged) {
 #pragma unroll
-        for (int j = 0; j < kMarkBatch; ++j) {
-            const int i = i0 + j * kBlock + static_cast<int>(threadIdx.x);
-            const int g = g_lo + min(i, g_cnt - 1);
-            from[j] = part_ptr[g];
-            to[j] = part_ptr[g + 1];
-            row[j] = i >= g_cnt ? -1 : staged ? static_cast<int>(s_row[i] & 0x7fffffffu) : part2node[g];
-        }
-#pragma unroll
-        for (int j = 0; j < kMarkBatch; ++j) {
-            if (i0 + j * kBlock >= g_cnt) break;         // the same for the whole workgroup
-            int n = row[j] < 0 ? 0 : kept_before(to[j] - base) - kept_before(from[j] - base);
-            const int prev_row = __shfl_up(row[j], 1, kWave);
-            const uint64_t heads = __ballot(lane == 0 || prev_row != row[j]);
-            n = wave_run_sum(n, heads);
-            if (((heads >> lane) & 1ull) && n > 0) atomicAdd(node_degs + row[j], n);
-        }
-    }
-    const bool by_bits = s_starts_in_tile >= 0;
-    // lane k: word k of this wave
-    const int my_word = (lane < kItems ? lane : 0) * (kBlock / kWave) + wave;
-    const uint64_t start_word = s_starts[my_word], kept_word = s_kept[my_word];
-    const int start_before = s_starts_before[my_word] + before - 1;
-    const int place = s_kept_before[my_word] + s_prefix;
-    auto row_of = [&](int k) {                               // row of this thread's slot k; bit 31 as in s_row
-        int a = 0;
-        if (by_bits) {
-            const uint64_t word = lane_value(start_word, k);
-            a = __builtin_amdgcn_readlane(start_before, k) + ballot_rank(word) + static_cast<int>((word >> lane) & 1ull);
+            for (int j = 0; j < kBatch; ++j) row[j] = s_row[min(i0 + j * kBlock + static_cast<int>(threadIdx.x), g_cnt - 1)];
         } else {
-            const int e = static_cast<int>(base + k * kBlock + threadIdx.x);
-            int b = g_cnt;
-            while (b - a > 1) {
-                const int mid = (a + b) >> 1;
-                if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
-            }
+            load_rows(row, i0);
         }
-        a = max(a, 0);                                       // a slot before the first group (it is never used)
-        if (staged) return s_row[a];
-        const int row = part2node[g_lo + a];
-        return static_cast<unsigned>(row) | (!is_last && in_mask<kBits>(src, row) ? 0x80000000u : 0u);
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            if (i0 + j * kBlock >= g_cnt) break;             // the same for the whole workgroup
+            const bool some = i0 + j * kBlock + static_cast<int>(threadIdx.x) < g_cnt;
+            const int r = some ? static_cast<int>(row[j] & 0x7fffffffu) : -1;
+            int n = some ? kept_before(g.to[j] - base) - kept_before(g.from[j] - base) : 0;
+            const int left = __builtin_amdgcn_update_dpp(-2, r, kDppWaveShr1, 0xF, 0xF, false);
+            n = wave_run_sum(n, __ballot(left != r));        // lane 0 starts a run
+            if (left != r && n > 0) atomicAdd(node_degs + r, n);
+            if (some && row[j] >> 31 && g.to[j] > g.from[j]) ngh_mask[r] = 1;
+        }
     };
-    const int owned_lo = part_ptr[0], owned_hi = min(part_ptr[g_lo + g_cnt], length);
-    constexpr int kChunk = kItems < 8 ? kItems : 8;
-#pragma unroll(kItems <= 16 ? kItems / kChunk : 1)
-    for (int k0 = 0; k0 < kItems; k0 += kChunk) {
-        int c[kChunk];
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const long long idx = base + (k0 + k) * kBlock + threadIdx.x;
-            c[k] = idx >= owned_lo && idx < owned_hi ? col[idx] : -1;
-        }
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const uint64_t ballot = lane_value(kept_word, k0 + k);
-            if (is_last && ballot == 0ull) continue;         // the same for the whole wave
-            const unsigned row = row_of(k0 + k);
-            if ((ballot >> lane) & 1ull) {
-                const int dst = __builtin_amdgcn_readlane(place, k0 + k) + ballot_rank(ballot);
-                const int r = static_cast<int>(row & 0x7fffffffu);
-                out_id[dst] = r;
-                out_edge[dst] = c[k];
-                if (self_kept && r == c[k]) self_kept[r] = 1;
-            }
-            // a vertex that already reads as marked is not stored again: hubs are neighbours of most rows
-            if (!is_last && c[k] >= 0 && (row >> 31) != 0u && ngh_mask[c[k]] == 0) ngh_mask[c[k]] = 1;
-        }
+    count_rows(first, 0);
+    for (int i0 = kBlock * kBatch; i0 < g_cnt; i0 += kBlock * kBatch) {
+        Groups g;
+        load_groups(g, i0);
+        count_rows(g, i0);
     }
+    // ---- zeros behind the kept slots of the whole input, written here and not by a pass of their own because they cost what
+    // their bytes cost.  As many words as this tile drops slots, counted from the end, behind those of the tiles before it
+    // (which dropped base - s_prefix slots).
+    const long long end = length - (base - s_prefix);
+    const long long from = end - (inside - s_kept_before[kWords]);
+    zero_from(out_id, from, end, threadIdx.x, kBlock);
+    zero_from(out_edge, from, end, threadIdx.x, kBlock);
 }
 
 // ---------------------------------------------------------------- the pass with everything a path needs around it
@@ -589,11 +644,11 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
 __global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __restrict__ src_mask, int num_nodes, int words,
                                                              uint32_t* __restrict__ bits, uint32_t* __restrict__ self_kept,
                                                              const int* __restrict__ part_ptr, int num_parts, int num_tiles,
-                                                             int tile_slots, int* __restrict__ first, ScanState* st)
+                                                             int* __restrict__ first, ScanState* st)
 {
     const int i0 = blockIdx.x * 256 + threadIdx.x, stride = gridDim.x * 256;
     if (i0 == 0) *st = ScanState{};
-    for (int t = i0; t <= num_tiles; t += stride) find_tile_groups(part_ptr, num_parts, num_tiles, tile_slots, first, t);
+    mark_tile_groups(part_ptr, num_parts, num_tiles, first, i0, stride);
     // a thread packs 4 bytes into 4 bits of a word, 8 lanes a word (vertices past the end count as unmarked)
     const bool quads = reinterpret_cast<uintptr_t>(src_mask) % 4 == 0;
     for (int q0 = blockIdx.x * 256; q0 < words * 8; q0 += stride) {
@@ -623,21 +678,24 @@ __global__ __launch_bounds__(256) void mark_path_init_kernel(const uint8_t* __re
 // (0.58 ms for 126 M of them).  st->pad: [0] vertices of the mask, [1] not all of them kept their self-loop, [2] rows with
 // kept slots.
 // counts[1]: groups of at most group_size slots that the kept slots of the rows make (group_size 0: not counted).  Every
-// workgroup ends in three or four atomics on one line (12 ns each, serial).
-constexpr int kFinishCountBlocks = 256;
-__global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* __restrict__ bits, const uint4* __restrict__ self_kept,
-                                                               int words, uint32_t* __restrict__ gathered,
-                                                               const int* __restrict__ node_degs, int num_nodes,
-                                                               int group_size, ScanState* st)
+// workgroup ends in four atomics on one line (12 ns each, serial), so there are few of them and they are large.
+constexpr int kFinishBlock = 1024, kFinishBlocks = 128;
+__global__ __launch_bounds__(kFinishBlock) void mark_path_finish_kernel(const uint32_t* __restrict__ bits,
+                                                                        const uint4* __restrict__ self_kept, int words,
+                                                                        uint32_t* __restrict__ gathered,
+                                                                        const int* __restrict__ node_degs, int num_nodes,
+                                                                        int group_size, ScanState* st)
 {
-    const int i0 = blockIdx.x * 256 + threadIdx.x, count_stride = gridDim.x * 256;
+    constexpr int kWaves = kFinishBlock / kWave;
+    __shared__ int s_sum[4][kWaves];
+    const int i0 = blockIdx.x * kFinishBlock + threadIdx.x, stride = gridDim.x * kFinishBlock;
     int marked = 0, missing = 0, rows = 0, groups = 0;
     const unsigned gs = static_cast<unsigned>(max(group_size, 1));
     auto count_row = [&](int d) {
         rows += d != 0;
         groups += d > 0 ? static_cast<int>((static_cast<unsigned>(d) + gs - 1u) / gs) : 0;
     };
-    for (int w = i0; w < words; w += count_stride) {
+    for (int w = i0; w < words; w += stride) {
         const uint32_t b = bits[w];
         const uint4 lo = self_kept[2 * static_cast<size_t>(w)], hi = self_kept[2 * static_cast<size_t>(w) + 1];
         const uint32_t seen = nonzero_bytes(lo.x) | nonzero_bytes(lo.y) << 4 | nonzero_bytes(lo.z) << 8 |
@@ -649,22 +707,29 @@ __global__ __launch_bounds__(256) void mark_path_finish_kernel(const uint32_t* _
     }
     if (reinterpret_cast<uintptr_t>(node_degs) % 16 == 0) {
         const int4* quads = reinterpret_cast<const int4*>(node_degs);
-        for (int v = i0; v < num_nodes / 4; v += count_stride) {
+#pragma unroll 4
+        for (int v = i0; v < num_nodes / 4; v += stride) {
             const int4 d = quads[v];
             count_row(d.x); count_row(d.y); count_row(d.z); count_row(d.w);
         }
         if (i0 < num_nodes % 4) count_row(node_degs[num_nodes / 4 * 4 + i0]);
     } else {
-        for (int v = i0; v < num_nodes; v += count_stride) count_row(node_degs[v]);
+        for (int v = i0; v < num_nodes; v += stride) count_row(node_degs[v]);
     }
-    add_block_count(marked, &st->pad[0]);
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int sums[4] = {wave_inclusive_scan(marked), wave_inclusive_scan(missing), wave_inclusive_scan(rows), wave_inclusive_scan(groups)};
+    if (lane == kWave - 1) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s_sum[j][wave] = sums[j];
+    }
     __syncthreads();
-    add_block_count(missing, &st->pad[1]);
-    __syncthreads();
-    add_block_count(rows, &st->pad[2]);
-    if (group_size <= 0) return;
-    __syncthreads();
-    add_block_count(groups, &st->counts[1]);
+    if (threadIdx.x < 4) {
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) sum += s_sum[threadIdx.x][w];
+        int* const to[4] = {&st->pad[0], &st->pad[1], &st->pad[2], &st->counts[1]};
+        if (sum && (threadIdx.x < 3 || group_size > 0)) atomicAdd(to[threadIdx.x], sum);
+    }
 }
 
 
@@ -1126,16 +1191,15 @@ int launch_compact_mask_static(const int* in_id, int* out_id, const int* in_edge
 // for launch_mark_path the bit map of the source mask and one byte per vertex (its self-loop was kept), in whole words.
 struct MarkLayout {
     size_t kept, counts, first, bits, self_kept, total;
-    int tile_slots, num_tiles, words;
+    int num_tiles, words;
 };
 static MarkLayout mark_layout(long long length, long long num_nodes)
 {
     MarkLayout l;
-    l.tile_slots = mark_tile_slots(length);
-    l.num_tiles = static_cast<int>((length + l.tile_slots - 1) / l.tile_slots);
+    l.num_tiles = static_cast<int>((length + kMarkTile - 1) / kMarkTile);
     l.words = static_cast<int>((num_nodes + 31) / 32);
     l.kept = sizeof(ScanState);
-    l.counts = l.kept + static_cast<size_t>(l.num_tiles) * (l.tile_slots / 8);
+    l.counts = l.kept + static_cast<size_t>(l.num_tiles) * (kMarkTile / 8);
     l.first = l.counts + 4 * static_cast<size_t>(l.num_tiles);
     l.bits = (l.first + 4 * (static_cast<size_t>(l.num_tiles) + 1) + 15) / 16 * 16;
     l.self_kept = (l.bits + 4 * static_cast<size_t>(l.words) + 15) / 16 * 16;
@@ -1160,29 +1224,27 @@ static int launch_mark_pass(const int* part2node, const int* part_ptr, const int
     const int* first = reinterpret_cast<const int*>(workspace + l.first);
     const dim3 grid(l.num_tiles);
     const int len = static_cast<int>(length);
-#define EPPGCN_MARK(ITEMS_, PLACE_BLOCK_, SCANNED_)                                                                       \
-    do {                                                                                                                \
-        hipLaunchKernelGGL((keep_slots_kernel<ITEMS_, kBits>), grid, dim3(kMarkBlock), 0, stream, part_ptr, col, src,      \
-                           num_parts, len, kept, counts);                                                                 \
-        EPPGCN_HIP(hipGetLastError());                                                                                    \
-        if (SCANNED_)                                                                                                     \
-            hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, stream, counts, l.num_tiles);                  \
-        EPPGCN_HIP(hipGetLastError());                                                                                    \
-        hipLaunchKernelGGL((place_slots_kernel<PLACE_BLOCK_, kMarkBlock / PLACE_BLOCK_ * ITEMS_, SCANNED_, kBits>), grid, \
-                           dim3(PLACE_BLOCK_), 0, stream, part2node, part_ptr, col, src, ngh_mask, node_degs, out_id,     \
-                           out_edge, self_kept, len, l.num_tiles, is_last, first, kept, counts, st);                      \
-        EPPGCN_HIP(hipGetLastError());                                                                                    \
-    } while (0)
-    // place_slots walks a small tile from barrier to barrier.  1024 threads do that fastest as long as the chip holds all tiles
-    // at once (two workgroups on a CU: 512 tiles), beyond that four workgroups of 512 threads hide each other's waits better:
-    // 27 tiles 13.5 us with 1024 threads, 15.5 with 512, 21.5 with 256; 2250 tiles 63, 50, 54.  Tiles of 16 384 slots (scale
-    // 22, the mean of two layers): 450, 474, 522.  At the line, a whole marking with 1024 / 512 threads, us: 256 tiles 25.7 /
-    // 27.9, 500 tiles 32.8 / 33.5, 520 tiles 42.4 / 36.4, 1024 tiles 55.7 / 45.9 (a tenth kept: 24.0 / 24.8, 30.6 / 29.8,
-    // 36.4 / 32.1, 49.2 / 40.2).
-    if (l.tile_slots == kMarkBlock * kMarkItemsLarge) EPPGCN_MARK(kMarkItemsLarge, 1024, true);
-    else if (l.num_tiles > 512) EPPGCN_MARK(kMarkItemsSmall, 512, false);
-    else EPPGCN_MARK(kMarkItemsSmall, 1024, false);
-#undef EPPGCN_MARK
+    hipLaunchKernelGGL(keep_slots_kernel<kBits>, grid, dim3(kKeepBlock), 0, stream, part_ptr, col, src, num_parts, len, kept, counts);
+    EPPGCN_HIP(hipGetLastError());
+#define EPPGCN_PLACE(BLOCK_, SCANNED_)                                                                                    \
+    hipLaunchKernelGGL((place_slots_kernel<BLOCK_, SCANNED_, kBits>), grid, dim3(BLOCK_), 0, stream, part2node, part_ptr,  \
+                       col, src, ngh_mask, node_degs, out_id, out_edge, self_kept, num_parts, len, l.num_tiles, is_last,    \
+                       first, kept, counts, st)
+    // place_slots walks a tile from barrier to barrier.  1024 threads do that fastest as long as the chip holds all tiles at once
+    // (two workgroups on a CU: 512 tiles), beyond that smaller workgroups hide each other's waits better.  The kernel, us, with
+    // 1024 / 512 / 256 threads: 27 tiles 12 / 13 / -, 2253 tiles - / 41 / 46, 32 thousand tiles, the mean of two layers, - / 413 /
+    // 392; a whole marking: 564 tiles 37 / 33 / 38, 4395 tiles 143 / 123 / 119, 10 thousand tiles 315 / 274 / 275.
+    if (l.num_tiles >= kMarkScannedTiles) {
+        hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, stream, counts, l.num_tiles);
+        EPPGCN_HIP(hipGetLastError());
+        EPPGCN_PLACE(256, true);
+    } else if (l.num_tiles > 512) {
+        EPPGCN_PLACE(512, false);
+    } else {
+        EPPGCN_PLACE(1024, false);
+    }
+    EPPGCN_HIP(hipGetLastError());
+#undef EPPGCN_PLACE
     return kOk;
 }
 
@@ -1202,8 +1264,9 @@ int launch_mark_compact(const int* part2node, const int* part_ptr, const int* co
         return kOk;
     }
     ScanState* st = static_cast<ScanState*>(workspace);
-    hipLaunchKernelGGL(tile_groups_kernel, dim3((l.num_tiles + 1 + 255) / 256), dim3(256), 0, stream, part_ptr, num_parts,
-                       l.num_tiles, l.tile_slots, reinterpret_cast<int*>(base + l.first), st);
+    const int blocks = num_parts / 1024 + 1 < 4096 ? num_parts / 1024 + 1 : 4096;
+    hipLaunchKernelGGL(tile_groups_kernel, dim3(blocks), dim3(256), 0, stream, part_ptr, num_parts,
+                       l.num_tiles, reinterpret_cast<int*>(base + l.first), st);
     EPPGCN_HIP(hipGetLastError());
     if (int rc = launch_mark_pass<false>(part2node, part_ptr, col, src_mask, ngh_mask, node_degs, out_id, out_edge, nullptr,
                                          num_parts, length, is_last, l, base, stream))
@@ -1223,17 +1286,17 @@ int launch_mark_path(const int* part2node, const int* part_ptr, const int* col, 
     ScanState* st = static_cast<ScanState*>(workspace);
     uint32_t* bits = reinterpret_cast<uint32_t*>(base + l.bits);
     uint8_t* self_kept = reinterpret_cast<uint8_t*>(base + l.self_kept);
-    const int most = l.words * 8 > l.num_tiles + 1 ? l.words * 8 : l.num_tiles + 1;
-    const int init_blocks = most / 256 + 1 < 2048 ? most / 256 + 1 : 2048;
+    const int most = l.words * 8 > num_parts / 4 ? l.words * 8 : num_parts / 4;
+    const int init_blocks = most / 256 + 1 < 4096 ? most / 256 + 1 : 4096;
     hipLaunchKernelGGL(mark_path_init_kernel, dim3(init_blocks), dim3(256), 0, stream, src_mask, num_nodes, l.words, bits,
-                       reinterpret_cast<uint32_t*>(self_kept), part_ptr, num_parts, l.num_tiles, l.tile_slots,
+                       reinterpret_cast<uint32_t*>(self_kept), part_ptr, num_parts, l.num_tiles,
                        reinterpret_cast<int*>(base + l.first), st);
     EPPGCN_HIP(hipGetLastError());
     if (int rc = launch_mark_pass<true>(part2node, part_ptr, col, bits, ngh_mask, node_degs, out_id, out_edge, self_kept,
                                         num_parts, length, is_last, l, base, stream))
         return rc;
-    const int count_blocks = num_nodes / 1024 + 1 < kFinishCountBlocks ? num_nodes / 1024 + 1 : kFinishCountBlocks;
-    hipLaunchKernelGGL(mark_path_finish_kernel, dim3(count_blocks), dim3(256), 0, stream, bits,
+    const int count_blocks = num_nodes / 16384 + 1 < kFinishBlocks ? num_nodes / 16384 + 1 : kFinishBlocks;
+    hipLaunchKernelGGL(mark_path_finish_kernel, dim3(count_blocks), dim3(kFinishBlock), 0, stream, bits,
                        reinterpret_cast<const uint4*>(self_kept), l.words, gathered, node_degs, num_nodes, group_size,
                        st);
     EPPGCN_HIP(hipGetLastError());

@@ -58,8 +58,8 @@ def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shi
 
 
 @pytest.mark.parametrize("n,slots_per_row,loops,ps", [
-    (2300000, 15, True, 16), (9, 6000000, False, 32),               # two and three thousand large tiles (from 2^25 slots on)
-    (34000000, 0, True, 1)])                                        # more groups in a large tile than are staged
+    (2300000, 15, True, 16), (9, 6000000, False, 32),               # nine and thirteen thousand tiles (scanned from 2^25 slots on)
+    (34000000, 0, True, 1)])                                        # more groups in a tile than are staged
 @pytest.mark.parametrize("is_last", [False, True])
 def test_path_marking_in_large_tiles(api, n, slots_per_row, loops, ps, is_last):
     assert _check_marking(api, n, slots_per_row, loops, ps, is_last, 1) >= 1 << 25
@@ -70,6 +70,50 @@ def test_path_marking_in_large_tiles(api, n, slots_per_row, loops, ps, is_last):
 def test_path_marking_where_the_workgroups_get_smaller(api, n, is_last):
     """512 and 513 tiles of 4096 slots, the last one full, one slot short and one slot long."""
     assert _check_marking(api, n, 0, True, 4, is_last, 0) == n
+
+
+@pytest.mark.parametrize("slots", [(1 << 25) - 4096, (1 << 25) - 4095])
+def test_path_marking_where_the_counts_are_scanned(api, slots):
+    """8191 full tiles add up the counts before theirs, 8192 (the last one with a single slot) have them scanned."""
+    assert _check_marking(api, slots, 0, True, 64, False, 0) == slots
+
+
+@pytest.mark.parametrize("e", [40, 4096, 4097, 30000, 9000000])
+@pytest.mark.parametrize("is_last", [False, True])
+def test_path_marking_with_empty_groups_and_slots_of_no_group(api, e, is_last):
+    """Runs of empty groups, also at the start of a tile and at both ends, and slots before the first group and behind the last
+    one, which are never kept and mark nobody.  A row whose groups are all empty is not its own neighbour."""
+    rng = np.random.default_rng(e)
+    n = max(8, e // 9)
+    cuts = np.unique(np.concatenate([rng.integers(3, e - 5, e // 7 + 1), [3, e - 5], np.arange(4096, e - 5, 4096)])).astype(np.int64)
+    again = rng.integers(0, 4, cuts.size) * (rng.random(cuts.size) < 0.2)          # empty groups in front of a group
+    again[[0, -1]] = 2
+    pp = np.repeat(cuts, 1 + again)
+    p2n = np.sort(rng.integers(0, n, pp.size - 1)).astype(np.int32)
+    slots = np.arange(e)
+    row = np.full(e, -1)
+    filled = np.flatnonzero(np.diff(pp) > 0)
+    inside = (slots >= 3) & (slots < e - 5)
+    row[inside] = p2n[filled[np.searchsorted(pp[filled], slots[inside], side="right") - 1]]
+    col = rng.integers(0, n, e).astype(np.int32)
+    src = rng.random(n) < 0.3
+    keep = inside & src[col]
+    ngh = np.zeros(n, bool)
+    if not is_last:
+        marked = inside & src[np.maximum(row, 0)]
+        ngh[row[marked]] = True
+        ngh[col[marked]] = True
+    want = np.zeros((2, e), np.int32)
+    v = int(keep.sum())
+    want[0, :v], want[1, :v] = row[keep], col[keep]
+    degs_want = np.bincount(row[keep], minlength=n)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    for call in (api.mark_path, api.mark_compact):
+        degs, got_ngh = torch.zeros(n, dtype=torch.int32, device="cuda"), torch.zeros(n, dtype=torch.bool, device="cuda")
+        got = call(d(p2n), d(pp.astype(np.int32)), d(col), d(src), None if is_last else got_ngh, degs, is_last)
+        assert got[2] == v and np.array_equal(degs.cpu().numpy(), degs_want)
+        assert np.array_equal(got[0].cpu().numpy(), want[0]) and np.array_equal(got[1].cpu().numpy(), want[1])
+        assert np.array_equal(got_ngh.cpu().numpy(), ngh)
 
 
 def _check_marking(api, n, slots_per_row, loops, ps, is_last, shift):
