@@ -59,7 +59,9 @@ __device__ __forceinline__ void load_row_piece(float (&x)[VW], const float* __re
 {
     if (k + VW <= K) {
         if constexpr (VW == 4) {
-            const float4 t = *reinterpret_cast<const float4*>(row + k);
+            // read once: the caches are left to what the product writes, which the aggregation gathers next (R-MAT scale 20,
+            // 96 x 16: the two aggregations 165 -> 154 us, this product 94 -> 97; 16 x 22 at scale 22 alone: 197 -> 189)
+            const floatx4 t = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(row + k));
             x[0] = t.x; x[1] = t.y; x[2] = t.z; x[3] = t.w;
         } else if constexpr (VW == 2) {
             const float2 t = *reinterpret_cast<const float2*>(row + k);
@@ -292,12 +294,17 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
     int mt_cap = 8;                                     // 16-column tiles one launch covers
     while (mt_cap > 1 && lds_per_tile * mt_cap > kMaxOperandLds) mt_cap /= 2;
     const long long tiles = (n + kTileRows - 1) / kTileRows;
-    long long blocks = (tiles + kUpdateWaves - 1) / kUpdateWaves;
-    if (blocks > 256 * 8) blocks = 256 * 8;
     for (int c0 = 0; c0 < out_cols; c0 += 16 * mt_cap) {
         const int cols = out_cols - c0 < 16 * mt_cap ? out_cols - c0 : 16 * mt_cap;
         int mt = 1;
         while (16 * mt < cols) mt *= 2;
+        const size_t lds = lds_per_tile * mt;
+        // Workgroups: more than the chip holds, so that one that falls behind does not end the launch, as long as each still
+        // spreads the filling of its operand over some tiles.  4.2 M rows, 16 x 22 (2 KB), us with 8 / 12 / 24 / 48 / 64 / 256
+        // workgroups per CU: 197, 170, 167, 163, 169, 221; 1 M rows, 96 x 16 (8 KB), with 8 / 24 / 32 / 48 / 64: 94, 92, 95, 103, 114.
+        const long long cap = 256ll * (lds <= 2048 ? 48 : lds <= 8192 ? 24 : 8);
+        long long blocks = (tiles + kUpdateWaves - 1) / kUpdateWaves;
+        if (blocks > cap) blocks = cap;
         RowsArgs a;
         a.out = out + c0;
         a.x = x;
@@ -324,7 +331,6 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         // [N, 32] results unchanged or slower
         if (a.vec_store && out_cols >= 64) a.vec_store = 2;
         a.tile_store = (a.vec_store && ld_out == 32 && cols == 32 && c0 == 0 && n < (1ll << 32)) ? 1 : 0;
-        const size_t lds = lds_per_tile * mt;
         hipError_t e;
         if (vw == 4) e = launch_rows_mt<4>(a, mt, cu, grid, lds, stream);
         else if (vw == 2) e = launch_rows_mt<2>(a, mt, cu, grid, lds, stream);
@@ -425,6 +431,14 @@ __global__ __launch_bounds__(64 * kReduceSlices) void reduce_partials_kernel(flo
     float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
     if (e < count) {
         int b = slice;
+        constexpr int kUnder = 16;                       // loads under way; the additions keep the order of four at a time
+        for (; b + (kUnder - 1) * kReduceSlices < num_blocks; b += kUnder * kReduceSlices) {
+            float v[kUnder];
+#pragma unroll
+            for (int u = 0; u < kUnder; ++u) v[u] = partial[static_cast<size_t>(b + u * kReduceSlices) * count + e];
+#pragma unroll
+            for (int u = 0; u < kUnder; u += 4) s0 += v[u], s1 += v[u + 1], s2 += v[u + 2], s3 += v[u + 3];
+        }
         for (; b + 3 * kReduceSlices < num_blocks; b += 4 * kReduceSlices) {
             s0 += partial[static_cast<size_t>(b) * count + e];
             s1 += partial[static_cast<size_t>(b + kReduceSlices) * count + e];
@@ -487,9 +501,10 @@ int launch_dense_weight(float* dw, const float* x, int ld_x, const float* g, int
     const int ktiles = (K + 15) / 16;
     int ktb = 8 / dt;
     while (ktb > 1 && ktb / 2 >= ktiles) ktb /= 2;
+    if (ktb == 8 && ktiles <= 6) ktb = 6;               // no products of columns that do not exist: 1 M rows, 96 x 16, 87 -> 77 us
     hipError_t e;
 #define EPPGCN_W(KTB_, DT_) launch_weight<KTB_, DT_>(partial, x, ld_x, g, ld_g, relu_in, n, K, D, rows_per_wave, blocks, stream, rows)
-    if (dt == 1) e = ktb == 8 ? EPPGCN_W(8, 1) : ktb == 4 ? EPPGCN_W(4, 1) : ktb == 2 ? EPPGCN_W(2, 1) : EPPGCN_W(1, 1);
+    if (dt == 1) e = ktb == 8 ? EPPGCN_W(8, 1) : ktb == 6 ? EPPGCN_W(6, 1) : ktb == 4 ? EPPGCN_W(4, 1) : ktb == 2 ? EPPGCN_W(2, 1) : EPPGCN_W(1, 1);
     else if (dt == 2) e = ktb == 4 ? EPPGCN_W(4, 2) : ktb == 2 ? EPPGCN_W(2, 2) : EPPGCN_W(1, 2);
     else e = ktb == 2 ? EPPGCN_W(2, 4) : EPPGCN_W(1, 4);
 #undef EPPGCN_W

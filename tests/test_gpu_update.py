@@ -350,3 +350,25 @@ def test_pruned_backward_clears_and_scales_in_one_launch(api, n, m, offset, list
                       dev(np.ones(n, np.float32)), parts, out=out.view(n, m), gathered_rows=bitmap)
     assert np.array_equal(out.cpu().numpy().reshape(n, m), want.astype(np.float32))
     assert (whole[:32 + offset] == 7).all() and (whole[32 + offset + n * m:] == 7).all()
+
+
+# inputs around the 16-column tiles of the weight kernel (six tiles in one pass up to 96), rows around the 256 block sums that
+# the last kernel loads together (a block per 64 rows)
+@pytest.mark.parametrize("k", [65, 80, 81, 96, 97, 112, 128])
+@pytest.mark.parametrize("m", [1, 16])
+@pytest.mark.parametrize("n", [1, 255 * 64, 255 * 64 + 1, 256 * 64, 257 * 64 + 5])
+def test_weight_gradient_at_the_ends_of_its_tiles(api, n, k, m):
+    """Whole numbers: every sum is exact in fp32."""
+    rng = np.random.default_rng(n + k + m)
+    x, g = dev(rng.integers(-4, 5, (n, k)).astype(np.float32)), dev(rng.integers(-4, 5, (n, m)).astype(np.float32))
+    assert torch.equal(api.update_backward_weight(x, g).double(), x.double().T.contiguous() @ g.double())
+
+
+@pytest.mark.parametrize("k,m", [(3, 2), (4, 1), (16, 22), (33, 9), (96, 16), (130, 20)])
+def test_products_of_more_rows_than_the_workgroups_take_at_once(api, k, m):
+    """A workgroup takes 64 rows at a time, at most 12 288 of them run (operands of up to 2 KB; 6144 up to 8 KB, else 2048)."""
+    n = 12288 * 64 + 17 if k < 33 else 6144 * 64 + 17 if k < 130 else 2048 * 64 + 17
+    gen = torch.Generator("cuda").manual_seed(k)
+    x = torch.randint(-4, 5, (n, k), device="cuda", generator=gen).float()
+    w = torch.randint(-4, 5, (k, m), device="cuda", generator=gen).float()
+    assert torch.equal(api.update_forward(x, w).double(), x.double() @ w.double())
