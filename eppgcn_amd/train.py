@@ -59,6 +59,9 @@ class _TrainingLoss(torch.autograd.Function):
         return gnnadvisor().nll_backward(d_loss.contiguous(), logits, labels, ctx.num_rows), None, None
 
 
+_LOSS, _LOSS_STEPS = _TrainingLoss, (_TrainingLoss.forward, _TrainingLoss.backward)
+
+
 class Net(torch.nn.Module):
     """The reference's model (EPPGCN/gcn_main.py:190-208): conv -> relu -> ... -> conv.  With
     ``fuse_relu`` (default) the activation between two layers is applied by the consuming layer
@@ -150,6 +153,7 @@ class Trainer:
         self.for_time = self.loss_time = self.back_time = self.build_time = 0.0
         self.losses: List[float] = []
         self.train_idx = self.train_y = None       # set by the first epoch, or by the caller
+        self._unit_gradient = None                 # a one like the loss, and what it is valid for
         self.kept_edges = [None] * num_layers      # per conv layer, filled by build_back_part
 
     def build_back_part(self):
@@ -207,9 +211,37 @@ class Trainer:
         selected = self.row_labels is not None and self._row_versions == (self.train_idx._version, self.train_y._version)
         if (selected and out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous()
                 and out.shape[0] == self.row_labels.numel()):
+            ops = gnnadvisor()
+            if (_TrainingLoss is _LOSS and (_TrainingLoss.forward, _TrainingLoss.backward) == _LOSS_STEPS
+                    and getattr(ops, "native_functions", ())[3:] == (ops.nll_forward, ops.nll_backward)
+                    and type(out) is torch.Tensor):
+                loss = ops.training_loss(out, self.train_idx, self.row_labels)      # _TrainingLoss in native code
+                if loss is not None:
+                    return loss
             return _TrainingLoss.apply(out, self.train_idx, self.row_labels)
         logp = F.log_softmax(out.index_select(0, self.train_idx), dim=1)
         return -logp.gather(1, self.train_y.unsqueeze(1)).mean()
+
+    def _zero_grad(self):
+        """``optimizer.zero_grad()``, without torch's way round its own Adam (14 us, a fifteenth of a small graph's epoch)."""
+        opt = self.optimizer
+        if (type(opt) is not torch.optim.Adam or "zero_grad" in vars(opt) or not _is_torchs(torch.optim.Adam.zero_grad)
+                or any(type(w) is not torch.nn.Parameter for group in opt.param_groups for w in group["params"])):
+            return opt.zero_grad()
+        for group in opt.param_groups:
+            self.GNNA.drop_gradients(group["params"])
+
+    def _backward(self, loss):
+        """``loss.backward()`` with a gradient of one that is kept, where autograd would make one (a launch per epoch): for a
+        plain scalar whose gradient nobody is handed, and outside a capture, whose graph may outlive the trainer."""
+        if (type(loss) is not torch.Tensor or loss.dim() or not loss.is_cuda or loss.dtype != torch.float32
+                or loss._backward_hooks or loss.retains_grad or torch.cuda.is_current_stream_capturing()):
+            return loss.backward()
+        kept = self._unit_gradient
+        if kept is None or kept[1:] != (kept[0]._version, loss.device):
+            one = torch.ones_like(loss, requires_grad=False)
+            kept = self._unit_gradient = one, one._version, loss.device
+        loss.backward(kept[0])
 
     def _adam_in_one_launch(self):
         """The optimizer's step in the library's kernel, with the rounding and the state of torch's own; False, with nothing
@@ -247,7 +279,7 @@ class Trainer:
         ds = self.dataset
         sync = torch.cuda.synchronize if phase_timers else (lambda: None)
         self.model.train()
-        self.optimizer.zero_grad()
+        self._zero_grad()
         t = time.perf_counter()
         out = self.model(ds.x, self.inputInfo, self.mask_props, self.back_props, is_first_iter, False)
         sync()
@@ -264,7 +296,7 @@ class Trainer:
         sync()
         self.loss_time += time.perf_counter() - t
         t = time.perf_counter()
-        loss.backward()
+        self._backward(loss)
         sync()
         self.back_time += time.perf_counter() - t
         if not self._adam_in_one_launch():
