@@ -238,9 +238,10 @@ class Trainer:
                 or loss._backward_hooks or loss.retains_grad or torch.cuda.is_current_stream_capturing()):
             return loss.backward()
         kept = self._unit_gradient
-        if kept is None or kept[1:] != (kept[0]._version, loss.device):
+        stream = torch.cuda.current_stream(loss.device)      # a fill on another stream may not have run yet
+        if kept is None or kept[1:] != (kept[0]._version, loss.device, stream):
             one = torch.ones_like(loss, requires_grad=False)
-            kept = self._unit_gradient = one, one._version, loss.device
+            kept = self._unit_gradient = one, one._version, loss.device, stream
         loss.backward(kept[0])
 
     def _adam_in_one_launch(self):

@@ -304,6 +304,23 @@ def test_kept_unit_gradient(trained, monkeypatch):
     assert handed and handed[0] != tr._unit_gradient[0].data_ptr()
 
 
+def test_unit_gradient_of_another_stream():
+    tr = _trainer()
+    tr.train_step(False)
+    kept = tr._unit_gradient[0]
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        tr.train_step(False)
+        assert tr._unit_gradient[0] is not kept          # its fill is ordered before the work of its own stream only
+        there = tr._unit_gradient[0]
+        tr.train_step(False)
+        assert tr._unit_gradient[0] is there
+    torch.cuda.current_stream().wait_stream(other)
+    torch.cuda.synchronize()
+    assert float(there) == 1.0
+
+
 @pytest.mark.parametrize("how", ["plain", "instance", "subclass", "parameter"])
 def test_gradients_are_dropped(how):
     tr = _trainer()
