@@ -59,9 +59,7 @@ __device__ __forceinline__ void load_row_piece(float (&x)[VW], const float* __re
 {
     if (k + VW <= K) {
         if constexpr (VW == 4) {
-            // read once: the caches are left to what the product writes, which the aggregation gathers next (R-MAT scale 20,
-            // 96 x 16: the two aggregations 165 -> 154 us, this product 94 -> 97; 16 x 22 at scale 22 alone: 197 -> 189)
-            const floatx4 t = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(row + k));
+            const float4 t = *reinterpret_cast<const float4*>(row + k);
             x[0] = t.x; x[1] = t.y; x[2] = t.z; x[3] = t.w;
         } else if constexpr (VW == 2) {
             const float2 t = *reinterpret_cast<const float2*>(row + k);
@@ -299,12 +297,18 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         int mt = 1;
         while (16 * mt < cols) mt *= 2;
         const size_t lds = lds_per_tile * mt;
-        // Workgroups: more than the chip holds, so that one that falls behind does not end the launch, as long as each still
-        // spreads the filling of its operand over some tiles.  4.2 M rows, 16 x 22 (2 KB), us with 8 / 12 / 24 / 48 / 64 / 256
-        // workgroups per CU: 197, 170, 167, 163, 169, 221; 1 M rows, 96 x 16 (8 KB), with 8 / 24 / 32 / 48 / 64: 94, 92, 95, 103, 114.
-        const long long cap = 256ll * (lds <= 2048 ? 48 : lds <= 8192 ? 24 : 8);
+        // Workgroups: up to 24 per CU, more than the chip holds, so that one that falls behind does not end the launch, while a
+        // wave still has two tiles and the operand that a workgroup fills in LDS is small; else 8 per CU.  us with 8 / 24:
+        // 4.2 M rows, 96 x 16 (8 KB) 387 / 374, 16 x 22 (2 KB) 204 / 171; 1 M rows 99 / 95, 39 / 33; 0.26 M rows, where 24 leave a
+        // wave one tile, 26 / 28, 12 / 13; 2.1 M rows, 200 x 32 (26 KB) 440 / 484.  Input rows are not read past the caches: an
+        // instruction takes half a line of each row, and the other half is fetched anew (4.2 M rows, 96 x 16, 374 -> 430;
+        // 200 x 32 853 -> 1126).
+        const long long cap = 256ll * 8, wide_cap = lds <= 8192 ? 256ll * 24 : cap;
         long long blocks = (tiles + kUpdateWaves - 1) / kUpdateWaves;
-        if (blocks > cap) blocks = cap;
+        if (blocks > cap) {
+            const long long pairs = (tiles + 2 * kUpdateWaves - 1) / (2 * kUpdateWaves);
+            blocks = pairs < cap ? cap : pairs < wide_cap ? pairs : wide_cap;
+        }
         RowsArgs a;
         a.out = out + c0;
         a.x = x;
