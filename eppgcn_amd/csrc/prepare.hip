@@ -256,7 +256,10 @@ __global__ __launch_bounds__(kCompactBlock) void compact_mask_kernel(
 //                        per 64 slots queued ten thousand on one address.
 constexpr int kMarkTile = 4096;           // slots of a tile
 constexpr int kKeepBlock = 1024;
-constexpr int kMarkStagedRows = kMarkTile;     // groups of a tile whose rows are staged (more: read where they are needed)
+// Groups of a tile whose rows are staged (more, which takes empty groups: read where they are needed).  The first group of the next
+// tile counts, so a tile of one-slot groups has one more than slots.  Without room for it, us for a whole marking: 34 M rows of
+// one slot 832, now 503; R-MAT scale 22 in groups of one slot 2724, now 1530.
+constexpr int kMarkStagedRows = kMarkTile + 1;
 constexpr int kMarkScannedTiles = 8192;   // tiles from which on their counts are scanned by a launch of its own
 
 // first[t] = last group starting at or before slot t * kMarkTile (group 0 for slots before all groups); first[num_tiles] = last
@@ -506,7 +509,7 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     }
     __syncthreads();
     // The owner of slot e is g_lo - 1 + (number of groups of the tile that start at or before e).
-    // When no two groups start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
+    // When no two groups of the tile start at the same slot (no empty groups, as build_part guarantees) that number is a prefix
     // population count over the map of group starts; otherwise every slot does a binary search over the group starts.
     if (wave < 2) {
         const unsigned long long* words = wave == 0 ? s_kept : s_starts;
@@ -542,26 +545,34 @@ __global__ __launch_bounds__(kBlock, 8) void place_slots_kernel(
     const int start_before = s_starts_before[my_word] + before - 1;
     const int place = s_kept_before[my_word] + s_prefix;
     unsigned row[kItems];                                    // bit 31 as in s_row
+    // starts at or before the lane: those below it in the word without its first bit, and the first bit
+    auto group_by_bits = [&](int k) {
+        const uint64_t word = lane_value(start_word, k);
+        const int head = __builtin_amdgcn_readlane(start_before, k) + static_cast<int>(word & 1ull);
+        return max(head + ballot_rank(word >> 1), 0);        // a slot before the first group is never used
+    };
     if (by_bits && staged) {
 #pragma unroll
-        for (int k = 0; k < kItems; ++k) {
-            // starts at or before the lane: those below it in the word without its first bit, and the first bit
-            const uint64_t word = lane_value(start_word, k);
-            const int head = __builtin_amdgcn_readlane(start_before, k) + static_cast<int>(word & 1ull);
-            const int a = head + ballot_rank(word >> 1);
-            row[k] = s_row[max(a, 0)];                       // a slot before the first group is never used
-        }
+        for (int k = 0; k < kItems; ++k) row[k] = s_row[group_by_bits(k)];
     } else {
 #pragma unroll 1
         for (int k = 0; k < kItems; ++k) {
-            const int e = static_cast<int>(base + mine + k * kWave);
-            int a = 0, b = g_cnt;
-            while (b - a > 1) {
-                const int mid = (a + b) >> 1;
-                if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
+            unsigned found = 0u;
+            if (!is_last || lane_value(kept_word, k) != 0ull) {      // the same for the whole wave; the last layer marks nobody
+                int a = 0;
+                if (by_bits) {
+                    a = group_by_bits(k);
+                } else {
+                    const int e = static_cast<int>(base + mine + k * kWave);
+                    int b = g_cnt;
+                    while (b - a > 1) {
+                        const int mid = (a + b) >> 1;
+                        if (part_ptr[g_lo + mid] <= e) a = mid; else b = mid;
+                    }
+                }
+                const int r = part2node[g_lo + a];
+                found = static_cast<unsigned>(r) | (!is_last && in_mask<kBits>(src, r) ? 0x80000000u : 0u);
             }
-            const int r = part2node[g_lo + a];
-            const unsigned found = static_cast<unsigned>(r) | (!is_last && in_mask<kBits>(src, r) ? 0x80000000u : 0u);
 #pragma unroll
             for (int j = 0; j < kItems; ++j) row[j] = j == k ? found : row[j];
         }

@@ -59,7 +59,7 @@ def test_path_marking_in_one_pass(api, n, slots_per_row, loops, ps, is_last, shi
 
 @pytest.mark.parametrize("n,slots_per_row,loops,ps", [
     (2300000, 15, True, 16), (9, 6000000, False, 32),               # nine and thirteen thousand tiles (scanned from 2^25 slots on)
-    (34000000, 0, True, 1)])                                        # more groups in a tile than are staged
+    (34000000, 0, True, 1)])                                        # as many groups in a tile as slots
 @pytest.mark.parametrize("is_last", [False, True])
 def test_path_marking_in_large_tiles(api, n, slots_per_row, loops, ps, is_last):
     assert _check_marking(api, n, slots_per_row, loops, ps, is_last, 1) >= 1 << 25
@@ -90,10 +90,16 @@ def test_path_marking_with_empty_groups_and_slots_of_no_group(api, e, is_last):
     again[[0, -1]] = 2
     pp = np.repeat(cuts, 1 + again)
     p2n = np.sort(rng.integers(0, n, pp.size - 1)).astype(np.int32)
+    _check_groups(api, pp, p2n, e, n, is_last, rng)
+
+
+def _check_groups(api, pp, p2n, e, n, is_last, rng):
+    """Marking of e slots with random columns and sources against the groups' definition: slot s belongs to the group with slots
+    that starts last at or before s."""
     slots = np.arange(e)
     row = np.full(e, -1)
     filled = np.flatnonzero(np.diff(pp) > 0)
-    inside = (slots >= 3) & (slots < e - 5)
+    inside = (slots >= pp[0]) & (slots < pp[-1])
     row[inside] = p2n[filled[np.searchsorted(pp[filled], slots[inside], side="right") - 1]]
     col = rng.integers(0, n, e).astype(np.int32)
     src = rng.random(n) < 0.3
@@ -114,6 +120,48 @@ def test_path_marking_with_empty_groups_and_slots_of_no_group(api, e, is_last):
         assert got[2] == v and np.array_equal(degs.cpu().numpy(), degs_want)
         assert np.array_equal(got[0].cpu().numpy(), want[0]) and np.array_equal(got[1].cpu().numpy(), want[1])
         assert np.array_equal(got_ngh.cpu().numpy(), ngh)
+
+
+@pytest.mark.parametrize("at", [(4096,), (8192,), (5000,), (4096, 5000, 8192)])
+@pytest.mark.parametrize("e", [12388, 3000000, 34000000])
+@pytest.mark.parametrize("is_last", [False, True])
+def test_path_marking_where_a_tile_has_more_groups_than_slots(api, at, e, is_last):
+    """Five thousand empty groups at a slot: a tile's rows are not staged then.  Where they start with the next tile, no two
+    groups of this one share a slot; in the middle they do.  In each of the three sizes of workgroups."""
+    rng = np.random.default_rng(e + len(at))
+    cuts = np.unique(np.concatenate([rng.integers(0, e, e // 5), [0, e], at])).astype(np.int64)
+    pp = np.repeat(cuts, 1 + 5000 * np.isin(cuts, at))
+    n = max(8, e // 9)
+    p2n = np.sort(rng.integers(0, n, pp.size - 1)).astype(np.int32)
+    _check_groups(api, pp, p2n, e, n, is_last, rng)
+
+
+def _marking_us(api, pp, p2n, col, n, is_last):
+    """Shortest of ten markings."""
+    src = torch.arange(n, device="cuda") % 10 == 0
+    best = float("inf")
+    for _ in range(10):
+        ngh, degs = torch.zeros(n, dtype=torch.bool, device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        torch.cuda.synchronize()
+        start.record()
+        pending = api.mark_path_begin(p2n, pp, col, src, None if is_last else ngh, degs, is_last)
+        end.record()
+        pending()
+        best = min(best, start.elapsed_time(end) * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("is_last", [False, True])
+def test_one_slot_groups_are_staged(api, is_last):
+    """A tile of one-slot groups has 4097 of them, with the next tile's first.  With their rows staged, 33.5 M slots take 1.25 to
+    1.3 times as long in groups of one slot as in groups of two; with a search per slot it is 2.06 to 2.27 times."""
+    n = 1 << 22
+    indptr = torch.arange(0, 8 * n + 1, 8, dtype=torch.int32, device="cuda")
+    col = torch.randint(0, n, (8 * n,), dtype=torch.int32, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    one, two = (_marking_us(api, *api.build_part(ps, indptr, 8 * n), col, n, is_last) for ps in (1, 2))
+    print("groups of 1 and 2 slots:", one, two, "us")
+    assert one < 1.6 * two
 
 
 def _check_marking(api, n, slots_per_row, loops, ps, is_last, shift):
