@@ -23,6 +23,7 @@
 //     kept: eight, and more while they are small); it affects speed only.
 #include <torch/extension.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -550,38 +551,140 @@ bool plain_eager(std::initializer_list<const Tensor*> tensors)
     return true;
 }
 
-// The Python records of a layer, which are read when a pass runs: a layer's backward path is filled in after its first forward
-// pass.  An autograd node holds them by the storage of a one-element tensor, since that is a kind of saved data that compiled
-// autograd can hand on; the element is its own address, so that a copy of the tensor is recognised.
-struct LayerRecords {
+// What the Python functions keep on ctx, which a caller finds - and can set - on a result's grad_fn, and which the backward pass
+// reads when it runs: a layer's backward path is filled in after its first forward pass.  It becomes a dict when somebody looks
+// (made in each pass, an epoch of 2 708 vertices took 175 us for 170).  A node holds it by the storage of a one-element tensor,
+// since that is a kind of saved data that compiled autograd can hand on; the element is its own address, so that a copy of the
+// tensor is recognised.
+struct Attributes {
+    static constexpr int kMost = 6;
     int64_t address;
-    pybind11::object info, back;
-    static Tensor held(pybind11::object info, pybind11::object back)
+    const char* const* names;                            // kMost, the unused ones null
+    pybind11::object kept[kMost];                        // their values until there is a dict
+    pybind11::object dict;
+    static Tensor held(Attributes* a)
     {
-        auto* r = new LayerRecords{0, std::move(info), std::move(back)};
-        r->address = reinterpret_cast<int64_t>(r);
-        return torch::from_blob(&r->address, {1}, [r](void*) { let_go(r); }, torch::kInt64);
+        a->address = reinterpret_cast<int64_t>(a);
+        return torch::from_blob(&a->address, {1}, [a](void*) { let_go(a); }, torch::kInt64);
     }
-    static const LayerRecords& of(const Tensor& held)
+    static Attributes& of(const Tensor& held)
     {
         const int64_t* at = held.data_ptr<int64_t>();
-        TORCH_CHECK(*at == reinterpret_cast<int64_t>(at), "the layer's records were copied");
-        return *reinterpret_cast<const LayerRecords*>(at);
+        TORCH_CHECK(*at == reinterpret_cast<int64_t>(at), "the function's attributes were copied");
+        return *reinterpret_cast<Attributes*>(*at);
     }
-    static void let_go(LayerRecords* r)
+    pybind11::dict as_dict()
+    {
+        if (!dict) {
+            pybind11::dict made;
+            for (int k = 0; k < kMost && names[k]; ++k) made[names[k]] = kept[k];
+            dict = std::move(made);
+            for (auto& value : kept) value = pybind11::object();
+        }
+        return pybind11::reinterpret_borrow<pybind11::dict>(dict);
+    }
+    pybind11::object get(int k) const
+    {
+        if (!dict) return kept[k];
+        PyObject* value = PyDict_GetItemString(dict.ptr(), names[k]);
+        if (!value) {
+            PyErr_Format(PyExc_AttributeError, "the function has no attribute '%s'", names[k]);
+            throw pybind11::error_already_set();
+        }
+        return pybind11::reinterpret_borrow<pybind11::object>(value);
+    }
+    static void let_go(Attributes* a)
     {
         if (!Py_IsInitialized()) return;                 // nothing is left to give the objects back to
         pybind11::gil_scoped_acquire gil;
-        delete r;
+        delete a;
     }
 };
-static_assert(offsetof(LayerRecords, address) == 0, "the element's address is the object's");
+static_assert(offsetof(Attributes, address) == 0, "the element's address is the object's");
+
+// grad_fn of a native function F with kInputs inputs: the saved tensors, the inputs that need gradients, and the attributes above.
+template <class F, int kInputs>
+struct NodeType {
+    using Node = torch::autograd::CppNode<F>;
+    static PyTypeObject type;
+    static Node& node(PyObject* self)
+    {
+        return dynamic_cast<Node&>(*reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata);
+    }
+    static pybind11::dict attributes(PyObject* self)
+    {
+        return F::attributes(node(self).ctx_).as_dict();
+    }
+    static PyObject* get(PyObject* self, PyObject* name)
+    {
+        HANDLE_TH_ERRORS
+        PyObject* found = PyObject_GenericGetAttr(self, name);
+        if (found || !PyErr_ExceptionMatches(PyExc_AttributeError)) return found;
+        pybind11::error_already_set missing;
+        PyObject* value = PyDict_GetItemWithError(attributes(self).ptr(), name);
+        if (!value && !PyErr_Occurred()) missing.restore();
+        Py_XINCREF(value);
+        return value;
+        END_HANDLE_TH_ERRORS
+    }
+    static int set(PyObject* self, PyObject* name, PyObject* value)
+    {
+        HANDLE_TH_ERRORS
+        if (PyObject_HasAttr(reinterpret_cast<PyObject*>(&type), name)) return PyObject_GenericSetAttr(self, name, value);
+        const pybind11::dict values = attributes(self);
+        if (value) return PyObject_SetItem(values.ptr(), name, value);
+        if (PyDict_Contains(values.ptr(), name) == 0) {
+            PyErr_SetObject(PyExc_AttributeError, name);
+            return -1;
+        }
+        return PyObject_DelItem(values.ptr(), name);
+        END_HANDLE_TH_ERRORS_RET(-1)
+    }
+    static PyObject* dict(PyObject* self, void*)
+    {
+        HANDLE_TH_ERRORS
+        return attributes(self).release().ptr();
+        END_HANDLE_TH_ERRORS
+    }
+    static PyObject* saved_tensors(PyObject* self, void*)
+    {
+        HANDLE_TH_ERRORS
+        return pybind11::tuple(pybind11::cast(node(self).ctx_.get_saved_variables())).release().ptr();
+        END_HANDLE_TH_ERRORS
+    }
+    static PyObject* needs_input_grad(PyObject* self, void*)
+    {
+        HANDLE_TH_ERRORS
+        const Node& n = node(self);
+        pybind11::tuple needs(kInputs);
+        for (uint32_t k = 0; k < kInputs; ++k) needs[k] = pybind11::bool_(k < n.num_outputs() && n.next_edge(k).is_valid());
+        return needs.release().ptr();
+        END_HANDLE_TH_ERRORS
+    }
+    static pybind11::object add(const char* name)
+    {
+        using namespace torch::autograd;                 // for the names in the macro
+        static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                           {"saved_tensors", saved_tensors, nullptr, nullptr, nullptr},
+                                           {"needs_input_grad", needs_input_grad, nullptr, nullptr, nullptr},
+                                           {"__dict__", dict, nullptr, nullptr, nullptr},
+                                           {nullptr}};
+        type.tp_getattro = get;
+        type.tp_setattro = set;
+        _initFunctionPyTypeObject(type, name, properties, nullptr);
+        registerCppFunction(typeid(Node), &type);
+        const auto added = pybind11::reinterpret_borrow<pybind11::object>(reinterpret_cast<PyObject*>(&type));
+        pybind11::module_::import("torch.autograd.graph").attr("Node").attr("register")(added);      // isinstance, as for Python's
+        return added;
+    }
+};
+template <class F, int kInputs>
+PyTypeObject NodeType<F, kInputs>::type{};
 
 // An attribute of a record, with the error that the Python function's call of the module gives for one of another type.
 template <class T>
-T arg_of(const pybind11::object& record, const char* name)
+T value_of(const pybind11::object& value, const char* name)
 {
-    const pybind11::object value = record.attr(name);
     try {
         return value.cast<T>();
     } catch (const pybind11::cast_error&) {
@@ -589,15 +692,23 @@ T arg_of(const pybind11::object& record, const char* name)
         throw pybind11::error_already_set();
     }
 }
+template <class T>
+T arg_of(const pybind11::object& record, const char* name)
+{
+    return value_of<T>(record.attr(name), name);
+}
 
 struct GraphArgs {
     Tensor row_pointers, column_index, degrees, part_ptr, part2node;
+    pybind11::object hints[3];                           // the last three as the record has them
     int part_size, dim_worker, warp_per_block;
     explicit GraphArgs(const pybind11::object& info)
         : row_pointers(arg_of<Tensor>(info, "row_pointers")), column_index(arg_of<Tensor>(info, "column_index")),
           degrees(arg_of<Tensor>(info, "degrees")), part_ptr(arg_of<Tensor>(info, "partPtr")),
-          part2node(arg_of<Tensor>(info, "part2Node")), part_size(arg_of<int>(info, "partSize")),
-          dim_worker(arg_of<int>(info, "dimWorker")), warp_per_block(arg_of<int>(info, "warpPerBlock")) {}
+          part2node(arg_of<Tensor>(info, "part2Node")),
+          hints{info.attr("partSize"), info.attr("dimWorker"), info.attr("warpPerBlock")},
+          part_size(value_of<int>(hints[0], "partSize")), dim_worker(value_of<int>(hints[1], "dimWorker")),
+          warp_per_block(value_of<int>(hints[2], "warpPerBlock")) {}
 };
 
 struct PathArgs {
@@ -611,40 +722,49 @@ struct PathArgs {
 };
 
 struct GNNAFunction : torch::autograd::Function<GNNAFunction> {
+    enum { kInfo, kBack, kRelu };
+    static constexpr const char* kNames[Attributes::kMost] = {"inputInfo", "backInfo", "reluInput",
+                                                              "partSize", "dimWorker", "warpPerBlock"};
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& X, const Tensor& W,
                           const pybind11::object& info, const pybind11::object& back, bool relu_input)
     {
         ctx->save_for_backward({X, W});
         const GraphArgs g(info);
-        ctx->saved_data["relu_input"] = relu_input;
-        ctx->saved_data["records"] = LayerRecords::held(info, back);
+        ctx->saved_data["attributes"] = Attributes::held(
+            new Attributes{0, kNames, {info, back, pybind11::bool_(relu_input), g.hints[0], g.hints[1], g.hints[2]}, {}});
         return ::forward(X, W, g.row_pointers, g.column_index, g.degrees, g.part_ptr, g.part2node, g.part_size, g.dim_worker,
                          g.warp_per_block, relu_input)[0];
+    }
+    static Attributes& attributes(torch::autograd::AutogradContext& ctx)
+    {
+        return Attributes::of(ctx.saved_data.at("attributes").toTensor());
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
         const Tensor &X = saved[0], &W = saved[1], d_output = grads[0].contiguous();
-        const bool relu_input = ctx->saved_data["relu_input"].toBool(), need_dx = ctx->needs_input_grad(0);
-        const Tensor held = ctx->saved_data["records"].toTensor();
-        const auto& records = LayerRecords::of(held);
+        const bool need_dx = ctx->needs_input_grad(0);
         std::vector<Tensor> d;
         pybind11::gil_scoped_acquire gil;                // for the records, and for the caches above as in every other call
-        const pybind11::object unpruned = pybind11::getattr(records.back, "unpruned", pybind11::none());
+        const Attributes& kept = attributes(*ctx);
+        const pybind11::object back = kept.get(kBack);
+        const bool relu_input = value_of<bool>(kept.get(kRelu), kNames[kRelu]);
+        const pybind11::object unpruned = pybind11::getattr(back, "unpruned", pybind11::none());
         const int all_edges = PyObject_IsTrue(unpruned.ptr());
         if (all_edges < 0) throw pybind11::error_already_set();
         if (all_edges) {
-            const GraphArgs g(records.info);
+            const GraphArgs g(kept.get(kInfo));
             d = ::backward(d_output, X, W, g.row_pointers, g.column_index, g.degrees, g.part_ptr, g.part2node, g.part_size,
                            g.dim_worker, g.warp_per_block, need_dx, relu_input);
         } else {
-            const PathArgs p(records.back);
+            const PathArgs p(back);
             d = ours_backward(d_output, X, W, p.id, p.part_pointer, p.edge_list, p.degrees, p.part_size, p.num_parts, p.layer,
                               p.blockx, p.blocky, need_dx, relu_input);
         }
         return {need_dx ? d[0] : Tensor(), d[1], Tensor(), Tensor(), Tensor()};
     }
 };
+using GNNAFunctionBackward = NodeType<GNNAFunction, 8>;      // the Python function takes eight inputs
 
 // The layer's forward pass with the autograd function above; nullopt: the caller takes the Python function.
 std::optional<Tensor> gcn_layer(const Tensor& X, const Tensor& W, pybind11::object info, pybind11::object back, bool relu_input)
@@ -654,21 +774,31 @@ std::optional<Tensor> gcn_layer(const Tensor& X, const Tensor& W, pybind11::obje
 }
 
 struct TrainingLoss : torch::autograd::Function<TrainingLoss> {
+    static constexpr const char* kNames[Attributes::kMost] = {"num_rows"};
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& logits, const Tensor& rows, const Tensor& labels)
     {
         ctx->save_for_backward({logits, labels});
         ctx->saved_data["num_rows"] = rows.numel();
         return nll_forward(logits, rows, labels);
     }
+    static Attributes& attributes(torch::autograd::AutogradContext& ctx)
+    {
+        auto& held = ctx.saved_data["attributes"];
+        if (!held.isTensor()) held = Attributes::held(new Attributes{0, kNames, {pybind11::int_(ctx.saved_data.at("num_rows").toInt())}, {}});
+        return Attributes::of(held.toTensor());
+    }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads)
     {
         const auto saved = ctx->get_saved_variables();
         const bool twice = torch::GradMode::is_enabled() && grads[0].requires_grad();
+        const bool looked_at = ctx->saved_data.find("attributes") != ctx->saved_data.end();
         Tensor d;
         {
             torch::NoGradGuard no_grad;
             pybind11::gil_scoped_acquire gil;            // one call into the library at a time, as from Python
-            d = nll_backward(grads[0].contiguous(), saved[0], saved[1], ctx->saved_data["num_rows"].toInt());
+            const int64_t num_rows = looked_at ? value_of<int64_t>(attributes(*ctx).get(0), kNames[0])
+                                               : ctx->saved_data["num_rows"].toInt();
+            d = nll_backward(grads[0].contiguous(), saved[0], saved[1], num_rows);
         }
         if (twice) {                                     // as Python's once_differentiable: an error if it is differentiated
             auto error = std::make_shared<torch::autograd::DelayedError>(
@@ -678,6 +808,8 @@ struct TrainingLoss : torch::autograd::Function<TrainingLoss> {
         return {d, Tensor(), Tensor()};
     }
 };
+
+using TrainingLossBackward = NodeType<TrainingLoss, 3>;
 
 std::optional<Tensor> training_loss(const Tensor& logits, const Tensor& rows, const Tensor& labels)
 {
@@ -956,6 +1088,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           py::arg("input"), py::arg("weight"), py::arg("info"), py::arg("back"), py::arg("relu_input"));
     m.def("training_loss", torch::wrap_pybind_function(training_loss), "nll_forward with its autograd function in native code (HIP); None: not for these inputs",
           py::arg("logits"), py::arg("rows"), py::arg("labels"));
+    GNNAFunctionBackward::add("GNNAFunctionBackward");
+    TrainingLossBackward::add("_TrainingLossBackward");
     // what the two call, for callers that replace functions of this module
     m.attr("native_functions") = py::make_tuple(m.attr("forward"), m.attr("backward"), m.attr("ours_backward"),
                                                 m.attr("nll_forward"), m.attr("nll_backward"));

@@ -147,6 +147,68 @@ def test_records_are_read_in_the_pass_and_let_go(trained):
     assert gone() is None
 
 
+@pytest.mark.parametrize("needs_dx", [False, True])
+def test_grad_fn_shows_what_the_python_function_keeps(trained, needs_dx):
+    """Records, launch hints and saved tensors are read from and set on a result's grad_fn as on the Python function's ctx."""
+    import copy
+    tr = trained
+    X = _input(tr).requires_grad_(needs_dx)
+    weights, back = tr.model.convs[1].weights, tr.back_props[1]
+    outs = [run(tr, X) for run in (_call, _python)]      # a Python node's saved tensors go with its output
+    nodes = [out.grad_fn for out in outs]
+    ours, theirs = nodes
+    assert vars(ours) == vars(theirs) and type(ours).__name__ == type(theirs).__name__
+    for node in nodes:
+        assert node.inputInfo is tr.inputInfo and node.backInfo is back and node.reluInput is tr.model.convs[1].relu_input
+        assert (node.partSize, node.dimWorker, node.warpPerBlock) == (tr.inputInfo.partSize, tr.inputInfo.dimWorker,
+                                                                      tr.inputInfo.warpPerBlock)
+        assert type(node.saved_tensors) is tuple and [a is b for a, b in zip(node.saved_tensors, (X, weights))] == [True, True]
+        assert node.needs_input_grad == (needs_dx, True) + (False,) * 6
+        assert isinstance(node, torch.autograd.graph.Node)
+        with pytest.raises(AttributeError):
+            node.nothing
+        with pytest.raises(AttributeError):
+            del node.nothing
+        with pytest.raises(AttributeError):
+            node.saved_tensors = ()
+    del node, nodes, ours, theirs, outs
+    for run in (_call, _python):
+        out = run(tr, X)
+        out.grad_fn.note = 3
+        gc.collect()
+        assert out.grad_fn.note == 3                     # it is the node's, not the Python object's
+        del out.grad_fn.note
+        assert not hasattr(out.grad_fn, "note")
+        other = copy.copy(back)
+        del other.id
+        out.grad_fn.backInfo = other                     # read when the backward pass runs
+        d = _path_gradient(tr, out.shape)
+        with pytest.raises(AttributeError, match="id"):
+            torch.autograd.grad(out, weights, d, retain_graph=True)
+        out.grad_fn.backInfo = back
+        torch.autograd.grad(out, weights, d)
+        assert out.grad_fn.backInfo is back
+        with pytest.raises(RuntimeError, match="second time"):
+            out.grad_fn.saved_tensors
+        gone = weakref.ref(other)
+        del other, out
+        gc.collect()
+        assert gone() is None
+
+
+def test_grad_fn_of_the_loss_shows_what_the_python_function_keeps(trained):
+    from eppgcn_amd import train
+    tr = trained
+    out = tr.model(tr.dataset.x, tr.inputInfo, tr.mask_props, tr.back_props, False, False).detach().requires_grad_()
+    losses = tr._loss(out), train._TrainingLoss.apply(out, tr.train_idx, tr.row_labels)
+    nodes = [loss.grad_fn for loss in losses]
+    for node in nodes:
+        assert node.num_rows == tr.train_idx.numel() and node.saved_tensors[0] is out
+        assert torch.equal(node.saved_tensors[1], tr.row_labels) and node.needs_input_grad == (True, False, False)
+        assert isinstance(node, torch.autograd.graph.Node)
+    assert vars(nodes[0]) == vars(nodes[1]) and type(nodes[0]).__name__ == type(nodes[1]).__name__
+
+
 def test_saved_tensor_hooks_and_checkpoint(trained):
     from torch.utils.checkpoint import checkpoint
     tr = trained
