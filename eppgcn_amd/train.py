@@ -13,7 +13,7 @@ import torch.nn.functional as F
 import torch.optim.optimizer as torch_optimizer
 
 from . import gnnadvisor, graphs
-from .gcn_conv import GCNConv
+from .gcn_conv import GCNConv, _is_as_defined, _is_torchs
 from .param import backInputProperty, inputProperty, maskInputProperty
 
 
@@ -59,7 +59,7 @@ class _TrainingLoss(torch.autograd.Function):
         return gnnadvisor().nll_backward(d_loss.contiguous(), logits, labels, ctx.num_rows), None, None
 
 
-_LOSS, _LOSS_STEPS = _TrainingLoss, (_TrainingLoss.forward, _TrainingLoss.backward)
+_LOSS, _LOSS_PARTS = _TrainingLoss, dict(vars(_TrainingLoss))
 
 
 class Net(torch.nn.Module):
@@ -96,15 +96,6 @@ def _step_hooks(opt):
     """Where torch keeps the callables that run around an optimizer's step."""
     return ((opt, "_optimizer_step_pre_hooks"), (opt, "_optimizer_step_post_hooks"),
             (torch_optimizer, "_global_optimizer_pre_hooks"), (torch_optimizer, "_global_optimizer_post_hooks"))
-
-
-def _is_torchs(step):
-    """No function of another module's is ``step`` or one that it wraps (torch puts wrappers of its own around it)."""
-    while step is not None:
-        if not getattr(step, "__globals__", {}).get("__name__", "").startswith("torch."):
-            return False
-        step = getattr(step, "__wrapped__", None)
-    return True
 
 
 class Trainer:
@@ -212,7 +203,7 @@ class Trainer:
         if (selected and out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous()
                 and out.shape[0] == self.row_labels.numel()):
             ops = gnnadvisor()
-            if (_TrainingLoss is _LOSS and (_TrainingLoss.forward, _TrainingLoss.backward) == _LOSS_STEPS
+            if (_TrainingLoss is _LOSS and _is_as_defined(_TrainingLoss, _LOSS_PARTS)
                     and getattr(ops, "native_functions", ())[3:] == (ops.nll_forward, ops.nll_backward)
                     and type(out) is torch.Tensor):
                 loss = ops.training_loss(out, self.train_idx, self.row_labels)      # _TrainingLoss in native code

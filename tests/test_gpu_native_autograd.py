@@ -296,6 +296,27 @@ def test_python_function_where_the_call_is_looked_into(trained, how, monkeypatch
     assert not _is_native(out)
 
 
+@pytest.mark.parametrize("where", ["own", "torch"])
+@pytest.mark.parametrize("what", ["layer", "loss"])
+def test_a_replaced_apply_is_called_in_every_pass(trained, what, where, monkeypatch):
+    from eppgcn_amd import gcn_conv, train
+    tr, X = trained, _input(trained)
+    logits = tr.model(tr.dataset.x, tr.inputInfo, tr.mask_props, tr.back_props, False, False).detach().requires_grad_()
+    function = gcn_conv.GNNAFunction if what == "layer" else train._TrainingLoss
+    run = (lambda: _call(tr, X)) if what == "layer" else (lambda: tr._loss(logits))
+    torchs, calls = torch.autograd.Function.apply.__func__, []
+
+    def counted(cls, *args):
+        calls.append(cls)
+        return torchs(cls, *args)
+
+    monkeypatch.setattr(function if where == "own" else torch.autograd.Function, "apply", classmethod(counted))
+    for k in range(2):
+        assert not _is_native(run()) and calls == [function] * (k + 1)
+    monkeypatch.undo()
+    assert _is_native(run()) and len(calls) == 2
+
+
 def test_function_transforms_refuse_as_before(trained):
     X = _input(trained)
     with pytest.raises(RuntimeError):
