@@ -219,8 +219,7 @@ class Trainer:
         if (type(opt) is not torch.optim.Adam or "zero_grad" in vars(opt) or not _is_torchs(torch.optim.Adam.zero_grad)
                 or any(type(w) is not torch.nn.Parameter for group in opt.param_groups for w in group["params"])):
             return opt.zero_grad()
-        for group in opt.param_groups:
-            self.GNNA.drop_gradients(group["params"])
+        self.GNNA.drop_gradients([w for group in opt.param_groups for w in group["params"]])
 
     def _backward(self, loss):
         """``loss.backward()`` with a gradient of one that is kept, where autograd would make one (a launch per epoch): for a

@@ -151,3 +151,22 @@ def test_a_profile_has_the_range_of_the_optimizer():
         with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
             tr.train_step(epoch == 0)
         assert [e.count for e in profile.key_averages() if e.key == "Optimizer.step#Adam.step"] == [1], epoch
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3])
+def test_a_profile_has_one_range_of_dropped_gradients(groups):
+    """Torch's zero_grad and the trainer's way round it are the same range of a profile, once whatever the groups."""
+    from eppgcn_amd import graphs, train
+    trainer = train.Trainer(graphs.uniform_graph(200, 400, seed=1, device="cuda"), dim=8, hidden=4, num_classes=3)
+    for k in range(groups - 1):
+        trainer.optimizer.add_param_group({"params": [torch.nn.Parameter(torch.ones(k + 2, device="cuda"))]})
+    counts = []
+    for drop in (trainer._zero_grad, trainer.optimizer.zero_grad):
+        for group in trainer.optimizer.param_groups:
+            for w in group["params"]:
+                w.grad = torch.ones_like(w)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as profile:
+            drop()
+        counts.append([e.count for e in profile.key_averages() if e.key == "Optimizer.zero_grad#Adam.zero_grad"])
+        assert all(w.grad is None for group in trainer.optimizer.param_groups for w in group["params"])
+    assert counts == [[1], [1]]
