@@ -817,6 +817,15 @@ std::optional<Tensor> training_loss(const Tensor& logits, const Tensor& rows, co
     return TrainingLoss::apply(logits, rows, labels);
 }
 
+// A loss that is training_loss's own result, with no hook on its node: its backward pass starts in the library, which only reads
+// the gradient it is given, and nobody else is handed it.
+bool gradient_stays_unseen(const Tensor& loss)
+{
+    const auto node = loss.defined() ? loss.grad_fn() : nullptr;
+    return dynamic_cast<TrainingLossBackward::Node*>(node.get()) && node->pre_hooks().empty() &&
+           node->tensor_pre_hooks().empty() && node->post_hooks().empty();
+}
+
 // ---------------------------------------------------------------- optimizer
 // One Adam step of all weights in one launch, in the rounding of torch's grouped operations; `steps` are the optimizer's CPU
 // counters.  False, with nothing changed, for weights, gradients or state of another form than fp32, contiguous and on one
@@ -1090,6 +1099,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
           py::arg("logits"), py::arg("rows"), py::arg("labels"));
     GNNAFunctionBackward::add("GNNAFunctionBackward");
     TrainingLossBackward::add("_TrainingLossBackward");
+    m.def("gradient_stays_unseen", &gradient_stays_unseen, "the loss is training_loss's own and has no hooks on its node");
     // what the two call, for callers that replace functions of this module
     m.attr("native_functions") = py::make_tuple(m.attr("forward"), m.attr("backward"), m.attr("ours_backward"),
                                                 m.attr("nll_forward"), m.attr("nll_backward"));

@@ -222,10 +222,11 @@ class Trainer:
         self.GNNA.drop_gradients([w for group in opt.param_groups for w in group["params"]])
 
     def _backward(self, loss):
-        """``loss.backward()`` with a gradient of one that is kept, where autograd would make one (a launch per epoch): for a
-        plain scalar whose gradient nobody is handed, and outside a capture, whose graph may outlive the trainer."""
-        if (type(loss) is not torch.Tensor or loss.dim() or not loss.is_cuda or loss.dtype != torch.float32
-                or loss._backward_hooks or loss.retains_grad or torch.cuda.is_current_stream_capturing()):
+        """``loss.backward()`` with a gradient of one that is kept, where autograd would make one (a launch per epoch): for the
+        library's own loss whose gradient nobody is handed - a function of another's may write to it unseen, through ``data`` -
+        and outside a capture, whose graph may outlive the trainer."""
+        if (type(loss) is not torch.Tensor or loss._backward_hooks or loss.retains_grad
+                or not self.GNNA.gradient_stays_unseen(loss) or torch.cuda.is_current_stream_capturing()):
             return loss.backward()
         kept = self._unit_gradient
         stream = torch.cuda.current_stream(loss.device)      # a fill on another stream may not have run yet

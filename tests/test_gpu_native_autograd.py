@@ -387,6 +387,46 @@ def test_kept_unit_gradient(trained, monkeypatch):
     assert handed and handed[0] != tr._unit_gradient[0].data_ptr()
 
 
+class _WritesIntoItsGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, d):
+        d.data.mul_(3.0)
+        return d
+
+
+@pytest.mark.parametrize("how", ["function", "prehook", "hook", "tensor_hook"])
+def test_each_epoch_starts_from_one(how, monkeypatch):
+    """Whoever is handed the gradient that the backward pass starts from may write into it; no write is seen in another epoch."""
+    tr = _trainer()
+    tr.train_step(False)                                 # a gradient of one is kept now
+    loss_of, starts = tr._loss, []
+
+    def changed(out):
+        loss = loss_of(out)
+        if how == "function":
+            loss = _WritesIntoItsGradient.apply(loss)
+        elif how == "prehook":
+            loss.grad_fn.register_prehook(lambda grads: grads[0].data.mul_(3.0) and None)
+        elif how == "hook":
+            loss.grad_fn.register_hook(lambda ins, outs: outs[0].data.mul_(3.0) and None)
+        else:
+            loss.register_hook(lambda grad: grad.data.mul_(3.0) and None)
+        loss.grad_fn.register_prehook(lambda grads: starts.append(float(grads[0])))
+        return loss
+
+    monkeypatch.setattr(tr, "_loss", changed)
+    for _ in range(3):
+        tr.train_step(False)
+    assert starts == [3.0 if how in ("prehook", "tensor_hook") else 1.0] * 3
+    monkeypatch.undo()
+    tr.train_step(False)
+    assert float(tr._unit_gradient[0]) == 1.0
+
+
 def test_unit_gradient_of_another_stream():
     tr = _trainer()
     tr.train_step(False)
