@@ -260,6 +260,31 @@ def test_group_split_at_the_ends_of_tiles(api, n, top, ps):
         assert np.array_equal(got[:parts + 1], want) and not got[parts + 1:].any()
 
 
+@pytest.mark.parametrize("groups", [1, 4, 5, 63, 64, 65, 127, 128, 129, 5000])
+@pytest.mark.parametrize("ps", [1, 3])
+def test_groups_of_a_hub(api, groups, ps):
+    """A wave writes the first 64 groups of a vertex in one step and those behind them in loops that end at the capacity."""
+    deg = np.array([2, groups * ps - ps // 2, 0, 7], np.int32)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    count = (deg + ps - 1) // ps
+    want = np.concatenate([start + ps * np.arange(c) for start, c in zip(indptr, count)] + [[indptr[-1]]]).astype(np.int32)
+    pp, p2n = api.build_part(ps, torch.from_numpy(indptr).cuda(), int(indptr[-1]))
+    assert np.array_equal(pp.cpu().numpy(), want) and np.array_equal(p2n.cpu().numpy(), np.repeat(np.arange(4), count))
+    lib = api.load()
+    nbytes = lib.eppgcn_split_workspace_bytes(4)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    for capacity in sorted({1, 2, 3, 66, 67, 68, groups, want.size - 1, want.size, want.size + 9}):
+        whole = torch.full((capacity + 200,), 7, dtype=torch.int32, device="cuda")
+        parts, slots = ctypes.c_int64(), ctypes.c_int64()
+        rc = lib.eppgcn_split_back_part(torch.from_numpy(deg).cuda().data_ptr(), 4, ps, whole[100:].data_ptr(), capacity,
+                                        ws.data_ptr(), nbytes, None, ctypes.byref(parts), ctypes.byref(slots),
+                                        torch.cuda.current_stream().cuda_stream)
+        got = whole.cpu().numpy()
+        assert rc == (0 if capacity >= want.size else -4) and (got[:100] == 7).all() and (got[100 + capacity:] == 7).all()
+        inside = min(capacity, want.size)
+        assert np.array_equal(got[100:100 + inside], want[:inside]) and not got[100 + inside:100 + capacity].any()
+
+
 @pytest.mark.parametrize("layers", [2, 6])
 def test_preparing_several_layers_holds_one_build_workspace(api, layers):
     """All plans of a run are under way before the host waits for the first one, but their builds follow one another on the
