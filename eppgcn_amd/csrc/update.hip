@@ -297,13 +297,19 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         int mt = 1;
         while (16 * mt < cols) mt *= 2;
         const size_t lds = lds_per_tile * mt;
-        // Workgroups: up to 24 per CU, more than the chip holds, so that one that falls behind does not end the launch, while a
-        // wave still has two tiles and the operand that a workgroup fills in LDS is small; else 8 per CU.  us with 8 / 24:
-        // 4.2 M rows, 96 x 16 (8 KB) 387 / 374, 16 x 22 (2 KB) 204 / 171; 1 M rows 99 / 95, 39 / 33; 0.26 M rows, where 24 leave a
-        // wave one tile, 26 / 28, 12 / 13; 2.1 M rows, 200 x 32 (26 KB) 440 / 484.  Input rows are not read past the caches: an
-        // instruction takes half a line of each row, and the other half is fetched anew (4.2 M rows, 96 x 16, 374 -> 430;
-        // 200 x 32 853 -> 1126).
-        const long long cap = 256ll * 8, wide_cap = lds <= 8192 ? 256ll * 24 : cap;
+        // Workgroups: 8 per CU, or 24, more than the chip holds, so that one that falls behind does not end the launch.  24 pay while
+        // the operand that each fills in LDS is small and its waves have work: us with 24 over us with 8, columns in -> out,
+        //   from 2^20 rows, operands up to 8 KB, 32 columns and more: 96 -> 16 0.94-0.97, 16 -> 96 1.03 at 1 M rows and 0.87-0.97
+        //     above, 64 <-> 32 0.88-0.99, 16 -> 22 0.94, 22 -> 16 0.97-1.05, 128 -> 16 0.97, 16 -> 128 0.83-0.96, 33 <-> 9 0.93-0.99
+        //     (0.85 M rows: 64 -> 32 1.06, 16 -> 96 1.05, but 96 -> 16 0.96, 16 -> 128 0.89);
+        //   fewer rows: 16 -> 96 1.03-1.09, 96 -> 16 0.99-1.04, 70 -> 12 1.02-1.09, 22 -> 16 1.07, but operands up to 4 KB with more
+        //     columns out than in: 16 -> 22 0.95-1.00, 9 -> 33 0.95-1.01 (and 12 -> 20, 8 -> 24 0.95);
+        //   fewer columns: 8 <-> 7, 8 -> 8, 12 <-> 8 1.00-1.10 at any number of rows, 16 -> 8 1.02-1.07;
+        //   operands of 12 KB (47 -> 47) 1.00, of 16 KB (96 <-> 32, 64 -> 64) 1.04-1.2 up to 1.5 M rows, 0.93-1.03 at 3 M.
+        // Input rows are not read past the caches: an instruction takes half a line of each row, and the other half is fetched anew
+        // (4.2 M rows, 96 x 16, 374 -> 430 us; 200 x 32 853 -> 1126).
+        const bool many = lds <= 8192 && K + cols >= 32 && (n >= 1 << 20 || (lds <= 4096 && cols > K));
+        const long long cap = 256ll * 8, wide_cap = many ? 256ll * 24 : cap;
         long long blocks = (tiles + kUpdateWaves - 1) / kUpdateWaves;
         if (blocks > cap) {
             const long long pairs = (tiles + 2 * kUpdateWaves - 1) / (2 * kUpdateWaves);

@@ -364,11 +364,17 @@ def test_weight_gradient_at_the_ends_of_its_tiles(api, n, k, m):
     assert torch.equal(api.update_backward_weight(x, g).double(), x.double().T.contiguous() @ g.double())
 
 
-@pytest.mark.parametrize("k,m", [(3, 2), (4, 1), (16, 22), (33, 9), (96, 16), (130, 20)])
-def test_products_of_more_rows_than_the_workgroups_take_at_once(api, k, m):
-    """A workgroup takes 64 rows at a time, at most 12 288 of them run (operands of up to 2 KB; 6144 up to 8 KB, else 2048)."""
-    n = 12288 * 64 + 17 if k < 33 else 6144 * 64 + 17 if k < 130 else 2048 * 64 + 17
+# a workgroup takes 64 rows at a time; 2048 workgroups, or up to 6144 while each of their waves has two tiles of 16 rows: from 2^20
+# rows, and from 2048 * 128 on for more columns out than in, in each case with 32 columns and more and an operand of at most 8 KB (4)
+@pytest.mark.parametrize("k,m,n", [(3, 2, 2048 * 64 + 17), (4, 1, (1 << 20) + 17), (130, 20, (1 << 20) + 17),       # 2048
+                                   (16, 22, 2048 * 128 - 1), (16, 22, 2048 * 128 + 17), (16, 22, 6144 * 64 + 17),   # 2048, 2049, 3073
+                                   (16, 22, 6144 * 128 + 17), (9, 33, 6144 * 128 + 17),                             # 6144
+                                   (33, 9, (1 << 20) - 1), (33, 9, (1 << 20) + 17), (96, 16, (1 << 20) - 1),        # 2048, 6144, 2048
+                                   (96, 16, (1 << 20) + 17), (12, 20, (1 << 20) + 1), (12, 19, (1 << 20) + 1)])     # 6144, 6144, 2048
+def test_products_of_more_rows_than_the_workgroups_take_at_once(api, k, m, n):
     gen = torch.Generator("cuda").manual_seed(k)
     x = torch.randint(-4, 5, (n, k), device="cuda", generator=gen).float()
     w = torch.randint(-4, 5, (k, m), device="cuda", generator=gen).float()
     assert torch.equal(api.update_forward(x, w).double(), x.double() @ w.double())
+    g = torch.randint(-4, 5, (n, m), device="cuda", generator=gen).float()
+    assert torch.equal(api.update_backward_input(g, w).double(), g.double() @ w.double().T)
