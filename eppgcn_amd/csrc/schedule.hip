@@ -255,9 +255,9 @@ __global__ __launch_bounds__(256) void plan_init_kernel(StreamHeader* h, PlanSca
 
 // Sets bit (row & 31) of touched[row >> 5] for the lanes with `set`, and of single[row >> 5] for those with `alone` too: the
 // lanes of a wave whose rows share a word (rows ascend along the groups, so they are neighbours) combine their bits first,
-// one atomic per run.  One atomic per group was most of the classification kernel before (0.7 ms per run at R-MAT scale 22);
-// combining the bits in six shuffle steps per map cost plan_keys 22 of 401 us more than these sums.  A row's bit is counted in its first lane, so the bits of a run are distinct and their sum is their union;
-// rows that do not ascend are set one by one.
+// one atomic per run.  A row's bit is counted in its first lane, so the bits of a run are distinct and their sum is their union;
+// rows that do not ascend are set one by one.  One atomic per group was most of the classification kernel before (0.7 ms per run
+// at R-MAT scale 22); combining the bits in six shuffle steps per map cost plan_keys 22 of 401 us more than these sums.
 __device__ __forceinline__ void or_row_bits(uint32_t* __restrict__ touched, uint32_t* __restrict__ single, int row, bool set,
                                             bool alone)
 {
@@ -299,9 +299,9 @@ __device__ __forceinline__ int4 pack_group(int beg, int size, int row, int p, bo
 // after two or three groups.  It runs over pointers and rows in LDS, those of the tile and of the 64 groups on either side of it
 // (a step was a round trip to memory, one round of groups after the other: 48 us for the 705 tiles of R-MAT scale 20, all of
 // which run at once; with the sorted path of that scale 81 -> 52 us, with 256 threads 69, with 1024 48 but 6 % slower at scale
-// 22), and the columns that decide the keys are loaded together.  What is left at scale 22 (7.8 M groups 202 -> 190 us) is one cache line
-// of `col` per group, and one of `ids` where the rows are looked up there: 5.9 M groups of a path 347 us with ids, 172 with the
-// rows that the split left (eppgcn_split_and_plan).
+// 22), and the columns that decide the keys are loaded together.  What is left at scale 22 (7.8 M groups 202 -> 190 us) is one
+// cache line of `col` per group, and one of `ids` where the rows are looked up there: 5.9 M groups of a path 347 us with ids, 172
+// with the rows that the split left (eppgcn_split_and_plan).
 constexpr int kMaxRowWalk = 64;
 constexpr int kKeysBlock = 512;
 constexpr int kKeysRounds = kSortTile / kKeysBlock;

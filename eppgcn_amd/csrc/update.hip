@@ -511,7 +511,9 @@ int launch_dense_weight(float* dw, const float* x, int ld_x, const float* g, int
     const int ktiles = (K + 15) / 16;
     int ktb = 8 / dt;
     while (ktb > 1 && ktb / 2 >= ktiles) ktb /= 2;
-    if (ktb == 8 && ktiles <= 6) ktb = 6;               // no products of columns that do not exist: 1 M rows, 96 x 16, 87 -> 77 us
+    // 65 to 96 inputs (and at most 16 gradient columns) take six tiles of inputs in their pass, not eight: up to one of products with
+    // inputs that do not exist, not three.  1 M rows, 96 x 16, 87 -> 77 us.  Other widths keep theirs: 96 x 32 two of eight.
+    if (ktb == 8 && ktiles <= 6) ktb = 6;
     hipError_t e;
 #define EPPGCN_W(KTB_, DT_) launch_weight<KTB_, DT_>(partial, x, ld_x, g, ld_g, relu_in, n, K, D, rows_per_wave, blocks, stream, rows)
     if (dt == 1) e = ktb == 8 ? EPPGCN_W(8, 1) : ktb == 6 ? EPPGCN_W(6, 1) : ktb == 4 ? EPPGCN_W(4, 1) : ktb == 2 ? EPPGCN_W(2, 1) : EPPGCN_W(1, 1);

@@ -354,8 +354,8 @@ def test_pruned_backward_clears_and_scales_in_one_launch(api, n, m, offset, list
 
 # inputs around the 16-column tiles of the weight kernel (six tiles in one pass up to 96), rows around the 256 block sums that
 # the last kernel loads together (a block per 64 rows)
-@pytest.mark.parametrize("k", [65, 80, 81, 96, 97, 112, 128])
-@pytest.mark.parametrize("m", [1, 16])
+@pytest.mark.parametrize("k", [64, 65, 80, 81, 96, 97, 112, 128, 129, 192, 193])
+@pytest.mark.parametrize("m", [1, 16, 17])
 @pytest.mark.parametrize("n", [1, 255 * 64, 255 * 64 + 1, 256 * 64, 257 * 64 + 5])
 def test_weight_gradient_at_the_ends_of_its_tiles(api, n, k, m):
     """Whole numbers: every sum is exact in fp32."""
