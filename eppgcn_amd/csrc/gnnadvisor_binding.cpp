@@ -532,8 +532,9 @@ Tensor nll_backward(Tensor d_loss, Tensor logits, Tensor labels, int64_t num_row
 // the engine's thread, which has to get the interpreter for each).  They are for plain tensors in ordinary eager autograd; for
 // anything that looks into or changes how functions run - function transforms, forward-mode gradients, dispatch and function
 // modes, tracing, profiling, subclasses - the callers take the Python functions, which behave as torch defines it for those.
-// A small graph's epoch is bound by the host that issues its 17 launches: 215 us at 2 708 vertices with the Python functions, 181
-// with these (and 163 with the kept unit gradient and drop_gradients below in place of torch's own); its kernels take 70.
+// A small graph's epoch is bound by the host that issues its 17 launches: 216-240 us at 2 708 vertices with the Python functions over
+// eight processes, 177-189 with these, the kept unit gradient and drop_gradients below in place of torch's own (single processes
+// 215, these alone 181, all 163); its kernels take 66.
 bool plain_eager(std::initializer_list<const Tensor*> tensors)
 {
     using c10::DispatchKey;
