@@ -297,18 +297,24 @@ int launch_dense_rows(float* out, int ld_out, int out_cols, const float* x, int 
         int mt = 1;
         while (16 * mt < cols) mt *= 2;
         const size_t lds = lds_per_tile * mt;
-        // Workgroups: 8 per CU, or 24, more than the chip holds, so that one that falls behind does not end the launch.  24 pay while
-        // the operand that each fills in LDS is small and its waves have work: us with 24 over us with 8, columns in -> out,
-        //   from 2^20 rows, operands up to 8 KB, 32 columns and more: 96 -> 16 0.94-0.97, 16 -> 96 1.03 at 1 M rows and 0.87-0.97
-        //     above, 64 <-> 32 0.88-0.99, 16 -> 22 0.94, 22 -> 16 0.97-1.05, 128 -> 16 0.97, 16 -> 128 0.83-0.96, 33 <-> 9 0.93-0.99
-        //     (0.85 M rows: 64 -> 32 1.06, 16 -> 96 1.05, but 96 -> 16 0.96, 16 -> 128 0.89);
-        //   fewer rows: 16 -> 96 1.03-1.09, 96 -> 16 0.99-1.04, 70 -> 12 1.02-1.09, 22 -> 16 1.07, but operands up to 4 KB with more
-        //     columns out than in: 16 -> 22 0.95-1.00, 9 -> 33 0.95-1.01 (and 12 -> 20, 8 -> 24 0.95);
-        //   fewer columns: 8 <-> 7, 8 -> 8, 12 <-> 8 1.00-1.10 at any number of rows, 16 -> 8 1.02-1.07;
-        //   operands of 12 KB (47 -> 47) 1.00, of 16 KB (96 <-> 32, 64 -> 64) 1.04-1.2 up to 1.5 M rows, 0.93-1.03 at 3 M.
+        // Workgroups: 8 per CU, or 24, more than the chip holds, so that one that falls behind does not end the launch, as far as a
+        // wave keeps two tiles.  24 pay where the operand that each workgroup fills in LDS is small and a tile is some work: for
+        // operands up to 8 KB and 32 columns and more, in and out together.  us with 24 over us with 8, in -> out, 0.5 to 4.2 M rows:
+        //   a masked result (a third stream) of more than one tile 0.72-1.00 (30 -> 44 at 0.5 M rows 1.05); of one tile (22 -> 16) 1.02-1.07;
+        //   any other from 2^20 rows on: 96 -> 16 0.93-0.97, 16 -> 96 1.03 at 1.05 M rows, then 0.88-0.94, 64 -> 32 1.02, then 0.90-0.97,
+        //     16 -> 32 0.83-0.93, 48 -> 20 1.03, then 0.85-0.96, 33 <-> 9 0.92-0.99, 64 -> 16 0.96-1.02; but rows read in pairs with
+        //     more than 32 columns out (30 -> 40, 44, 64) 1.01-1.12;
+        //   fewer rows: 16 -> 96 1.05-1.13, 96 -> 16 0.97-1.08, 64 -> 32 1.05-1.10, 70 -> 12 0.95-1.08, 22 -> 16 1.06-1.11, but up to 4 KB
+        //     with more columns out than in (16 -> 22 0.96, 16 -> 32 0.92-1.01, 9 -> 33 0.96-0.99, 20 -> 32 0.99-1.03) and up to 6 KB with
+        //     rows read float by float (33 -> 9, 57 -> 7, 41 -> 21, 25 -> 20 0.91-1.01, 35 -> 25 0.95-1.03);
+        //   fewer columns (8 <-> 7, 8 -> 8, 12 <-> 8, 12 -> 12, 16 <-> 8) 0.98-1.17 at any number of rows;
+        //   operands of 10 KB 0.94-0.99, of 12 KB 1.00, of 16 KB (96 <-> 32, 64 -> 64) 1.04-1.2 up to 1.5 M rows, 0.93-1.03 at 3 M.
         // Input rows are not read past the caches: an instruction takes half a line of each row, and the other half is fetched anew
         // (4.2 M rows, 96 x 16, 374 -> 430 us; 200 x 32 853 -> 1126).
-        const bool many = lds <= 8192 && K + cols >= 32 && (n >= 1 << 20 || (lds <= 4096 && cols > K));
+        const bool many = lds <= 8192 && K + cols >= 32 &&
+                          (relu_ref ? mt >= 2
+                                    : n >= 1 << 20 ? !(vw == 2 && mt >= 4)
+                                                   : vw == 1 ? lds <= 6144 : lds <= 4096 && cols > K);
         const long long cap = 256ll * 8, wide_cap = many ? 256ll * 24 : cap;
         long long blocks = (tiles + kUpdateWaves - 1) / kUpdateWaves;
         if (blocks > cap) {

@@ -364,17 +364,20 @@ def test_weight_gradient_at_the_ends_of_its_tiles(api, n, k, m):
     assert torch.equal(api.update_backward_weight(x, g).double(), x.double().T.contiguous() @ g.double())
 
 
-# a workgroup takes 64 rows at a time; 2048 workgroups, or up to 6144 while each of their waves has two tiles of 16 rows: from 2^20
-# rows, and from 2048 * 128 on for more columns out than in, in each case with 32 columns and more and an operand of at most 8 KB (4)
+# a workgroup takes 64 rows at a time; 2048 workgroups, or up to 6144 while each of their waves has two tiles of 16 rows, by the shape,
+# the operand's size, how a row is read (four, two or one float at a time) and whether the result is masked
 @pytest.mark.parametrize("k,m,n", [(3, 2, 2048 * 64 + 17), (4, 1, (1 << 20) + 17), (130, 20, (1 << 20) + 17),       # 2048
                                    (16, 22, 2048 * 128 - 1), (16, 22, 2048 * 128 + 17), (16, 22, 6144 * 64 + 17),   # 2048, 2049, 3073
-                                   (16, 22, 6144 * 128 + 17), (9, 33, 6144 * 128 + 17),                             # 6144
-                                   (33, 9, (1 << 20) - 1), (33, 9, (1 << 20) + 17), (96, 16, (1 << 20) - 1),        # 2048, 6144, 2048
-                                   (96, 16, (1 << 20) + 17), (12, 20, (1 << 20) + 1), (12, 19, (1 << 20) + 1)])     # 6144, 6144, 2048
+                                   (16, 22, 6144 * 128 + 17), (9, 33, 6144 * 128 + 17), (33, 9, 6144 * 128 + 17),   # 6144
+                                   (96, 16, (1 << 20) - 1), (96, 16, (1 << 20) + 17),                               # 2048, 6144
+                                   (30, 40, (1 << 20) + 17), (40, 30, (1 << 20) + 17), (41, 21, 6144 * 64 + 17),    # 2048, 6144, 3073
+                                   (12, 20, (1 << 20) + 1), (12, 19, (1 << 20) + 1)])                               # 6144, 2048
 def test_products_of_more_rows_than_the_workgroups_take_at_once(api, k, m, n):
     gen = torch.Generator("cuda").manual_seed(k)
     x = torch.randint(-4, 5, (n, k), device="cuda", generator=gen).float()
     w = torch.randint(-4, 5, (k, m), device="cuda", generator=gen).float()
     assert torch.equal(api.update_forward(x, w).double(), x.double() @ w.double())
     g = torch.randint(-4, 5, (n, m), device="cuda", generator=gen).float()
-    assert torch.equal(api.update_backward_input(g, w).double(), g.double() @ w.double().T)
+    want = g.double() @ w.double().T
+    assert torch.equal(api.update_backward_input(g, w).double(), want)
+    assert torch.equal(api.update_backward_input(g, w, relu_ref=x).double(), torch.where(x > 0, want, 0.0))
