@@ -552,16 +552,40 @@ bool plain_eager(std::initializer_list<const Tensor*> tensors)
     return true;
 }
 
+// An attribute of a record, with the error that the Python function's call of the module gives for one of another type.
+template <class T>
+T value_of(const pybind11::object& value, const char* name)
+{
+    try {
+        return value.cast<T>();
+    } catch (const pybind11::cast_error&) {
+        PyErr_Format(PyExc_TypeError, "%s of the layer's record has a type that the operation does not take", name);
+        throw pybind11::error_already_set();
+    }
+}
+template <class T>
+T arg_of(const pybind11::object& record, const char* name)
+{
+    return value_of<T>(record.attr(name), name);
+}
+
 // What the Python functions keep on ctx, which a caller finds - and can set - on a result's grad_fn, and which the backward pass
 // reads when it runs: a layer's backward path is filled in after its first forward pass.  It becomes a dict when somebody looks
 // (made in each pass, an epoch of 2 708 vertices took 175 us for 170).  A node holds it by the storage of a one-element tensor,
 // since that is a kind of saved data that compiled autograd can hand on; the element is its own address, so that a copy of the
 // tensor is recognised.
 struct Attributes {
-    static constexpr int kMost = 6;
+    enum Kind { kObject, kNumber, kTruth };
+    struct Name {
+        const char* name;
+        Kind kind;
+        int at;                                          // in objects (an object) or numbers (the others)
+    };
     int64_t address;
-    const char* const* names;                            // kMost, the unused ones null
-    pybind11::object kept[kMost];                        // their values until there is a dict
+    const Name* names;
+    int count;
+    pybind11::object objects[2];                         // the values until there is a dict
+    int64_t numbers[4];
     pybind11::object dict;
     static Tensor held(Attributes* a)
     {
@@ -578,21 +602,31 @@ struct Attributes {
     {
         if (!dict) {
             pybind11::dict made;
-            for (int k = 0; k < kMost && names[k]; ++k) made[names[k]] = kept[k];
+            for (int k = 0; k < count; ++k) {
+                const Name& n = names[k];
+                if (n.kind == kObject) made[n.name] = objects[n.at];
+                else if (n.kind == kTruth) made[n.name] = pybind11::bool_(numbers[n.at] != 0);
+                else made[n.name] = pybind11::int_(numbers[n.at]);
+            }
             dict = std::move(made);
-            for (auto& value : kept) value = pybind11::object();
+            for (auto& value : objects) value = pybind11::object();
         }
         return pybind11::reinterpret_borrow<pybind11::dict>(dict);
     }
-    pybind11::object get(int k) const
+    pybind11::object in_dict(int k) const
     {
-        if (!dict) return kept[k];
-        PyObject* value = PyDict_GetItemString(dict.ptr(), names[k]);
+        PyObject* value = PyDict_GetItemString(dict.ptr(), names[k].name);
         if (!value) {
-            PyErr_Format(PyExc_AttributeError, "the function has no attribute '%s'", names[k]);
+            PyErr_Format(PyExc_AttributeError, "the function has no attribute '%s'", names[k].name);
             throw pybind11::error_already_set();
         }
         return pybind11::reinterpret_borrow<pybind11::object>(value);
+    }
+    pybind11::object object(int k) const { return dict ? in_dict(k) : objects[names[k].at]; }
+    template <class T>
+    T number(int k) const
+    {
+        return dict ? value_of<T>(in_dict(k), names[k].name) : static_cast<T>(numbers[names[k].at]);
     }
     static void let_go(Attributes* a)
     {
@@ -682,34 +716,14 @@ struct NodeType {
 template <class F, int kInputs>
 PyTypeObject NodeType<F, kInputs>::type{};
 
-// An attribute of a record, with the error that the Python function's call of the module gives for one of another type.
-template <class T>
-T value_of(const pybind11::object& value, const char* name)
-{
-    try {
-        return value.cast<T>();
-    } catch (const pybind11::cast_error&) {
-        PyErr_Format(PyExc_TypeError, "%s of the layer's record has a type that the operation does not take", name);
-        throw pybind11::error_already_set();
-    }
-}
-template <class T>
-T arg_of(const pybind11::object& record, const char* name)
-{
-    return value_of<T>(record.attr(name), name);
-}
-
 struct GraphArgs {
     Tensor row_pointers, column_index, degrees, part_ptr, part2node;
-    pybind11::object hints[3];                           // the last three as the record has them
     int part_size, dim_worker, warp_per_block;
     explicit GraphArgs(const pybind11::object& info)
         : row_pointers(arg_of<Tensor>(info, "row_pointers")), column_index(arg_of<Tensor>(info, "column_index")),
           degrees(arg_of<Tensor>(info, "degrees")), part_ptr(arg_of<Tensor>(info, "partPtr")),
-          part2node(arg_of<Tensor>(info, "part2Node")),
-          hints{info.attr("partSize"), info.attr("dimWorker"), info.attr("warpPerBlock")},
-          part_size(value_of<int>(hints[0], "partSize")), dim_worker(value_of<int>(hints[1], "dimWorker")),
-          warp_per_block(value_of<int>(hints[2], "warpPerBlock")) {}
+          part2node(arg_of<Tensor>(info, "part2Node")), part_size(arg_of<int>(info, "partSize")),
+          dim_worker(arg_of<int>(info, "dimWorker")), warp_per_block(arg_of<int>(info, "warpPerBlock")) {}
 };
 
 struct PathArgs {
@@ -724,15 +738,16 @@ struct PathArgs {
 
 struct GNNAFunction : torch::autograd::Function<GNNAFunction> {
     enum { kInfo, kBack, kRelu };
-    static constexpr const char* kNames[Attributes::kMost] = {"inputInfo", "backInfo", "reluInput",
-                                                              "partSize", "dimWorker", "warpPerBlock"};
+    static constexpr Attributes::Name kNames[] = {
+        {"inputInfo", Attributes::kObject, 0}, {"backInfo", Attributes::kObject, 1}, {"reluInput", Attributes::kTruth, 0},
+        {"partSize", Attributes::kNumber, 1}, {"dimWorker", Attributes::kNumber, 2}, {"warpPerBlock", Attributes::kNumber, 3}};
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& X, const Tensor& W,
                           const pybind11::object& info, const pybind11::object& back, bool relu_input)
     {
         ctx->save_for_backward({X, W});
         const GraphArgs g(info);
-        ctx->saved_data["attributes"] = Attributes::held(
-            new Attributes{0, kNames, {info, back, pybind11::bool_(relu_input), g.hints[0], g.hints[1], g.hints[2]}, {}});
+        ctx->saved_data["attributes"] = Attributes::held(new Attributes{
+            0, kNames, 6, {info, back}, {relu_input, g.part_size, g.dim_worker, g.warp_per_block}, {}});
         return ::forward(X, W, g.row_pointers, g.column_index, g.degrees, g.part_ptr, g.part2node, g.part_size, g.dim_worker,
                          g.warp_per_block, relu_input)[0];
     }
@@ -748,13 +763,13 @@ struct GNNAFunction : torch::autograd::Function<GNNAFunction> {
         std::vector<Tensor> d;
         pybind11::gil_scoped_acquire gil;                // for the records, and for the caches above as in every other call
         const Attributes& kept = attributes(*ctx);
-        const pybind11::object back = kept.get(kBack);
-        const bool relu_input = value_of<bool>(kept.get(kRelu), kNames[kRelu]);
+        const pybind11::object back = kept.object(kBack);
+        const bool relu_input = kept.number<bool>(kRelu);
         const pybind11::object unpruned = pybind11::getattr(back, "unpruned", pybind11::none());
         const int all_edges = PyObject_IsTrue(unpruned.ptr());
         if (all_edges < 0) throw pybind11::error_already_set();
         if (all_edges) {
-            const GraphArgs g(kept.get(kInfo));
+            const GraphArgs g(kept.object(kInfo));
             d = ::backward(d_output, X, W, g.row_pointers, g.column_index, g.degrees, g.part_ptr, g.part2node, g.part_size,
                            g.dim_worker, g.warp_per_block, need_dx, relu_input);
         } else {
@@ -775,7 +790,7 @@ std::optional<Tensor> gcn_layer(const Tensor& X, const Tensor& W, pybind11::obje
 }
 
 struct TrainingLoss : torch::autograd::Function<TrainingLoss> {
-    static constexpr const char* kNames[Attributes::kMost] = {"num_rows"};
+    static constexpr Attributes::Name kNames[] = {{"num_rows", Attributes::kNumber, 0}};
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& logits, const Tensor& rows, const Tensor& labels)
     {
         ctx->save_for_backward({logits, labels});
@@ -785,7 +800,7 @@ struct TrainingLoss : torch::autograd::Function<TrainingLoss> {
     static Attributes& attributes(torch::autograd::AutogradContext& ctx)
     {
         auto& held = ctx.saved_data["attributes"];
-        if (!held.isTensor()) held = Attributes::held(new Attributes{0, kNames, {pybind11::int_(ctx.saved_data.at("num_rows").toInt())}, {}});
+        if (!held.isTensor()) held = Attributes::held(new Attributes{0, kNames, 1, {}, {ctx.saved_data.at("num_rows").toInt()}, {}});
         return Attributes::of(held.toTensor());
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads)
@@ -797,8 +812,7 @@ struct TrainingLoss : torch::autograd::Function<TrainingLoss> {
         {
             torch::NoGradGuard no_grad;
             pybind11::gil_scoped_acquire gil;            // one call into the library at a time, as from Python
-            const int64_t num_rows = looked_at ? value_of<int64_t>(attributes(*ctx).get(0), kNames[0])
-                                               : ctx->saved_data["num_rows"].toInt();
+            const int64_t num_rows = looked_at ? attributes(*ctx).number<int64_t>(0) : ctx->saved_data["num_rows"].toInt();
             d = nll_backward(grads[0].contiguous(), saved[0], saved[1], num_rows);
         }
         if (twice) {                                     // as Python's once_differentiable: an error if it is differentiated

@@ -13,7 +13,7 @@ import torch.nn.functional as F
 import torch.optim.optimizer as torch_optimizer
 
 from . import gnnadvisor, graphs
-from .gcn_conv import GCNConv, _is_as_defined, _is_torchs
+from .gcn_conv import GCNConv, _is_torchs, _parts
 from .param import backInputProperty, inputProperty, maskInputProperty
 
 
@@ -59,7 +59,7 @@ class _TrainingLoss(torch.autograd.Function):
         return gnnadvisor().nll_backward(d_loss.contiguous(), logits, labels, ctx.num_rows), None, None
 
 
-_LOSS, _LOSS_PARTS = _TrainingLoss, dict(vars(_TrainingLoss))
+_LOSS, _LOSS_PARTS = _TrainingLoss, _parts(_TrainingLoss) if _is_torchs(_TrainingLoss.apply) else None
 
 
 class Net(torch.nn.Module):
@@ -203,7 +203,7 @@ class Trainer:
         if (selected and out.dtype == torch.float32 and out.dim() == 2 and out.is_contiguous()
                 and out.shape[0] == self.row_labels.numel()):
             ops = gnnadvisor()
-            if (_TrainingLoss is _LOSS and _is_as_defined(_TrainingLoss, _LOSS_PARTS)
+            if (_TrainingLoss is _LOSS and _parts(_TrainingLoss) == _LOSS_PARTS
                     and getattr(ops, "native_functions", ())[3:] == (ops.nll_forward, ops.nll_backward)
                     and type(out) is torch.Tensor):
                 loss = ops.training_loss(out, self.train_idx, self.row_labels)      # _TrainingLoss in native code
