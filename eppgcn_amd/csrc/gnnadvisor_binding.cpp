@@ -696,9 +696,10 @@ struct NodeType {
         return needs.release().ptr();
         END_HANDLE_TH_ERRORS
     }
-    static pybind11::object add(const char* name)
+    static void add(const char* name)
     {
         using namespace torch::autograd;                 // for the names in the macro
+        if (type.tp_flags & Py_TPFLAGS_READY) return;    // the module is imported under a second name
         static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
                                            {"saved_tensors", saved_tensors, nullptr, nullptr, nullptr},
                                            {"needs_input_grad", needs_input_grad, nullptr, nullptr, nullptr},
@@ -708,9 +709,9 @@ struct NodeType {
         type.tp_setattro = set;
         _initFunctionPyTypeObject(type, name, properties, nullptr);
         registerCppFunction(typeid(Node), &type);
+        Py_INCREF(&type);                                // it is never freed
         const auto added = pybind11::reinterpret_borrow<pybind11::object>(reinterpret_cast<PyObject*>(&type));
         pybind11::module_::import("torch.autograd.graph").attr("Node").attr("register")(added);      // isinstance, as for Python's
-        return added;
     }
 };
 template <class F, int kInputs>
